@@ -46,9 +46,14 @@ struct HostTopo {
   std::vector<int4> tri;
   std::vector<int> lra_fixed;
   std::vector<float> lra_l0;
-  std::vector<int> tstart, eprefix;  // Jacobi tiles (empty: slot-parallel solve)
-  std::vector<TileEntry> entries;
-  std::vector<int> ecid;  // per entry: constraint index, bit 31 set for a bend
+  std::vector<int> patch;    // the vertices in runs of neighbours (patch_order)
+  std::vector<int> pstart;   // where each cloth's run begins, and n
+  // Jacobi tiles in solver order (hdr empty: slot-parallel solve); see TileBufs
+  std::vector<int> order, rank, sprefix, halo, scid, bcid;
+  std::vector<int4> hdr;
+  std::vector<uint4> sent, bent;
+  std::vector<float2> bpar;
+  int max_local = 0, lds_slots = 0;
   std::vector<float> k_dist, k_bend;  // stiffness per constraint (before the kp mapping)
 };
 
@@ -66,7 +71,12 @@ struct AdjState {
   int64_t arena_cap = 0;
   int* ctl = nullptr;  // 2 + every
   AdjBufs ab;
-  int* ecid = nullptr;
+};
+
+// How a body's vertices are cut into tiles: at most tile_v vertices, in patches of sub
+// vertices (0: one patch), worked on by `threads` threads
+struct TileShape {
+  int tile_v, sub, threads;
 };
 
 }  // namespace
@@ -79,7 +89,7 @@ struct cm_body {
   hipStream_t stream = nullptr;
   std::vector<void*> allocs;
   // state
-  float4 *x = nullptr, *p = nullptr, *p2 = nullptr, *v = nullptr;
+  float4 *x = nullptr, *p = nullptr, *q0 = nullptr, *q1 = nullptr, *v = nullptr;
   uint8_t* pinned = nullptr;
   float* mass = nullptr;
   // topology
@@ -89,10 +99,7 @@ struct cm_body {
   float2* b_kpphi0 = nullptr;
   int* vprefix = nullptr;
   uint32_t* vslot = nullptr;
-  int ntiles = 0;
-  int* tstart = nullptr;
-  int* eprefix = nullptr;
-  TileEntry* entries = nullptr;
+  TileBufs tl;
   int* lra_fixed = nullptr;
   float* lra_l0 = nullptr;
   uint8_t* lra_flag = nullptr;
@@ -123,7 +130,7 @@ struct cm_body {
   bool use_graph = true;
   // launch shapes (cm_autotune): Jacobi tile vertices; traversal tiles per XCD chunk
   // and the traversal's visit budget live in lb
-  int tile_v = kTileV;
+  TileShape shape{128, 0, 256};
   // host copies
   std::vector<float> inv_mass_h;
   std::vector<uint8_t> pinned_h;
@@ -160,6 +167,29 @@ int upload(cm_body* b, T** out, const std::vector<T>& h) {
   int rc = dalloc(b, out, h.size());
   if (rc) return rc;
   if (!h.empty()) CM_HIP(hipMemcpy(*out, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice));
+  return CM_OK;
+}
+
+// the tiles of h on the device (none: the slot-parallel form)
+int upload_tiles(cm_body* b, const HostTopo& h) {
+  if (h.hdr.empty()) return CM_OK;
+  TileBufs t;
+  int rc;
+  if ((rc = tile_lds_allow(tile_lds_bytes(h.max_local, h.lds_slots, true))) ||
+      (rc = upload(b, &t.order, h.order)) || (rc = upload(b, &t.rank, h.rank)) ||
+      (rc = upload(b, &t.prefix, h.sprefix)) || (rc = upload(b, &t.hdr, h.hdr)) ||
+      (rc = upload(b, &t.halo, h.halo)) || (rc = upload(b, &t.sent, h.sent)) ||
+      (rc = upload(b, &t.bent, h.bent)) || (rc = upload(b, &t.bpar, h.bpar)) ||
+      (rc = upload(b, &t.scid, h.scid)) || (rc = upload(b, &t.bcid, h.bcid)))
+    return rc;
+  t.max_local = h.max_local;
+  t.lds_slots = h.lds_slots;
+  t.nsent = (int)h.sent.size();
+  t.nbent = (int)h.bent.size();
+  t.n = (int)h.hdr.size() / 2;
+  t.threads = b->shape.threads;
+  b->tl = t;
+  b->nb.rank = t.rank;
   return CM_OK;
 }
 
@@ -211,73 +241,166 @@ inline uint64_t edge_key(int a, int b) {
   return ((uint64_t)lo << 32) | hi;
 }
 
-// Cut the vertices into tiles of at most kTileV consecutive vertices and kTileSlots
-// slots, and list for each tile every constraint that touches it once, with the
-// tile-local slot of each of its roles. Leaves the tiles empty when one vertex has
-// more slots than a tile holds.
-void build_tiles(int n, HostTopo& h, int tile_v = kTileV) {
-  const std::vector<int>& pre = h.prefix;
+// Orders the vertices ids[0, n) into runs of neighbours by halving them along the
+// longest axis of their box, at multiples of 128 (then 64, 32, 16), so that every
+// aligned run of up to 128 is a compact patch of the rest shape.
+void patch_order(const float* xyz, int* ids, int n) {
+  if (n <= 16) {
+    std::sort(ids, ids + n);
+    return;
+  }
+  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  for (int i = 0; i < n; ++i)
+    for (int k = 0; k < 3; ++k) {
+      lo[k] = std::fmin(lo[k], xyz[3 * (size_t)ids[i] + k]);
+      hi[k] = std::fmax(hi[k], xyz[3 * (size_t)ids[i] + k]);
+    }
+  int ax = 0;
+  for (int k = 1; k < 3; ++k)
+    if (hi[k] - lo[k] > hi[ax] - lo[ax]) ax = k;
+  const int unit = n > 128 ? 128 : (n > 64 ? 64 : (n > 32 ? 32 : 16));
+  const int left = ((n + unit - 1) / unit + 1) / 2 * unit;
+  // sort keys: an ordered integer of the coordinate, so that any value (also NaN) has
+  // its place, then the vertex
+  auto key = [&](int v) {
+    uint32_t u;
+    std::memcpy(&u, &xyz[3 * (size_t)v + ax], 4);
+    u = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+    return ((uint64_t)u << 32) | (uint32_t)v;
+  };
+  std::nth_element(ids, ids + left, ids + n, [&](int p, int q) { return key(p) < key(q); });
+  patch_order(xyz, ids, left);
+  patch_order(xyz, ids + left, n - left);
+}
+
+// Cut the vertices into tiles (TileBufs) of at most tile_v vertices and kTileSlots
+// slots, none across two cloths. sub > 0: a tile is made of patches of `sub` vertices
+// from tile_v / sub places of the cloth, else it is one patch. Leaves the tiles empty
+// when a vertex has more slots than a tile holds.
+void build_tiles(int n, HostTopo& h, int tile_v, int sub) {
+  h.order.clear();
+  h.hdr.clear();
+  h.halo.clear();
+  h.sent.clear();
+  h.bent.clear();
+  h.bpar.clear();
+  h.scid.clear();
+  h.bcid.clear();
+  h.max_local = h.lds_slots = 0;
+  for (int v = 0; v < n; ++v)
+    if (h.prefix[v + 1] - h.prefix[v] > kTileSlots) return;
   std::vector<int> ts{0};
-  for (int v = 0; v < n;) {
-    const int start = v;
-    while (v < n && v - start < tile_v && pre[v + 1] - pre[start] <= kTileSlots) ++v;
-    if (v == start) return;  // a vertex with more than kTileSlots slots
-    ts.push_back(v);
+  int slots = 0;
+  auto close = [&]() {
+    if ((int)h.order.size() > ts.back()) ts.push_back((int)h.order.size());
+    slots = 0;
+  };
+  h.order.reserve(n);
+  for (size_t c = 0; c + 1 < h.pstart.size(); ++c) {
+    const int b = h.pstart[c], len = h.pstart[c + 1] - b;
+    const int unit = sub > 0 ? std::min(sub, tile_v) : tile_v;
+    const int nsub = (len + unit - 1) / unit, per = tile_v / unit, nt = (nsub + per - 1) / per;
+    for (int t = 0; t < nt; ++t) {
+      for (int u = t; u < nsub; u += nt)
+        for (int k = u * unit; k < std::min(len, (u + 1) * unit); ++k) {
+          const int v = h.patch[b + k], c1 = h.prefix[v + 1] - h.prefix[v];
+          if (slots + c1 > kTileSlots) close();
+          h.order.push_back(v);
+          slots += c1;
+        }
+      close();
+    }
   }
   const int nt = (int)ts.size() - 1;
-  std::vector<int> seen_s(h.sid.size(), -1), seen_b(h.bid.size(), -1);  // entry of this tile
-  std::vector<int> ep{0};
-  std::vector<TileEntry> ent;
-  std::vector<int> cid;
-  for (int tile = 0; tile < nt; ++tile) {
-    const int s0 = pre[ts[tile]], s1 = pre[ts[tile + 1]];
-    const int base = (int)ent.size();
-    for (int k = s0; k < s1; ++k) {
-      const uint32_t w = h.vslot[k];
-      const int idx = (int)(w & 0x1fffffffu), role = (int)((w >> 29) & 3u);
-      const bool bend = (w & 0x80000000u) != 0;
-      int& seen = bend ? seen_b[idx] : seen_s[idx];
-      if (seen < base) {  // first slot of this constraint in this tile
-        seen = (int)ent.size();
-        TileEntry e;
-        if (bend) {
-          e.ids = h.bid[idx];
-          e.a = h.b_kpphi0[idx].x;
-          e.b = h.b_kpphi0[idx].y;
-        } else {
-          e.ids = make_int4(h.sid[idx].x, h.sid[idx].y, -1, -1);
-          e.a = h.s_l0kp[idx].x;
-          e.b = h.s_l0kp[idx].y;
-        }
-        e.s01 = e.s23 = 0xffffffffu;
-        ent.push_back(e);
-        cid.push_back(bend ? (int)(0x80000000u | (uint32_t)idx) : idx);
-      }
-      TileEntry& e = ent[seen];
-      const uint32_t off = (uint32_t)(k - s0);
-      uint32_t& word = role < 2 ? e.s01 : e.s23;
-      const int sh = (role & 1) * 16;
-      word = (word & ~(0xffffu << sh)) | (off << sh);
-    }
-    // distance constraints first, then bends: a wave then mostly runs one path
-    std::vector<int> order((size_t)ent.size() - base);
-    for (size_t k = 0; k < order.size(); ++k) order[k] = base + (int)k;
-    std::stable_partition(order.begin(), order.end(),
-                          [&](int k) { return ent[k].ids.z < 0; });
-    std::vector<TileEntry> te(order.size());
-    std::vector<int> tc(order.size());
-    for (size_t k = 0; k < order.size(); ++k) {
-      te[k] = ent[order[k]];
-      tc[k] = cid[order[k]];
-    }
-    std::copy(te.begin(), te.end(), ent.begin() + base);
-    std::copy(tc.begin(), tc.end(), cid.begin() + base);
-    ep.push_back((int)ent.size());
+  h.rank.resize(n);
+  h.sprefix.assign(n + 1, 0);
+  for (int k = 0; k < n; ++k) {
+    const int v = h.order[k];
+    h.rank[v] = k;
+    h.sprefix[k + 1] = h.sprefix[k] + h.prefix[v + 1] - h.prefix[v];
   }
-  h.tstart = std::move(ts);
-  h.eprefix = std::move(ep);
-  h.entries = std::move(ent);
-  h.ecid = std::move(cid);
+  // entry of this tile (distance, bend) and tile-local id (halo) last given to each
+  std::vector<int> seen_s(h.sid.size(), -1), seen_b(h.bid.size(), -1), lt(n, -1), lid(n, 0);
+  h.sent.reserve(h.sid.size() * 3 / 2);
+  h.bent.reserve(h.bid.size() * 3 / 2);
+  for (int t = 0; t < nt; ++t) {
+    const int v0 = ts[t], v1 = ts[t + 1], slot0 = h.sprefix[v0];
+    const int s_base = (int)h.sent.size(), b_base = (int)h.bent.size(), h_base = (int)h.halo.size();
+    auto local = [&](int v) -> uint32_t {
+      const int k = h.rank[v];
+      if (k >= v0 && k < v1) return (uint32_t)(k - v0);
+      if (lt[v] != t) {
+        lt[v] = t;
+        lid[v] = v1 - v0 + (int)h.halo.size() - h_base;
+        h.halo.push_back(k);
+      }
+      return (uint32_t)lid[v];
+    };
+    for (int k = v0; k < v1; ++k) {
+      const int v = h.order[k];
+      for (int q = h.prefix[v]; q < h.prefix[v + 1]; ++q) {
+        const uint32_t w = h.vslot[q];
+        const int idx = (int)(w & 0x1fffffffu), role = (int)((w >> 29) & 3u);
+        const uint32_t slot = (uint32_t)(h.sprefix[k] - slot0 + q - h.prefix[v]);
+        auto put = [&](uint32_t& word, int r) {
+          word = (word & ~(0xffffu << (16 * r))) | (slot << (16 * r));
+        };
+        if (w & 0x80000000u) {
+          int& seen = seen_b[idx];
+          if (seen < b_base) {  // first slot of this constraint in this tile
+            seen = (int)h.bent.size();
+            const int4 e = h.bid[idx];
+            const uint32_t i0 = local(e.x), i1 = local(e.y), i2 = local(e.z), i3 = local(e.w);
+            h.bent.push_back(make_uint4(i0 | (i1 << 16), i2 | (i3 << 16), 0xffffffffu, 0xffffffffu));
+            h.bpar.push_back(h.b_kpphi0[idx]);
+            h.bcid.push_back(idx);
+          }
+          put(role < 2 ? h.bent[seen].z : h.bent[seen].w, role & 1);
+        } else {
+          int& seen = seen_s[idx];
+          if (seen < s_base) {
+            seen = (int)h.sent.size();
+            const uint32_t i0 = local(h.sid[idx].x), i1 = local(h.sid[idx].y);
+            uint4 e = make_uint4(i0 | (i1 << 16), 0xffffffffu, 0, 0);
+            std::memcpy(&e.z, &h.s_l0kp[idx].x, 4);
+            std::memcpy(&e.w, &h.s_l0kp[idx].y, 4);
+            h.sent.push_back(e);
+            h.scid.push_back(idx);
+          }
+          put(h.sent[seen].y, role & 1);
+        }
+      }
+    }
+    const int nh = (int)h.halo.size() - h_base;
+    h.max_local = std::max(h.max_local, v1 - v0 + nh);
+    h.lds_slots = std::max(h.lds_slots, h.sprefix[v1] - slot0);
+    h.hdr.push_back(make_int4(v0, v1 - v0, h_base, nh));
+    h.hdr.push_back(make_int4(s_base, (int)h.sent.size() - s_base, b_base,
+                              (int)h.bent.size() - b_base));
+  }
+  // dynamic records pass through the same LDS, 1,024 of them or more at a time
+  h.lds_slots = std::max((h.lds_slots + 3) & ~3, 1024);
+  if (h.max_local > 0xffff ||
+      tile_lds_bytes(h.max_local, h.lds_slots, true) > (size_t)(150 << 10)) {
+    if (tile_v > 1) return build_tiles(n, h, tile_v / 2, 0);
+    h.hdr.clear();
+  }
+}
+
+// The tile shape of a body, from k_solve's launches measured on the draped 256^2 and
+// 131x97 cloths (contacts) and on cloths without contacts:
+// - from 2,048 tiles of 128 up, or without self-collision, plain 128-vertex patches
+//   with 256 threads: the fewest repeated evaluations, and the tiles per CU even out
+//   their contacts (1024^2: 122 us, 180 as below; 96 cloths: 91 against 101 us);
+// - smaller colliding cloths: 512 threads and tiles of 32-vertex patches from all over
+//   the cloth (draped 256^2: 23 us; 41 us as plain patches of 256 threads, whose
+//   heaviest tile holds 5,800 of the 344,000 records; without contacts 13.6 against
+//   11.8 us);
+// - fewer vertices per tile where the tiles would not fill the CUs (131x97: 14.5 us
+//   with 64, 15.4 with 128; 64^2: 6.0 us with 32, 7.0 with 64, 8.4 with 128).
+TileShape default_shape(int n, bool collides) {
+  if (!collides || n >= 262144) return {128, 0, 256};
+  return {n < 12288 ? 32 : (n < 32768 ? 64 : 128), kSubPatch, 512};
 }
 
 int build_topology(const cm_params& P, const float* xyz, int n, const uint32_t* tri, int t,
@@ -389,7 +512,6 @@ int build_topology(const cm_params& P, const float* xyz, int n, const uint32_t* 
     for (int j = 0; j < F; ++j)
       if (!pinned[i])
         h.lra_l0[(size_t)i * F + j] = host_dist(xyz, i, h.lra_fixed[j]) * (1.f + P.strain_limit);
-  build_tiles(n, h);
   return CM_OK;
 }
 
@@ -401,7 +523,8 @@ PbdBufs pbd_bufs(cm_body* b) {
   pb.F = b->F;
   pb.x = b->x;
   pb.p = b->p;
-  pb.p2 = b->p2;
+  pb.q0 = b->q0;
+  pb.q1 = b->q1;
   pb.v = b->v;
   pb.pinned = b->pinned;
   pb.sid = b->sid;
@@ -410,10 +533,7 @@ PbdBufs pbd_bufs(cm_body* b) {
   pb.b_kpphi0 = b->b_kpphi0;
   pb.vprefix = b->vprefix;
   pb.vslot = b->vslot;
-  pb.ntiles = b->ntiles;
-  pb.tstart = b->tstart;
-  pb.eprefix = b->eprefix;
-  pb.entries = b->entries;
+  pb.tl = b->tl;
   pb.lra_fixed = b->lra_fixed;
   pb.lra_l0 = b->lra_l0;
   pb.lra_flag = b->lra_flag;
@@ -684,12 +804,17 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
         h.k_bend[i] = batch->k_bend[cloth_of[h.bid[i].x]];
         h.b_kpphi0[i].x = kp_of(h.k_bend[i], I);
       }
-    build_tiles(n, h);  // tile entries carry the stiffness
   }
+  h.patch.resize(n);
+  for (int i = 0; i < n; ++i) h.patch[i] = i;
+  h.pstart = batch ? batch->vstart : std::vector<int>{0, n};
+  for (size_t c = 0; c + 1 < h.pstart.size(); ++c)
+    patch_order(xyz, h.patch.data() + h.pstart[c], h.pstart[c + 1] - h.pstart[c]);
+  b->shape = default_shape(n, (b->prm.flags & CM_F_SELF_COLLISION) != 0);
+  build_tiles(n, h, b->shape.tile_v, b->shape.sub);
   b->S = (int)h.sid.size();
   b->B = (int)h.bid.size();
   b->F = (int)h.lra_fixed.size();
-  b->ntiles = h.tstart.empty() ? 0 : (int)h.tstart.size() - 1;
   b->nslots = h.prefix[n];
   for (auto& e : h.sid) {
     b->h_sid.push_back(e.x);
@@ -710,16 +835,14 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
     mass[i] = b->pinned_h[i] ? params->pinned_mass
                              : (inv_mass[i] > 0 ? 1.f / inv_mass[i] : params->pinned_mass);
   }
-  if ((rc = upload(b, &b->x, x4)) || (rc = upload(b, &b->p, x4)) || (rc = dalloc(b, &b->p2, n)) ||
+  if ((rc = upload(b, &b->x, x4)) || (rc = upload(b, &b->p, x4)) || (rc = dalloc(b, &b->q0, n)) ||
+      (rc = dalloc(b, &b->q1, n)) ||
       (rc = upload(b, &b->v, v4)) || (rc = upload(b, &b->pinned, b->pinned_h)) ||
       (rc = upload(b, &b->mass, mass)) || (rc = upload(b, &b->sid, h.sid)) ||
       (rc = upload(b, &b->s_l0kp, h.s_l0kp)) || (rc = upload(b, &b->bid, h.bid)) ||
       (rc = upload(b, &b->b_kpphi0, h.b_kpphi0)) || (rc = upload(b, &b->vprefix, h.prefix)) ||
       (rc = upload(b, &b->vslot, h.vslot)) || (rc = upload(b, &b->lra_fixed, h.lra_fixed)) ||
-      (!h.tstart.empty() && ((rc = upload(b, &b->tstart, h.tstart)) ||
-                             (rc = upload(b, &b->eprefix, h.eprefix)) ||
-                             (rc = upload(b, &b->entries, h.entries)) ||
-                             (rc = upload(b, &b->adj.ecid, h.ecid)))) ||
+      (rc = upload_tiles(b, h)) ||
       (rc = upload(b, &b->lra_l0, h.lra_l0)) ||
       (rc = dalloc(b, &b->lra_flag, (size_t)n * std::max(b->F, 1))) ||
       (rc = dalloc(b, &b->ground, n)) ||
@@ -1334,10 +1457,7 @@ int adj_alloc(cm_body* b, T** out, size_t count) {
 void adj_release(cm_body* b) {
   AdjState& a = b->adj;
   for (void* ptr : a.allocs) hipFree(ptr);
-  int* ecid = a.ecid;
   a = AdjState();
-  a.ecid = ecid;
-  a.ab.ecid = ecid;
 }
 
 int adj_check(cm_body* b, const char* who) {
@@ -1348,7 +1468,7 @@ int adj_check(cm_body* b, const char* who) {
                                  "attachments, sphere, damping, friction or contact-time rollback");
     return CM_ERR_ARG;
   }
-  if (b->ntiles <= 0) {
+  if (b->tl.n <= 0) {
     set_error(std::string(who) + ": a vertex has more constraint slots than a Jacobi tile holds");
     return CM_ERR_ARG;
   }
@@ -1370,8 +1490,8 @@ int adj_setup(cm_body* b, int nsub, int every) {
       (rc = adj_alloc(b, &a.dpre, (size_t)every * (n + 1))) ||
       (rc = adj_alloc(b, &a.ctl, 2 + (size_t)every)) || (rc = adj_alloc(b, &a.ab.lx, n)) ||
       (rc = adj_alloc(b, &a.ab.lv, n)) || (rc = adj_alloc(b, &a.ab.lp, n)) ||
-      (rc = adj_alloc(b, &a.ab.la, n)) || (rc = adj_alloc(b, &a.ab.av, n)) ||
-      (rc = adj_alloc(b, &a.ab.dcnt, (size_t)I * n)) ||
+      (rc = adj_alloc(b, &a.ab.la, n)) ||
+      (rc = adj_alloc(b, &a.ab.cnt, (size_t)I * n)) ||
       (rc = adj_alloc(b, &a.ab.gks, (size_t)b->S)) || (rc = adj_alloc(b, &a.ab.gkb, (size_t)b->B)))
     return rc;
   const int64_t per = b->prm.reserved[3] > 0 ? b->prm.reserved[3] : std::max<int64_t>(b->n, 65536);
@@ -1454,16 +1574,13 @@ int cm_set_stiffness(cm_body* b, const float* k_dist, const float* k_bend) {
     h.k_bend[i] = k_bend[i];
     h.b_kpphi0[i].x = kp_of(k_bend[i], I);
   }
-  if (b->ntiles > 0) build_tiles(b->n, h, b->tile_v);
   CM_HIP(hipStreamSynchronize(b->stream));
   if (b->S)
     CM_HIP(hipMemcpy(b->s_l0kp, h.s_l0kp.data(), sizeof(float2) * b->S, hipMemcpyHostToDevice));
   if (b->B)
     CM_HIP(hipMemcpy(b->b_kpphi0, h.b_kpphi0.data(), sizeof(float2) * b->B,
                      hipMemcpyHostToDevice));
-  if (b->ntiles > 0)
-    CM_HIP(hipMemcpy(b->entries, h.entries.data(), sizeof(TileEntry) * h.entries.size(),
-                     hipMemcpyHostToDevice));
+  if (b->tl.n > 0 && (rc = launch_tile_stiffness(pbd_bufs(b), b->stream))) return rc;
   b->adj.ready = false;  // a recorded forward used the old stiffness
   return CM_OK;
 }
@@ -1602,32 +1719,25 @@ void drop_graph(cm_body* b) {
 // current ones (the substep graph is dropped: it holds the old buffers)
 int set_tiles(cm_body* b, int tile_v) {
   HostTopo& h = b->topo;
-  build_tiles(b->n, h, tile_v);
-  if (h.tstart.empty()) {
+  build_tiles(b->n, h, tile_v, b->shape.sub);
+  if (h.hdr.empty()) {
     set_error("cm_autotune: the mesh has no tiled Jacobi layout");
     return CM_ERR_STATE;
   }
   CM_HIP(hipStreamSynchronize(b->stream));
   drop_graph(b);
-  free_alloc(b, b->tstart);
-  free_alloc(b, b->eprefix);
-  free_alloc(b, b->entries);
-  free_alloc(b, b->adj.ecid);
+  for (void* p : {(void*)b->tl.order, (void*)b->tl.rank, (void*)b->tl.prefix, (void*)b->tl.hdr,
+                  (void*)b->tl.halo, (void*)b->tl.sent, (void*)b->tl.bent, (void*)b->tl.bpar,
+                  (void*)b->tl.scid, (void*)b->tl.bcid})
+    free_alloc(b, p);
   // until the new tiles are in place the body uses the slot-parallel Jacobi form,
   // which needs no tiles (and stays so if an upload fails)
-  b->ntiles = 0;
-  b->tstart = b->eprefix = nullptr;
-  b->entries = nullptr;
-  b->adj.ecid = nullptr;
-  b->adj.ab.ecid = nullptr;
+  b->tl = TileBufs();
+  b->nb.rank = nullptr;
   b->adj.ready = false;
-  int rc;
-  if ((rc = upload(b, &b->tstart, h.tstart)) || (rc = upload(b, &b->eprefix, h.eprefix)) ||
-      (rc = upload(b, &b->entries, h.entries)) || (rc = upload(b, &b->adj.ecid, h.ecid)))
-    return rc;
-  b->adj.ab.ecid = b->adj.ecid;
-  b->ntiles = (int)h.tstart.size() - 1;
-  b->tile_v = tile_v;
+  const int rc = upload_tiles(b, h);
+  if (rc) return rc;
+  b->shape.tile_v = tile_v;
   return CM_OK;
 }
 
@@ -1709,9 +1819,9 @@ int cm_autotune(cm_body* b, int32_t substeps, int32_t* chosen) {
   float ms = 0.f;
   if ((rc = trial(&ms))) return fail(rc);  // warm-up
   // one parameter at a time, each over its candidates, keeping the fastest
-  if (b->ntiles > 0) {
-    const int cand[3] = {64, 128, 256};
-    int best = b->tile_v;
+  if (b->tl.n > 0) {
+    const int cand[4] = {b->shape.tile_v, 64, 128, 256};
+    int best = b->shape.tile_v;
     float best_ms = 1e30f;
     for (int c : cand) {
       if ((rc = set_tiles(b, c)) || (rc = trial(&ms))) return fail(rc);
@@ -1746,7 +1856,7 @@ int cm_autotune(cm_body* b, int32_t substeps, int32_t* chosen) {
   CM_HIP(hipStreamSynchronize(b->stream));
   cleanup();
   if (chosen) {
-    chosen[0] = b->tile_v;
+    chosen[0] = b->shape.tile_v;
     chosen[1] = b->lb.trav_chunk;
     chosen[2] = b->lb.trav_budget;
   }

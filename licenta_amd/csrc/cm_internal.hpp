@@ -177,7 +177,9 @@ struct NarrowBufs {
   int4 *vf_v = nullptr, *ee_v = nullptr;      // compacted contacts
   float4 *vf_w = nullptr, *vf_tn = nullptr, *ee_w = nullptr, *ee_tn = nullptr;
   int *d_nvf = nullptr, *d_nee = nullptr;
-  // per-vertex dynamic record CSR
+  // per-vertex dynamic record CSR, in solver order (rank: solver position of a vertex,
+  // null: its id); the payloads' vertex ids are solver positions too
+  const int* rank = nullptr;
   int *dcount = nullptr, *dprefix = nullptr, *dcursor = nullptr;  // n + 1, n + 1, n
   uint32_t* drec = nullptr;  // 4 * (vf_out_cap + ee_out_cap)
   uint32_t* dtmp = nullptr;  // same size: staging for very long record lists
@@ -205,20 +207,39 @@ int launch_narrow(const NarrowBufs& nb, const int4* tri, const float4* x, const 
 int launch_dynamic_csr(const NarrowBufs& nb, hipStream_t s);
 
 // ---- PBD (k_pbd.hip) -------------------------------------------------------
-// Vertex tiles of the Jacobi kernel: at most kTileV consecutive vertices holding at
-// most kTileSlots constraint slots. Each tile lists the constraints touching it once.
-constexpr int kTileV = 128;
+// Jacobi tiles: the solver numbers the vertices in an order of its own (order[k] =
+// vertex at solver position k, rank = its inverse) in which a tile is a run of
+// consecutive positions: a patch of at most tile_v vertices that holds at most
+// kTileSlots constraint slots. A tile lists the constraints touching it once, distance
+// and bend apart, in tile-local vertex numbers: its own vertices first, then its halo
+// (the other vertices of its constraints), whose solver positions are listed.
 constexpr int kTileSlots = 3072;
-struct alignas(16) TileEntry {
-  int4 ids;            // vertex ids; ids.z < 0 marks a distance constraint (ids.x, ids.y)
-  float a, b;          // distance: l0, kp; bend: kp, phi0
-  uint32_t s01, s23;   // tile-local slot of roles 0..3, 16 bits each, 0xffff = not in tile
+// patches of neighbouring vertices a tile is made of when tiles are few: contacts
+// gather in a few regions, and a tile of several small patches from all over the
+// cloth holds about as many as any other
+constexpr int kSubPatch = 32;
+struct TileBufs {
+  int n = 0;  // 0: no tiles (a vertex has more slots than a tile holds)
+  int threads = 256;                 // of a workgroup (256 or 512)
+  int max_local = 0, lds_slots = 0;  // LDS per workgroup: positions and slots
+  int* order = nullptr;   // n vertices (null: solver numbering = vertex ids)
+  int* rank = nullptr;
+  int* prefix = nullptr;  // n + 1: constraint slots before each solver position
+  int4* hdr = nullptr;    // 2 per tile: {v0, nv, halo0, nhalo}, {s0, ns, b0, nb}
+  int* halo = nullptr;    // solver positions
+  // distance entries {id0 | id1 << 16, slot0 | slot1 << 16, l0, kp}; bend entries
+  // {id0 | id1 << 16, id2 | id3 << 16, slot0 | slot1 << 16, slot2 | slot3 << 16} with
+  // {kp, phi0}; tile-local ids and slots, slot 0xffff = not a vertex of the tile
+  uint4 *sent = nullptr, *bent = nullptr;
+  float2* bpar = nullptr;
+  int *scid = nullptr, *bcid = nullptr;  // constraint of each entry
+  int nsent = 0, nbent = 0;
 };
-static_assert(sizeof(TileEntry) == 32, "TileEntry is two 16-byte loads");
 
 struct PbdBufs {
   int n = 0, S = 0, B = 0, F = 0;
-  float4 *x = nullptr, *p = nullptr, *p2 = nullptr, *v = nullptr;  // .w of x/p = inverse mass
+  float4 *x = nullptr, *p = nullptr, *v = nullptr;  // .w of x/p = inverse mass
+  float4 *q0 = nullptr, *q1 = nullptr;  // the solver's iterates, in solver order
   const uint8_t* pinned = nullptr;
   const int2* sid = nullptr;
   const float2* s_l0kp = nullptr;
@@ -226,10 +247,7 @@ struct PbdBufs {
   const float2* b_kpphi0 = nullptr;
   const int* vprefix = nullptr;
   const uint32_t* vslot = nullptr;
-  int ntiles = 0;  // 0: slot-parallel solve (a vertex has more than kTileSlots slots)
-  const int* tstart = nullptr;
-  const int* eprefix = nullptr;
-  const TileEntry* entries = nullptr;
+  TileBufs tl;
   const int* lra_fixed = nullptr;
   const float* lra_l0 = nullptr;
   uint8_t* lra_flag = nullptr;
@@ -253,25 +271,28 @@ int launch_solver(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, h
 int launch_solve_only(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, int iters,
                       hipStream_t s);
 int launch_integrate(const PbdBufs& b, const PbdParams& pp, hipStream_t s);
+// kp of every tile entry from the per-constraint parameters
+int launch_tile_stiffness(const PbdBufs& b, hipStream_t s);
+// LDS that the tiled kernels take (host check at tile building)
+size_t tile_lds_bytes(int max_local, int lds_slots, bool adjoint);
+int tile_lds_allow(size_t bytes);
 int launch_integrate_from(const PbdBufs& b, const PbdParams& pp, const float4* pfin,
                           hipStream_t s);
 int launch_friction(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, hipStream_t s);
 int launch_revert_toc(const PbdBufs& b, const NarrowBufs& nb, hipStream_t s);
 int launch_vertex_normals(int n, const int* vt_prefix, const int4* vt_tri, const float4* pos,
                           float4* nrm, int carry, int unit, hipStream_t s);
-// the solver stage with every iterate kept: pk[k * n, (k + 1) * n) = positions
-// entering iteration k, pk[iters * n ...) the result
+// the solver stage with every iterate kept, in solver order: pk[k * n, (k + 1) * n) =
+// positions entering iteration k, pk[iters * n ...) the result
 int launch_solver_rec(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, float4* pk,
                       hipStream_t s);
 
 // ---- adjoint (k_pbd.hip) ---------------------------------------------------
 struct AdjBufs {
   float4 *lx = nullptr, *lv = nullptr;  // dL/dx, dL/dv (n)
-  float4 *lp = nullptr, *la = nullptr;  // dL/dp of the iterates (n each, alternating)
-  float4* av = nullptr;                 // lp / count per vertex (n)
-  int* dcnt = nullptr;                  // non-zero contact records per iteration and vertex (iters * n)
+  float4 *lp = nullptr, *la = nullptr;  // dL/dp of the iterates (n each, alternating; solver order)
+  int* cnt = nullptr;  // Jacobi count per iteration and vertex (iters * n), solver order
   double *gks = nullptr, *gkb = nullptr;  // dL/dkp per distance / bend constraint
-  const int* ecid = nullptr;              // per tile entry: constraint index (bit 31: bend)
 };
 // The contact set of substep `slot`: the per-vertex records (dprefix[n] of them) are
 // appended to arena; ctl[0] = records used, ctl[1] = overflow, ctl[2 + slot] = first.

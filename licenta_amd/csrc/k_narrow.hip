@@ -737,15 +737,21 @@ __global__ void __launch_bounds__(kBlock) k_ccd_write(
   if (over) atomicOr(warn, (uint32_t)CM_WARN_CANDIDATE_CAP);
 }
 
+// vertex ids as solver positions
+__device__ __forceinline__ int4 ranked(int4 q, const int* __restrict__ rank) {
+  return rank ? make_int4(rank[q.x], rank[q.y], rank[q.z], rank[q.w]) : q;
+}
+
 __global__ void __launch_bounds__(kBlock) k_dyn_count(const int4* __restrict__ vfv,
                                                       const int4* __restrict__ eev,
                                                       const int* __restrict__ d_nvf,
                                                       const int* __restrict__ d_nee,
+                                                      const int* __restrict__ rank,
                                                       int* __restrict__ dcount, int n) {
   const int nvf = *d_nvf, nee = *d_nee;
   if (blockIdx.x == 0 && threadIdx.x == 0) dcount[n] = 0;  // long-list counter of k_dyn_sort
   for (int c = blockIdx.x * kBlock + threadIdx.x; c < nvf + nee; c += gridDim.x * kBlock) {
-    const int4 q = c < nvf ? vfv[c] : eev[c - nvf];
+    const int4 q = ranked(c < nvf ? vfv[c] : eev[c - nvf], rank);
     atomicAdd(&dcount[q.x], 1);
     atomicAdd(&dcount[q.y], 1);
     atomicAdd(&dcount[q.z], 1);
@@ -757,6 +763,7 @@ __global__ void __launch_bounds__(kBlock) k_dyn_fill(const int4* __restrict__ vf
                                                      const int4* __restrict__ eev,
                                                      const int* __restrict__ d_nvf,
                                                      const int* __restrict__ d_nee,
+                                                     const int* __restrict__ rank,
                                                      const int* __restrict__ prefix,
                                                      int* __restrict__ dcount,
                                                      uint32_t* __restrict__ drec) {
@@ -764,7 +771,7 @@ __global__ void __launch_bounds__(kBlock) k_dyn_fill(const int4* __restrict__ vf
   // k_dyn_sort orders them), which leaves the counts cleared for the next substep
   const int nvf = *d_nvf, nee = *d_nee;
   for (int c = blockIdx.x * kBlock + threadIdx.x; c < nvf + nee; c += gridDim.x * kBlock) {
-    const int4 q = c < nvf ? vfv[c] : eev[c - nvf];
+    const int4 q = ranked(c < nvf ? vfv[c] : eev[c - nvf], rank);
     const int vv[4] = {q.x, q.y, q.z, q.w};
     for (int r = 0; r < 4; ++r)
       drec[prefix[vv[r]] + atomicSub(&dcount[vv[r]], 1) - 1] = 4u * (uint32_t)c + r;
@@ -772,6 +779,7 @@ __global__ void __launch_bounds__(kBlock) k_dyn_fill(const int4* __restrict__ vf
 }
 
 __device__ __forceinline__ void put_payload(uint32_t r, int k, int nvf,
+                                            const int* __restrict__ rank,
                                             const int4* __restrict__ vf_v,
                                             const float4* __restrict__ vf_w,
                                             const int4* __restrict__ ee_v,
@@ -779,7 +787,7 @@ __device__ __forceinline__ void put_payload(uint32_t r, int k, int nvf,
                                             RecPayload* __restrict__ out) {
   const int ci = (int)(r >> 2), role = (int)(r & 3u);
   const bool isvf = ci < nvf;
-  int4 ids = isvf ? vf_v[ci] : ee_v[ci - nvf];
+  int4 ids = ranked(isvf ? vf_v[ci] : ee_v[ci - nvf], rank);
   const float4 w = isvf ? vf_w[ci] : ee_w[ci - nvf];
   ids.x |= (role << 29) | (isvf ? (int)0x80000000u : 0);
   RecPayload rp;
@@ -799,6 +807,7 @@ __global__ void __launch_bounds__(kBlock) k_dyn_sort(int n, const int* __restric
                                                      int* __restrict__ nlong,
                                                      int* __restrict__ long_list,
                                                      const int* __restrict__ d_nvf,
+                                                     const int* __restrict__ rank,
                                                      const int4* __restrict__ vf_v,
                                                      const float4* __restrict__ vf_w,
                                                      const int4* __restrict__ ee_v,
@@ -828,7 +837,7 @@ __global__ void __launch_bounds__(kBlock) k_dyn_sort(int n, const int* __restric
   for (int j = 0; j < k; ++j) {
     const uint32_t r = sk[j][tid];
     drec[b + j] = r;
-    put_payload(r, b + j, nvf, vf_v, vf_w, ee_v, ee_w, rec);
+    put_payload(r, b + j, nvf, rank, vf_v, vf_w, ee_v, ee_w, rec);
   }
 }
 
@@ -840,6 +849,7 @@ __global__ void __launch_bounds__(kBlock) k_dyn_sort_long(const int* __restrict_
                                                           uint32_t* __restrict__ drec,
                                                           uint32_t* __restrict__ tmp,
                                                           const int* __restrict__ d_nvf,
+                                                          const int* __restrict__ rank,
                                                           const int4* __restrict__ vf_v,
                                                           const float4* __restrict__ vf_w,
                                                           const int4* __restrict__ ee_v,
@@ -860,7 +870,7 @@ __global__ void __launch_bounds__(kBlock) k_dyn_sort_long(const int* __restrict_
         int r = 0;
         for (int m = 0; m < k; ++m) r += sl[m] < key;
         drec[b + r] = key;
-        put_payload(key, b + r, nvf, vf_v, vf_w, ee_v, ee_w, rec);
+        put_payload(key, b + r, nvf, rank, vf_v, vf_w, ee_v, ee_w, rec);
       }
     } else {
       for (int j = threadIdx.x; j < k; j += kBlock) {
@@ -872,7 +882,7 @@ __global__ void __launch_bounds__(kBlock) k_dyn_sort_long(const int* __restrict_
       __syncthreads();
       for (int j = threadIdx.x; j < k; j += kBlock) {
         drec[b + j] = tmp[b + j];
-        put_payload(tmp[b + j], b + j, nvf, vf_v, vf_w, ee_v, ee_w, rec);
+        put_payload(tmp[b + j], b + j, nvf, rank, vf_v, vf_w, ee_v, ee_w, rec);
       }
     }
     __syncthreads();
@@ -886,13 +896,14 @@ __global__ void __launch_bounds__(kBlock) k_rec_keys(const int4* __restrict__ vf
                                                      const int4* __restrict__ eev,
                                                      const int* __restrict__ d_nvf,
                                                      const int* __restrict__ d_nee,
+                                                     const int* __restrict__ rank,
                                                      uint4* __restrict__ keys,
                                                      uint4* __restrict__ vals,
                                                      int* __restrict__ d_nrec) {
   const int nvf = *d_nvf, nee = *d_nee;
   if (blockIdx.x == 0 && threadIdx.x == 0) *d_nrec = 4 * (nvf + nee);
   for (int c = blockIdx.x * kBlock + threadIdx.x; c < nvf + nee; c += gridDim.x * kBlock) {
-    const int4 q = c < nvf ? vfv[c] : eev[c - nvf];
+    const int4 q = ranked(c < nvf ? vfv[c] : eev[c - nvf], rank);
     keys[c] = make_uint4((uint32_t)q.x, (uint32_t)q.y, (uint32_t)q.z, (uint32_t)q.w);
     const uint32_t r = 4u * (uint32_t)c;
     vals[c] = make_uint4(r, r + 1u, r + 2u, r + 3u);
@@ -906,6 +917,7 @@ __global__ void __launch_bounds__(kBlock) k_rec_place(int n, const uint32_t* __r
                                                       const uint32_t* vals,
                                                       const int* __restrict__ d_nrec,
                                                       const int* __restrict__ d_nvf,
+                                                      const int* __restrict__ rank,
                                                       const int4* __restrict__ vf_v,
                                                       const float4* __restrict__ vf_w,
                                                       const int4* __restrict__ ee_v,
@@ -928,7 +940,7 @@ __global__ void __launch_bounds__(kBlock) k_rec_place(int n, const uint32_t* __r
     if (i < R) {
       const uint32_t r = vals[i];
       drec[i] = r;
-      put_payload(r, i, nvf, vf_v, vf_w, ee_v, ee_w, rec);
+      put_payload(r, i, nvf, rank, vf_v, vf_w, ee_v, ee_w, rec);
     }
   }
 }
@@ -1017,7 +1029,7 @@ int launch_dynamic_csr(const NarrowBufs& nb, hipStream_t s) {
     uint32_t* keys = nb.skey;
     uint32_t* kalt = nb.skey + rcap;
     hipLaunchKernelGGL(k_rec_keys, dim3(gc), dim3(kBlock), 0, s, nb.vf_v, nb.ee_v, nb.d_nvf,
-                       nb.d_nee, (uint4*)keys, (uint4*)nb.drec, nb.d_nrec);
+                       nb.d_nee, nb.rank, (uint4*)keys, (uint4*)nb.drec, nb.d_nrec);
     int bits = 1;
     while (bits < 32 && ((int64_t)1 << bits) < nb.n) ++bits;
     int in_alt = 0;
@@ -1026,27 +1038,27 @@ int launch_dynamic_csr(const NarrowBufs& nb, hipStream_t s) {
     if (rc) return rc;
     hipLaunchKernelGGL(k_rec_place, dim3(grid_for(std::max<int64_t>(rcap, nb.n + 1))),
                        dim3(kBlock), 0, s, nb.n, in_alt ? kalt : keys, in_alt ? nb.dtmp : nb.drec,
-                       nb.d_nrec, nb.d_nvf, nb.vf_v, nb.vf_w, nb.ee_v, nb.ee_w, nb.dprefix,
-                       nb.drec, nb.rec);
+                       nb.d_nrec, nb.d_nvf, nb.rank, nb.vf_v, nb.vf_w, nb.ee_v, nb.ee_w,
+                       nb.dprefix, nb.drec, nb.rec);
     CM_LAUNCH_CHECK();
     return CM_OK;
   }
   // per-vertex counts, a scan, atomic placement, then each vertex's list ordered;
   // dcount[0, n) is zero here: cleared at creation, then by every k_dyn_fill
   hipLaunchKernelGGL(k_dyn_count, dim3(gc), dim3(kBlock), 0, s, nb.vf_v, nb.ee_v, nb.d_nvf,
-                     nb.d_nee, nb.dcount, nb.n);
+                     nb.d_nee, nb.rank, nb.dcount, nb.n);
   CM_LAUNCH_CHECK();
   int rc = scan_exclusive(nb.dcount, nb.dprefix, nb.n, nullptr, nb.dprefix + nb.n, nb.scan_temp,
                           s);
   if (rc) return rc;
   hipLaunchKernelGGL(k_dyn_fill, dim3(gc), dim3(kBlock), 0, s, nb.vf_v, nb.ee_v, nb.d_nvf,
-                     nb.d_nee, nb.dprefix, nb.dcount, nb.drec);
+                     nb.d_nee, nb.rank, nb.dprefix, nb.dcount, nb.drec);
   hipLaunchKernelGGL(k_dyn_sort, dim3(nblocks(nb.n)), dim3(kBlock), 0, s, nb.n, nb.dprefix,
-                     nb.drec, nb.dcount + nb.n, nb.dlong, nb.d_nvf, nb.vf_v, nb.vf_w, nb.ee_v,
-                     nb.ee_w, nb.rec);
+                     nb.drec, nb.dcount + nb.n, nb.dlong, nb.d_nvf, nb.rank, nb.vf_v, nb.vf_w,
+                     nb.ee_v, nb.ee_w, nb.rec);
   hipLaunchKernelGGL(k_dyn_sort_long, dim3(512), dim3(kBlock), 0, s, nb.dprefix, nb.dcount + nb.n,
-                     nb.dlong, nb.drec, nb.dtmp, nb.d_nvf, nb.vf_v, nb.vf_w, nb.ee_v, nb.ee_w,
-                     nb.rec);
+                     nb.dlong, nb.drec, nb.dtmp, nb.d_nvf, nb.rank, nb.vf_v, nb.vf_w, nb.ee_v,
+                     nb.ee_w, nb.rec);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }

@@ -11,8 +11,8 @@
 //  k_solve        <- one Jacobi iteration of PBDStepSolver (:648-659): ground, LRA,
 //                    static (stretch :986-1022, bend :1024-1147), dynamic (VF :1212-1311,
 //                    EE :1313-1415) corrections and FinalCorrectionStep (:1690-1698)
-//                    in one launch: a workgroup evaluates the slots of a tile of up to
-//                    128 consecutive vertices in parallel into LDS, then each vertex sums its slots in
+//                    in one launch: a workgroup evaluates the constraints of a patch of
+//                    vertices in parallel into LDS, then each vertex sums its slots in
 //                    the reference's slot order, so the per-vertex sums are the
 //                    reference's gathers (:1417-1475) without the global slot buffer.
 //  k_integrate    <- _FinalUpdate (:1916-1932) + _WorldConstraints
@@ -435,6 +435,7 @@ __device__ __forceinline__ f3 ee_corr(float4 P0, float4 P1, float4 P2, float4 P3
 
 struct SolveArgs {
   int n, F, abs_mode, ground_on, bend_fp64;
+  int max_local, lds_slots;
   float th;
   const float4* ground;
   const int* lra_fixed;
@@ -448,10 +449,13 @@ struct SolveArgs {
   const float2* b_kpphi0;
   const int* dprefix;
   const RecPayload* rec;  // dynamic records in per-vertex order
-  // vertex tiles: tstart[ntiles + 1] vertex ranges, eprefix[ntiles + 1] entry ranges
-  const int* tstart;
-  const int* eprefix;
-  const TileEntry* entries;
+  const int* order;  // vertex of each solver position (tiles), and the inverse
+  const int* rank;
+  const int4* hdr;
+  const int* halo;
+  const uint4* sent;
+  const uint4* bent;
+  const float2* bpar;
 };
 
 // one static slot's correction: slot word = bend flag (bit 31), role (bits 29-30),
@@ -474,211 +478,329 @@ __device__ __forceinline__ f3 rec_corr(const RecPayload& rp, const float4 (&P)[4
                       : ee_corr(P[0], P[1], P[2], P[3], rp.w, role, th);
 }
 
-constexpr int kSolveV = 64;  // vertices per workgroup (slot-parallel form)
-constexpr int kLds = kTileSlots;  // slot corrections staged in LDS per pass
-constexpr int kBatch = 4;         // constraint entries / records per thread in flight
+constexpr int kSolveV = 64;       // vertices per workgroup (slot-parallel form)
+constexpr int kLds = kTileSlots;  // slot corrections staged in LDS per pass (slot-parallel form)
+constexpr int kBatch = 2;         // records per thread in flight
 
 __device__ __forceinline__ void lds_put(float* cx, float* cy, float* cz, uint32_t off, f3 c) {
   cx[off] = c.x;
   cy[off] = c.y;
   cz[off] = c.z;
 }
+// c to the tile-local slot off, unless its vertex is not in the tile
+__device__ __forceinline__ void tile_put(float* cx, float* cy, float* cz, uint32_t off, f3 c) {
+  if (off != 0xffffu) lds_put(cx, cy, cz, off, c);
+}
 
-// One Jacobi iteration over a range of consecutive vertices. The range's static
-// corrections are staged in LDS: in the tiled form (kTiles) each constraint that
-// touches the tile is evaluated once, from the tile's entry list, and its
-// corrections go to the slots of the tile's vertices; in the slot-parallel form
-// every slot re-evaluates its constraint, kLds slots per pass. The range's dynamic
-// records follow the same way. Each vertex then adds its own entries in slot
-// order, so every per-vertex sum has the reference's order and rounding.
-template <bool kTiles>
-__global__ void __launch_bounds__(kBlock) k_solve(SolveArgs a, const float4* __restrict__ pin,
-                                                  float4* __restrict__ pout) {
-  __shared__ float cx[kLds], cy[kLds], cz[kLds];
-  int v0, v1, tile = 0;
-  if (kTiles) {
-    // each XCD takes a contiguous range of tiles, so the positions that neighbouring
-    // tiles share are fetched into one L2
-    tile = xcd_block(blockIdx.x, gridDim.x);
-    v0 = a.tstart[tile];
-    v1 = a.tstart[tile + 1];
-  } else {
-    v0 = blockIdx.x * kSolveV;
-    v1 = min(v0 + kSolveV, a.n);
+// ground and long-range corrections of vertex `vid` at pi; the pinned vertices are
+// read at fixed_at(j)
+template <class FixedAt>
+__device__ __forceinline__ void ground_lra(const SolveArgs& a, int vid, float4 pi,
+                                           FixedAt fixed_at, f3& total, int& cnt) {
+  if (a.ground_on) {
+    const float4 gq = a.ground[vid];
+    if (gq.w != 0.f) {
+      const f3 nc = mk3(0.f, 1.f, 0.f);
+      const float cv = dot(sub(xyz(pi), xyz(gq)), nc);
+      if (cv < 0) {
+        total = add(total, mul(nc, -cv));
+        cnt += 1;
+      }
+    }
   }
+  if (a.F) {
+    f3 acc = mk3(0, 0, 0);
+    int c = 0;
+    for (int j = 0; j < a.F; ++j) {
+      if (a.lra_flag[(int64_t)vid * a.F + j]) {
+        const f3 diff = sub(xyz(pi), xyz(fixed_at(j)));
+        const float l = len(diff);
+        const f3 nn = divs(diff, l);
+        acc = add(acc, mul(nn, -(l - a.lra_l0[(int64_t)vid * a.F + j])));
+        ++c;
+      }
+    }
+    total = add(total, acc);
+    cnt += c;
+  }
+}
+
+// The corrections of the dynamic records [c0, c1) into the LDS slots. kBatch records
+// per thread: their loads, then their positions' loads, are in flight together before
+// any of them is evaluated. at(id): the position of a record's vertex; put(slot, c).
+template <int kT, class At, class Put>
+__device__ __forceinline__ void eval_records(const SolveArgs& a, int c0, int c1, At at, Put put) {
+  for (int q0 = c0 + threadIdx.x; q0 < c1; q0 += kT * kBatch) {
+    RecPayload rp[kBatch];
+    float4 P[kBatch][4];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (q0 + u * kT < c1) rp[u] = a.rec[q0 + u * kT];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (q0 + u * kT >= c1) continue;
+      P[u][0] = at(rp[u].ids.x & 0x1fffffff);
+      P[u][1] = at(rp[u].ids.y);
+      P[u][2] = at(rp[u].ids.z);
+      P[u][3] = at(rp[u].ids.w);
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (q0 + u * kT < c1) put(q0 + u * kT - c0, rec_corr(rp[u], P[u], a.th));
+  }
+}
+
+// acc plus the values c[k, e) one after the other (LDS reads batched ahead of the
+// dependent adds)
+template <class T>
+__device__ __forceinline__ T sum_run(T acc, const T* c, int k, int e) {
+  for (; k + 8 <= e; k += 8) {
+    T v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = c[k + u];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc = acc + v[u];
+  }
+  for (; k < e; ++k) acc = acc + c[k];
+  return acc;
+}
+
+// LDS of a tile workgroup: positions (kPos arrays), four slot arrays (x, y, z and, for
+// the records, whether the correction counts), and the tile's slot and record prefixes
+struct TileLds {
+  float *c[3];
+  int *cn, *sp, *rp;
+};
+template <int kPos>
+__device__ __forceinline__ TileLds tile_lds(float4* base, int max_local, int lds_slots) {
+  TileLds l;
+  float* f = (float*)(base + kPos * max_local);
+  for (int k = 0; k < 3; ++k) l.c[k] = f + k * lds_slots;
+  l.cn = (int*)(f + 3 * lds_slots);
+  l.sp = l.cn + lds_slots;
+  l.rp = l.sp + kBlock + 1;
+  return l;
+}
+
+// The per-vertex sums of a tile are serial chains in slot order, up to hundreds of
+// records long, but their components are independent: a wave takes one component (or
+// the record count, component 3) of 64 vertices at a time. f(u, component, vertex) is
+// called for the wave's u-th such job.
+// jobs of a wave: 4 components x up to 4 x 64 vertices
+template <int kT>
+__host__ __device__ constexpr int tile_job_count() { return 16 / (kT / 64); }
+template <int kT, class F>
+__device__ __forceinline__ void tile_jobs(int nv, F f) {
+  const int groups = (nv + 63) >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+  for (int u = 0; u < tile_job_count<kT>(); ++u) {
+    const int job = wave + (kT / 64) * u;
+    if (job >= 4 * groups) break;
+    const int v = (job >> 2) * 64 + lane;
+    if (v < nv) f(u, job & 3, v);
+  }
+}
+
+// One Jacobi iteration over a tile (TileBufs). The tile's positions and its halo's are
+// staged in LDS; each constraint that touches the tile is evaluated once from there
+// and its corrections go to the slots of the tile's vertices; each vertex then adds
+// its slots in slot order, so every per-vertex sum has the reference's order and
+// rounding. The dynamic records follow the same way, their positions from memory; only
+// non-zero corrections are counted (adding a zero one changes nothing: a sum that
+// starts at +0 is never -0). kFirst: pin is in vertex order; else, and pout always, in
+// solver order.
+// The launch is bound by the bends' FP64 chains (about 540 instructions each) and, with
+// contacts, by the tile with the most records. Evaluating from LDS-staged patches
+// instead of strips of 128 vertex ids cut the repeated evaluations from 1.75 (distance)
+// and 2.34 (bend) per constraint to 1.13 and 1.24 and the entries from 32 to 16 and 24
+// bytes; one wave per component of the sums took the records' chains (up to 182 on the
+// draped 256^2 cloth, each with a branch) off one wave. Per launch, before -> now:
+// 1024^2 236 -> 122 us, 96 cloths 147 -> 91, 192x301 without contacts 15.9 -> 11.9,
+// draped 256^2 31.3 -> 23.2, draped 131x97 27.9 -> 14.5, 64^2 9.1 -> 6.0. More waves per
+// SIMD (96 registers: five) spill and are slower (1024^2: 43 against 30 ms a pass).
+template <bool kFirst, int kT>
+__global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float4* __restrict__ pin,
+                                                  float4* __restrict__ pout) {
+  constexpr int kJobs = tile_job_count<kT>();
+  extern __shared__ float4 lpos[];
+  const TileLds l = tile_lds<1>(lpos, a.max_local, a.lds_slots);
+  // each XCD takes a contiguous range of tiles, so the positions that neighbouring
+  // tiles share are fetched into one L2
+  const int tile = xcd_block(blockIdx.x, gridDim.x);
+  const int4 h0 = a.hdr[2 * tile], h1 = a.hdr[2 * tile + 1];
+  const int v0 = h0.x, nv = h0.y, nh = h0.w;
+  const int tid = threadIdx.x;
+  auto at = [&](int k) { return pin[kFirst ? a.order[k] : k]; };
+  for (int k = tid; k < nv + nh; k += kT) lpos[k] = at(k < nv ? v0 + k : a.halo[h0.z + k - nv]);
+  const int s0 = a.vprefix[v0];
+  int r0 = 0, r1 = 0;
+  if (a.dprefix) {
+    r0 = a.dprefix[v0];
+    r1 = a.dprefix[v0 + nv];
+  }
+  for (int k = tid; k <= nv; k += kT) {  // tiles hold at most kBlock vertices
+    l.sp[k] = a.vprefix[v0 + k] - s0;
+    l.rp[k] = a.dprefix ? a.dprefix[v0 + k] : 0;
+  }
+  __syncthreads();
+  for (int q = tid; q < h1.w; q += kT) {
+    const uint4 t = a.bent[h1.z + q];
+    const float2 par = a.bpar[h1.z + q];
+    f3 cr[4];
+    if (a.bend_fp64)
+      bend_all<double>(lpos[t.x & 0xffffu], lpos[t.x >> 16], lpos[t.y & 0xffffu], lpos[t.y >> 16],
+                       par, a.abs_mode, cr);
+    else
+      bend_all<float>(lpos[t.x & 0xffffu], lpos[t.x >> 16], lpos[t.y & 0xffffu], lpos[t.y >> 16],
+                      par, a.abs_mode, cr);
+    tile_put(l.c[0], l.c[1], l.c[2], t.z & 0xffffu, cr[0]);
+    tile_put(l.c[0], l.c[1], l.c[2], t.z >> 16, cr[1]);
+    tile_put(l.c[0], l.c[1], l.c[2], t.w & 0xffffu, cr[2]);
+    tile_put(l.c[0], l.c[1], l.c[2], t.w >> 16, cr[3]);
+  }
+  // the distance entries are dealt to the waves in reverse: the last waves, which the
+  // bends' remainder leaves idle, take the first of them
+  for (int q = tid ^ (kT - 64); q < h1.y; q += kT) {
+    const uint4 t = a.sent[h1.x + q];
+    f3 c0, c1;
+    stretch_both(lpos[t.x & 0xffffu], lpos[t.x >> 16],
+                 make_float2(__uint_as_float(t.z), __uint_as_float(t.w)), c0, c1);
+    tile_put(l.c[0], l.c[1], l.c[2], t.y & 0xffffu, c0);
+    tile_put(l.c[0], l.c[1], l.c[2], t.y >> 16, c1);
+  }
+  __syncthreads();
+  float accs[kJobs], accd[kJobs];  // of this thread's jobs: slots, records
+  int accn[kJobs];
+#pragma unroll
+  for (int u = 0; u < kJobs; ++u) {
+    accs[u] = accd[u] = 0.f;
+    accn[u] = 0;
+  }
+  tile_jobs<kT>(nv, [&](int u, int comp, int v) {
+    if (comp < 3) accs[u] = sum_run(0.f, l.c[comp], l.sp[v], l.sp[v + 1]);
+  });
+  __syncthreads();
+  for (int c0 = r0; c0 < r1; c0 += a.lds_slots) {
+    const int c1 = min(c0 + a.lds_slots, r1);
+    eval_records<kT>(a, c0, c1, at, [&](int q, f3 c) {
+      lds_put(l.c[0], l.c[1], l.c[2], q, c);
+      l.cn[q] = is_zero(c) ? 0 : 1;
+    });
+    __syncthreads();
+    tile_jobs<kT>(nv, [&](int u, int comp, int v) {
+      const int k = max(l.rp[v], c0) - c0, e = min(l.rp[v + 1], c1) - c0;
+      if (comp < 3) accd[u] = sum_run(accd[u], l.c[comp], k, e);
+      else accn[u] = sum_run(accn[u], l.cn, k, e);
+    });
+    __syncthreads();
+  }
+  // the sums to LDS, component by component: slots at [0, kBlock), records after them
+  tile_jobs<kT>(nv, [&](int u, int comp, int v) {
+    if (comp < 3) {
+      l.c[comp][v] = accs[u];
+      l.c[comp][kBlock + v] = accd[u];
+    } else {
+      l.cn[v] = accn[u];
+    }
+  });
+  __syncthreads();
+  if (tid >= nv) return;
+  const int i = v0 + tid;
+  const float4 pi = lpos[tid];
+  f3 total = mk3(0, 0, 0);
+  int cnt = 0;
+  if (a.ground_on | a.F)
+    ground_lra(a, a.order[i], pi,
+               [&](int j) { return pin[kFirst ? a.lra_fixed[j] : a.rank[a.lra_fixed[j]]]; },
+               total, cnt);
+  total = add(total, mk3(l.c[0][tid], l.c[1][tid], l.c[2][tid]));
+  cnt += l.sp[tid + 1] - l.sp[tid];
+  if (l.rp[tid + 1] > l.rp[tid]) {
+    total = add(total, mk3(l.c[0][kBlock + tid], l.c[1][kBlock + tid], l.c[2][kBlock + tid]));
+    cnt += l.cn[tid];
+  }
+  pout[i] = f4(add(xyz(pi), divs(total, (float)cnt)), pi.w);
+}
+
+// One Jacobi iteration over kSolveV consecutive vertices for meshes without tiles:
+// every slot re-evaluates its constraint, kLds slots per pass.
+__global__ void __launch_bounds__(kBlock) k_solve_slots(SolveArgs a,
+                                                        const float4* __restrict__ pin,
+                                                        float4* __restrict__ pout) {
+  __shared__ float cx[kLds], cy[kLds], cz[kLds];
+  const int v0 = blockIdx.x * kSolveV, v1 = min(v0 + kSolveV, a.n);
   const int tid = threadIdx.x;
   const int i = v0 + tid;
-  const bool mine = i < v1;  // tiles hold at most kBlock vertices
+  const bool mine = i < v1;
   float4 pi = make_float4(0.f, 0.f, 0.f, 0.f);
   f3 total = mk3(0, 0, 0);
   int cnt = 0;
   if (mine) {
     pi = pin[i];
-    if (a.ground_on) {
-      const float4 gq = a.ground[i];
-      if (gq.w != 0.f) {
-        const f3 nc = mk3(0.f, 1.f, 0.f);
-        const float cv = dot(sub(xyz(pi), xyz(gq)), nc);
-        if (cv < 0) {
-          total = add(total, mul(nc, -cv));
-          cnt += 1;
-        }
-      }
-    }
-    if (a.F) {
-      f3 acc = mk3(0, 0, 0);
-      int c = 0;
-      for (int j = 0; j < a.F; ++j) {
-        if (a.lra_flag[(int64_t)i * a.F + j]) {
-          const f3 diff = sub(xyz(pi), xyz(pin[a.lra_fixed[j]]));
-          const float l = len(diff);
-          const f3 nn = divs(diff, l);
-          acc = add(acc, mul(nn, -(l - a.lra_l0[(int64_t)i * a.F + j])));
-          ++c;
-        }
-      }
-      total = add(total, acc);
-      cnt += c;
-    }
+    ground_lra(a, i, pi, [&](int j) { return pin[a.lra_fixed[j]]; }, total, cnt);
   }
-  // static slots
-  {
-    const int s0 = a.vprefix[v0], s1 = a.vprefix[v1];
-    int k = mine ? a.vprefix[i] : 0;
-    const int e = mine ? a.vprefix[i + 1] : 0;
-    f3 acc = mk3(0, 0, 0);
-    for (int c0 = s0; c0 < s1; c0 += kLds) {
-      const int c1 = min(c0 + kLds, s1);
-      if (kTiles) {  // a tile's slots fit one pass (c0 == s0)
-        const int eb = a.eprefix[tile], ee = a.eprefix[tile + 1];
-        // kBatch entries per thread at a time: their loads, then their positions'
-        // loads, are in flight together before any of them is evaluated
-        for (int q0 = eb + tid; q0 < ee; q0 += kBlock * kBatch) {
-          TileEntry te[kBatch];
-          float4 P[kBatch][4];
-#pragma unroll
-          for (int u = 0; u < kBatch; ++u)
-            if (q0 + u * kBlock < ee) te[u] = a.entries[q0 + u * kBlock];
-#pragma unroll
-          for (int u = 0; u < kBatch; ++u) {
-            if (q0 + u * kBlock >= ee) continue;
-            P[u][0] = pin[te[u].ids.x];
-            P[u][1] = pin[te[u].ids.y];
-            if (te[u].ids.z >= 0) {
-              P[u][2] = pin[te[u].ids.z];
-              P[u][3] = pin[te[u].ids.w];
-            }
-          }
-#pragma unroll
-          for (int u = 0; u < kBatch; ++u) {
-            if (q0 + u * kBlock >= ee) continue;
-            const TileEntry& t = te[u];
-            if (t.ids.z < 0) {
-              f3 c0v, c1v;
-              stretch_both(P[u][0], P[u][1], make_float2(t.a, t.b), c0v, c1v);
-              if ((t.s01 & 0xffffu) != 0xffffu) lds_put(cx, cy, cz, t.s01 & 0xffffu, c0v);
-              if ((t.s01 >> 16) != 0xffffu) lds_put(cx, cy, cz, t.s01 >> 16, c1v);
-            } else {
-              f3 cr[4];
-              if (a.bend_fp64)
-                bend_all<double>(P[u][0], P[u][1], P[u][2], P[u][3], make_float2(t.a, t.b),
-                                 a.abs_mode, cr);
-              else
-                bend_all<float>(P[u][0], P[u][1], P[u][2], P[u][3], make_float2(t.a, t.b),
-                                a.abs_mode, cr);
-              if ((t.s01 & 0xffffu) != 0xffffu) lds_put(cx, cy, cz, t.s01 & 0xffffu, cr[0]);
-              if ((t.s01 >> 16) != 0xffffu) lds_put(cx, cy, cz, t.s01 >> 16, cr[1]);
-              if ((t.s23 & 0xffffu) != 0xffffu) lds_put(cx, cy, cz, t.s23 & 0xffffu, cr[2]);
-              if ((t.s23 >> 16) != 0xffffu) lds_put(cx, cy, cz, t.s23 >> 16, cr[3]);
-            }
-            // evaluate the batch's entries one after the other (bounded registers)
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
-      } else {
-        for (int q = c0 + tid; q < c1; q += kBlock)
-          lds_put(cx, cy, cz, q - c0, slot_corr(a, a.vslot[q], pin));
-      }
-      __syncthreads();
-      const int kend = min(e, c1);
-      // LDS reads batched ahead of the dependent adds; the add order is unchanged
-      for (; k + 4 <= kend; k += 4) {
-        const int q = k - c0;
-        const f3 e0 = mk3(cx[q], cy[q], cz[q]), e1 = mk3(cx[q + 1], cy[q + 1], cz[q + 1]);
-        const f3 e2 = mk3(cx[q + 2], cy[q + 2], cz[q + 2]), e3 = mk3(cx[q + 3], cy[q + 3], cz[q + 3]);
-        acc = add(add(add(add(acc, e0), e1), e2), e3);
-      }
-      for (; k < kend; ++k) acc = add(acc, mk3(cx[k - c0], cy[k - c0], cz[k - c0]));
-      __syncthreads();
-    }
-    if (mine) {
-      total = add(total, acc);
-      cnt += e - (int)a.vprefix[i];
-    }
+  const int s0 = a.vprefix[v0], s1 = a.vprefix[v1];
+  int k = mine ? a.vprefix[i] : 0;
+  const int e = mine ? a.vprefix[i + 1] : 0;
+  f3 acc = mk3(0, 0, 0);
+  if (mine) cnt += e - k;
+  for (int c0 = s0; c0 < s1; c0 += kLds) {
+    const int c1 = min(c0 + kLds, s1);
+    for (int q = c0 + tid; q < c1; q += kBlock)
+      lds_put(cx, cy, cz, q - c0, slot_corr(a, a.vslot[q], pin));
+    __syncthreads();
+    const int kend = min(e, c1);
+    for (; k < kend; ++k) acc = add(acc, mk3(cx[k - c0], cy[k - c0], cz[k - c0]));
+    __syncthreads();
   }
-  // dynamic records: only non-zero corrections are summed and counted
+  if (mine) total = add(total, acc);
   if (a.dprefix) {
     const int r0 = a.dprefix[v0], r1 = a.dprefix[v1];
-    if (r1 > r0) {
-      int k = mine ? a.dprefix[i] : 0;
-      const int e = mine ? a.dprefix[i + 1] : 0;
-      const bool any = mine && e > k;
-      f3 acc = mk3(0, 0, 0);
-      int c = 0;
-      for (int c0 = r0; c0 < r1; c0 += kLds) {
-        const int c1 = min(c0 + kLds, r1);
-        for (int q0 = c0 + tid; q0 < c1; q0 += kBlock * kBatch) {
-          RecPayload rp[kBatch];
-          float4 P[kBatch][4];
-#pragma unroll
-          for (int u = 0; u < kBatch; ++u)
-            if (q0 + u * kBlock < c1) rp[u] = a.rec[q0 + u * kBlock];
-#pragma unroll
-          for (int u = 0; u < kBatch; ++u) {
-            if (q0 + u * kBlock >= c1) continue;
-            P[u][0] = pin[rp[u].ids.x & 0x1fffffff];
-            P[u][1] = pin[rp[u].ids.y];
-            P[u][2] = pin[rp[u].ids.z];
-            P[u][3] = pin[rp[u].ids.w];
-          }
-#pragma unroll
-          for (int u = 0; u < kBatch; ++u)
-            if (q0 + u * kBlock < c1)
-              lds_put(cx, cy, cz, q0 + u * kBlock - c0, rec_corr(rp[u], P[u], a.th));
-        }
-        __syncthreads();
-        const int kend = min(e, c1);
-        for (; k + 4 <= kend; k += 4) {
-          const int q = k - c0;
-          f3 ev[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) ev[u] = mk3(cx[q + u], cy[q + u], cz[q + u]);
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (!is_zero(ev[u])) {
-              acc = add(acc, ev[u]);
-              ++c;
-            }
-        }
-        for (; k < kend; ++k) {
-          const f3 val = mk3(cx[k - c0], cy[k - c0], cz[k - c0]);
-          if (!is_zero(val)) {
-            acc = add(acc, val);
-            ++c;
-          }
-        }
-        __syncthreads();
+    int rk = mine ? a.dprefix[i] : 0;
+    const int re = mine ? a.dprefix[i + 1] : 0;
+    const bool any = re > rk;
+    f3 racc = mk3(0, 0, 0);
+    int c = 0;
+    for (int c0 = r0; c0 < r1; c0 += kLds) {
+      const int c1 = min(c0 + kLds, r1);
+      eval_records<kBlock>(a, c0, c1, [&](int id) { return pin[id]; },
+                   [&](int q, f3 v) { lds_put(cx, cy, cz, q, v); });
+      __syncthreads();
+      for (const int kend = min(re, c1); rk < kend; ++rk) {
+        const f3 val = mk3(cx[rk - c0], cy[rk - c0], cz[rk - c0]);
+        racc = add(racc, val);
+        c += !is_zero(val);
       }
-      if (any) {
-        total = add(total, acc);
-        cnt += c;
-      }
+      __syncthreads();
+    }
+    if (any) {
+      total = add(total, racc);
+      cnt += c;
     }
   }
   if (mine) pout[i] = f4(add(xyz(pi), divs(total, (float)cnt)), pi.w);
 }
 
-__global__ void __launch_bounds__(kBlock) k_integrate(int n, const float4* __restrict__ pfin,
+// kp of the tile entries from the per-constraint parameters
+__global__ void __launch_bounds__(kBlock) k_tile_stiffness(
+    int ns, int nb, const int* __restrict__ scid, const int* __restrict__ bcid,
+    const float2* __restrict__ s_l0kp, const float2* __restrict__ b_kpphi0,
+    uint4* __restrict__ sent, float2* __restrict__ bpar) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < ns) sent[i].w = __float_as_uint(s_l0kp[scid[i]].y);
+  if (i < nb) bpar[i].x = b_kpphi0[bcid[i]].x;
+}
+
+// p in vertex order <-> q in solver order
+__global__ void __launch_bounds__(kBlock) k_to_order(int n, const int* __restrict__ order,
+                                                     const float4* __restrict__ p,
+                                                     float4* __restrict__ q) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) q[i] = p[order ? order[i] : i];
+}
+
+__global__ void __launch_bounds__(kBlock) k_integrate(int n, const int* __restrict__ rank,
+                                                      const float4* __restrict__ pfin,
                                                       float4* __restrict__ x,
                                                       float4* __restrict__ v,
                                                       float4* __restrict__ p,
@@ -686,7 +808,7 @@ __global__ void __launch_bounds__(kBlock) k_integrate(int n, const float4* __res
                                                       float dt, int clamp, f3 lo, f3 hi) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  float4 pi = pfin[i];
+  float4 pi = pfin[rank ? rank[i] : i];  // pfin is in solver order
   if (pinned[i]) {
     v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
   } else {
@@ -719,8 +841,8 @@ __global__ void __launch_bounds__(kBlock) k_integrate(int n, const float4* __res
 // (:1700-1723) keeps the tangential velocity along fn and reflects the normal part
 // scaled by (1 - kf)^c.
 __global__ void __launch_bounds__(kBlock) k_friction(
-    int n, int rigid_n, const float4* __restrict__ ground, const int* __restrict__ dprefix,
-    const uint32_t* __restrict__ drec, const int* __restrict__ d_nvf,
+    int n, int rigid_n, const float4* __restrict__ ground, const int* __restrict__ rank,
+    const int* __restrict__ dprefix, const uint32_t* __restrict__ drec, const int* __restrict__ d_nvf,
     const float4* __restrict__ vf_tn, const float4* __restrict__ ee_tn, float4* __restrict__ v,
     float kf) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
@@ -734,7 +856,8 @@ __global__ void __launch_bounds__(kBlock) k_friction(
     vel = reflect(add(vt, mul(vn, 1.f - kf)), nc);
   }
   if (dprefix) {
-    const int b = dprefix[i], e = dprefix[i + 1];
+    const int r = rank ? rank[i] : i;
+    const int b = dprefix[r], e = dprefix[r + 1];
     if (e > b) {
       const int nvf = *d_nvf;
       f3 acc = mk3(0.f, 0.f, 0.f);
@@ -760,7 +883,8 @@ __global__ void __launch_bounds__(kBlock) k_friction(
 // (the reference starts its minimum at 100) and moves to (1 - t) x + t p
 // (CudaUtils::AdvancePositionInTimePos, Core/CudaUtils.cu:396-399). The contact t is
 // the time of contact in seconds, used as the blend weight as the reference does.
-__global__ void __launch_bounds__(kBlock) k_revert_toc(int n, const int* __restrict__ dprefix,
+__global__ void __launch_bounds__(kBlock) k_revert_toc(int n, const int* __restrict__ rank,
+                                                       const int* __restrict__ dprefix,
                                                        const uint32_t* __restrict__ drec,
                                                        const int* __restrict__ d_nvf,
                                                        const float4* __restrict__ vf_tn,
@@ -769,7 +893,8 @@ __global__ void __launch_bounds__(kBlock) k_revert_toc(int n, const int* __restr
                                                        float4* __restrict__ p) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  const int b = dprefix[i], e = dprefix[i + 1];
+  const int r = rank ? rank[i] : i;
+  const int b = dprefix[r], e = dprefix[r + 1];
   if (e == b) return;
   const int nvf = *d_nvf;
   float tmin = 100.f;
@@ -815,41 +940,43 @@ __global__ void __launch_bounds__(kBlock) k_vertex_normals(int n, const int* __r
 // are piecewise constant. Cotangents run in FP32; stiffness gradients sum in FP64.
 
 // x' = p_I, v' = (p_I - x) / dt; pinned: x' = x, v' = 0
-__global__ void __launch_bounds__(kBlock) k_adj_integrate(int n, const uint8_t* __restrict__ pinned,
+__global__ void __launch_bounds__(kBlock) k_adj_integrate(int n, const int* __restrict__ rank,
+                                                          const uint8_t* __restrict__ pinned,
                                                           float4* __restrict__ lx,
                                                           const float4* __restrict__ lv,
                                                           float4* __restrict__ lp, float dt) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   if (pinned[i]) {
-    lp[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    lp[rank[i]] = make_float4(0.f, 0.f, 0.f, 0.f);
     return;
   }
   const f3 gv = divs(xyz(lv[i]), dt);
-  lp[i] = f4(add(xyz(lx[i]), gv), 0.f);
+  lp[rank[i]] = f4(add(xyz(lx[i]), gv), 0.f);
   lx[i] = f4(neg(gv), 0.f);
 }
 
 // p0 = x + dt v', v' = v + dt g
-__global__ void __launch_bounds__(kBlock) k_adj_predict(int n, float4* __restrict__ lx,
+__global__ void __launch_bounds__(kBlock) k_adj_predict(int n, const int* __restrict__ rank,
+                                                        float4* __restrict__ lx,
                                                         float4* __restrict__ lv,
                                                         const float4* __restrict__ lp, float dt) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  const f3 g = xyz(lp[i]);
+  const f3 g = xyz(lp[rank[i]]);
   lx[i] = f4(add(xyz(lx[i]), g), 0.f);
   lv[i] = f4(mul(g, dt), 0.f);
 }
 
 // The dynamic part of every iteration's Jacobi counts, all iterations at once (the
-// substep's iterates are on the tape): record q adds one to dcnt[it * n + v], v its
-// vertex, when its correction at the iterate pk[it] is non-zero, as k_solve counts it.
+// substep's iterates are on the tape): record q adds one to cnt[it * n + v], v its
+// vertex's solver position, when its correction at the iterate pk[it] is non-zero, as k_solve counts it.
 // Integer sums, so the order of the atomics does not matter.
 __global__ void __launch_bounds__(kBlock) k_adj_counts(int n, int iters,
                                                        const int* __restrict__ dprefix,
                                                        const RecPayload* __restrict__ rec,
                                                        const float4* __restrict__ pk,
-                                                       int* __restrict__ dcnt, float th) {
+                                                       int* __restrict__ cnt, float th) {
   const int nrec = dprefix[n];
   const int64_t total = (int64_t)nrec * iters;
   for (int64_t k = blockIdx.x * (int64_t)kBlock + threadIdx.x; k < total;
@@ -862,21 +989,19 @@ __global__ void __launch_bounds__(kBlock) k_adj_counts(int n, int iters,
     const float4 P[4] = {ps[id0], ps[rp.ids.y], ps[rp.ids.z], ps[rp.ids.w]};
     if (!is_zero(rec_corr(rp, P, th))) {
       const int v = role == 0 ? id0 : (role == 1 ? rp.ids.y : (role == 2 ? rp.ids.z : rp.ids.w));
-      atomicAdd(&dcnt[(int64_t)it * n + v], 1);
+      atomicAdd(&cnt[(int64_t)it * n + v], 1);
     }
   }
 }
 
-// per vertex: the iteration's count (static slots plus the non-zero dynamic records
-// counted by k_adj_counts; dcnt null: no contacts) and av = lp / count
-__global__ void __launch_bounds__(kBlock) k_adj_scale(int n, const int* __restrict__ vprefix,
-                                                      const int* __restrict__ dcnt,
-                                                      const float4* __restrict__ lp,
-                                                      float4* __restrict__ av) {
+// every iteration's Jacobi counts before the dynamic part: the static slots
+__global__ void __launch_bounds__(kBlock) k_adj_counts_init(int n, int iters,
+                                                            const int* __restrict__ prefix,
+                                                            int* __restrict__ cnt) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  const int cnt = vprefix[i + 1] - vprefix[i] + (dcnt ? dcnt[i] : 0);
-  av[i] = cnt ? f4(divs(xyz(lp[i]), (float)cnt), 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
+  const int c = prefix[i + 1] - prefix[i];
+  for (int it = 0; it < iters; ++it) cnt[(int64_t)it * n + i] = c;
 }
 
 // Distance constraint: c0 = -w1 t, c1 = w2 t with t = f kp / ws, f = (l - l0) n.
@@ -1041,96 +1166,116 @@ __device__ __forceinline__ f3 rec_vjp(const RecPayload& rp, const float4 (&P)[4]
 }
 
 struct AdjArgs {
-  int abs_mode, bend_fp64;
+  int abs_mode, bend_fp64, max_local, lds_slots;
   float th;
-  const int* vprefix;
-  const int* tstart;
-  const int* eprefix;
-  const TileEntry* entries;
-  const int* ecid;  // per entry: constraint index, bit 31 set for a bend
+  TileBufs tl;
   const int* dprefix;
   const RecPayload* rec;
   double* gks;  // dL/dkp per distance constraint
   double* gkb;  // dL/dkp per bend constraint
 };
 
-// One reverse Jacobi iteration over a vertex tile, in the layout of k_solve<true>:
-// every constraint touching the tile is differentiated once, its vertex cotangents
-// go to the tile's slots, and each vertex adds its slots in slot order, then its
-// dynamic records in record order: la = lp + sum over slots and records. The tile
-// holding a constraint's role-0 vertex adds its dL/dkp (one owner per constraint).
+// One reverse Jacobi iteration over a vertex tile, in the layout of k_solve: the
+// cotangents of the corrections are lp / count (zero without a count), formed where
+// they are staged or gathered; every constraint touching the tile is differentiated
+// once, its vertex cotangents go to the tile's slots, and each vertex adds its slots in
+// slot order, then its dynamic records in record order: la = lp + sum over slots and
+// records. The tile holding a constraint's role-0 vertex adds its dL/dkp (one owner per
+// constraint). Bound by the FP64 bend VJP at two waves per SIMD (246 registers). 128^2:
+// 13.7 us a launch (21.1 in strips of 128 ids, plus 4.2 for a scaling launch of its
+// own), 24 cloths of 64^2: 29 us (38 + 5).
 __global__ void __launch_bounds__(kBlock) k_adj_iter(AdjArgs a, const float4* __restrict__ ps,
-                                                     const float4* __restrict__ av,
+                                                     const int* __restrict__ cnt,
                                                      const float4* __restrict__ lp,
                                                      float4* __restrict__ la) {
-  __shared__ float cx[kLds], cy[kLds], cz[kLds];
+  constexpr int kJobs = tile_job_count<kBlock>();
+  extern __shared__ float4 lpos[];
+  float4* lav = lpos + a.max_local;
+  const TileLds l = tile_lds<2>(lpos, a.max_local, a.lds_slots);
   const int tile = xcd_block(blockIdx.x, gridDim.x);  // contiguous tiles per XCD
-  const int v0 = a.tstart[tile], v1 = a.tstart[tile + 1];
+  const int4 h0 = a.tl.hdr[2 * tile], h1 = a.tl.hdr[2 * tile + 1];
+  const int v0 = h0.x, nv = h0.y, nh = h0.w;
   const int tid = threadIdx.x;
-  const int i = v0 + tid;
-  const bool mine = i < v1;
-  f3 total = mk3(0, 0, 0);
-  {
-    const int s0 = a.vprefix[v0];
-    const int eb = a.eprefix[tile], ee = a.eprefix[tile + 1];
-    for (int q = eb + tid; q < ee; q += kBlock) {
-      const TileEntry t = a.entries[q];
-      const int cid = a.ecid[q];
-      float gkp;
-      if (t.ids.z < 0) {
-        const float4 P0 = ps[t.ids.x], P1 = ps[t.ids.y];
-        const float4 G0 = av[t.ids.x], G1 = av[t.ids.y];
-        const f3 gd = stretch_vjp(P0, P1, G0, G1, t.a, t.b, gkp);
-        if ((t.s01 & 0xffffu) != 0xffffu) {
-          lds_put(cx, cy, cz, t.s01 & 0xffffu, gd);
-          a.gks[cid] += (double)gkp;
-        }
-        if ((t.s01 >> 16) != 0xffffu) lds_put(cx, cy, cz, t.s01 >> 16, neg(gd));
-      } else {
-        const float4 P[4] = {ps[t.ids.x], ps[t.ids.y], ps[t.ids.z], ps[t.ids.w]};
-        const float4 G[4] = {av[t.ids.x], av[t.ids.y], av[t.ids.z], av[t.ids.w]};
-        f3 o[4];
-        if (a.bend_fp64)
-          bend_vjp<double>(P, G, t.a, t.b, a.abs_mode, o, gkp);
-        else
-          bend_vjp<float>(P, G, t.a, t.b, a.abs_mode, o, gkp);
-        if ((t.s01 & 0xffffu) != 0xffffu) {
-          lds_put(cx, cy, cz, t.s01 & 0xffffu, o[0]);
-          a.gkb[cid & 0x7fffffff] += (double)gkp;
-        }
-        if ((t.s01 >> 16) != 0xffffu) lds_put(cx, cy, cz, t.s01 >> 16, o[1]);
-        if ((t.s23 & 0xffffu) != 0xffffu) lds_put(cx, cy, cz, t.s23 & 0xffffu, o[2]);
-        if ((t.s23 >> 16) != 0xffffu) lds_put(cx, cy, cz, t.s23 >> 16, o[3]);
-      }
-    }
-    __syncthreads();
-    if (mine) {
-      const int e = a.vprefix[i + 1];
-      for (int k = a.vprefix[i]; k < e; ++k)
-        total = add(total, mk3(cx[k - s0], cy[k - s0], cz[k - s0]));
-    }
-    __syncthreads();
+  auto scaled = [&](int k) {
+    const int c = cnt[k];
+    return c ? f4(divs(xyz(lp[k]), (float)c), 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
+  };
+  for (int k = tid; k < nv + nh; k += kBlock) {
+    const int v = k < nv ? v0 + k : a.tl.halo[h0.z + k - nv];
+    lpos[k] = ps[v];
+    lav[k] = scaled(v);
   }
+  const int s0 = a.tl.prefix[v0];
+  for (int k = tid; k <= nv; k += kBlock) {
+    l.sp[k] = a.tl.prefix[v0 + k] - s0;
+    l.rp[k] = a.dprefix ? a.dprefix[v0 + k] : 0;
+  }
+  __syncthreads();
+  for (int q = tid; q < h1.w; q += kBlock) {
+    const uint4 t = a.tl.bent[h1.z + q];
+    const float2 par = a.tl.bpar[h1.z + q];
+    const uint32_t id[4] = {t.x & 0xffffu, t.x >> 16, t.y & 0xffffu, t.y >> 16};
+    const float4 P[4] = {lpos[id[0]], lpos[id[1]], lpos[id[2]], lpos[id[3]]};
+    const float4 G[4] = {lav[id[0]], lav[id[1]], lav[id[2]], lav[id[3]]};
+    f3 o[4];
+    float gkp;
+    if (a.bend_fp64)
+      bend_vjp<double>(P, G, par.x, par.y, a.abs_mode, o, gkp);
+    else
+      bend_vjp<float>(P, G, par.x, par.y, a.abs_mode, o, gkp);
+    if ((t.z & 0xffffu) != 0xffffu) {
+      lds_put(l.c[0], l.c[1], l.c[2], t.z & 0xffffu, o[0]);
+      a.gkb[a.tl.bcid[h1.z + q]] += (double)gkp;
+    }
+    tile_put(l.c[0], l.c[1], l.c[2], t.z >> 16, o[1]);
+    tile_put(l.c[0], l.c[1], l.c[2], t.w & 0xffffu, o[2]);
+    tile_put(l.c[0], l.c[1], l.c[2], t.w >> 16, o[3]);
+  }
+  for (int q = tid ^ (kBlock - 64); q < h1.y; q += kBlock) {
+    const uint4 t = a.tl.sent[h1.x + q];
+    const uint32_t i0 = t.x & 0xffffu, i1 = t.x >> 16;
+    float gkp;
+    const f3 gd = stretch_vjp(lpos[i0], lpos[i1], lav[i0], lav[i1], __uint_as_float(t.z),
+                              __uint_as_float(t.w), gkp);
+    if ((t.y & 0xffffu) != 0xffffu) {
+      lds_put(l.c[0], l.c[1], l.c[2], t.y & 0xffffu, gd);
+      a.gks[a.tl.scid[h1.x + q]] += (double)gkp;
+    }
+    tile_put(l.c[0], l.c[1], l.c[2], t.y >> 16, neg(gd));
+  }
+  __syncthreads();
+  float acc[kJobs];
+#pragma unroll
+  for (int u = 0; u < kJobs; ++u) acc[u] = 0.f;
+  tile_jobs<kBlock>(nv, [&](int u, int comp, int v) {
+    if (comp < 3) acc[u] = sum_run(0.f, l.c[comp], l.sp[v], l.sp[v + 1]);
+  });
+  __syncthreads();
   if (a.dprefix) {
-    const int r0 = a.dprefix[v0], r1 = a.dprefix[v1];
-    int k = mine ? a.dprefix[i] : 0;
-    const int e = mine ? a.dprefix[i + 1] : 0;
-    for (int c0 = r0; c0 < r1; c0 += kLds) {
-      const int c1 = min(c0 + kLds, r1);
+    const int r0 = a.dprefix[v0], r1 = a.dprefix[v0 + nv];
+    for (int c0 = r0; c0 < r1; c0 += a.lds_slots) {
+      const int c1 = min(c0 + a.lds_slots, r1);
       for (int q = c0 + tid; q < c1; q += kBlock) {
         const RecPayload rp = a.rec[q];
         const int id0 = rp.ids.x & 0x1fffffff;
         const float4 P[4] = {ps[id0], ps[rp.ids.y], ps[rp.ids.z], ps[rp.ids.w]};
-        const float4 G[4] = {av[id0], av[rp.ids.y], av[rp.ids.z], av[rp.ids.w]};
-        lds_put(cx, cy, cz, q - c0, rec_vjp(rp, P, G, a.th));
+        const float4 G[4] = {scaled(id0), scaled(rp.ids.y), scaled(rp.ids.z), scaled(rp.ids.w)};
+        lds_put(l.c[0], l.c[1], l.c[2], q - c0, rec_vjp(rp, P, G, a.th));
       }
       __syncthreads();
-      const int kend = min(e, c1);
-      for (; k < kend; ++k) total = add(total, mk3(cx[k - c0], cy[k - c0], cz[k - c0]));
+      tile_jobs<kBlock>(nv, [&](int u, int comp, int v) {
+        if (comp < 3)
+          acc[u] = sum_run(acc[u], l.c[comp], max(l.rp[v], c0) - c0, min(l.rp[v + 1], c1) - c0);
+      });
       __syncthreads();
     }
   }
-  if (mine) la[i] = f4(add(xyz(lp[i]), total), 0.f);
+  tile_jobs<kBlock>(nv, [&](int u, int comp, int v) {
+    if (comp < 3) l.c[comp][v] = acc[u];
+  });
+  __syncthreads();
+  if (tid < nv)
+    la[v0 + tid] = f4(add(xyz(lp[v0 + tid]), mk3(l.c[0][tid], l.c[1][tid], l.c[2][tid])), 0.f);
 }
 
 // Tape of a recorded substep's contact set: slot `slot` of ctl ([0] records used, [1]
@@ -1192,11 +1337,17 @@ static SolveArgs solve_args(const PbdBufs& b, const PbdParams& pp, const NarrowB
   a.lra_fixed = b.lra_fixed;
   a.lra_l0 = b.lra_l0;
   a.lra_flag = b.lra_flag;
-  a.vprefix = b.vprefix;
+  a.vprefix = b.tl.n > 0 ? b.tl.prefix : b.vprefix;
   a.vslot = b.vslot;
-  a.tstart = b.tstart;
-  a.eprefix = b.eprefix;
-  a.entries = b.entries;
+  a.max_local = b.tl.max_local;
+  a.lds_slots = b.tl.lds_slots;
+  a.order = b.tl.order;
+  a.rank = b.tl.rank;
+  a.hdr = b.tl.hdr;
+  a.halo = b.tl.halo;
+  a.sent = b.tl.sent;
+  a.bent = b.tl.bent;
+  a.bpar = b.tl.bpar;
   a.sid = b.sid;
   a.s_l0kp = b.s_l0kp;
   a.bid = b.bid;
@@ -1207,18 +1358,58 @@ static SolveArgs solve_args(const PbdBufs& b, const PbdParams& pp, const NarrowB
   return a;
 }
 
-// `iters` Jacobi iterations ping-ponging p -> p2 -> p ...
-static int launch_iterations(const PbdBufs& b, const SolveArgs& a, int iters, hipStream_t s) {
-  float4* src = b.p;
-  float4* dst = b.p2;
-  for (int it = 0; it < iters; ++it) {
-    if (b.ntiles > 0)
-      hipLaunchKernelGGL(k_solve<true>, dim3(b.ntiles), dim3(kBlock), 0, s, a, src, dst);
-    else
-      hipLaunchKernelGGL(k_solve<false>, dim3((b.n + kSolveV - 1) / kSolveV), dim3(kBlock), 0, s,
-                         a, src, dst);
-    std::swap(src, dst);
+// One Jacobi iteration src -> dst; first: src is in vertex order (dst never is)
+static void launch_iteration(const PbdBufs& b, const SolveArgs& a, bool first, const float4* src,
+                             float4* dst, hipStream_t s) {
+  if (b.tl.n <= 0) {
+    hipLaunchKernelGGL(k_solve_slots, dim3((b.n + kSolveV - 1) / kSolveV), dim3(kBlock), 0, s, a,
+                       src, dst);
+    return;
   }
+  const size_t lds = tile_lds_bytes(b.tl.max_local, b.tl.lds_slots, false);
+  const dim3 grid(b.tl.n), wg(b.tl.threads);
+  if (b.tl.threads == 512) {
+    if (first) hipLaunchKernelGGL((k_solve<true, 512>), grid, wg, lds, s, a, src, dst);
+    else hipLaunchKernelGGL((k_solve<false, 512>), grid, wg, lds, s, a, src, dst);
+  } else {
+    if (first) hipLaunchKernelGGL((k_solve<true, 256>), grid, wg, lds, s, a, src, dst);
+    else hipLaunchKernelGGL((k_solve<false, 256>), grid, wg, lds, s, a, src, dst);
+  }
+}
+
+// `iters` Jacobi iterations p -> q0 -> q1 -> q0 ...
+static int launch_iterations(const PbdBufs& b, const SolveArgs& a, int iters, hipStream_t s) {
+  const float4* src = b.p;
+  for (int it = 0; it < iters; ++it) {
+    float4* dst = (it & 1) ? b.q1 : b.q0;
+    launch_iteration(b, a, it == 0, src, dst, s);
+    src = dst;
+  }
+  CM_LAUNCH_CHECK();
+  return CM_OK;
+}
+
+size_t tile_lds_bytes(int max_local, int lds_slots, bool adjoint) {
+  return (adjoint ? 2 : 1) * sizeof(float4) * (size_t)max_local +
+         4 * sizeof(float) * (size_t)lds_slots + 2 * sizeof(int) * (kBlock + 1);
+}
+
+// more than 64 KiB of LDS per workgroup has to be asked for (meshes with a vertex of
+// very many constraints)
+int tile_lds_allow(size_t bytes) {
+  if (bytes <= (64u << 10)) return CM_OK;
+  for (const void* f :
+       {(const void*)k_solve<true, 256>, (const void*)k_solve<false, 256>,
+        (const void*)k_solve<true, 512>, (const void*)k_solve<false, 512>, (const void*)k_adj_iter})
+    CM_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  return CM_OK;
+}
+
+int launch_tile_stiffness(const PbdBufs& b, hipStream_t s) {
+  const int m = std::max(b.tl.nsent, b.tl.nbent);
+  if (m <= 0) return CM_OK;
+  hipLaunchKernelGGL(k_tile_stiffness, dim3(nblocks(m)), dim3(kBlock), 0, s, b.tl.nsent,
+                     b.tl.nbent, b.tl.scid, b.tl.bcid, b.s_l0kp, b.b_kpphi0, b.tl.sent, b.tl.bpar);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
@@ -1238,17 +1429,23 @@ int launch_solver(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, h
 
 int launch_solve_only(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, int iters,
                       hipStream_t s) {
-  return launch_iterations(b, solve_args(b, pp, nb), iters, s);
+  const int rc = launch_iterations(b, solve_args(b, pp, nb), iters, s);
+  if (rc) return rc;
+  // back to p: vertex i is at solver position rank[i]
+  hipLaunchKernelGGL(k_to_order, dim3(nblocks(b.n)), dim3(kBlock), 0, s, b.n, b.tl.rank,
+                     (iters & 1) ? b.q0 : b.q1, b.p);
+  CM_LAUNCH_CHECK();
+  return CM_OK;
 }
 
 int launch_integrate(const PbdBufs& b, const PbdParams& pp, hipStream_t s) {
-  return launch_integrate_from(b, pp, (pp.iters & 1) ? b.p2 : b.p, s);
+  return launch_integrate_from(b, pp, (pp.iters & 1) ? b.q0 : b.q1, s);
 }
 
 int launch_integrate_from(const PbdBufs& b, const PbdParams& pp, const float4* pfin,
                           hipStream_t s) {
-  hipLaunchKernelGGL(k_integrate, dim3(nblocks(b.n)), dim3(kBlock), 0, s, b.n, pfin, b.x, b.v,
-                     b.p, b.pinned, pp.dt, (pp.flags & CM_F_WORLD_CLAMP) ? 1 : 0, pp.wmin,
+  hipLaunchKernelGGL(k_integrate, dim3(nblocks(b.n)), dim3(kBlock), 0, s, b.n, b.tl.rank, pfin,
+                     b.x, b.v, b.p, b.pinned, pp.dt, (pp.flags & CM_F_WORLD_CLAMP) ? 1 : 0, pp.wmin,
                      pp.wmax);
   CM_LAUNCH_CHECK();
   return CM_OK;
@@ -1263,8 +1460,8 @@ int launch_vertex_normals(int n, const int* vt_prefix, const int4* vt_tri, const
 }
 
 int launch_revert_toc(const PbdBufs& b, const NarrowBufs& nb, hipStream_t s) {
-  hipLaunchKernelGGL(k_revert_toc, dim3(nblocks(b.n)), dim3(kBlock), 0, s, b.n, nb.dprefix,
-                     nb.drec, nb.d_nvf, nb.vf_tn, nb.ee_tn, b.x, b.p);
+  hipLaunchKernelGGL(k_revert_toc, dim3(nblocks(b.n)), dim3(kBlock), 0, s, b.n, nb.rank,
+                     nb.dprefix, nb.drec, nb.d_nvf, nb.vf_tn, nb.ee_tn, b.x, b.p);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
@@ -1276,7 +1473,7 @@ int launch_friction(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb,
   const float4* ground = (pp.flags & CM_F_GROUND) ? b.ground : nullptr;
   const bool coll = (pp.flags & CM_F_SELF_COLLISION) && nb.dprefix;
   hipLaunchKernelGGL(k_friction, dim3(g), dim3(kBlock), 0, s, b.n, rigid_n, ground,
-                     coll ? nb.dprefix : nullptr, nb.drec, nb.d_nvf, nb.vf_tn, nb.ee_tn, b.v,
+                     nb.rank, coll ? nb.dprefix : nullptr, nb.drec, nb.d_nvf, nb.vf_tn, nb.ee_tn, b.v,
                      pp.kf);
   CM_LAUNCH_CHECK();
   return CM_OK;
@@ -1293,17 +1490,10 @@ int launch_solver_rec(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& n
   if (pp.flags & CM_F_SPHERE)
     hipLaunchKernelGGL(k_sphere, dim3(g), dim3(kBlock), 0, s, b.n, b.x, b.p, pp.sc, pp.sr + pp.th);
   CM_LAUNCH_CHECK();
-  CM_HIP(hipMemcpyAsync(pk, b.p, sizeof(float4) * b.n, hipMemcpyDeviceToDevice, s));
+  hipLaunchKernelGGL(k_to_order, dim3(g), dim3(kBlock), 0, s, b.n, b.tl.order, b.p, pk);
   const SolveArgs a = solve_args(b, pp, nb);
-  for (int it = 0; it < pp.iters; ++it) {
-    const float4* src = pk + (int64_t)it * b.n;
-    float4* dst = pk + (int64_t)(it + 1) * b.n;
-    if (b.ntiles > 0)
-      hipLaunchKernelGGL(k_solve<true>, dim3(b.ntiles), dim3(kBlock), 0, s, a, src, dst);
-    else
-      hipLaunchKernelGGL(k_solve<false>, dim3((b.n + kSolveV - 1) / kSolveV), dim3(kBlock), 0, s,
-                         a, src, dst);
-  }
+  for (int it = 0; it < pp.iters; ++it)
+    launch_iteration(b, a, false, pk + (int64_t)it * b.n, pk + (int64_t)(it + 1) * b.n, s);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
@@ -1319,41 +1509,39 @@ int launch_tape_records(int n, const int* dprefix, const RecPayload* rec, RecPay
 
 int launch_adj_substep(const PbdBufs& b, const PbdParams& pp, const AdjBufs& ab, const float4* pk,
                        const int* dprefix, const RecPayload* rec, hipStream_t s) {
-  if (b.ntiles <= 0) {
+  if (b.tl.n <= 0) {
     set_error("adjoint: needs the tiled Jacobi layout");
     return CM_ERR_ARG;
   }
   const int g = nblocks(b.n);
-  hipLaunchKernelGGL(k_adj_integrate, dim3(g), dim3(kBlock), 0, s, b.n, b.pinned, ab.lx, ab.lv,
-                     ab.lp, pp.dt);
+  hipLaunchKernelGGL(k_adj_integrate, dim3(g), dim3(kBlock), 0, s, b.n, b.tl.rank, b.pinned, ab.lx,
+                     ab.lv, ab.lp, pp.dt);
   AdjArgs a;
   a.abs_mode = (pp.ref_compat & CM_RC_BEND_ABS) ? 1 : 0;
   a.bend_fp64 = (pp.flags & CM_F_BEND_FP64) ? 1 : 0;
+  a.max_local = b.tl.max_local;
+  a.lds_slots = b.tl.lds_slots;
   a.th = pp.th;
-  a.vprefix = b.vprefix;
-  a.tstart = b.tstart;
-  a.eprefix = b.eprefix;
-  a.entries = b.entries;
-  a.ecid = ab.ecid;
+  a.tl = b.tl;
   a.dprefix = dprefix;
   a.rec = rec;
   a.gks = ab.gks;
   a.gkb = ab.gkb;
-  if (dprefix) {
-    CM_HIP(hipMemsetAsync(ab.dcnt, 0, sizeof(int) * (size_t)pp.iters * b.n, s));
+  hipLaunchKernelGGL(k_adj_counts_init, dim3(g), dim3(kBlock), 0, s, b.n, pp.iters, b.tl.prefix,
+                     ab.cnt);
+  if (dprefix)
     hipLaunchKernelGGL(k_adj_counts, dim3(1024), dim3(kBlock), 0, s, b.n, pp.iters, dprefix, rec,
-                       pk, ab.dcnt, pp.th);
-  }
+                       pk, ab.cnt, pp.th);
+  const size_t lds = tile_lds_bytes(b.tl.max_local, b.tl.lds_slots, true);
   float4* src = ab.lp;
   float4* dst = ab.la;
   for (int it = pp.iters - 1; it >= 0; --it) {
-    const float4* ps = pk + (int64_t)it * b.n;
-    hipLaunchKernelGGL(k_adj_scale, dim3(g), dim3(kBlock), 0, s, b.n, b.vprefix,
-                       dprefix ? ab.dcnt + (int64_t)it * b.n : nullptr, src, ab.av);
-    hipLaunchKernelGGL(k_adj_iter, dim3(b.ntiles), dim3(kBlock), 0, s, a, ps, ab.av, src, dst);
+    hipLaunchKernelGGL(k_adj_iter, dim3(b.tl.n), dim3(kBlock), lds, s, a, pk + (int64_t)it * b.n,
+                       ab.cnt + (int64_t)it * b.n, src, dst);
     std::swap(src, dst);
   }
-  hipLaunchKernelGGL(k_adj_predict, dim3(g), dim3(kBlock), 0, s, b.n, ab.lx, ab.lv, src, pp.dt);
+  hipLaunchKernelGGL(k_adj_predict, dim3(g), dim3(kBlock), 0, s, b.n, b.tl.rank, ab.lx, ab.lv, src,
+                     pp.dt);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
