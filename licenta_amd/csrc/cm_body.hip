@@ -117,7 +117,8 @@ struct cm_body {
   void* sort_temp = nullptr;
   float4 *cen = nullptr, *box = nullptr, *tmp_min = nullptr, *tmp_max = nullptr;
   LbvhBufs lb;
-  int2 *chunk = nullptr, *pairs = nullptr;
+  int* chunk = nullptr;
+  int2* pairs = nullptr;
   int *leaf_cnt = nullptr, *leaf_off = nullptr;
   int* counters = nullptr;  // [0] npairs [1] ncand_vf [2] ncand_ee [3] nvf [4] nee ... [8] traversal hand-over count
   void* lb_temp = nullptr;  // LBVH build/refit scratch (carve_build)
@@ -621,6 +622,8 @@ int record_substep(cm_body* b, hipEvent_t* ev = nullptr, const TapeSlot* tape = 
   }
   mark(CM_STAGE_PAIRS);
   if (coll) {
+    rc = launch_pack_nodes(b->lb, false, s);
+    if (rc) return rc;
     rc = launch_pairs(b->lb, b->cap, b->chunk, b->leaf_cnt, b->leaf_off, b->pairs, b->counters,
                       b->scan_temp, s);
     if (rc) return rc;

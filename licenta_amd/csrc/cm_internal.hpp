@@ -85,6 +85,8 @@ int fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s);
 // ---- LBVH (k_lbvh.hip) -----------------------------------------------------
 // ints per traversal hand-over record (leaf, pairs, depth, node, cap, visits, stack)
 constexpr int kTravRec = 72;
+// trees of fewer leaves are walked through their quantised nodes (26-bit ids)
+constexpr int kQuantLeaves = 1 << 26;
 // ints per leaf for the traversal stack entries below its LDS part
 constexpr int kTravSpill = 47;
 
@@ -98,7 +100,8 @@ struct LbvhBufs {
   int *state = nullptr, *top_list = nullptr, *top_index = nullptr, *ntop = nullptr;
   float4 *tmin = nullptr, *tmax = nullptr;  // deferred-node scratch (large trees)
   int *trm = nullptr, *tdone = nullptr;
-  float4* nodes = nullptr;  // 4 float4 per internal node (children, rightmost leaves, boxes)
+  uint4* qnodes = nullptr;  // quantised record of each internal node, 2 uint4 (k_lbvh.hip)
+  int* irr = nullptr;       // set when the tree has to be walked through its exact boxes
   int trav_chunk = 4;       // traversal: tiles per chunk dealt to one XCD (launch shape only)
   // traversal: visits a leaf makes in the first pass before a wave takes it over (0:
   // one pass); records of kTravRec ints for up to rcap such leaves; hctl[0] their
@@ -131,12 +134,14 @@ int launch_tri_update_batch(const LbvhBufs& b, const float4* x, const float4* p,
                             hipStream_t s);
 int launch_build(const LbvhBufs& b, const uint64_t* keys, int midpoint, hipStream_t s);
 int launch_refit(const LbvhBufs& b, hipStream_t s);
-int launch_pack_nodes(const LbvhBufs& b, hipStream_t s);
-// pairs: traversal into chunk (T*cap int2) + per-leaf counts, then compaction.
-int launch_pairs(const LbvhBufs& b, int cap, int2* chunk, int* counts, int* offsets,
+// the traversal's node records; from_caller: check the caller's tree first
+int launch_pack_nodes(const LbvhBufs& b, bool from_caller, hipStream_t s);
+// pairs: traversal into chunk (T * cap ints: the pairs' second leaves) + per-leaf counts,
+// then compaction.
+int launch_pairs(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offsets,
                  int2* pairs, int* d_npairs, void* scan_temp, hipStream_t s);
 // the traversal kernel alone on the current tree (it rewrites the same pair chunk)
-int launch_traverse_only(const LbvhBufs& b, int cap, int2* chunk, int* counts, int* offsets,
+int launch_traverse_only(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offsets,
                          hipStream_t s);
 int launch_gather_tris(int t, const uint32_t* perm, const int4* tri_in, int4* tri_out,
                        int fix_leaves, float4* amin, float4* amax, float4* tmp_min,

@@ -207,7 +207,8 @@ __device__ __forceinline__ int sgn(int a) { return signbit((float)a) ? -1 : 1; }
 
 __global__ void __launch_bounds__(kBlock) k_build_init(int t, int* __restrict__ cnt,
                                                        int* __restrict__ hi,
-                                                       int* __restrict__ ntop, int ncloth,
+                                                       int* __restrict__ ntop,
+                                                       int* __restrict__ irr, int ncloth,
                                                        int* __restrict__ croot) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i < 2 * t - 1) {
@@ -215,7 +216,10 @@ __global__ void __launch_bounds__(kBlock) k_build_init(int t, int* __restrict__ 
     hi[i] = -1;
   }
   if (i < ncloth) croot[i] = -1;
-  if (i == 0) *ntop = 0;  // deferred-node count of the refit
+  if (i == 0) {
+    *ntop = 0;  // deferred-node count of the refit
+    *irr = 0;
+  }
 }
 
 __global__ void __launch_bounds__(kBlock) k_build(int t, const uint64_t* __restrict__ k,
@@ -281,18 +285,6 @@ __global__ void __launch_bounds__(kBlock) k_parents(int t, const int* __restrict
 }
 
 // ---- bottom-up refit ------------------------------------------------------------
-// Packed node record read by the traversal, 4 float4 per internal node:
-//   [0] left, right, rmll, rmlr (int bits)   [1] left min xyz, left max x
-//   [2] left max yz, right min xy             [3] right min z, right max xyz
-__device__ __forceinline__ void write_node(float4* __restrict__ nodes, int q, int l, int r,
-                                           int a, int b, f3 lmn, f3 lmx, f3 rmn, f3 rmx) {
-  float4* o = nodes + 4 * (int64_t)q;
-  o[0] = make_float4(__int_as_float(l), __int_as_float(r), __int_as_float(a), __int_as_float(b));
-  o[1] = make_float4(lmn.x, lmn.y, lmn.z, lmx.x);
-  o[2] = make_float4(lmx.y, lmx.z, rmn.x, rmn.y);
-  o[3] = make_float4(rmn.z, rmx.x, rmx.y, rmx.z);
-}
-
 constexpr int kRefitCH = 1024;  // leaves (and node ids) per refit workgroup
 constexpr int kTopCap = 2048;   // deferred nodes the top pass keeps in LDS
 constexpr int kTopList = 8192;  // pending deferred nodes the top pass lists in LDS
@@ -308,8 +300,7 @@ constexpr int kTopList = 8192;  // pending deferred nodes the top pass lists in 
 __global__ void __launch_bounds__(kRefitCH) k_refit_local(
     int t, const int* __restrict__ lefts, const int* __restrict__ rights,
     const int2* __restrict__ ranges, float4* __restrict__ amin, float4* __restrict__ amax,
-    int* __restrict__ rmll, int* __restrict__ rmlr, float4* __restrict__ nodes,
-    int* __restrict__ state, int* __restrict__ top_list, int* __restrict__ top_index,
+    int* __restrict__ rmll, int* __restrict__ rmlr, int* __restrict__ state, int* __restrict__ top_list, int* __restrict__ top_index,
     int* __restrict__ ntop, int* __restrict__ gdone) {
   __shared__ float4 lmin[kRefitCH], lmax[kRefitCH];  // leaf boxes of the chunk
   __shared__ float4 nmin[kRefitCH], nmax[kRefitCH];  // node boxes of the chunk
@@ -371,7 +362,6 @@ __global__ void __launch_bounds__(kRefitCH) k_refit_local(
     amax[q] = nmax[tid];
     rmll[q] = a;
     rmlr[q] = b;
-    write_node(nodes, q, l, r, a, b, lmn, lmx, rmn, rmx);
     state[q] = 1;
   } else {
     state[q] = 0;
@@ -403,12 +393,11 @@ __device__ __forceinline__ void top_child(int c, int nin, const int* __restrict_
 
 // a finished deferred node j (node qq): its box and rightmost leaf in the deferred
 // scratch (for its parent) and in the tree
-__device__ __forceinline__ void put_deferred(int j, int qq, int ll, int rr, int a, int b, f3 lmn,
-                                             f3 lmx, f3 rmn, f3 rmx, float4* __restrict__ gmin,
+__device__ __forceinline__ void put_deferred(int j, int qq, int a, int b, f3 lmn, f3 lmx,
+                                             f3 rmn, f3 rmx, float4* __restrict__ gmin,
                                              float4* __restrict__ gmax, int* __restrict__ grm,
                                              float4* __restrict__ amin, float4* __restrict__ amax,
-                                             int* __restrict__ rmll, int* __restrict__ rmlr,
-                                             float4* __restrict__ nodes) {
+                                             int* __restrict__ rmll, int* __restrict__ rmlr) {
   gmin[j] = f4(vmin(lmn, rmn), 0.f);
   gmax[j] = f4(vmax(lmx, rmx), 0.f);
   grm[j] = max(a, b);
@@ -416,7 +405,6 @@ __device__ __forceinline__ void put_deferred(int j, int qq, int ll, int rr, int 
   amax[qq] = gmax[j];
   rmll[qq] = a;
   rmlr[qq] = b;
-  write_node(nodes, qq, ll, rr, a, b, lmn, lmx, rmn, rmx);
 }
 
 constexpr int kSuper = 64 * kRefitCH;  // leaves per workgroup of the middle pass
@@ -431,8 +419,7 @@ constexpr int kMidCap = 8192;          // deferred nodes one middle workgroup ho
 __global__ void __launch_bounds__(1024) k_refit_mid(
     int t, const int* __restrict__ lefts, const int* __restrict__ rights,
     const int2* __restrict__ ranges, float4* __restrict__ amin, float4* __restrict__ amax,
-    int* __restrict__ rmll, int* __restrict__ rmlr, float4* __restrict__ nodes,
-    const int* __restrict__ state, const int* __restrict__ top_list,
+    int* __restrict__ rmll, int* __restrict__ rmlr, const int* __restrict__ state, const int* __restrict__ top_list,
     const int* __restrict__ top_index, const int* __restrict__ ntop, float4* __restrict__ gmin,
     float4* __restrict__ gmax, int* __restrict__ grm, int* __restrict__ gdone) {
   __shared__ int own[kMidCap];
@@ -472,8 +459,8 @@ __global__ void __launch_bounds__(1024) k_refit_mid(
       if (rt && !(inside(rr) && gdone[b] < 0 && -gdone[b] < pass)) continue;
       if (lt) { lmn = xyz(gmin[a]); lmx = xyz(gmax[a]); a = grm[a]; }
       if (rt) { rmn = xyz(gmin[b]); rmx = xyz(gmax[b]); b = grm[b]; }
-      put_deferred(j, qq, ll, rr, a, b, lmn, lmx, rmn, rmx, gmin, gmax, grm, amin, amax, rmll,
-                   rmlr, nodes);
+      put_deferred(j, qq, a, b, lmn, lmx, rmn, rmx, gmin, gmax, grm, amin, amax, rmll,
+                   rmlr);
       __threadfence_block();
       gdone[j] = -pass;
       changed = true;
@@ -489,10 +476,10 @@ __global__ void __launch_bounds__(1024) k_refit_mid(
 __global__ void __launch_bounds__(1024) k_refit_top(
     int t, const int* __restrict__ lefts, const int* __restrict__ rights,
     float4* __restrict__ amin, float4* __restrict__ amax, int* __restrict__ rmll,
-    int* __restrict__ rmlr, float4* __restrict__ nodes, const int* __restrict__ state,
+    int* __restrict__ rmlr, const int* __restrict__ state,
     const int* __restrict__ top_list, const int* __restrict__ top_index, int* __restrict__ ntop,
     float4* __restrict__ gmin, float4* __restrict__ gmax, int* __restrict__ grm,
-    int* __restrict__ gdone, uint32_t* __restrict__ warn) {
+    int* __restrict__ gdone, uint32_t* __restrict__ warn, int* __restrict__ irr) {
   __shared__ float4 smin[kTopCap], smax[kTopCap];
   __shared__ int srm[kTopCap], sdone[kTopCap];
   __shared__ int plist[kTopList];
@@ -558,7 +545,6 @@ __global__ void __launch_bounds__(1024) k_refit_top(
       amax[q[k]] = smax[j];
       rmll[q[k]] = la[k];
       rmlr[q[k]] = ra[k];
-      write_node(nodes, q[k], l[k], r[k], la[k], ra[k], lmn[k], lmx[k], rmn[k], rmx[k]);
     }
   } else {
     // gdone: 0 pending (set by k_refit_local), < 0 finished by k_refit_mid, > 0 the
@@ -590,8 +576,8 @@ __global__ void __launch_bounds__(1024) k_refit_top(
         if (rt && !(gdone[b] != 0 && gdone[b] < pass)) continue;
         if (lt) { lmn = xyz(gmin[a]); lmx = xyz(gmax[a]); a = grm[a]; }
         if (rt) { rmn = xyz(gmin[b]); rmx = xyz(gmax[b]); b = grm[b]; }
-        put_deferred(j, qq, ll, rr, a, b, lmn, lmx, rmn, rmx, gmin, gmax, grm, amin, amax, rmll,
-                     rmlr, nodes);
+        put_deferred(j, qq, a, b, lmn, lmx, rmn, rmx, gmin, gmax, grm, amin, amax, rmll,
+                     rmlr);
         __threadfence_block();
         gdone[j] = pass;
         changed = true;
@@ -601,83 +587,68 @@ __global__ void __launch_bounds__(1024) k_refit_top(
     for (int k = tid; k < nloop; k += 1024)
       if (gdone[listed ? plist[k] : k] == 0) left_over = true;
   }
-  if (__syncthreads_or(left_over) && tid == 0) atomicOr(warn, (uint32_t)CM_WARN_REFIT_LIMIT);
+  if (__syncthreads_or(left_over) && tid == 0) {
+    atomicOr(warn, (uint32_t)CM_WARN_REFIT_LIMIT);
+    atomicOr(irr, 1);  // an unfinished node's box need not hold its children's
+  }
   if (tid == 0) *ntop = 0;
 }
 
 // ---- traversal ----------------------------------------------------------------
 constexpr int kTravBlock = 128;  // 2 waves
 constexpr int kStack = 63;       // usable entries, as the reference's int[64] with its -1 sentinel
-// The first kLdsStack entries of a lane's stack live in LDS (8 KiB per workgroup, so
-// LDS leaves room for 8 waves per SIMD); deeper entries, rare, go to the lane's
-// global spill row of kStack - kLdsStack ints.
+// The first kLdsStack rows of a lane's stack live in LDS (8 KiB per workgroup, so
+// LDS leaves room for 8 waves per SIMD); deeper ones, rare, go to the lane's global
+// spill row of kStack - kLdsStack ints.
 constexpr int kLdsStack = 16;
 constexpr int kSpill = kStack - kLdsStack;
 static_assert(kSpill == kTravSpill, "spill row");
 
-__device__ __forceinline__ void put_pair(int2* p, int a, int b) {
-  // a plain store: a leaf's chunk fills whole lines in L2 before they go out (streamed
-  // stores left each 8-byte pair a partial-line write; the 512-cloth batch traversal
-  // took 2.2 ms with them, 1.36 ms without)
-  *(long long*)p = (long long)(uint32_t)a | ((long long)b << 32);
-}
-
-// State of one leaf's DFS between two visits: the node to visit next, the stack
-// depth, the pairs written and the visits made.
-struct DfsState {
-  int node, top, ncol;
-  long long visits;
+// The tree as the traversal kernels take it
+struct WalkTree {
+  int t;
+  const uint4* qnodes;  // null: the exact walk
+  const int *irr, *lefts, *rights, *rmll, *rmlr;
+  const float4 *amin, *amax;
+  const int *slot_cloth, *croot, *ccap;  // batch (null: one cloth)
 };
 
-// DFS of one leaf (Collision/CudaBVH.cu:23-113) from state st: its pairs in the
-// reference's order into out (at most cap), stack entry k in sstk[k][col]. Returns
-// true when the walk ended (stack empty, the first dropped pair, or the visit limit);
-// false when `budget` visits had been made first, with st at the next visit.
-// The stack's first kLds entries are sstk[k][col], the rest spill[k - kLds].
+// DFS of one leaf (Collision/CudaBVH.cu:23-113) from the root through the exact boxes:
+// the second leaves of its pairs in the reference's order into out (at most cap); the
+// stack is sstk[k][col]. Returns their number.
 template <int kRow, int kLds>
-__device__ __forceinline__ bool dfs_run(int nin, int me, int leaf, f3 mn, f3 mx,
-                                        const float4* __restrict__ nodes, int cap,
-                                        int2* __restrict__ out, long long limit,
-                                        long long budget, DfsState& st, uint32_t& w,
-                                        int (*sstk)[kRow], int col, int* __restrict__ spill) {
-  int node = st.node, top = st.top, ncol = st.ncol;
-  long long visits = st.visits;
-  bool done = true;
-  while (true) {
-    if (visits >= budget) {
-      done = false;
-      break;
-    }
+__device__ __forceinline__ int walk_exact(const WalkTree& T, int leaf, int root, f3 mn, f3 mx, int cap,
+                          int* __restrict__ out, uint32_t& w, int (*sstk)[kRow], int col,
+                          int* __restrict__ spill) {
+  const int nin = T.t - 1, me = nin + leaf;
+  const long long limit = 64ll * T.t + 4096;
+  int node = root, top = 0, ncol = 0;
+  for (long long visits = 0;;) {
     if (++visits > limit) {
       w |= CM_WARN_TRAVERSAL_LIMIT;
       break;
     }
-    // One 64-byte record per node: children, rightmost leaves, both child boxes.
-    // Both tests use & so that all four loads are issued together.
-    const float4* nd = nodes + 4 * (int64_t)node;
-    const float4 r0 = nd[0], r1 = nd[1], r2 = nd[2], r3 = nd[3];
-    const int l = __float_as_int(r0.x), r = __float_as_int(r0.y);
-    const int rml = __float_as_int(r0.z), rmr = __float_as_int(r0.w);
-    const bool ol = (rml > me) & overlap(mn, mx, mk3(r1.x, r1.y, r1.z), mk3(r1.w, r2.x, r2.y));
-    const bool orr = (rmr > me) & overlap(mn, mx, mk3(r2.z, r2.w, r3.x), mk3(r3.y, r3.z, r3.w));
+    const int l = T.lefts[node], r = T.rights[node];
+    const bool ol = (T.rmll[node] > me) & overlap(mn, mx, xyz(T.amin[l]), xyz(T.amax[l]));
+    const bool orr = (T.rmlr[node] > me) & overlap(mn, mx, xyz(T.amin[r]), xyz(T.amax[r]));
     const bool el = ol & (l >= nin), er = orr & (r >= nin);
-    if (el | er) {
-      // Past the cap the reference keeps walking but drops every further pair, so
-      // stopping at the first dropped pair yields the same list.
-      if (ncol + (int)el + (int)er > cap) {
-        if (el && ncol < cap) put_pair(out + ncol++, leaf, l - nin);
-        else if (er && ncol < cap) put_pair(out + ncol++, leaf, r - nin);
-        w |= CM_WARN_PAIR_CAP;
-        break;
-      }
-      if (el) put_pair(out + ncol++, leaf, l - nin);
-      if (er) put_pair(out + ncol++, leaf, r - nin);
+    // Past the cap the reference keeps walking but drops every further pair, so
+    // stopping at the first dropped pair yields the same list.
+    if (ncol + (int)el + (int)er > cap) {
+      if (el && ncol < cap) out[ncol++] = l - nin;
+      else if (er && ncol < cap) out[ncol++] = r - nin;
+      w |= CM_WARN_PAIR_CAP;
+      break;
     }
+    if (el) out[ncol++] = l - nin;
+    if (er) out[ncol++] = r - nin;
     const bool tl = ol & (l < nin), tr = orr & (r < nin);
     if (tl | tr) {
       node = tl ? l : r;
       if (tl & tr) {
-        if (top < kStack) {
+        if (top >= kStack) {
+          w |= CM_WARN_STACK_OVERFLOW;  // the push is dropped, as in the reference
+        } else {
           if constexpr (kLds < kStack) {
             if (top < kLds) sstk[top][col] = r;
             else spill[top - kLds] = r;
@@ -685,8 +656,6 @@ __device__ __forceinline__ bool dfs_run(int nin, int me, int leaf, f3 mn, f3 mx,
             sstk[top][col] = r;
           }
           ++top;
-        } else {
-          w |= CM_WARN_STACK_OVERFLOW;  // the push is dropped, as in the reference
         }
       }
     } else {
@@ -696,12 +665,184 @@ __device__ __forceinline__ bool dfs_run(int nin, int me, int leaf, f3 mn, f3 mx,
       else node = sstk[top][col];
     }
   }
-  st.node = node;
-  st.top = top;
-  st.ncol = ncol;
-  st.visits = visits;
-  return done;
+  return ncol;
 }
+
+// ---- the walk through quantised nodes ----------------------------------------------
+// The walk is bound by its instructions (nearly every branch is taken by some lane of a
+// wave) and, where the nodes outgrow an L2, by the bytes of its gathers. A node's record
+// is therefore 32 bytes, two loads:
+//   .x  split (bits 0-25; the children are split and split + 1, as the build lays them),
+//       bit 26 / 27: the left / right child is a leaf, bit 28: see .y
+//   .y  the right child's rightmost leaf; the left one's is split (of a node with two
+//       parents it can be another: then bit 28 is set and .y is the larger of the two)
+//   then three words per child: its box in 16 bits a bound, (min x, min y),
+//       (min z, 65535 - max x), (65535 - max y, 65535 - max z)
+// Bounds are quantised by one monotone function over the root's box, the leaf's own box
+// by the same one as (max x, max y), (max z, 65535 - min x), ..., so boxes that overlap
+// have no word larger than the leaf's: three saturating 16-bit subtractions, an or and a
+// compare. The test can pass boxes that do not overlap, so the leaves it finds are
+// candidates: their exact boxes are tested after the walk (by 8 at a time, off its chain
+// of loads), in order, and those that fail are dropped. The pairs and their order are
+// walk_exact's: where a node's box holds its children's (irr clear), a leaf whose exact
+// box passes has ancestors that pass. A walk that reaches the stack limit or the visit
+// limit is given up (kRedo) and done exactly.
+// k_traverse with what finishes its long walks, exact records of 64 bytes and pairs
+// stored as they are found -> now: flat 256^2 614 -> 353 us, draped 319 -> 331, draped
+// 131x97 217 -> 179, 64^2 134 -> 100, 2 M leaves 1,070 -> 815, crumpled 1024^2 1,825 ->
+// 1,860 (there 65 vector and 30 scalar instructions a visit at 43% of the lanes bound
+// it; refilling the lanes that finish early from a wave's queue of leaves was slower,
+// 2,320, as is stepping two levels at a time: 650 instructions a step, or loading both
+// children's records ahead).
+constexpr uint32_t kSplitMask = (1u << 26) - 1, kLeftLeaf = 1u << 26, kRightLeaf = 1u << 27,
+                   kOtherRight = 1u << 28;
+struct Quant {
+  f3 lo, scale;
+};
+__device__ __forceinline__ Quant quant_frame(float4 lo, float4 hi) {
+  auto sc = [](float a, float b) { return b > a ? 65535.f / (b - a) : 0.f; };
+  return {xyz(lo), mk3(sc(lo.x, hi.x), sc(lo.y, hi.y), sc(lo.z, hi.z))};
+}
+// monotone in v, whatever the frame (a frame without extent, or past the float range,
+// gives one value for all)
+__device__ __forceinline__ uint32_t q16(float v, float lo, float scale) {
+  return (uint32_t)fminf(fmaxf((v - lo) * scale, 0.f), 65535.f);
+}
+// the three words of a box; of the leaf's own box with min and max exchanged
+__device__ __forceinline__ uint3 q_box(Quant q, f3 mn, f3 mx) {
+  return make_uint3(q16(mn.x, q.lo.x, q.scale.x) | (q16(mn.y, q.lo.y, q.scale.y) << 16),
+                    q16(mn.z, q.lo.z, q.scale.z) | ((65535u - q16(mx.x, q.lo.x, q.scale.x)) << 16),
+                    (65535u - q16(mx.y, q.lo.y, q.scale.y)) |
+                        ((65535u - q16(mx.z, q.lo.z, q.scale.z)) << 16));
+}
+// per half: how far a is above b, 0 if it is not
+__device__ __forceinline__ uint32_t above16(uint32_t a, uint32_t b) {
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(us2, a),
+                                                                    __builtin_bit_cast(us2, b)));
+}
+__device__ __forceinline__ bool q_overlap(uint32_t a, uint32_t b, uint32_t c, uint3 q) {
+  return (above16(a, q.x) | above16(b, q.y) | above16(c, q.z)) == 0;
+}
+
+struct QNode {
+  int split;
+  bool l, r, lleaf, rleaf;  // child passes, child is a leaf
+};
+__device__ __forceinline__ QNode q_visit(const uint4* __restrict__ qnodes, int node, int leaf,
+                                         uint3 q) {
+  const uint4* p = (const uint4*)((const char*)qnodes + ((uint32_t)node << 5));
+  const uint4 a = p[0], b = p[1];
+  QNode n;
+  n.split = (int)(a.x & kSplitMask);
+  const int rml = (a.x & kOtherRight) ? (int)a.y : n.split;
+  n.l = (rml > leaf) & q_overlap(a.z, a.w, b.x, q);
+  n.r = ((int)a.y > leaf) & q_overlap(b.y, b.z, b.w, q);
+  n.lleaf = (a.x & kLeftLeaf) != 0;
+  n.rleaf = (a.x & kRightLeaf) != 0;
+  return n;
+}
+
+enum WalkEnd { kDone, kBudget, kRedo };
+// State of a walk between two visits: the node to visit next (-1: none), the pending
+// nodes (the last in tos, the one below it in row top - 1, the first in row 1), the
+// candidates or pairs written, the visits made
+struct WalkState {
+  int node, top, tos, n, visits;
+};
+
+// One visit: the node's leaf children that pass join the candidates cand[n][col], st goes
+// to the next node. The candidates are collected in LDS: a store to memory in the walk
+// would have each visit wait for it, as loads and stores share one counter. Returns
+// false when the stack limit is reached.
+template <int kRow>
+__device__ __forceinline__ bool quant_step(const uint4* __restrict__ qnodes, int leaf, uint3 q,
+                                           WalkState& st, int& n, int (*sstk)[kRow],
+                                           int (*cand)[kRow], int col, int* __restrict__ spill) {
+  bool fits = true;
+  ++st.visits;
+  const QNode v = q_visit(qnodes, st.node, leaf, q);
+  if (v.l & v.lleaf) cand[n++][col] = v.split;
+  if (v.r & v.rleaf) cand[n++][col] = v.split + 1;
+  const bool tl = v.l & !v.lleaf, tr = v.r & !v.rleaf;
+  if (tl & tr) {
+    if (st.top < kLdsStack) sstk[st.top][col] = st.tos;
+    else if (st.top < kStack) spill[st.top - kLdsStack] = st.tos;
+    else fits = false;
+    st.tos = v.split + 1;
+    ++st.top;
+  }
+  st.node = tl ? v.split : v.split + 1;
+  if (!(tl | tr)) {
+    st.node = st.top > 0 ? st.tos : -1;
+    st.top = max(st.top - 1, 0);
+    st.tos = sstk[min(st.top, kLdsStack - 1)][col];
+    if (st.top >= kLdsStack) st.tos = spill[st.top - kLdsStack];
+  }
+  return fits;
+}
+
+// The exact boxes of the n candidates, kVerify at a time: the second leaves of those that
+// pass go to out[m...), at most cap. Returns the pairs found, also past the cap.
+template <int kVerify, int kRow>
+__device__ __forceinline__ int verify(const WalkTree& T, f3 mn, f3 mx, int n, int m, int cap,
+                                      int* __restrict__ out, int (*cand)[kRow], int col) {
+  const int nin = T.t - 1;
+  for (int k = 0; k < n; k += kVerify) {
+    int c[kVerify];
+    float4 a[kVerify], b[kVerify];
+#pragma unroll
+    for (int u = 0; u < kVerify; ++u) {
+      c[u] = cand[min(k + u, n - 1)][col];
+      a[u] = T.amin[nin + c[u]];
+      b[u] = T.amax[nin + c[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < kVerify; ++u)
+      if (k + u < n && overlap(mn, mx, xyz(a[u]), xyz(b[u]))) {
+        if (m < cap) out[m] = c[u];
+        ++m;
+      }
+  }
+  return m;
+}
+
+__device__ __forceinline__ int visit_limit(int t) {
+  return (int)min(64ll * t + 4096, (long long)INT_MAX - 1);
+}
+
+// Walks on from st until it ends or `budget` visits were made; the second leaves of its
+// pairs go to out[0, st.n), at most cap.
+template <int kCand, int kVerify, int kRow>
+__device__ __forceinline__ WalkEnd walk_quant(const WalkTree& T, int leaf, f3 mn, f3 mx, uint3 q,
+                                              int cap, int* __restrict__ out, int budget,
+                                              WalkState& st, uint32_t& w, int (*sstk)[kRow],
+                                              int (*cand)[kRow], int col,
+                                              int* __restrict__ spill) {
+  const int limit = visit_limit(T.t);
+  const int bound = min(budget, limit);
+  for (;;) {
+    int n = 0;
+    const int room = min(kCand - 2, cap - st.n);  // past the cap one more is looked for
+    bool fits = true;
+    while (st.node >= 0 && st.visits < bound && n <= room && fits)
+      fits = quant_step(T.qnodes, leaf, q, st, n, sstk, cand, col, spill);
+    const int m = verify<kVerify>(T, mn, mx, n, st.n, cap, out, cand, col);
+    st.n = min(m, cap);
+    if (!fits) return kRedo;
+    if (m > cap) {  // the reference drops every pair past the cap
+      w |= CM_WARN_PAIR_CAP;
+      return kDone;
+    }
+    if (st.node < 0) return kDone;
+    if (st.visits >= bound) return st.visits >= limit ? kRedo : kBudget;
+  }
+}
+
+// The first pass's budget is given in exact visits; quantised ones are cheaper, and 1.7
+// for one give the shortest two passes (draped 256^2: 342 us at 200 visits, 331 at 340,
+// 362 at 400; flat 256^2: 500, 353, 320).
+constexpr int quant_budget(int budget) { return budget + budget * 7 / 10; }
 
 // A leaf whose walk outlasts the first pass's visit budget leaves its state in a
 // record of kRec ints: leaf, pairs written, stack depth, next node, cap, visits, then
@@ -709,89 +850,99 @@ __device__ __forceinline__ bool dfs_run(int nin, int me, int leaf, f3 mn, f3 mx,
 constexpr int kRec = kTravRec;
 static_assert(kRec >= 6 + kStack, "record holds the stack");
 
+template <int kRow>
+__device__ __forceinline__ void put_record(int* __restrict__ R, int leaf, int cap,
+                                           const WalkState& st, int (*sstk)[kRow], int col,
+                                           const int* __restrict__ spill) {
+  R[0] = leaf;
+  R[1] = st.n;
+  R[2] = st.top;
+  R[3] = st.node;
+  R[4] = cap;
+  R[5] = st.visits;
+  for (int k = 1; k <= st.top; ++k)
+    R[5 + k] = k == st.top ? st.tos : (k < kLdsStack ? sstk[k][col] : spill[k - kLdsStack]);
+}
+
 // First pass: one lane per leaf, at most `budget` visits (no budget: budget <= 0 or
 // no record buffer). A leaf still walking then takes a record slot, if one is left,
 // and counts zero pairs here; past the slots it walks on to the end.
-__global__ void __launch_bounds__(kTravBlock) k_traverse(int t, const float4* __restrict__ nodes,
-                                                         const float4* __restrict__ amin,
-                                                         const float4* __restrict__ amax, int cap,
-                                                         int2* __restrict__ chunk,
+template <int kCand, int kVerify>
+__global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap,
+                                                         int* __restrict__ chunk,
                                                          int* __restrict__ counts,
                                                          uint32_t* __restrict__ warn,
-                                                         const int* __restrict__ slot_cloth,
-                                                         const int* __restrict__ croot,
-                                                         const int* __restrict__ ccap,
                                                          int* __restrict__ tile_sum,
                                                          int xchunk, int budget,
                                                          int* __restrict__ rec, int rcap,
                                                          int* __restrict__ hctl,
                                                          int* __restrict__ spill) {
-  // Entry k of every lane's stack is one row, so a wave's pushes and pops at equal
+  // Row k of every lane's stack is one LDS row, so a wave's pushes and pops at equal
   // depths hit 64 consecutive banks.
-  __shared__ int sstk[kLdsStack][kTravBlock];
+  __shared__ int sstk[kLdsStack][kTravBlock], cand[kCand][kTravBlock];
   // Workgroups are dealt to the 8 XCDs in turn. Each XCD takes every eighth chunk of
   // `xchunk` consecutive tiles (Morton-ordered leaves), so its L2 serves compact
   // subtrees while the dense regions of the cloth, whose leaves visit many more
   // nodes, are shared evenly between the XCDs. The grid is padded to whole rounds.
   const int j = blockIdx.x / kXcds, xcd = blockIdx.x % kXcds;
   const int tile = ((j / xchunk) * kXcds + xcd) * xchunk + j % xchunk;
+  const int t = T.t;
   if (tile >= (t + kTravBlock - 1) / kTravBlock) return;
   const int leaf = tile * kTravBlock + threadIdx.x;
-  int ncol = 0;
   const int stride = cap;  // every leaf's chunk holds the body's cap (a cloth's may be less)
   uint32_t w = 0;
-  const int nin = t - 1;
-  const int me = nin + leaf;
-  DfsState st{0, 0, 0, 0};  // root (a batch: the root of the leaf's cloth, its cap)
+  const int me = t - 1 + leaf;
+  int root = 0, ncol = 0;
   bool walk = leaf < t;
-  if (walk && croot) {
-    const int c = slot_cloth[leaf];
-    st.node = croot[c];
-    cap = ccap[c];
-    walk = st.node >= 0;  // a one-triangle cloth has no pairs
+  if (walk && T.croot) {  // a batch: the root of the leaf's cloth, its cap
+    const int c = T.slot_cloth[leaf];
+    root = T.croot[c];
+    cap = T.ccap[c];
+    walk = root >= 0;  // a one-triangle cloth has no pairs
   }
-  f3 mn = mk3(0, 0, 0), mx = mk3(0, 0, 0);
-  int2* out = chunk + (int64_t)leaf * stride;
+  int* out = chunk + (int64_t)leaf * stride;
   int* sp = spill + (int64_t)leaf * kSpill;
-  const long long limit = 64ll * t + 4096;
-  bool done = true;
+  f3 mn = mk3(0, 0, 0), mx = mk3(0, 0, 0);
+  uint3 q = make_uint3(0, 0, 0);
+  WalkState st{root, 0, 0, 0, 0};
+  WalkEnd end = kDone;
   if (walk) {
-    mn = xyz(amin[me]);
-    mx = xyz(amax[me]);
-    const bool budgeted = budget > 0 && rec;
-    done = dfs_run<kTravBlock, kLdsStack>(nin, me, leaf, mn, mx, nodes, cap, out, limit,
-                                          budgeted ? (long long)budget : LLONG_MAX, st, w, sstk,
-                                          threadIdx.x, sp);
+    mn = xyz(T.amin[me]);
+    mx = xyz(T.amax[me]);
+    end = kRedo;
+    if (T.qnodes && *T.irr == 0) {
+      q = q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn);
+      end = walk_quant<kCand, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out,
+                                   budget > 0 && rec ? budget : INT_MAX, st, w, sstk, cand,
+                                   threadIdx.x, sp);
+    }
   }
   // Leaves still walking claim record slots with one atomic per wave (thousands of
   // lanes on one counter would queue at its L2 channel).
   const int lane = threadIdx.x & 63;
-  const uint64_t want = __ballot(!done);
+  const uint64_t want = __ballot(end == kBudget);
   bool handed = false;
   if (want) {
     int base = 0;
     if (lane == 0) base = atomicAdd(hctl, __popcll(want));
     base = __shfl(base, 0, 64);
-    if (!done) {
+    if (end == kBudget) {
       const int slot = base + __popcll(want & ((1ull << lane) - 1));
       if (slot < rcap) {
-        int* R = rec + (int64_t)slot * kRec;
-        R[0] = leaf;
-        R[1] = st.ncol;
-        R[2] = st.top;
-        R[3] = st.node;
-        R[4] = cap;
-        R[5] = (int)st.visits;
-        for (int k = 0; k < st.top; ++k)
-          R[6 + k] = k < kLdsStack ? sstk[k][threadIdx.x] : sp[k - kLdsStack];
+        put_record(rec + (int64_t)slot * kRec, leaf, cap, st, sstk, threadIdx.x, sp);
         handed = true;
       } else {
-        dfs_run<kTravBlock, kLdsStack>(nin, me, leaf, mn, mx, nodes, cap, out, limit, LLONG_MAX,
-                                       st, w, sstk, threadIdx.x, sp);
+        end = walk_quant<kCand, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out, INT_MAX, st, w, sstk,
+                                     cand, threadIdx.x, sp);
       }
     }
   }
-  if (walk) ncol = handed ? 0 : st.ncol;
+  if (walk) ncol = handed ? 0 : st.n;
+  if (end == kRedo) {
+    w = 0;
+    ncol = walk_exact<kTravBlock, kLdsStack>(T, leaf, root, mn, mx, cap, out, w, sstk,
+                                             threadIdx.x, sp);
+  }
   if (leaf < t) counts[leaf] = ncol;
   // one warning atomic per wave: two thirds of the leaves of a draped cloth hit the cap
 #pragma unroll
@@ -806,7 +957,7 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(int t, const float4* __
   __syncthreads();
   if (threadIdx.x == 0) {
     int tot = 0;
-    for (int q = 0; q < kTravBlock / 64; ++q) tot += wsum[q];
+    for (int k = 0; k < kTravBlock / 64; ++k) tot += wsum[k];
     tile_sum[tile] = tot;
   }
 }
@@ -815,7 +966,8 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(int t, const float4* __
 // The reference's DFS visits nodes in preorder and emits a node's left leaf child
 // before its right one, so a pair's place in the leaf's list is the preorder place of
 // the node that emits it. The wave expands up to 64 pending nodes at once, in any
-// order, and tags every pair with a 64-bit key that sorts in that preorder:
+// order, and tags every pair (a candidate whose exact box passes) with a 64-bit key
+// that sorts in that preorder:
 //   bits 63..58  rank of the pending subtree handed over (0 = the next node to visit,
 //                then the stack entries from the top down: they are visited in that
 //                order, each subtree before the next)
@@ -827,12 +979,9 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(int t, const float4* __
 // right one. Pending nodes are kept sorted by key (the smallest on top), so every pair
 // below the top pending node's key is final. The wave stops once more than the
 // remaining cap of pairs are final: the first `cap` are the leaf's list and one more
-// means the reference dropped pairs (CM_WARN_PAIR_CAP). A push the reference would
-// drop (stack full) is mirrored by tracking each pending node's stack depth: a node
-// whose children are both walked at depth kStack loses its right child, and
-// CM_WARN_STACK_OVERFLOW is raised when such a node precedes the point where the
-// reference's walk stopped. A leaf that overflows this pass's buffers or path bits,
-// or could reach the visit limit, is walked by lane 0 alone from its record.
+// means the reference dropped pairs (CM_WARN_PAIR_CAP). A leaf that overflows this
+// pass's buffers or path bits, or could reach the stack limit (each pending node
+// carries its stack depth) or the visit limit, is walked exactly by lane 0 alone.
 constexpr int kPend = 512;     // pending nodes per leaf
 constexpr int kHits = 256;     // pairs kept per leaf
 constexpr int kPathBits = 50;
@@ -863,10 +1012,8 @@ __device__ __forceinline__ int wave_sum(int v) {
 // at once.
 constexpr int kLaneModeMin = 16384;
 
-__global__ void __launch_bounds__(64) k_traverse_resume(int t, const float4* __restrict__ nodes,
-                                                        const float4* __restrict__ amin,
-                                                        const float4* __restrict__ amax,
-                                                        int2* __restrict__ chunk, int stride,
+__global__ void __launch_bounds__(64) k_traverse_resume(WalkTree T,
+                                                        int* __restrict__ chunk, int stride,
                                                         int* __restrict__ counts,
                                                         uint32_t* __restrict__ warn,
                                                         int* __restrict__ tile_sum,
@@ -877,10 +1024,9 @@ __global__ void __launch_bounds__(64) k_traverse_resume(int t, const float4* __r
   __shared__ uint64_t hk[kHits];
   __shared__ int hp[kHits];
   __shared__ int fstk[kStack][1];
-  __shared__ unsigned long long s_ovf, s_stop;
   const int lane = threadIdx.x;
-  const int nin = t - 1;
-  const long long limit = 64ll * t + 4096;
+  const int nin = T.t - 1;
+  const long long limit = 64ll * T.t + 4096;
   const int nres = min(hctl[0], rcap);
   if (nres > kLaneModeMin) return;  // k_traverse_lanes takes them
   uint32_t wacc = 0;
@@ -888,19 +1034,15 @@ __global__ void __launch_bounds__(64) k_traverse_resume(int t, const float4* __r
     const int* R = rec + (int64_t)rid * kRec;
     const int leaf = R[0], ncol0 = R[1], top0 = R[2], cur = R[3], cap = R[4];
     const long long visits0 = R[5];
-    const int me = nin + leaf;
-    const f3 mn = xyz(amin[me]), mx = xyz(amax[me]);
+    const f3 mn = xyz(T.amin[nin + leaf]), mx = xyz(T.amax[nin + leaf]);
+    const uint3 q = q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn);
     const int capr = cap - ncol0;  // pairs still to find (0: only whether one more exists)
-    int2* out = chunk + (int64_t)leaf * stride;
+    int* out = chunk + (int64_t)leaf * stride;
     // pending: the stack entries bottom-up, then the next node on top
     const int m = top0 + 1;
     for (int k = lane; k < m; k += 64) {
       pe[k] = (k < top0 ? R[6 + k] : cur) | (k << 26);  // visited at stack depth k
       pk[k] = (uint64_t)(top0 - k) << 58;
-    }
-    if (lane == 0) {
-      s_ovf = ~0ull;
-      s_stop = ~0ull;
     }
     __syncthreads();
     int np = m, nh = 0;
@@ -913,9 +1055,9 @@ __global__ void __launch_bounds__(64) k_traverse_resume(int t, const float4* __r
       int node = 0, sd = 0;
       uint64_t key = 0;
       if (act) {
-        const int e = pe[np - 1 - lane];
-        node = e & 0x3ffffff;
-        sd = e >> 26;
+        const uint32_t e = (uint32_t)pe[np - 1 - lane];
+        node = (int)(e & kSplitMask);
+        sd = (int)(e >> 26);
         key = pk[np - 1 - lane];
       }
       __syncthreads();
@@ -924,39 +1066,34 @@ __global__ void __launch_bounds__(64) k_traverse_resume(int t, const float4* __r
       uint64_t ck[2] = {0, 0}, ek[2] = {0, 0};
       bool deep = false;
       if (act) {
-        const float4* nd = nodes + 4 * (int64_t)node;
-        const float4 r0 = nd[0], r1 = nd[1], r2 = nd[2], r3 = nd[3];
-        const int l = __float_as_int(r0.x), r = __float_as_int(r0.y);
-        const int rml = __float_as_int(r0.z), rmr = __float_as_int(r0.w);
-        const bool ol = (rml > me) & overlap(mn, mx, mk3(r1.x, r1.y, r1.z), mk3(r1.w, r2.x, r2.y));
-        const bool orr =
-            (rmr > me) & overlap(mn, mx, mk3(r2.z, r2.w, r3.x), mk3(r3.y, r3.z, r3.w));
-        if (ol & (l >= nin)) {
+        const QNode v = q_visit(T.qnodes, node, leaf, q);
+        auto passes = [&](int c) {
+          return overlap(mn, mx, xyz(T.amin[nin + c]), xyz(T.amax[nin + c]));
+        };
+        const bool el = (v.l & v.lleaf) && passes(v.split);
+        const bool er = (v.r & v.rleaf) && passes(v.split + 1);
+        if (el) {
           ek[ne] = key;
-          ep[ne++] = l - nin;
+          ep[ne++] = v.split;
         }
-        if (orr & (r >= nin)) {
+        if (er) {
           ek[ne] = key | 1ull;
-          ep[ne++] = r - nin;
+          ep[ne++] = v.split + 1;
         }
-        const bool tl = ol & (l < nin), tr = orr & (r < nin);
+        const bool tl = v.l & !v.lleaf, tr = v.r & !v.rleaf;
         if (tl | tr) {
           const int d = (int)((key >> 1) & 127ull);
-          if (d + 1 > kPathBits) deep = true;
+          const bool both = tl & tr;
+          if (d + 1 > kPathBits || (both && sd >= kStack)) deep = true;
           const uint64_t kl = (key & ~0xffull) | ((uint64_t)(d + 1) << 1);
           const uint64_t kr = kl | (1ull << (57 - d));
-          const bool both = tl & tr;
           if (tl) {
-            ce[nc] = l | ((both && sd < kStack ? sd + 1 : sd) << 26);
+            ce[nc] = v.split | ((both ? sd + 1 : sd) << 26);
             ck[nc++] = kl;
           }
           if (tr) {
-            if (both && sd >= kStack) {
-              atomicMin(&s_ovf, (unsigned long long)key);
-            } else {
-              ce[nc] = r | (sd << 26);
-              ck[nc++] = kr;
-            }
+            ce[nc] = (v.split + 1) | (sd << 26);
+            ck[nc++] = kr;
           }
         }
       }
@@ -1020,11 +1157,8 @@ __global__ void __launch_bounds__(64) k_traverse_resume(int t, const float4* __r
       __syncthreads();
       nout = 0;
       if (lane == 0) {
-        for (int k = 0; k < top0; ++k) fstk[k][0] = R[6 + k];
-        DfsState st{cur, top0, ncol0, visits0};
-        dfs_run<1, kStack>(nin, me, leaf, mn, mx, nodes, cap, out, limit, LLONG_MAX, st, w, fstk,
-                           0, nullptr);
-        nout = st.ncol;
+        const int root = T.croot ? T.croot[T.slot_cloth[leaf]] : 0;
+        nout = walk_exact<1, kStack>(T, leaf, root, mn, mx, cap, out, w, fstk, 0, nullptr);
       }
     } else {
       // each pair's place is the number of smaller keys (keys are distinct)
@@ -1032,13 +1166,11 @@ __global__ void __launch_bounds__(64) k_traverse_resume(int t, const float4* __r
         const uint64_t ki = hk[i];
         int rank = 0;
         for (int j2 = 0; j2 < nh; ++j2) rank += hk[j2] < ki;
-        if (rank < capr) put_pair(out + ncol0 + rank, leaf, hp[i]);
-        if (rank == capr) s_stop = ki & ~1ull;  // the node where the reference stopped
+        if (rank < capr) out[ncol0 + rank] = hp[i];
       }
       __syncthreads();
       nout = ncol0 + min(nh, capr);
       if (nh > capr) w |= CM_WARN_PAIR_CAP;
-      if (s_ovf != ~0ull && s_ovf < s_stop) w |= CM_WARN_STACK_OVERFLOW;
     }
     if (lane == 0) {
       counts[leaf] = nout;
@@ -1054,35 +1186,43 @@ __global__ void __launch_bounds__(64) k_traverse_resume(int t, const float4* __r
 
 // Second pass when there are more than kLaneModeMin records: one lane per record
 // walks on serially from the record's state (next node, stack, pairs written,
-// visits), exactly as the first pass would have without a budget.
+// visits), as the first pass would have without a budget.
+template <int kCand, int kVerify>
 __global__ void __launch_bounds__(kTravBlock) k_traverse_lanes(
-    int t, const float4* __restrict__ nodes, const float4* __restrict__ amin,
-    const float4* __restrict__ amax, int2* __restrict__ chunk, int stride,
-    int* __restrict__ counts, uint32_t* __restrict__ warn, int* __restrict__ tile_sum,
-    const int* __restrict__ rec, int rcap, const int* __restrict__ hctl,
-    int* __restrict__ spill) {
-  __shared__ int sstk[kLdsStack][kTravBlock];
+    WalkTree T, int* __restrict__ chunk, int stride, int* __restrict__ counts,
+    uint32_t* __restrict__ warn, int* __restrict__ tile_sum, const int* __restrict__ rec, int rcap,
+    const int* __restrict__ hctl, int* __restrict__ spill) {
+  __shared__ int sstk[kLdsStack][kTravBlock], cand[kCand][kTravBlock];
   const int nres = min(hctl[0], rcap);
   if (nres <= kLaneModeMin) return;  // k_traverse_resume takes them
-  const int nin = t - 1;
-  const long long limit = 64ll * t + 4096;
+  const int nin = T.t - 1;
   uint32_t w = 0;
   for (int rid = blockIdx.x * kTravBlock + threadIdx.x; rid < nres;
        rid += gridDim.x * kTravBlock) {
     const int* R = rec + (int64_t)rid * kRec;
-    const int leaf = R[0], top0 = R[2];
-    const int me = nin + leaf;
+    const int leaf = R[0], top = R[2], cap = R[4];
     int* sp = spill + (int64_t)leaf * kSpill;
-    for (int k = 0; k < top0; ++k) {
-      if (k < kLdsStack) sstk[k][threadIdx.x] = R[6 + k];
-      else sp[k - kLdsStack] = R[6 + k];
+    int* out = chunk + (int64_t)leaf * stride;
+    for (int k = 1; k < top; ++k) {
+      if (k < kLdsStack) sstk[k][threadIdx.x] = R[5 + k];
+      else sp[k - kLdsStack] = R[5 + k];
     }
-    DfsState st{R[3], top0, R[1], (long long)R[5]};
-    dfs_run<kTravBlock, kLdsStack>(nin, me, leaf, xyz(amin[me]), xyz(amax[me]), nodes, R[4],
-                                   chunk + (int64_t)leaf * stride, limit, LLONG_MAX, st, w, sstk,
-                                   threadIdx.x, sp);
-    counts[leaf] = st.ncol;
-    atomicAdd(&tile_sum[leaf / kTravBlock], st.ncol);
+    const f3 mn = xyz(T.amin[nin + leaf]), mx = xyz(T.amax[nin + leaf]);
+    WalkState st{R[3], top, top > 0 ? R[5 + top] : 0, R[1], R[5]};
+    uint32_t wl = 0;
+    int ncol;
+    if (walk_quant<kCand, kVerify, kTravBlock>(T, leaf, mn, mx, q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn),
+                               cap, out, INT_MAX, st, wl, sstk, cand, threadIdx.x, sp) == kRedo) {
+      wl = 0;
+      const int root = T.croot ? T.croot[T.slot_cloth[leaf]] : 0;
+      ncol = walk_exact<kTravBlock, kLdsStack>(T, leaf, root, mn, mx, cap, out, wl, sstk,
+                                               threadIdx.x, sp);
+    } else {
+      ncol = st.n;
+    }
+    w |= wl;
+    counts[leaf] = ncol;
+    atomicAdd(&tile_sum[leaf / kTravBlock], ncol);
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) w |= __shfl_xor(w, o, 64);
@@ -1093,30 +1233,53 @@ __global__ void k_clear_records(int* __restrict__ hctl) {
   if (threadIdx.x == 0) hctl[0] = 0;
 }
 
-// packed node records from separate arrays (unit-level pair query)
+// box b lies in box a (false when a bound is NaN)
+__device__ __forceinline__ bool holds(f3 amn, f3 amx, f3 bmn, f3 bmx) {
+  return amn.x <= bmn.x && amn.y <= bmn.y && amn.z <= bmn.z && amx.x >= bmx.x &&
+         amx.y >= bmx.y && amx.z >= bmx.z;
+}
+// The quantised node records, and whether they can be walked: every node's box has to
+// hold its children's. kCaller (unit-level pair query, the caller's own tree): also its
+// children have to lie side by side as the build lays them, and its rightmost leaves
+// must not shrink upwards.
+template <bool kCaller>
 __global__ void __launch_bounds__(kBlock) k_pack_nodes(int t, const int* __restrict__ lefts,
                                                        const int* __restrict__ rights,
                                                        const float4* __restrict__ amin,
                                                        const float4* __restrict__ amax,
                                                        const int* __restrict__ rmll,
                                                        const int* __restrict__ rmlr,
-                                                       float4* __restrict__ nodes) {
-  const int q = blockIdx.x * kBlock + threadIdx.x;
-  if (q >= t - 1) return;
-  const int l = lefts[q], r = rights[q];
-  write_node(nodes, q, l, r, rmll[q], rmlr[q], xyz(amin[l]), xyz(amax[l]), xyz(amin[r]),
-             xyz(amax[r]));
+                                                       uint4* __restrict__ qnodes,
+                                                       int* __restrict__ irr) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const int nin = t - 1;
+  if (i >= nin) return;
+  const int l = lefts[i], r = rights[i], a = rmll[i], b = rmlr[i];
+  const f3 lmn = xyz(amin[l]), lmx = xyz(amax[l]), rmn = xyz(amin[r]), rmx = xyz(amax[r]);
+  const f3 mn = xyz(amin[i]), mx = xyz(amax[i]);
+  const bool ll = l >= nin, rl = r >= nin;
+  const int sp = ll ? l - nin : l;
+  bool ok = holds(mn, mx, lmn, lmx) && holds(mn, mx, rmn, rmx);
+  if (kCaller && ok)
+    ok = sp + 1 == (rl ? r - nin : r) && (ll ? a == l : a >= max(rmll[l], rmlr[l])) &&
+         (rl ? b == r : b >= max(rmll[r], rmlr[r]));
+  if (!ok) atomicOr(irr, 1);
+  const Quant q = quant_frame(amin[0], amax[0]);
+  const uint3 bl = q_box(q, lmn, lmx), br = q_box(q, rmn, rmx);
+  const bool other = a != nin + sp;
+  qnodes[2 * (int64_t)i] =
+      make_uint4((uint32_t)sp | (ll ? kLeftLeaf : 0u) | (rl ? kRightLeaf : 0u) |
+                     (other ? kOtherRight : 0u),
+                 (uint32_t)((other ? max(a, b) : b) - nin), bl.x, bl.y);
+  qnodes[2 * (int64_t)i + 1] = make_uint4(bl.z, br.x, br.y, br.z);
 }
 
-// One wave per leaf copies its chunk to the compacted list. The leaf's offset is its
-// tile's prefix plus the counts of the tile's earlier leaves (at most 127, summed by
-// the wave).
 // One workgroup per traversal tile of kTravBlock leaves: the first wave scans the
 // leaves' counts, then the workgroup writes the tile's pairs in order, kBlock
 // consecutive output slots at a time (each thread finds its slot's leaf by binary
 // search over the tile's prefixes), so reads and writes are contiguous runs.
-__global__ void __launch_bounds__(kBlock) k_compact_pairs(int t, int cap,
-                                                          const int2* __restrict__ chunk,
+__global__ void __launch_bounds__(kBlock) k_compact_pairs(int t, int stride,
+                                                          const int* __restrict__ chunk,
                                                           const int* __restrict__ counts,
                                                           const int* __restrict__ tile_pre,
                                                           int2* __restrict__ pairs,
@@ -1152,7 +1315,7 @@ __global__ void __launch_bounds__(kBlock) k_compact_pairs(int t, int cap,
       if (pre[mid] <= k) lo = mid;
       else hi = mid - 1;
     }
-    pairs[out0 + k] = chunk[(int64_t)(l0 + lo) * cap + (k - pre[lo])];
+    pairs[out0 + k] = make_int2(l0 + lo, chunk[(int64_t)(l0 + lo) * stride + (k - pre[lo])]);
   }
 }
 
@@ -1228,7 +1391,7 @@ int launch_build(const LbvhBufs& b, const uint64_t* keys, int midpoint, hipStrea
   const int t = b.t;
   if (t < 2) return CM_OK;
   hipLaunchKernelGGL(k_build_init, dim3(nblocks(std::max(2 * t - 1, b.ncloth))), dim3(kBlock), 0,
-                     s, t, b.claim_cnt, b.claim_hi, b.ntop, b.ncloth, b.croot);
+                     s, t, b.claim_cnt, b.claim_hi, b.ntop, b.irr, b.ncloth, b.croot);
   hipLaunchKernelGGL(k_build, dim3(nblocks(t - 1)), dim3(kBlock), 0, s, t, keys, midpoint, b.lefts,
                      b.rights, b.claim_cnt, b.claim_hi, b.ranges, b.warn,
                      b.ncloth ? b.tstart : nullptr, b.croot);
@@ -1242,47 +1405,60 @@ int launch_refit(const LbvhBufs& b, hipStream_t s) {
   const int t = b.t;
   if (t < 2) return CM_OK;
   hipLaunchKernelGGL(k_refit_local, dim3((t + kRefitCH - 1) / kRefitCH), dim3(kRefitCH), 0, s, t,
-                     b.lefts, b.rights, b.ranges, b.amin, b.amax, b.rmll, b.rmlr, b.nodes, b.state,
+                     b.lefts, b.rights, b.ranges, b.amin, b.amax, b.rmll, b.rmlr, b.state,
                      b.top_list, b.top_index, b.ntop, b.tdone);
   if (t > 2 * kSuper)  // smaller trees defer at most a few hundred nodes
     hipLaunchKernelGGL(k_refit_mid, dim3((t + kSuper - 1) / kSuper), dim3(1024), 0, s, t, b.lefts,
-                       b.rights, b.ranges, b.amin, b.amax, b.rmll, b.rmlr, b.nodes, b.state,
+                       b.rights, b.ranges, b.amin, b.amax, b.rmll, b.rmlr, b.state,
                        b.top_list, b.top_index, b.ntop, b.tmin, b.tmax, b.trm, b.tdone);
   hipLaunchKernelGGL(k_refit_top, dim3(1), dim3(1024), 0, s, t, b.lefts, b.rights, b.amin, b.amax,
-                     b.rmll, b.rmlr, b.nodes, b.state, b.top_list, b.top_index, b.ntop, b.tmin,
-                     b.tmax, b.trm, b.tdone, b.warn);
+                     b.rmll, b.rmlr, b.state, b.top_list, b.top_index, b.ntop, b.tmin,
+                     b.tmax, b.trm, b.tdone, b.warn, b.irr);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
 
-// both traversal passes (the second only with a budget and record buffers)
-static int launch_traverse(const LbvhBufs& b, int cap, int2* chunk, int* counts, int* offsets,
+// Candidates a lane collects before it tests them, and how many it tests at a time: trees
+// of up to kFewLeaves leaves put at most two waves on a SIMD, so LDS and registers are
+// free, and each walk that stops to test holds up its wave (k_traverse, 66 by 8 against
+// 24 by 4: 64^2 90 against 120 us, 131x97 121 against 196); larger ones need the waves
+// (2 M leaves: 815 us with 16 by 4, 855 with 24 by 4, 1,370 with 66 by 4).
+constexpr int kFewLeaves = 1 << 18;
+
+// the second pass needs a budget, record buffers and quantised nodes
+static bool two_passes(const LbvhBufs& b) {
+  return b.t < kQuantLeaves && b.trav_budget > 0 && b.trec && b.hctl && b.rcap > 0;
+}
+
+static int launch_traverse(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offsets,
                            hipStream_t s) {
   const int t = b.t;
   const int nt = (t + kTravBlock - 1) / kTravBlock;
   const int xchunk = b.trav_chunk > 0 ? b.trav_chunk : 4;
   const int round = kXcds * xchunk;
-  const bool two = b.trav_budget > 0 && b.trec && b.hctl && b.rcap > 0;
-  hipLaunchKernelGGL(k_traverse, dim3((nt + round - 1) / round * round), dim3(kTravBlock), 0, s, t,
-                     b.nodes, b.amin, b.amax,
-                     cap, chunk, counts, b.warn, b.ncloth ? b.slot_cloth : nullptr,
-                     b.ncloth ? b.croot : nullptr, b.ccap, offsets, xchunk,
-                     two ? b.trav_budget : 0, two ? b.trec : nullptr, b.rcap, b.hctl, b.spill);
+  const bool two = two_passes(b);
+  const WalkTree T{t,      t < kQuantLeaves ? b.qnodes : nullptr, b.irr, b.lefts, b.rights, b.rmll,
+                   b.rmlr, b.amin, b.amax, b.ncloth ? b.slot_cloth : nullptr,
+                   b.ncloth ? b.croot : nullptr, b.ccap};
+  const bool few = t <= kFewLeaves;
+  hipLaunchKernelGGL((few ? k_traverse<66, 8> : k_traverse<16, 4>),
+                     dim3((nt + round - 1) / round * round), dim3(kTravBlock), 0, s, T, cap, chunk,
+                     counts, b.warn, offsets, xchunk, two ? quant_budget(b.trav_budget) : 0,
+                     two ? b.trec : nullptr, b.rcap, b.hctl, b.spill);
   if (two) {  // one of the two finishes the records, the other returns at once
-    hipLaunchKernelGGL(k_traverse_resume, dim3(std::min(b.rcap, kResumeBlocks)), dim3(64), 0, s,
-                       t, b.nodes, b.amin, b.amax, chunk, cap, counts, b.warn, offsets, b.trec,
-                       b.rcap, b.hctl);
+    hipLaunchKernelGGL(k_traverse_resume, dim3(std::min(b.rcap, kResumeBlocks)), dim3(64), 0, s, T,
+                       chunk, cap, counts, b.warn, offsets, b.trec, b.rcap, b.hctl);
     if (b.rcap > kLaneModeMin)
-      hipLaunchKernelGGL(k_traverse_lanes,
+      hipLaunchKernelGGL((few ? k_traverse_lanes<66, 8> : k_traverse_lanes<16, 4>),
                          dim3(std::min((b.rcap + kTravBlock - 1) / kTravBlock, 8192)),
-                         dim3(kTravBlock), 0, s, t, b.nodes, b.amin, b.amax, chunk, cap, counts,
-                         b.warn, offsets, b.trec, b.rcap, b.hctl, b.spill);
+                         dim3(kTravBlock), 0, s, T, chunk, cap, counts, b.warn, offsets, b.trec,
+                         b.rcap, b.hctl, b.spill);
   }
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
 
-int launch_pairs(const LbvhBufs& b, int cap, int2* chunk, int* counts, int* offsets, int2* pairs,
+int launch_pairs(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offsets, int2* pairs,
                  int* d_npairs, void* scan_temp, hipStream_t s) {
   const int t = b.t;
   if (t < 2) return fill_i32(d_npairs, 0, 1, s);
@@ -1294,28 +1470,28 @@ int launch_pairs(const LbvhBufs& b, int cap, int2* chunk, int* counts, int* offs
   rc = scan_tiles(nullptr, 1, nt, offsets, offsets + nt, 0, (int64_t)t * cap, 0, d_npairs,
                   nullptr, scan_temp, s);
   if (rc) return rc;
-  const bool two = b.trav_budget > 0 && b.trec && b.hctl && b.rcap > 0;
-  hipLaunchKernelGGL(k_compact_pairs, dim3(nt), dim3(kBlock), 0, s, t, cap, chunk, counts,
-                     offsets + nt, pairs, two ? b.hctl : nullptr);
+  hipLaunchKernelGGL(k_compact_pairs, dim3(nt), dim3(kBlock), 0, s, t, cap, chunk,
+                     counts, offsets + nt, pairs, two_passes(b) ? b.hctl : nullptr);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
 
-int launch_traverse_only(const LbvhBufs& b, int cap, int2* chunk, int* counts, int* offsets,
+int launch_traverse_only(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offsets,
                          hipStream_t s) {
   if (b.t < 2) return CM_OK;
   const int rc = launch_traverse(b, cap, chunk, counts, offsets, s);
-  if (rc || !(b.trav_budget > 0 && b.trec && b.hctl && b.rcap > 0)) return rc;
+  if (rc || !two_passes(b)) return rc;
   hipLaunchKernelGGL(k_clear_records, dim3(1), dim3(64), 0, s, b.hctl);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
 
-int launch_pack_nodes(const LbvhBufs& b, hipStream_t s) {
+int launch_pack_nodes(const LbvhBufs& b, bool from_caller, hipStream_t s) {
   const int t = b.t;
-  if (t < 2) return CM_OK;
-  hipLaunchKernelGGL(k_pack_nodes, dim3(nblocks(t - 1)), dim3(kBlock), 0, s, t, b.lefts, b.rights,
-                     b.amin, b.amax, b.rmll, b.rmlr, b.nodes);
+  if (t < 2 || t >= kQuantLeaves) return CM_OK;
+  hipLaunchKernelGGL(from_caller ? k_pack_nodes<true> : k_pack_nodes<false>, dim3(nblocks(t - 1)),
+                     dim3(kBlock), 0, s, t, b.lefts, b.rights, b.amin, b.amax, b.rmll, b.rmlr,
+                     b.qnodes, b.irr);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
@@ -1358,8 +1534,9 @@ size_t carve_build(int t, void* d_temp, LbvhBufs* b) {
   take(&o->top_list, sizeof(int) * tt);
   take(&o->top_index, sizeof(int) * tt);
   take(&o->ntop, sizeof(int));
+  take(&o->irr, sizeof(int));
   take(&o->ranges, sizeof(int2) * tt);
-  take(&o->nodes, 4 * sizeof(float4) * tt);
+  take(&o->qnodes, 2 * sizeof(uint4) * tt);
   take(&o->tmin, sizeof(float4) * tt);
   take(&o->tmax, sizeof(float4) * tt);
   take(&o->trm, sizeof(int) * tt);
@@ -1369,9 +1546,9 @@ size_t carve_build(int t, void* d_temp, LbvhBufs* b) {
 
 size_t lbvh_build_temp_bytes(int t) { return carve_build(t, nullptr, nullptr); }
 size_t lbvh_pairs_temp_bytes(int t, int cap) {
-  return align_up(sizeof(int2) * (size_t)t * cap) + 2 * align_up(sizeof(int) * (size_t)t) +
-         align_up(4 * sizeof(float4) * (size_t)t) + align_up(sizeof(int) * kSpill * (size_t)t) +
-         scan_temp_bytes(t);
+  return align_up(sizeof(int) * (size_t)t * cap) +
+         2 * align_up(sizeof(int) * (size_t)t) + align_up(2 * sizeof(uint4) * (size_t)t) +
+         align_up(sizeof(int) * kSpill * (size_t)t) + align_up(sizeof(int)) + scan_temp_bytes(t);
 }
 
 }  // namespace cm
@@ -1491,17 +1668,21 @@ extern "C" int cm_lbvh_pairs(int32_t t, const int32_t* d_lefts, const int32_t* d
   b.rmlr = (int*)d_rmlr;
   b.warn = d_warn;
   char* tp = (char*)d_temp;
-  int2* chunk = (int2*)tp;
-  tp += align_up(sizeof(int2) * (size_t)t * cap);
+  int* chunk = (int*)tp;
+  tp += align_up(sizeof(int) * (size_t)t * cap);
   int* counts = (int*)tp;
   tp += align_up(sizeof(int) * (size_t)t);
   int* offsets = (int*)tp;
   tp += align_up(sizeof(int) * (size_t)t);
-  b.nodes = (float4*)tp;
-  tp += align_up(4 * sizeof(float4) * (size_t)t);
+  b.qnodes = (uint4*)tp;
+  tp += align_up(2 * sizeof(uint4) * (size_t)t);
   b.spill = (int*)tp;
   tp += align_up(sizeof(int) * kSpill * (size_t)t);
-  int rc = launch_pack_nodes(b, (hipStream_t)stream);
+  b.irr = (int*)tp;
+  tp += align_up(sizeof(int));
+  int rc = fill_i32(b.irr, 0, 1, (hipStream_t)stream);
+  if (rc) return rc;
+  rc = launch_pack_nodes(b, true, (hipStream_t)stream);
   if (rc) return rc;
   rc = scan_temp_clear(tp, t, (hipStream_t)stream);
   if (rc) return rc;
