@@ -977,12 +977,13 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
     CM_HIP(hipMemset(b->scan_temp, 0, scan_temp_bytes((int)smax)));
   }
   nb.scan_temp = b->scan_temp;
-  // tiles of 256 pairs or candidates (their counts, then the counts' prefixes)
-  const int64_t ntile = (std::max<int64_t>(pcap, nb.vf_cap + nb.ee_cap) + 255) / 256;
+  // tiles of pairs or candidates (their counts, then the counts' prefixes)
+  const int64_t ccap = nb.vf_cap + nb.ee_cap;
+  const int64_t ntile = std::max(tile_max(kTileSmall, std::max(pcap, ccap)), tile_max(kTilePlan, ccap));
   if ((rc = dalloc(b, &nb.mask, pcap)) || (rc = dalloc(b, &nb.tile_sum, ntile)) ||
       (rc = dalloc(b, &nb.tile_pre, 2 * ntile)) || (rc = dalloc(b, &nb.cand_vf, nb.vf_cap)) ||
       (rc = dalloc(b, &nb.cand_ee, nb.ee_cap)) ||
-      (rc = dalloc(b, &nb.hit_flag, nb.vf_cap + nb.ee_cap)) ||
+      (rc = dalloc(b, &nb.near_mask, (ccap + 63) / 64)) || (rc = dalloc(b, &nb.hit_flag, ccap)) ||
       (rc = dalloc(b, &nb.near_ids, nb.vf_cap + nb.ee_cap)) ||
       (rc = dalloc(b, &nb.cplan, nb.vf_cap + nb.ee_cap)) ||
       (rc = dalloc(b, &nb.ccp, nb.vf_cap + nb.ee_cap)) ||

@@ -6,6 +6,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <string>
 
 #include "../../include/clothmi.h"
@@ -58,14 +59,38 @@ int scan_temp_clear(void* temp, int n_max, hipStream_t s);
 // *d_total (if non-null) receives the sum. out may alias in.
 int scan_exclusive(const int* in, int* out, int n_max, const int* d_n, int* d_total, void* temp,
                    hipStream_t s);
-// Exclusive scan of per-tile sums (tiles of per_tile items; ceil(*d_items / per_tile)
-// of them, at most ntile_max; all ntile_max when d_items is null). packed: each sum
-// holds two counts below 2^16, scanned into pre[2i] (low) and pre[2i+1] (high);
-// else pre[i]. The totals (below 2^31), clamped to cap0 / cap1, go to *d_tot0 /
-// *d_tot1. temp: a scan temp (scan_temp_bytes(n) with n >= ntile_max).
-int scan_tiles(const int* d_items, int per_tile, int ntile_max, const int* sums, int* pre,
-               int packed, int64_t cap0, int64_t cap1, int* d_tot0, int* d_tot1, void* temp,
-               hipStream_t s);
+// Tiles of the passes over a device-side number of items: one tile of 64 * R consecutive
+// items per wave, lane l taking items base + l + 64 * j, j < R. R grows with the count, so
+// that a short list still gives every SIMD a wave and a long one has few tile sums:
+//   kTileSmall  R = 1 up to 8,192 tiles, else 4 (R = 4 -> 1: 64^2 k_ccd_test 40 -> 13.5
+//               us, k_cand_count 8 -> 5.6; draped 131x97 k_ccd_test 48 -> 17)
+//   kTilePlan   R = as many as leave kPlanWaves tiles, 1 to 8: a tile gathers the long
+//               searches of its chunks, so long lists want large ones (R = 8 -> 1 at 64^2:
+//               59 -> 22 us; R up to 16: 486 -> 522 us draped 256^2)
+enum TileRule : int { kTileSmall, kTilePlan };
+constexpr int kSmallWaves = 8192, kPlanWaves = 3072, kPlanLanes = 8;
+__host__ __device__ inline int tile_lanes(TileRule rule, int items) {
+  if (rule == kTileSmall) return items <= 64 * kSmallWaves ? 1 : 4;
+  const int r = (int)(((int64_t)items + 64 * kPlanWaves - 1) / (64 * kPlanWaves));
+  return r < 1 ? 1 : r > kPlanLanes ? kPlanLanes : r;
+}
+// most tiles that up to item_cap items can make
+inline int64_t tile_max(TileRule rule, int64_t item_cap) {
+  const int64_t few = rule == kTileSmall ? kSmallWaves : kPlanWaves;
+  const int64_t per = 64 * (rule == kTileSmall ? 4 : kPlanLanes);
+  return std::max<int64_t>(std::min<int64_t>((item_cap + 63) / 64, few),
+                           (item_cap + per - 1) / per);
+}
+// Exclusive scan of n per-tile sums. packed: each sum holds two counts below 2^16,
+// scanned into pre[2i] (low) and pre[2i+1] (high); else pre[i]. The totals (below 2^31),
+// clamped to cap0 / cap1, go to *d_tot0 / *d_tot1. temp: a scan temp
+// (scan_temp_bytes(m) with m >= the number of tiles).
+int scan_tiles(int n, const int* sums, int* pre, int packed, int64_t cap0, int64_t cap1,
+               int* d_tot0, int* d_tot1, void* temp, hipStream_t s);
+// the same over the tiles of min(*d_items, item_cap) items
+int scan_tiles_dev(const int* d_items, TileRule rule, int64_t item_cap, const int* sums, int* pre,
+                   int packed, int64_t cap0, int64_t cap1, int* d_tot0, int* d_tot1, void* temp,
+                   hipStream_t s);
 size_t radix_sort_temp_bytes(int n);
 int radix_sort(uint64_t* keys, uint32_t* vals, int n, int key_bits, void* temp, hipStream_t s);
 int radix_sort_clear(void* temp, int n, hipStream_t s);  // before the first sort on a temp
@@ -165,11 +190,12 @@ struct NarrowBufs {
   const int2* pairs = nullptr;
   const int* d_npairs = nullptr;
   uint16_t* mask = nullptr;   // per pair
-  int* tile_sum = nullptr;  // per tile of 256 pairs / candidates: packed counts
+  int* tile_sum = nullptr;  // per tile of pairs / candidates: packed counts
   int* tile_pre = nullptr;  // per tile: exclusive prefixes of the two counts
   int4 *cand_vf = nullptr, *cand_ee = nullptr;
   int *d_ncand_vf = nullptr, *d_ncand_ee = nullptr;
-  uint8_t* hit_flag = nullptr;  // per candidate (VF then EE): near, then hit per near index
+  uint64_t* near_mask = nullptr;  // a bit per candidate (VF then EE): near
+  uint8_t* hit_flag = nullptr;    // per near index: hit
   int* near_ids = nullptr;       // candidates passing the box-gap rejection, in order
   int* d_nnear = nullptr;
   // CCD passes, per candidate (VF then EE, vf_cap + ee_cap), written for near

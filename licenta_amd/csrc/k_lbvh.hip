@@ -1467,8 +1467,7 @@ int launch_pairs(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offse
   const int nt = (t + kTravBlock - 1) / kTravBlock;
   int rc = launch_traverse(b, cap, chunk, counts, offsets, s);
   if (rc) return rc;
-  rc = scan_tiles(nullptr, 1, nt, offsets, offsets + nt, 0, (int64_t)t * cap, 0, d_npairs,
-                  nullptr, scan_temp, s);
+  rc = scan_tiles(nt, offsets, offsets + nt, 0, (int64_t)t * cap, 0, d_npairs, nullptr, scan_temp, s);
   if (rc) return rc;
   hipLaunchKernelGGL(k_compact_pairs, dim3(nt), dim3(kBlock), 0, s, t, cap, chunk,
                      counts, offsets + nt, pairs, two_passes(b) ? b.hctl : nullptr);

@@ -24,10 +24,7 @@ __device__ __forceinline__ int bit(int f, int b) { return (f >> b) & 1; }
 
 // Items are processed in tiles, one tile of 64 * R consecutive items per wave: lane
 // l takes items base + l + 64 * j, j < R, so every load is coalesced and a tile needs
-// no workgroup barrier. The pass over all candidates uses R = 8 (fewer tile sums to
-// scan); the passes over pairs and over the short list of near candidates use R = 4
-// (more waves share the work).
-constexpr int kBig = 8, kSmall = 4;
+// no workgroup barrier. R follows from the item count (tile_lanes).
 constexpr int kWavesPerBlock = kBlock / 64;
 
 __device__ __forceinline__ int wave_sum(int v) {
@@ -118,14 +115,14 @@ __global__ void __launch_bounds__(kBlock) k_cand_count(
     const int4* __restrict__ tri, const float4* __restrict__ x, const float4* __restrict__ p,
     float th, int ee_on, uint16_t* __restrict__ mask, int* __restrict__ tile_sum) {
   const int np = (int)min((int64_t)*d_npairs, pair_cap);
-  const int ntiles = (np + (64 * kSmall) - 1) / (64 * kSmall);
+  const int R = tile_lanes(kTileSmall, np);
+  const int ntiles = (np + 64 * R - 1) / (64 * R);
   const int lane = threadIdx.x & 63;
   for (int tile = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6); tile < ntiles;
        tile += gridDim.x * kWavesPerBlock) {
     int c = 0;
-#pragma unroll
-    for (int j = 0; j < kSmall; ++j) {
-      const int k = tile * (64 * kSmall) + j * 64 + lane;
+    for (int j = 0; j < R; ++j) {
+      const int k = tile * (64 * R) + j * 64 + lane;
       if (k < np) {
         const unsigned m = pair_mask(pairs[k], tri, x, p, th, ee_on);
         mask[k] = (uint16_t)m;
@@ -138,31 +135,31 @@ __global__ void __launch_bounds__(kBlock) k_cand_count(
 }
 
 // pass 2 (after the scan of the tile counts): candidates at their ordered positions
-__global__ void __launch_bounds__(kBlock) k_cand_write(
-    const int2* __restrict__ pairs, const int* __restrict__ d_npairs, int64_t pair_cap,
+template <int R>
+__device__ __forceinline__ void cand_write(
+    const int2* __restrict__ pairs, int np,
     const int4* __restrict__ tri, const uint16_t* __restrict__ mask,
     const int* __restrict__ tile_pre, int4* __restrict__ cand_vf, int4* __restrict__ cand_ee,
     int64_t vf_cap, int64_t ee_cap, uint32_t* __restrict__ warn) {
-  const int np = (int)min((int64_t)*d_npairs, pair_cap);
-  const int ntiles = (np + (64 * kSmall) - 1) / (64 * kSmall);
+  const int ntiles = (np + 64 * R - 1) / (64 * R);
   const int lane = threadIdx.x & 63;
   bool over = false;
   for (int tile = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6); tile < ntiles;
        tile += gridDim.x * kWavesPerBlock) {
-    unsigned m[kSmall];
-    int c[kSmall], off[kSmall];
+    unsigned m[R];
+    int c[R], off[R];
 #pragma unroll
-    for (int j = 0; j < kSmall; ++j) {
-      const int k = tile * (64 * kSmall) + j * 64 + lane;
+    for (int j = 0; j < R; ++j) {
+      const int k = tile * (64 * R) + j * 64 + lane;
       m[j] = k < np ? mask[k] : 0u;
       c[j] = mask_counts(m[j]);
     }
-    tile_offsets<kSmall>(c, off);
+    tile_offsets<R>(c, off);
     const int pvf = tile_pre[2 * tile], pee = tile_pre[2 * tile + 1];
 #pragma unroll
-    for (int j = 0; j < kSmall; ++j) {
+    for (int j = 0; j < R; ++j) {
       if (!m[j]) continue;
-      const int k = tile * (64 * kSmall) + j * 64 + lane;
+      const int k = tile * (64 * R) + j * 64 + lane;
       const int2 pr = pairs[k];
       const int4 t1 = tri[pr.x], t2 = tri[pr.y];
       const int v1[3] = {t1.x, t1.y, t1.z}, v2[3] = {t2.x, t2.y, t2.z};
@@ -184,6 +181,18 @@ __global__ void __launch_bounds__(kBlock) k_cand_write(
     }
   }
   if (over) atomicOr(warn, (uint32_t)CM_WARN_CANDIDATE_CAP);
+}
+
+__global__ void __launch_bounds__(kBlock) k_cand_write(
+    const int2* __restrict__ pairs, const int* __restrict__ d_npairs, int64_t pair_cap,
+    const int4* __restrict__ tri, const uint16_t* __restrict__ mask,
+    const int* __restrict__ tile_pre, int4* __restrict__ cand_vf, int4* __restrict__ cand_ee,
+    int64_t vf_cap, int64_t ee_cap, uint32_t* __restrict__ warn) {
+  const int np = (int)min((int64_t)*d_npairs, pair_cap);
+  if (tile_lanes(kTileSmall, np) == 1)
+    cand_write<1>(pairs, np, tri, mask, tile_pre, cand_vf, cand_ee, vf_cap, ee_cap, warn);
+  else
+    cand_write<4>(pairs, np, tri, mask, tile_pre, cand_vf, cand_ee, vf_cap, ee_cap, warn);
 }
 
 // ---- CCD (FP32, same arithmetic as the oracle) -------------------------------
@@ -354,7 +363,7 @@ __device__ __forceinline__ bool test_ee(f3 x1, f3 x2, f3 x3, f3 x4, Hit& h, floa
 //   k_ccd_plan    per candidate: cubic, f at the interval ends, plan word, the secant
 //                 root of each interval with a sign change, then the roots in order
 //                 with the same cumulative advance and only the box-gap rejection:
-//                 a near flag per candidate, near counts per tile. Plan word,
+//                 a near bit per candidate, near counts per tile. Plan word,
 //                 critical points and roots (interval i of candidate id in
 //                 roots[3 * id + i]) are stored for near candidates only, the only
 //                 ones the later passes read.
@@ -380,51 +389,6 @@ __device__ __forceinline__ int4 cand_of(int id, int nvf, const int4* __restrict_
                                         const int4* __restrict__ cand_ee, bool& isvf) {
   isvf = id < nvf;
   return isvf ? cand_vf[id] : cand_ee[id - nvf];
-}
-
-// Secant searches (Physics/CudaCubicSolver.cu:131-153, 20 steps) on the intervals
-// with a sign change, from x0 = start, x1 = end, f0 = f(x0), f1 = f(x1). The
-// reference evaluates f at both points every step; f(x0) of a step is f(x1) of the
-// previous one, and the first step's two values are the ones the plan computed at
-// the interval's ends, all from the same inputs, so they are carried over unchanged.
-// A search converges when |xc - x1| < EPS (root xc) or gives up after 20 steps (the
-// reference returns -15). A lane runs its searches one after the other in one loop,
-// so the wave waits for the lane with the most steps in all, not for the slowest
-// lane of every interval in turn.
-__device__ __forceinline__ void secants(const Cubic& q, int pl, const float (&fe)[4],
-                                        float (&r)[3]) {
-  auto next = [&](int i) {  // first interval >= i with a sign change, or 3
-    while (i <= q.cc && !(pl & (1 << (5 + i)))) ++i;
-    return i <= q.cc ? i : 3;
-  };
-  auto start = [&](int i, float& x0, float& x1, float& f0, float& f1) {
-    x0 = i == 0 ? 0.f : (i == 1 ? q.cp1 : q.cp2);
-    x1 = cubic_end(q.cp1, q.cp2, q.cc, i);
-    f0 = i == 0 ? fe[0] : (i == 1 ? fe[1] : fe[2]);
-    f1 = i == 0 ? fe[1] : (i == 1 ? fe[2] : fe[3]);
-  };
-  int i = next(0), k = 0;
-  float x0 = 0.f, x1 = 0.f, f0 = 0.f, f1 = 0.f;
-  if (i < 3) start(i, x0, x1, f0, f1);
-  while (i < 3) {
-    const float xc = (x0 * f1 - x1 * f0) / (f1 - f0);
-    const bool conv = fabsf(xc - x1) < kCubicEps;
-    if (conv) {
-      r[0] = i == 0 ? xc : r[0];
-      r[1] = i == 1 ? xc : r[1];
-      r[2] = i == 2 ? xc : r[2];
-    }
-    if (conv || ++k == 20) {
-      i = next(i + 1);
-      k = 0;
-      if (i < 3) start(i, x0, x1, f0, f1);
-      continue;
-    }
-    x0 = x1;
-    f0 = f1;
-    x1 = xc;
-    f1 = cubic_f(q, x1);
-  }
 }
 
 // Conservative rejections before the proximity tests. A VF hit puts the point within
@@ -498,145 +462,216 @@ __device__ __forceinline__ bool ccd_tests(bool isvf, int4 c, int pl, float2 cp, 
   return false;
 }
 
-// One candidate of k_ccd_plan: the plan of its roots and whether any root survives
-// the box-gap rejection after the same cumulative advance as ccd_tests (false: the
-// full tests cannot hit). Stores plan word, critical points and roots when near.
-__device__ __forceinline__ bool plan_near(bool isvf, int4 c, int id, const float4* __restrict__ x,
+// ---- k_ccd_plan ----
+// The pass is bound by vector instructions, most of them secant steps at few lanes: a wave
+// takes as many steps as its slowest lane (draped 256^2: 27 for 64 candidates whose lanes
+// need 5.9 on average, where 2.3% of the candidates take 20 or more). So a wave gives 64
+// candidates kBudget steps; those that need more go on a stack of ids in its LDS and are
+// run again from the start, 64 at a time (384 -> 368 us for the 96 cloths, 543 -> 486
+// draped 256^2, 97 -> 93 draped 131x97; 12 steps 380, 484, 94; 16 steps 391, 524, 97).
+// Tiles of one chunk run it to its end: a second round would cost them more than it saves.
+// From one loop over a candidate's roots with the checks unrolled, one tile of 512 a wave
+// and 2,048 workgroups -> now: 64^2 59 -> 10.4 us, flat 256^2 59 -> 14.7, draped 131x97
+// 129 -> 93, draped 256^2 600 -> 486, 96 cloths 476 -> 368, crumpled 1024^2 427 -> 375.
+// Handing single lanes new searches from a queue of set-up cubics in LDS was slower
+// (1,080 us draped 256^2): 53 KB a workgroup leave three waves a SIMD to hide its gathers.
+constexpr int kBudget = 8, kNoBudget = 1 << 20;
+struct PlanLds {
+  float root[3][64];  // secant roots of the 64 candidates under way, by interval
+  int stack[128];
+  alignas(8) uint32_t near[2 * kPlanLanes];  // near mask of the tile: 2 words for each 64 candidates
+};
+
+enum Plan : int { kFar, kNear, kMore };
+
+// One candidate: its cubic, f at the interval ends, the secant root of each interval with a
+// sign change, then whether any root survives the box-gap rejection after the same
+// cumulative advance as in ccd_tests (kFar: the full tests cannot hit). Stores plan word,
+// critical points and roots when one does. kMore: the searches need more than `budget`
+// steps, nothing is stored.
+__device__ __forceinline__ Plan plan_near(bool isvf, int4 c, int id, int budget, PlanLds& L,
+                                          const float4* __restrict__ x,
                                           const float4* __restrict__ v, float th, float dt,
                                           int dcd, int* __restrict__ plan,
                                           float2* __restrict__ cps, float* __restrict__ roots) {
-  if (!sane(isvf, c)) return false;
+  const int lane = threadIdx.x & 63;
+  if (!sane(isvf, c)) return kFar;
   const int4 q4 = cubic_ids(isvf, c);
-  const f3 o1 = xyz(x[q4.x]), o2 = xyz(x[q4.y]), o3 = xyz(x[q4.z]), o4 = xyz(x[q4.w]);
+  f3 p1 = xyz(x[q4.x]), p2 = xyz(x[q4.y]), p3 = xyz(x[q4.z]), p4 = xyz(x[q4.w]);
   if (dcd) {  // one test at x, no cubic
-    const bool nr = isvf ? !vf_far(o4, o1, o2, o3, th) : !ee_far(o1, o2, o3, o4, th);
-    if (nr) {
-      plan[id] = 0;
-      cps[id] = make_float2(0.f, 0.f);
-    }
-    return nr;
+    if (isvf ? vf_far(p4, p1, p2, p3, th) : ee_far(p1, p2, p3, p4, th)) return kFar;
+    plan[id] = 0;
+    cps[id] = make_float2(0.f, 0.f);
+    return kNear;
   }
   const f3 u1 = xyz(v[q4.x]), u2 = xyz(v[q4.y]), u3 = xyz(v[q4.z]), u4 = xyz(v[q4.w]);
   Cubic q;
-  cubic_setup(o1, o2, o3, o4, u1, u2, u3, u4, q);
-  // f at the interval ends: fe[i] at the start of interval i, fe[i + 1] at its end
-  int pl = q.cc;
-  float fe[4];
-  fe[0] = cubic_f(q, 0.f);
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    if (i > q.cc) break;
-    fe[i + 1] = cubic_f(q, cubic_end(q.cp1, q.cp2, q.cc, i));
-    if (fabsf(fe[i]) < kCubicEps) pl |= 1 << (2 + i);
-    if (fe[i] * fe[i + 1] < 0.f) pl |= 1 << (5 + i);
+  cubic_setup(p1, p2, p3, p4, u1, u2, u3, u4, q);
+  // f at the interval ends: e0 at 0, e1 to e3 at the ends of intervals 0 to 2
+  const int cc = q.cc;
+  const float e0 = cubic_f(q, 0.f), e1 = cubic_f(q, cubic_end(q.cp1, q.cp2, cc, 0));
+  float e2 = 0.f, e3 = 0.f;
+  if (cc >= 1) e2 = cubic_f(q, cubic_end(q.cp1, q.cp2, cc, 1));
+  if (cc >= 2) e3 = cubic_f(q, 1.f);
+  int starts = fabsf(e0) < kCubicEps ? 1 : 0;  // roots at the starts of intervals 0 to 2
+  int rem = e0 * e1 < 0.f ? 1 : 0;             // sign changes on them
+  if (cc >= 1) {
+    starts |= fabsf(e1) < kCubicEps ? 2 : 0;
+    rem |= e1 * e2 < 0.f ? 2 : 0;
   }
-  // the secant root of each interval with a sign change, with the cubic in registers
-  float r[3] = {kNoRoot, kNoRoot, kNoRoot};
-  secants(q, pl, fe, r);
-  f3 p1 = o1, p2 = o2, p3 = o3, p4 = o4;
-  auto near_at = [&](float root) {
-    const float t = root * dt;
-    if (isvf) {
-      p4 = add(p4, mul(u4, t));
-      p1 = add(p1, mul(u1, t));
-      p2 = add(p2, mul(u2, t));
-      p3 = add(p3, mul(u3, t));
-      return !vf_far(p4, p1, p2, p3, th);
+  if (cc >= 2) {
+    starts |= fabsf(e2) < kCubicEps ? 4 : 0;
+    rem |= e2 * e3 < 0.f ? 4 : 0;
+  }
+  const int pl = cc | starts << 2 | rem << 5;
+  // Secant searches (Physics/CudaCubicSolver.cu:131-153, 20 steps) on the intervals with a
+  // sign change, from x0 = start, x1 = end, f0 = f(x0), f1 = f(x1). The reference evaluates
+  // f at both points every step; f(x0) of a step is f(x1) of the previous one, and the first
+  // step's two values are the ones computed at the interval's ends, all from the same
+  // inputs, so they are carried over unchanged. A search converges when |xc - x1| < EPS
+  // (root xc) or gives up after 20 steps (the reference returns -15). A lane runs its
+  // searches one after the other in one loop, so the wave waits for the lane with the most
+  // steps in all, not for the slowest lane of every interval in turn.
+  // The two points of a step change places from one step to the next.
+  int found = 0, i = __ffs(rem) - 1, k = 0;
+  float xa = i <= 0 ? 0.f : (i == 1 ? q.cp1 : q.cp2), xb = cubic_end(q.cp1, q.cp2, cc, i);
+  float fa = i <= 0 ? e0 : (i == 1 ? e1 : e2), fb = i <= 0 ? e1 : (i == 1 ? e2 : e3);
+  // from the points (x0, f0) and (x1, f1): the next point goes to (x0, f0)
+  auto step = [&](float& x0, float& f0, float& x1, float& f1) {
+    const float xc = (x0 * f1 - x1 * f0) / (f1 - f0);
+    const bool conv = fabsf(xc - x1) < kCubicEps;
+    x0 = xc;
+    f0 = cubic_f(q, xc);
+    ++k;
+    if (conv || k == 20) {
+      if (conv && xc != kNoRoot) {
+        L.root[i][lane] = xc;
+        found |= 1 << i;
+      }
+      rem &= rem - 1;
+      k = 0;
+      i = rem == 4 ? 2 : 1;  // what is left: interval 1 or 2
+      const bool second = rem != 4;
+      const float sx = second ? q.cp1 : q.cp2, sf = second ? e1 : e2;
+      const float ex = second && cc == 2 ? q.cp2 : 1.f, ef = second ? e2 : e3;
+      x1 = sx;  // the next step's (x0, f0) and (x1, f1)
+      f1 = sf;
+      x0 = ex;
+      f0 = ef;
     }
+  };
+  for (int it = 0; rem && it < budget; it += 2) {
+    step(xa, fa, xb, fb);
+    if (rem) {
+      step(xb, fb, xa, fa);
+    }
+  }
+  if (rem) return kMore;
+  // the roots in order: that at the start of interval j (bit 2j), its secant root (2j + 1)
+  int order = 0;
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+    order |= ((starts >> j) & 1) << (2 * j) | ((found >> j) & 1) << (2 * j + 1);
+  bool nr = false;
+  while (order) {
+    const int b = __ffs(order) - 1, j = b >> 1;
+    order &= order - 1;
+    float r = j == 0 ? 0.f : (j == 1 ? q.cp1 : q.cp2);
+    if (b & 1) r = L.root[j][lane];
+    const float t = r * dt;
     p1 = add(p1, mul(u1, t));
     p2 = add(p2, mul(u2, t));
     p3 = add(p3, mul(u3, t));
     p4 = add(p4, mul(u4, t));
-    return !ee_far(p1, p2, p3, p4, th);
-  };
-  bool nr = false;
-  float ea = 0.f;
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    if (i > q.cc) break;
-    if ((pl & (1 << (2 + i))) && near_at(ea)) { nr = true; break; }
-    if ((pl & (1 << (5 + i))) && r[i] != kNoRoot && near_at(r[i])) { nr = true; break; }
-    ea = cubic_end(q.cp1, q.cp2, q.cc, i);
+    if (!(isvf ? vf_far(p4, p1, p2, p3, th) : ee_far(p1, p2, p3, p4, th))) {
+      nr = true;
+      break;
+    }
   }
-  if (nr) {
-    plan[id] = pl;
-    cps[id] = make_float2(q.cp1, q.cp2);
+  if (!nr) return kFar;
+  plan[id] = pl;
+  cps[id] = make_float2(q.cp1, q.cp2);
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-      if (i <= q.cc && (pl & (1 << (5 + i)))) roots[3 * (int64_t)id + i] = r[i];
-  }
-  return nr;
+  for (int j = 0; j < 3; ++j)
+    if (pl & (1 << (5 + j)))
+      roots[3 * (int64_t)id + j] = found & (1 << j) ? L.root[j][lane] : kNoRoot;
+  return kNear;
 }
 
-// pass 3: near flag per candidate (VF then EE ids), near counts per tile of ids
+// pass 3: near mask of the candidates (VF then EE ids), near counts per tile of ids
 __global__ void __launch_bounds__(kBlock) k_ccd_plan(
     const int4* __restrict__ cand_vf, const int4* __restrict__ cand_ee,
     const int* __restrict__ d_nvf, const int* __restrict__ d_nee, int64_t vf_cap,
     int64_t ee_cap, const float4* __restrict__ x, const float4* __restrict__ v, float th,
     float dt, int dcd, int* __restrict__ plan, float2* __restrict__ cps,
-    float* __restrict__ roots, int* __restrict__ d_ntotal, uint8_t* __restrict__ near_flag,
+    float* __restrict__ roots, int* __restrict__ d_ntotal, uint64_t* __restrict__ near_mask,
     int* __restrict__ tile_sum) {
+  __shared__ PlanLds lds[kWavesPerBlock];
+  PlanLds& L = lds[threadIdx.x >> 6];
   const int nvf = (int)min((int64_t)*d_nvf, vf_cap), nee = (int)min((int64_t)*d_nee, ee_cap);
   const int total = nvf + nee;
   if (blockIdx.x == 0 && threadIdx.x == 0) *d_ntotal = total;
-  const int ntiles = (total + (64 * kBig) - 1) / (64 * kBig);
+  const int R = tile_lanes(kTilePlan, total);
+  const int ntiles = total / (64 * R) + (total % (64 * R) != 0);
   const int lane = threadIdx.x & 63;
+  const uint64_t below = (1ull << lane) - 1ull;
+  // the lanes of a wave share L: their accesses stay in program order
+  auto order = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
   for (int tile = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6); tile < ntiles;
        tile += gridDim.x * kWavesPerBlock) {
-    int c = 0;
-    for (int j = 0; j < kBig; ++j) {
-      const int id = tile * (64 * kBig) + j * 64 + lane;
-      if (id >= total) break;
-      bool isvf;
-      const int4 q = cand_of(id, nvf, cand_vf, cand_ee, isvf);
-      const bool nr = plan_near(isvf, q, id, x, v, th, dt, dcd, plan, cps, roots);
-      near_flag[id] = (uint8_t)nr;
-      c += nr;
+    const int first = tile * R * 64;
+    const int chunks = min(R, (total - first + 63) >> 6);
+    if (lane < 2 * kPlanLanes) L.near[lane] = 0u;
+    int next = 0, depth = 0;  // chunks taken, ids on the stack
+    for (;;) {
+      order();
+      int id = -1, budget = kNoBudget;
+      if (depth >= 64 || next == chunks) {
+        if (depth == 0) break;
+        if (lane < depth) id = L.stack[depth - 1 - lane];
+        depth = max(0, depth - 64);
+      } else {
+        if (first + next * 64 + lane < total) id = first + next * 64 + lane;
+        ++next;
+        if (R > 1) budget = kBudget;
+      }
+      order();
+      Plan r = kFar;
+      if (id >= 0) {
+        bool isvf;
+        const int4 c = cand_of(id, nvf, cand_vf, cand_ee, isvf);
+        r = plan_near(isvf, c, id, budget, L, x, v, th, dt, dcd, plan, cps, roots);
+      }
+      const uint64_t more = __ballot(r == kMore);
+      if (r == kMore) L.stack[depth + __popcll(more & below)] = id;
+      depth += __popcll(more);
+      if (r == kNear) atomicOr(&L.near[(id - first) >> 5], 1u << ((id - first) & 31));
     }
-    c = wave_sum(c);
+    const uint64_t m = lane < chunks ? ((const uint64_t*)L.near)[lane] : 0ull;
+    if (lane < chunks) near_mask[tile * R + lane] = m;
+    const int c = wave_sum(__popcll(m));
     if (lane == 0) tile_sum[tile] = c;
   }
 }
 
-// pass 4: the near candidates' ids in order
+// pass 4: the near candidates' ids in order, from the 64-bit masks of the plan's tiles
 __global__ void __launch_bounds__(kBlock) k_near_list(const int* __restrict__ d_ntotal,
-                                                      const uint8_t* __restrict__ near_flag,
+                                                      const uint64_t* __restrict__ near_mask,
                                                       const int* __restrict__ tile_pre,
                                                       int* __restrict__ near_ids) {
-  // lane l takes the kBig consecutive ids from tile * 64 * kBig + l * kBig (one 8-byte
-  // load of their flags), so the ids leave in order: lane by lane, then within a lane
-  static_assert(kBig == 8, "one 8-byte load of near flags per lane");
   const int total = *d_ntotal;
-  const int ntiles = (total + (64 * kBig) - 1) / (64 * kBig);
+  const int R = tile_lanes(kTilePlan, total);
+  const int ntiles = total / (64 * R) + (total % (64 * R) != 0);
+  const int nmask = (total + 63) >> 6;
   const int lane = threadIdx.x & 63;
+  const uint64_t below = (1ull << lane) - 1ull;
   for (int tile = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6); tile < ntiles;
        tile += gridDim.x * kWavesPerBlock) {
-    const int b0 = tile * (64 * kBig) + lane * kBig;
-    uint32_t lo = 0, hi = 0;
-    if (b0 + kBig <= total) {
-      const uint2 u = *reinterpret_cast<const uint2*>(near_flag + b0);
-      lo = u.x;
-      hi = u.y;
-    } else {
-#pragma unroll
-      for (int j = 0; j < kBig; ++j) {
-        const uint32_t f = b0 + j < total ? near_flag[b0 + j] : 0u;
-        if (j < 4) lo |= f << (8 * j);
-        else hi |= f << (8 * (j - 4));
-      }
-    }
-    const int cnt = __popc(lo & 0x01010101u) + __popc(hi & 0x01010101u);
-    int inc = cnt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int u = __shfl_up(inc, o, 64);
-      if (lane >= o) inc += u;
-    }
-    int at = tile_pre[tile] + inc - cnt;
-#pragma unroll
-    for (int j = 0; j < kBig; ++j) {
-      const uint32_t f = ((j < 4 ? lo : hi) >> (8 * (j & 3))) & 1u;
-      if (f) near_ids[at++] = b0 + j;
+    int at = tile_pre[tile];
+    for (int j = 0; j < R && tile * R + j < nmask; ++j) {
+      const uint64_t m = near_mask[tile * R + j];
+      if ((m >> lane) & 1) near_ids[at + __popcll(m & below)] = (tile * R + j) * 64 + lane;
+      at += __popcll(m);
     }
   }
 }
@@ -652,14 +687,14 @@ __global__ void __launch_bounds__(kBlock) k_ccd_test(
     uint8_t* __restrict__ hit_flag, int* __restrict__ tile_sum, float4* __restrict__ hit_data,
     int64_t hit_cap) {
   const int nvf = (int)min((int64_t)*d_nvf, vf_cap), nn = *d_nnear;
-  const int ntiles = (nn + (64 * kSmall) - 1) / (64 * kSmall);
+  const int R = tile_lanes(kTileSmall, nn);
+  const int ntiles = (nn + 64 * R - 1) / (64 * R);
   const int lane = threadIdx.x & 63;
   for (int tile = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6); tile < ntiles;
        tile += gridDim.x * kWavesPerBlock) {
     int c = 0;
-#pragma unroll
-    for (int j = 0; j < kSmall; ++j) {
-      const int k = tile * (64 * kSmall) + j * 64 + lane;
+    for (int j = 0; j < R; ++j) {
+      const int k = tile * (64 * R) + j * 64 + lane;
       if (k < nn) {
         const int id = near_ids[k];
         bool isvf;
@@ -682,9 +717,9 @@ __global__ void __launch_bounds__(kBlock) k_ccd_test(
 // pass 6 (after the scan of the tile counts): each hit is written at its ordered
 // position among the VF or EE contacts, with the weights, time and normal k_ccd_test
 // kept for it (recomputed for near indices at or past hit_cap).
-__global__ void __launch_bounds__(kBlock) k_ccd_write(
-    const int4* __restrict__ cand_vf, const int4* __restrict__ cand_ee,
-    const int* __restrict__ d_nvf, int64_t vf_cap, const int* __restrict__ d_nnear,
+template <int R>
+__device__ __forceinline__ void ccd_write(
+    const int4* __restrict__ cand_vf, const int4* __restrict__ cand_ee, int nvf, int nn,
     const int* __restrict__ near_ids, const int* __restrict__ plan,
     const float2* __restrict__ cps, const float* __restrict__ roots,
     const uint8_t* __restrict__ hit_flag, const int* __restrict__ tile_pre, int64_t vf_out_cap,
@@ -693,24 +728,23 @@ __global__ void __launch_bounds__(kBlock) k_ccd_write(
     float4* __restrict__ vf_tn, int4* __restrict__ ee_v, float4* __restrict__ ee_w,
     float4* __restrict__ ee_tn, uint32_t* __restrict__ warn,
     const float4* __restrict__ hit_data, int64_t hit_cap) {
-  const int nvf = (int)min((int64_t)*d_nvf, vf_cap), nn = *d_nnear;
-  const int ntiles = (nn + (64 * kSmall) - 1) / (64 * kSmall);
+  const int ntiles = (nn + 64 * R - 1) / (64 * R);
   const int lane = threadIdx.x & 63;
   bool over = false;
   for (int tile = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6); tile < ntiles;
        tile += gridDim.x * kWavesPerBlock) {
-    int id[kSmall], c[kSmall], off[kSmall];
+    int id[R], c[R], off[R];
 #pragma unroll
-    for (int j = 0; j < kSmall; ++j) {
-      const int k = tile * (64 * kSmall) + j * 64 + lane;
+    for (int j = 0; j < R; ++j) {
+      const int k = tile * (64 * R) + j * 64 + lane;
       const bool hit = k < nn && hit_flag[k];
       id[j] = hit ? near_ids[k] : -1;
       c[j] = hit ? (id[j] < nvf ? 1 : (1 << 16)) : 0;
     }
-    tile_offsets<kSmall>(c, off);
+    tile_offsets<R>(c, off);
     const int pvf = tile_pre[2 * tile], pee = tile_pre[2 * tile + 1];
 #pragma unroll
-    for (int j = 0; j < kSmall; ++j) {
+    for (int j = 0; j < R; ++j) {
       if (id[j] < 0) continue;
       bool isvf;
       const int4 q = cand_of(id[j], nvf, cand_vf, cand_ee, isvf);
@@ -719,7 +753,7 @@ __global__ void __launch_bounds__(kBlock) k_ccd_write(
         over = true;
         continue;
       }
-      const int64_t k = (int64_t)tile * (64 * kSmall) + j * 64 + lane;
+      const int64_t k = (int64_t)tile * (64 * R) + j * 64 + lane;
       float4 w4, tn;
       if (k < hit_cap) {
         w4 = hit_data[2 * k];
@@ -735,6 +769,28 @@ __global__ void __launch_bounds__(kBlock) k_ccd_write(
     }
   }
   if (over) atomicOr(warn, (uint32_t)CM_WARN_CANDIDATE_CAP);
+}
+
+__global__ void __launch_bounds__(kBlock) k_ccd_write(
+    const int4* __restrict__ cand_vf, const int4* __restrict__ cand_ee,
+    const int* __restrict__ d_nvf, int64_t vf_cap, const int* __restrict__ d_nnear,
+    const int* __restrict__ near_ids, const int* __restrict__ plan,
+    const float2* __restrict__ cps, const float* __restrict__ roots,
+    const uint8_t* __restrict__ hit_flag, const int* __restrict__ tile_pre, int64_t vf_out_cap,
+    int64_t ee_out_cap, const float4* __restrict__ x, const float4* __restrict__ v, float th,
+    float dt, int dcd, int4* __restrict__ vf_v, float4* __restrict__ vf_w,
+    float4* __restrict__ vf_tn, int4* __restrict__ ee_v, float4* __restrict__ ee_w,
+    float4* __restrict__ ee_tn, uint32_t* __restrict__ warn,
+    const float4* __restrict__ hit_data, int64_t hit_cap) {
+  const int nvf = (int)min((int64_t)*d_nvf, vf_cap), nn = *d_nnear;
+  if (tile_lanes(kTileSmall, nn) == 1)
+    ccd_write<1>(cand_vf, cand_ee, nvf, nn, near_ids, plan, cps, roots, hit_flag, tile_pre,
+                 vf_out_cap, ee_out_cap, x, v, th, dt, dcd, vf_v, vf_w, vf_tn, ee_v, ee_w, ee_tn,
+                 warn, hit_data, hit_cap);
+  else
+    ccd_write<4>(cand_vf, cand_ee, nvf, nn, near_ids, plan, cps, roots, hit_flag, tile_pre,
+                 vf_out_cap, ee_out_cap, x, v, th, dt, dcd, vf_v, vf_w, vf_tn, ee_v, ee_w, ee_tn,
+                 warn, hit_data, hit_cap);
 }
 
 // vertex ids as solver positions
@@ -957,51 +1013,51 @@ static int grid_for(int64_t cap) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(g, 2048));
 }
 
-// workgroups for tiles of 64 * R items over up to `items` items
-static int tile_grid(int64_t items, int R) {
-  const int64_t g = (items + kBlock * R - 1) / (kBlock * R);
-  return (int)std::max<int64_t>(1, std::min<int64_t>(g, 2048));
+// Workgroups for the tiles of up to `items` items; a wave with no tile leaves at once. More
+// than the chip holds at once, so that the last round is short where tiles differ (2,048
+// -> 4,096 or 8,192: crumpled 1024^2 k_cand_count 478 -> 435 us, draped 256^2 97 -> 90 and
+// k_ccd_plan 612 -> 584), few enough that empty ones cost nothing.
+static int tile_grid(TileRule rule, int64_t items) {
+  const int64_t g = (tile_max(rule, items) + kWavesPerBlock - 1) / kWavesPerBlock;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(g, rule == kTilePlan ? 8192 : 4096));
 }
 
 int launch_narrow(const NarrowBufs& nb, const int4* tri, const float4* x, const float4* p,
                   const float4* v, float th, float dt, int ee_on, int dcd, hipStream_t s) {
   // candidates: masks and tile counts, tile prefixes (and the clamped totals), writes
-  const int ptiles = (int)((nb.pair_cap + 64 * kSmall - 1) / (64 * kSmall));
-  hipLaunchKernelGGL(k_cand_count, dim3(tile_grid(nb.pair_cap, kSmall)), dim3(kBlock), 0, s, nb.pairs,
+  hipLaunchKernelGGL(k_cand_count, dim3(tile_grid(kTileSmall, nb.pair_cap)), dim3(kBlock), 0, s, nb.pairs,
                      nb.d_npairs, nb.pair_cap, tri, x, p, th, ee_on, nb.mask, nb.tile_sum);
   CM_LAUNCH_CHECK();
-  int rc = scan_tiles(nb.d_npairs, 64 * kSmall, ptiles, nb.tile_sum, nb.tile_pre, 1, nb.vf_cap,
+  int rc = scan_tiles_dev(nb.d_npairs, kTileSmall, nb.pair_cap, nb.tile_sum, nb.tile_pre, 1, nb.vf_cap,
                       nb.ee_cap, nb.d_ncand_vf, nb.d_ncand_ee, nb.scan_temp, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_cand_write, dim3(tile_grid(nb.pair_cap, kSmall)), dim3(kBlock), 0, s, nb.pairs,
+  hipLaunchKernelGGL(k_cand_write, dim3(tile_grid(kTileSmall, nb.pair_cap)), dim3(kBlock), 0, s, nb.pairs,
                      nb.d_npairs, nb.pair_cap, tri, nb.mask, nb.tile_pre, nb.cand_vf, nb.cand_ee,
                      nb.vf_cap, nb.ee_cap, nb.warn);
   // CCD: plan with secant roots and near flags, near list, tests with tile hit
   // counts, tile prefixes, writes
   const int64_t ccap = nb.vf_cap + nb.ee_cap;
-  hipLaunchKernelGGL(k_ccd_plan, dim3(tile_grid(ccap, kBig)), dim3(kBlock), 0, s, nb.cand_vf,
+  hipLaunchKernelGGL(k_ccd_plan, dim3(tile_grid(kTilePlan, ccap)), dim3(kBlock), 0, s, nb.cand_vf,
                      nb.cand_ee, nb.d_ncand_vf, nb.d_ncand_ee, nb.vf_cap, nb.ee_cap, x, v, th, dt,
-                     dcd, nb.cplan, nb.ccp, nb.croot, nb.d_ntotal, nb.hit_flag, nb.tile_sum);
+                     dcd, nb.cplan, nb.ccp, nb.croot, nb.d_ntotal, nb.near_mask, nb.tile_sum);
   CM_LAUNCH_CHECK();
-  const int ctiles = (int)((ccap + 64 * kBig - 1) / (64 * kBig));
-  rc = scan_tiles(nb.d_ntotal, 64 * kBig, ctiles, nb.tile_sum, nb.tile_pre, 0, ccap, 0,
+  rc = scan_tiles_dev(nb.d_ntotal, kTilePlan, ccap, nb.tile_sum, nb.tile_pre, 0, ccap, 0,
                   nb.d_nnear, nullptr, nb.scan_temp, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_near_list, dim3(tile_grid(ccap, kBig)), dim3(kBlock), 0, s, nb.d_ntotal,
-                     nb.hit_flag, nb.tile_pre, nb.near_ids);
+  hipLaunchKernelGGL(k_near_list, dim3(tile_grid(kTilePlan, ccap)), dim3(kBlock), 0, s, nb.d_ntotal,
+                     nb.near_mask, nb.tile_pre, nb.near_ids);
   // the record payloads (32 B each) are free until k_rec_place refills them: they keep
   // each hit's weights, time and normal from k_ccd_test for k_ccd_write
   const int64_t hit_cap = 4 * (nb.vf_out_cap + nb.ee_out_cap);
-  hipLaunchKernelGGL(k_ccd_test, dim3(tile_grid(ccap, kSmall)), dim3(kBlock), 0, s, nb.cand_vf,
+  hipLaunchKernelGGL(k_ccd_test, dim3(tile_grid(kTileSmall, ccap)), dim3(kBlock), 0, s, nb.cand_vf,
                      nb.cand_ee, nb.d_ncand_vf, nb.vf_cap, nb.d_nnear, nb.near_ids, nb.cplan,
                      nb.ccp, nb.croot, x, v, th, dt, dcd, nb.hit_flag, nb.tile_sum,
                      (float4*)nb.rec, hit_cap);
   CM_LAUNCH_CHECK();
-  const int ntiles_near = (int)((ccap + 64 * kSmall - 1) / (64 * kSmall));
-  rc = scan_tiles(nb.d_nnear, 64 * kSmall, ntiles_near, nb.tile_sum, nb.tile_pre, 1, nb.vf_out_cap,
+  rc = scan_tiles_dev(nb.d_nnear, kTileSmall, ccap, nb.tile_sum, nb.tile_pre, 1, nb.vf_out_cap,
                   nb.ee_out_cap, nb.d_nvf, nb.d_nee, nb.scan_temp, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_ccd_write, dim3(tile_grid(ccap, kSmall)), dim3(kBlock), 0, s, nb.cand_vf,
+  hipLaunchKernelGGL(k_ccd_write, dim3(tile_grid(kTileSmall, ccap)), dim3(kBlock), 0, s, nb.cand_vf,
                      nb.cand_ee, nb.d_ncand_vf, nb.vf_cap, nb.d_nnear, nb.near_ids, nb.cplan,
                      nb.ccp, nb.croot, nb.hit_flag, nb.tile_pre, nb.vf_out_cap, nb.ee_out_cap, x,
                      v, th, dt, dcd, nb.vf_v, nb.vf_w, nb.vf_tn, nb.ee_v, nb.ee_w, nb.ee_tn,
@@ -1013,9 +1069,9 @@ int launch_narrow(const NarrowBufs& nb, const int4* tri, const float4* x, const 
 int launch_ccd_plan_only(const NarrowBufs& nb, const float4* x, const float4* v, float th,
                          float dt, int dcd, hipStream_t s) {
   const int64_t ccap = nb.vf_cap + nb.ee_cap;
-  hipLaunchKernelGGL(k_ccd_plan, dim3(tile_grid(ccap, kBig)), dim3(kBlock), 0, s, nb.cand_vf,
+  hipLaunchKernelGGL(k_ccd_plan, dim3(tile_grid(kTilePlan, ccap)), dim3(kBlock), 0, s, nb.cand_vf,
                      nb.cand_ee, nb.d_ncand_vf, nb.d_ncand_ee, nb.vf_cap, nb.ee_cap, x, v, th, dt,
-                     dcd, nb.cplan, nb.ccp, nb.croot, nb.d_ntotal, nb.hit_flag, nb.tile_sum);
+                     dcd, nb.cplan, nb.ccp, nb.croot, nb.d_ntotal, nb.near_mask, nb.tile_sum);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }

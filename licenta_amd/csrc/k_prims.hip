@@ -396,14 +396,18 @@ __device__ __forceinline__ unsigned long long unpack31(unsigned long long st) {
 }
 
 __global__ void __launch_bounds__(kBlock) k_scan_tiles(
-    const int* __restrict__ d_items, int per_tile, int ntile_max, const int* sums, int* pre,
-    int packed, int64_t cap0, int64_t cap1, int* __restrict__ d_tot0, int* __restrict__ d_tot1,
+    const int* __restrict__ d_items, TileRule rule, int n_max, const int* sums, int* pre, int packed,
+    int64_t cap0, int64_t cap1, int* __restrict__ d_tot0, int* __restrict__ d_tot1,
     int* __restrict__ ctr, unsigned long long* __restrict__ state) {
   __shared__ unsigned long long lds[kBlock / 64 + 1];
   __shared__ unsigned long long s_prefix;
   __shared__ int s_tile, s_last;
-  const int items = d_items ? max(0, *d_items) : ntile_max * per_tile;
-  const int n = min(ntile_max, (items + per_tile - 1) / per_tile);
+  int n = n_max;  // tiles; with d_items, the tiles of at most n_max items
+  if (d_items) {
+    const int items = min(max(0, *d_items), n_max);
+    const int per = 64 * tile_lanes(rule, items);
+    n = items / per + (items % per != 0);
+  }
   const int ntiles = (n + kScanTile - 1) / kScanTile;
   const int lane = lane_id(), wid = threadIdx.x >> 6;
   if (n == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
@@ -557,16 +561,29 @@ int scan_exclusive(const int* in, int* out, int n_max, const int* d_n, int* d_to
   return CM_OK;
 }
 
-int scan_tiles(const int* d_items, int per_tile, int ntile_max, const int* sums, int* pre,
-               int packed, int64_t cap0, int64_t cap1, int* d_tot0, int* d_tot1, void* temp,
-               hipStream_t s) {
+static int scan_tiles_grid(const int* d_items, TileRule rule, int n_max, int64_t ntile, const int* sums,
+                    int* pre, int packed, int64_t cap0, int64_t cap1, int* d_tot0, int* d_tot1,
+                    void* temp, hipStream_t s) {
   int* ctr = (int*)temp;
   unsigned long long* state = (unsigned long long*)((char*)temp + 256);
-  const int grid = std::min(lookback_tiles(ntile_max), kScanMaxGrid);
-  hipLaunchKernelGGL(k_scan_tiles, dim3(grid), dim3(kBlock), 0, s, d_items, per_tile, ntile_max,
-                     sums, pre, packed, cap0, cap1, d_tot0, d_tot1, ctr, state);
+  const int grid = std::min(lookback_tiles(ntile), kScanMaxGrid);
+  hipLaunchKernelGGL(k_scan_tiles, dim3(grid), dim3(kBlock), 0, s, d_items, rule, n_max, sums, pre,
+                     packed, cap0, cap1, d_tot0, d_tot1, ctr, state);
   CM_LAUNCH_CHECK();
   return CM_OK;
+}
+
+int scan_tiles(int n, const int* sums, int* pre, int packed, int64_t cap0, int64_t cap1,
+               int* d_tot0, int* d_tot1, void* temp, hipStream_t s) {
+  return scan_tiles_grid(nullptr, kTileSmall, n, n, sums, pre, packed, cap0, cap1, d_tot0, d_tot1,
+                         temp, s);
+}
+
+int scan_tiles_dev(const int* d_items, TileRule rule, int64_t item_cap, const int* sums, int* pre,
+                   int packed, int64_t cap0, int64_t cap1, int* d_tot0, int* d_tot1, void* temp,
+                   hipStream_t s) {
+  return scan_tiles_grid(d_items, rule, (int)item_cap, tile_max(rule, item_cap), sums, pre, packed,
+                         cap0, cap1, d_tot0, d_tot1, temp, s);
 }
 
 int fill_i32(int* p, int v, int64_t n, hipStream_t s) {
