@@ -1008,9 +1008,8 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
     if (sorted) {
       nb.sorted_csr = true;
       if ((rc = dalloc(b, &nb.skey, 2 * (size_t)rcap)) ||
-          (rc = dalloc(b, (char**)&nb.sort_temp, radix_sort_dev_temp_bytes())))
+          (rc = dalloc(b, (char**)&nb.sort_hist, radix_sort_dev_temp_bytes())))
         return fail(rc);
-      CM_HIP(hipMemset(nb.sort_temp, 0, radix_sort_dev_temp_bytes()));
     }
   }
   CM_HIP(hipMemset(nb.dprefix, 0, sizeof(int) * ((size_t)n + 1)));

@@ -97,12 +97,27 @@ int radix_sort_clear(void* temp, int n, hipStream_t s);  // before the first sor
 // Stable LSD sort of the first min(*d_n, n_max) 32-bit keys (key_bits <= 32) with
 // their values, with a launch shape independent of the count (graph-capturable). The
 // result ends in keys_alt / vals_alt when *in_alt is set (an odd number of passes),
-// else in keys / vals. temp: radix_sort_dev_temp_bytes(), cleared once before its
-// first sort by radix_sort_dev_clear.
+// else in keys / vals. hist (radix_sort_dev_temp_bytes()) holds the digit counts of the
+// low 8 bits by workgroup, hist[256 * block + digit] over dev_sort_range's keys: the
+// kernel that writes the keys counts them.
+constexpr int kSortItems = 8;                   // keys per thread per tile
+constexpr int kSortTile = kBlock * kSortItems;  // 2048 keys
+// 256 workgroups of a few tiles: 1.16 M records of 96 cloths 110 us for the list, as with
+// 1,024 and a scan in each pass (128: 124, 512: 121), none to 280,000 records 37 -> 22 (64^2)
+// and 52 -> 47 us (draped 256^2).
+constexpr int kDevSortBlocks = 256;
+struct DevSortRange {
+  int n, t0, t1, blocks;  // keys, this workgroup's tiles, workgroups that have any
+};
+__device__ __forceinline__ DevSortRange dev_sort_range(int n) {
+  const int ntiles = (n + kSortTile - 1) / kSortTile;
+  const int per = max(1, (ntiles + kDevSortBlocks - 1) / kDevSortBlocks);
+  const int t0 = min(ntiles, (int)blockIdx.x * per);
+  return {n, t0, min(ntiles, t0 + per), (ntiles + per - 1) / per};
+}
 size_t radix_sort_dev_temp_bytes();
-int radix_sort_dev_clear(void* temp, hipStream_t s);
 int radix_sort_dev(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt,
-                   int n_max, const int* d_n, int key_bits, void* temp, int* in_alt,
+                   int n_max, const int* d_n, int key_bits, int* hist, int* in_alt,
                    hipStream_t s);
 int fill_i32(int* p, int v, int64_t n, hipStream_t s);
 int fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s);
@@ -220,11 +235,11 @@ struct NarrowBufs {
   int* dlong = nullptr;      // n: vertices whose record lists are ordered by a workgroup
   // sorted_csr: the CSR comes from one radix sort of the records by vertex id
   // (else from per-vertex counts and atomic placement). skey: record keys then
-  // alternate keys (2 * 4 * (vf_out_cap + ee_out_cap)), sort_temp:
+  // alternate keys (2 * 4 * (vf_out_cap + ee_out_cap)), sort_hist:
   // radix_sort_dev_temp_bytes()
   bool sorted_csr = false;
   uint32_t* skey = nullptr;
-  void* sort_temp = nullptr;
+  int* sort_hist = nullptr;
   int* d_nrec = nullptr;     // records of the substep (sorted CSR)
   uint32_t* warn = nullptr;
   void* scan_temp = nullptr;

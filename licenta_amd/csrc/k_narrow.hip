@@ -947,7 +947,8 @@ __global__ void __launch_bounds__(kBlock) k_dyn_sort_long(const int* __restrict_
 
 // ---- sorted CSR: the records keyed by vertex id through the stable radix sort --------
 // record r = 4c + role of contact c (VF then EE) is keyed by that vertex; a stable
-// sort leaves each vertex's records in increasing r, the order k_dyn_sort gives
+// sort leaves each vertex's records in increasing r, the order k_dyn_sort gives. A
+// workgroup writes the keys of its tiles of the sort and counts their low 8 bits.
 __global__ void __launch_bounds__(kBlock) k_rec_keys(const int4* __restrict__ vfv,
                                                      const int4* __restrict__ eev,
                                                      const int* __restrict__ d_nvf,
@@ -955,15 +956,28 @@ __global__ void __launch_bounds__(kBlock) k_rec_keys(const int4* __restrict__ vf
                                                      const int* __restrict__ rank,
                                                      uint4* __restrict__ keys,
                                                      uint4* __restrict__ vals,
-                                                     int* __restrict__ d_nrec) {
-  const int nvf = *d_nvf, nee = *d_nee;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *d_nrec = 4 * (nvf + nee);
-  for (int c = blockIdx.x * kBlock + threadIdx.x; c < nvf + nee; c += gridDim.x * kBlock) {
+                                                     int* __restrict__ d_nrec,
+                                                     int* __restrict__ hist) {
+  __shared__ int h[256];
+  const int nvf = *d_nvf, nc = nvf + *d_nee;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *d_nrec = 4 * nc;
+  const DevSortRange r = dev_sort_range(4 * nc);
+  if (r.t0 >= r.t1) return;
+  h[threadIdx.x] = 0;
+  __syncthreads();
+  const int c1 = min(nc, r.t1 * (kSortTile / 4));
+  for (int c = r.t0 * (kSortTile / 4) + threadIdx.x; c < c1; c += kBlock) {
     const int4 q = ranked(c < nvf ? vfv[c] : eev[c - nvf], rank);
     keys[c] = make_uint4((uint32_t)q.x, (uint32_t)q.y, (uint32_t)q.z, (uint32_t)q.w);
-    const uint32_t r = 4u * (uint32_t)c;
-    vals[c] = make_uint4(r, r + 1u, r + 2u, r + 3u);
+    const uint32_t k = 4u * (uint32_t)c;
+    vals[c] = make_uint4(k, k + 1u, k + 2u, k + 3u);
+    atomicAdd(&h[q.x & 255], 1);
+    atomicAdd(&h[q.y & 255], 1);
+    atomicAdd(&h[q.z & 255], 1);
+    atomicAdd(&h[q.w & 255], 1);
   }
+  __syncthreads();
+  hist[blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
 }
 
 // From the sorted keys and values: dprefix[v] = the number of keys below v (binary
@@ -1084,13 +1098,14 @@ int launch_dynamic_csr(const NarrowBufs& nb, hipStream_t s) {
     const int64_t rcap = 4 * (nb.vf_out_cap + nb.ee_out_cap);
     uint32_t* keys = nb.skey;
     uint32_t* kalt = nb.skey + rcap;
-    hipLaunchKernelGGL(k_rec_keys, dim3(gc), dim3(kBlock), 0, s, nb.vf_v, nb.ee_v, nb.d_nvf,
-                       nb.d_nee, nb.rank, (uint4*)keys, (uint4*)nb.drec, nb.d_nrec);
+    hipLaunchKernelGGL(k_rec_keys, dim3(kDevSortBlocks), dim3(kBlock), 0, s, nb.vf_v, nb.ee_v,
+                       nb.d_nvf, nb.d_nee, nb.rank, (uint4*)keys, (uint4*)nb.drec, nb.d_nrec,
+                       nb.sort_hist);
     int bits = 1;
     while (bits < 32 && ((int64_t)1 << bits) < nb.n) ++bits;
     int in_alt = 0;
     int rc = radix_sort_dev(keys, nb.drec, kalt, nb.dtmp, (int)rcap, nb.d_nrec, bits,
-                            nb.sort_temp, &in_alt, s);
+                            nb.sort_hist, &in_alt, s);
     if (rc) return rc;
     hipLaunchKernelGGL(k_rec_place, dim3(grid_for(std::max<int64_t>(rcap, nb.n + 1))),
                        dim3(kBlock), 0, s, nb.n, in_alt ? kalt : keys, in_alt ? nb.dtmp : nb.drec,

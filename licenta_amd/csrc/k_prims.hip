@@ -173,12 +173,25 @@ __global__ void k_fill_i32(int* __restrict__ p, int v, int64_t n) {
 }
 
 // ---- radix sort ------------------------------------------------------------
-constexpr int kSortItems = 8;                    // keys per thread per tile
-constexpr int kSortTile = kBlock * kSortItems;   // 2048 keys per block
 constexpr int kWaves = kBlock / 64;
 
+// Lanes whose digit equals this lane's, among those in `valid`. A bit costs a shift, a
+// compare, and an xor and an and for each half of the mask (before, with a select for each
+// half: 2.1 M keys of 30 bits 231 us, now 172).
+__device__ __forceinline__ uint64_t match_digit(uint32_t d, uint64_t valid) {
+  uint64_t m = valid;
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const int sx = (int)(d << (31 - b)) >> 31;  // the bit in every place
+    m &= ~(__ballot(sx != 0) ^ (uint64_t)(int64_t)sx);
+  }
+  return m;
+}
+
+// Digit counts of each tile: hist[digit * nblk + tile] for the scan, or, with by_tile,
+// hist[tile * 256 + digit] for scatter kernels that add up the tiles before theirs.
 __global__ void __launch_bounds__(kBlock) k_radix_hist(const uint64_t* __restrict__ keys, int n,
-                                                       int shift, int nblk,
+                                                       int shift, int nblk, int by_tile,
                                                        int* __restrict__ hist) {
   __shared__ int h[256];
   h[threadIdx.x] = 0;
@@ -190,11 +203,39 @@ __global__ void __launch_bounds__(kBlock) k_radix_hist(const uint64_t* __restric
     if (i < n) atomicAdd(&h[(keys[i] >> shift) & 255u], 1);
   }
   __syncthreads();
-  hist[threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
+  hist[by_tile ? blockIdx.x * 256 + threadIdx.x : threadIdx.x * nblk + blockIdx.x] =
+      h[threadIdx.x];
+}
+
+// Up to this many tiles a scatter kernel adds up the tiles' digit counts itself, which costs
+// it about 1 us where the scan is a launch of 5: 32,258 keys of 30 bits 73 -> 53 us, 130,050
+// 79 -> 60. Every tile reads all counts, so many tiles are left to the scan: 500,000 keys
+// 91 us by the scan, 93 or more by the tiles.
+constexpr int kByTileMax = 64;
+
+// Where thread d's digit begins for block blk of nblk, from hist[block * 256 + digit]: the
+// digits below it and the blocks before this one.
+__device__ __forceinline__ int digit_start(const int* __restrict__ hist, int blk, int nblk) {
+  __shared__ int lds[kBlock / 64 + 1];
+  int before = 0, total = 0;
+  for (int b0 = 0; b0 < nblk; b0 += 16) {  // 16 loads at a time, also for the last few
+    int v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = hist[min(b0 + j, nblk - 1) * 256 + threadIdx.x];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      before += b0 + j < blk ? v[j] : 0;
+      total += b0 + j < nblk ? v[j] : 0;
+    }
+  }
+  int all;
+  return block_excl_scan(total, lds, all) + before;
 }
 
 // Stable scatter: wave w ranks the contiguous slice [w*64*ITEMS, (w+1)*64*ITEMS)
 // of the tile in order, using 8 ballots per 64-key chunk to find equal digits.
+// kByTile: offsets holds the tiles' digit counts, else where each (digit, tile) begins.
+template <bool kByTile>
 __global__ void __launch_bounds__(kBlock) k_radix_scatter(
     const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, int n, int shift, int nblk,
@@ -209,6 +250,8 @@ __global__ void __launch_bounds__(kBlock) k_radix_scatter(
   uint32_t val[kSortItems];
   int rank[kSortItems];
   const uint64_t lt = (1ull << lane) - 1ull;
+  const int start = kByTile ? digit_start(offsets, blockIdx.x, nblk)
+                            : offsets[threadIdx.x * nblk + blockIdx.x];
 #pragma unroll
   for (int c = 0; c < kSortItems; ++c) {
     const int i = base + c * 64 + lane;
@@ -216,13 +259,7 @@ __global__ void __launch_bounds__(kBlock) k_radix_scatter(
     key[c] = valid ? kin[i] : 0ull;
     val[c] = valid ? vin[i] : 0u;
     const uint32_t d = (uint32_t)(key[c] >> shift) & 255u;
-    uint64_t m = __ballot(valid);
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const bool bit = (d >> b) & 1u;
-      const uint64_t bb = __ballot(bit);
-      m &= bit ? bb : ~bb;
-    }
+    const uint64_t m = match_digit(d, __ballot(valid));
     int r = 0;
     if (valid) {
       const int before = __popcll(m & lt);
@@ -235,7 +272,7 @@ __global__ void __launch_bounds__(kBlock) k_radix_scatter(
   __syncthreads();
   {
     const int d = threadIdx.x;  // kBlock == 256 digits
-    int run = 0;
+    int run = start;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
       wbase[w][d] = run;
@@ -248,110 +285,206 @@ __global__ void __launch_bounds__(kBlock) k_radix_scatter(
     const int i = base + c * 64 + lane;
     if (i < n) {
       const uint32_t d = (uint32_t)(key[c] >> shift) & 255u;
-      const int pos = offsets[d * nblk + blockIdx.x] + wbase[wid][d] + rank[c];
+      const int pos = wbase[wid][d] + rank[c];
       kout[pos] = key[c];
       vout[pos] = val[c];
     }
   }
 }
 
-// ---- radix sort of 32-bit keys with a device-side count --------------------------
-// A fixed grid of kDevSortBlocks workgroups; workgroup b takes the contiguous run of
-// tiles [b * tpb, (b + 1) * tpb) of the n = min(*d_n, n_max) keys (tpb = ceil(tiles /
-// grid)), so one histogram per workgroup keeps the sort stable and the launch shape
-// does not depend on n.
-constexpr int kDevSortBlocks = 1024;
+// ---- radix sort in one workgroup ---------------------------------------------------
+// Up to kBlockSort keys are sorted by one workgroup, the keys (their low 32 bits where no
+// higher one is sorted by) and their 16-bit places in its LDS, in one launch for all
+// passes. A thread holds its keys in registers from one pass's read to the next one's
+// write. Bound by the ranking (about four vector instructions a bit for 64 keys) on one
+// CU, so longer sorts go to the whole chip. 6,962 keys of 30 bits 69 -> 33 us, of 63 bits
+// 136 -> 64; 8,192 keys 68 -> 37 (51 on the whole chip), 12,000 keys
+// 72 -> 51 there and 54 here.
+constexpr int kSortThreads = 1024, kSortWaves = kSortThreads / 64;
+constexpr int kBlockItems = 8;  // most keys per thread
+constexpr int kBlockSort = kBlockItems * kSortThreads;
+constexpr int kSortHead = sizeof(int) * (kSortWaves * 256 + 4);
 
-__device__ __forceinline__ void dev_sort_range(const int* d_n, int n_max, int& n, int& t0,
-                                               int& t1) {
-  n = min(*d_n, n_max);
-  const int ntiles = (n + kSortTile - 1) / kSortTile;
-  const int tpb = (ntiles + gridDim.x - 1) / gridDim.x;
-  t0 = min(ntiles, blockIdx.x * tpb);
-  t1 = min(ntiles, t0 + tpb);
+template <typename K>
+__global__ void __launch_bounds__(kSortThreads) k_sort_block(uint64_t* keys, uint32_t* vals, int n,
+                                                             int passes) {
+  extern __shared__ char sort_lds[];
+  int(*cnt)[256] = (int(*)[256])sort_lds;  // per wave and digit: count, then first place
+  int* wtot = (int*)(cnt + kSortWaves);    // 4: digit totals of 64 digits
+  K* skey = (K*)(wtot + 4);
+  uint16_t* sidx = (uint16_t*)(skey + n);
+  const int lane = lane_id(), wid = threadIdx.x >> 6;
+  const uint64_t below = (1ull << lane) - 1ull;
+  // wave w takes the n items in order from w * per
+  const int items = (n + kSortThreads - 1) / kSortThreads;
+  const int base = wid * 64 * items + lane;
+  K key[kBlockItems];
+  uint32_t at[kBlockItems];  // place in the caller's order (low half), rank in the wave (high)
+#pragma unroll
+  for (int c = 0; c < kBlockItems; ++c) {
+    const int i = base + c * 64;
+    key[c] = c < items && i < n ? (K)keys[i] : (K)0;
+    at[c] = (uint32_t)i & 0xffffu;
+  }
+  for (int pass = 0; pass < passes; ++pass) {
+    const int shift = 8 * pass;
+    for (int d = lane; d < 256; d += 64) cnt[wid][d] = 0;
+#pragma unroll
+    for (int c = 0; c < kBlockItems; ++c) {
+      if (c >= items) break;
+      const bool valid = base + c * 64 < n;
+      const uint32_t d = (uint32_t)(key[c] >> shift) & 255u;
+      const uint64_t m = match_digit(d, __ballot(valid));
+      const int before = __popcll(m & below);
+      if (valid) {
+        const int old = cnt[wid][d];
+        if (before == 0) cnt[wid][d] = old + __popcll(m);
+        at[c] |= (uint32_t)(old + before) << 16;
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < 256) {
+      int run = 0;
+#pragma unroll
+      for (int w = 0; w < kSortWaves; ++w) {
+        const int v = cnt[w][threadIdx.x];
+        cnt[w][threadIdx.x] = run;
+        run += v;
+      }
+      const int inc = wave_incl_scan(run);
+      if (lane == 63) wtot[wid] = inc;
+      cnt[0][threadIdx.x] = inc - run;  // wave 0's own base is 0: here the digit's base
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < kBlockItems; ++c) {
+      if (c >= items) break;
+      if (base + c * 64 < n) {
+        const uint32_t d = (uint32_t)(key[c] >> shift) & 255u;
+        int pos = cnt[0][d] + (int)(at[c] >> 16) + (wid ? cnt[wid][d] : 0);
+#pragma unroll
+        for (int w = 0; w < 3; ++w) pos += (int)(d >> 6) > w ? wtot[w] : 0;
+        skey[pos] = key[c];
+        sidx[pos] = (uint16_t)at[c];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < kBlockItems; ++c) {
+      const int i = base + c * 64;
+      if (c < items && i < n) {
+        key[c] = skey[i];
+        at[c] = sidx[i];
+      }
+    }
+  }
+  // whole keys and values from the caller's order; all are read before one is written
+  uint64_t k64[kBlockItems];
+  uint32_t v32[kBlockItems];
+#pragma unroll
+  for (int c = 0; c < kBlockItems; ++c)
+    if (c < items && base + c * 64 < n) {
+      k64[c] = keys[at[c]];
+      v32[c] = vals[at[c]];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < kBlockItems; ++c)
+    if (c < items && base + c * 64 < n) {
+      keys[base + c * 64] = k64[c];
+      vals[base + c * 64] = v32[c];
+    }
 }
 
+// ---- radix sort of 32-bit keys with a device-side count --------------------------
+// A fixed grid of kDevSortBlocks workgroups; workgroup b takes the run of tiles that
+// dev_sort_range gives it, so one histogram per workgroup keeps the sort stable and the
+// launch shape does not depend on n. A workgroup adds up the counts of the workgroups
+// before it (digit_start), which a few workgroups do faster than a scan's launch takes.
 __global__ void __launch_bounds__(kBlock) k_radix_hist_dev(const uint32_t* __restrict__ keys,
                                                            const int* __restrict__ d_n, int n_max,
                                                            int shift, int* __restrict__ hist) {
   __shared__ int h[256];
+  const DevSortRange r = dev_sort_range(min(*d_n, n_max));
+  if (r.t0 >= r.t1) return;
   h[threadIdx.x] = 0;
   __syncthreads();
-  int n, t0, t1;
-  dev_sort_range(d_n, n_max, n, t0, t1);
-  for (int tile = t0; tile < t1; ++tile) {
+  for (int tile = r.t0; tile < r.t1; ++tile) {
 #pragma unroll
     for (int k = 0; k < kSortItems; ++k) {
       const int i = tile * kSortTile + k * kBlock + threadIdx.x;
-      if (i < n) atomicAdd(&h[(keys[i] >> shift) & 255u], 1);
+      if (i < r.n) atomicAdd(&h[(keys[i] >> shift) & 255u], 1);
     }
   }
   __syncthreads();
-  hist[threadIdx.x * gridDim.x + blockIdx.x] = h[threadIdx.x];
+  hist[blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
 }
 
-// k_radix_scatter over the workgroup's run of tiles, each digit's running base carried
+// k_radix_scatter over the workgroup's run of tiles, each digit's running place carried
 // from tile to tile (thread d owns digit d of carry, wbase and the count sums)
 __global__ void __launch_bounds__(kBlock) k_radix_scatter_dev(
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, const int* __restrict__ d_n,
-    int n_max, int shift, const int* __restrict__ offsets) {
+    int n_max, int shift, const int* __restrict__ hist) {
   __shared__ int cnt[kWaves][256];
   __shared__ int wbase[kWaves][256];
-  __shared__ int carry[256];
+  const DevSortRange r = dev_sort_range(min(*d_n, n_max));
+  if (r.t0 >= r.t1) return;
   const int lane = lane_id(), wid = threadIdx.x >> 6;
-  int n, t0, t1;
-  dev_sort_range(d_n, n_max, n, t0, t1);
-  carry[threadIdx.x] = 0;
+  int carry = digit_start(hist, blockIdx.x, r.blocks);
   const uint64_t lt = (1ull << lane) - 1ull;
-  for (int tile = t0; tile < t1; ++tile) {
+  uint32_t nkey[kSortItems], nval[kSortItems];  // the next tile's, loaded a tile ahead
+  auto load = [&](int tile) {
+#pragma unroll
+    for (int c = 0; c < kSortItems; ++c) {
+      const int i = min(tile * kSortTile + (wid * kSortItems + c) * 64 + lane, r.n - 1);
+      nkey[c] = kin[i];
+      nval[c] = vin[i];
+    }
+  };
+  load(r.t0);
+  for (int tile = r.t0; tile < r.t1; ++tile) {
     for (int d = threadIdx.x; d < kWaves * 256; d += kBlock) (&cnt[0][0])[d] = 0;
-    __syncthreads();
     const int base = tile * kSortTile + wid * 64 * kSortItems;
-    uint32_t key[kSortItems];
-    uint32_t val[kSortItems];
+    uint32_t key[kSortItems], val[kSortItems];
     int rank[kSortItems];
 #pragma unroll
     for (int c = 0; c < kSortItems; ++c) {
-      const int i = base + c * 64 + lane;
-      const bool valid = i < n;
-      key[c] = valid ? kin[i] : 0u;
-      val[c] = valid ? vin[i] : 0u;
-      const uint32_t d = (key[c] >> shift) & 255u;
-      uint64_t m = __ballot(valid);
+      key[c] = nkey[c];
+      val[c] = nval[c];
+    }
+    if (tile + 1 < r.t1) load(tile + 1);
+    __syncthreads();
 #pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        const bool bit = (d >> b) & 1u;
-        const uint64_t bb = __ballot(bit);
-        m &= bit ? bb : ~bb;
-      }
-      int r = 0;
+    for (int c = 0; c < kSortItems; ++c) {
+      const bool valid = base + c * 64 + lane < r.n;
+      const uint32_t d = (key[c] >> shift) & 255u;
+      const uint64_t m = match_digit(d, __ballot(valid));
+      int q = 0;
       if (valid) {
         const int before = __popcll(m & lt);
         const int old = cnt[wid][d];
-        r = old + before;
+        q = old + before;
         if (before == 0) cnt[wid][d] = old + __popcll(m);
       }
-      rank[c] = r;
+      rank[c] = q;
     }
     __syncthreads();
     {
       const int d = threadIdx.x;  // kBlock == 256 digits
-      int run = carry[d];
 #pragma unroll
       for (int w = 0; w < kWaves; ++w) {
-        wbase[w][d] = run;
-        run += cnt[w][d];
+        wbase[w][d] = carry;
+        carry += cnt[w][d];
       }
-      carry[d] = run;
     }
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < kSortItems; ++c) {
       const int i = base + c * 64 + lane;
-      if (i < n) {
+      if (i < r.n) {
         const uint32_t d = (key[c] >> shift) & 255u;
-        const int pos = offsets[d * gridDim.x + blockIdx.x] + wbase[wid][d] + rank[c];
+        const int pos = wbase[wid][d] + rank[c];
         kout[pos] = key[c];
         vout[pos] = val[c];
       }
@@ -613,28 +746,18 @@ int radix_sort_clear(void* temp, int n, hipStream_t s) {
   return scan_temp_clear(tp, 256 * nb, s);
 }
 
-size_t radix_sort_dev_temp_bytes() {
-  return align_up(sizeof(int) * 256 * kDevSortBlocks) + scan_temp_bytes(256 * kDevSortBlocks);
-}
-
-int radix_sort_dev_clear(void* temp, hipStream_t s) {
-  return scan_temp_clear((char*)temp + align_up(sizeof(int) * 256 * kDevSortBlocks),
-                         256 * kDevSortBlocks, s);
-}
+size_t radix_sort_dev_temp_bytes() { return align_up(sizeof(int) * 256 * kDevSortBlocks); }
 
 int radix_sort_dev(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt,
-                   int n_max, const int* d_n, int key_bits, void* temp, int* in_alt,
+                   int n_max, const int* d_n, int key_bits, int* hist, int* in_alt,
                    hipStream_t s) {
-  int* hist = (int*)temp;
-  void* stemp = (char*)temp + align_up(sizeof(int) * 256 * kDevSortBlocks);
   const int passes = std::min(4, (key_bits + 7) / 8);
   uint32_t *ka = keys, *va = vals, *kb = keys_alt, *vb = vals_alt;
   for (int pass = 0; pass < passes; ++pass) {
     const int shift = 8 * pass;
-    hipLaunchKernelGGL(k_radix_hist_dev, dim3(kDevSortBlocks), dim3(kBlock), 0, s, ka, d_n, n_max,
-                       shift, hist);
-    int rc = scan_exclusive(hist, hist, 256 * kDevSortBlocks, nullptr, nullptr, stemp, s);
-    if (rc) return rc;
+    if (pass > 0)
+      hipLaunchKernelGGL(k_radix_hist_dev, dim3(kDevSortBlocks), dim3(kBlock), 0, s, ka, d_n,
+                         n_max, shift, hist);
     hipLaunchKernelGGL(k_radix_scatter_dev, dim3(kDevSortBlocks), dim3(kBlock), 0, s, ka, va, kb,
                        vb, d_n, n_max, shift, hist);
     CM_LAUNCH_CHECK();
@@ -642,6 +765,17 @@ int radix_sort_dev(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t*
     std::swap(va, vb);
   }
   *in_alt = passes & 1;
+  return CM_OK;
+}
+
+template <typename K>
+static int sort_block(uint64_t* keys, uint32_t* vals, int n, int passes, hipStream_t s) {
+  const size_t lds = kSortHead + (sizeof(K) + 2) * (size_t)n;
+  CM_HIP(hipFuncSetAttribute((const void*)k_sort_block<K>,
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(k_sort_block<K>, dim3(1), dim3(kSortThreads), lds, s, keys, vals, n,
+                     passes);
+  CM_LAUNCH_CHECK();
   return CM_OK;
 }
 
@@ -658,17 +792,26 @@ int radix_sort(uint64_t* keys, uint32_t* vals, int n, int key_bits, void* temp, 
   void* stemp = tp;
   int passes = (key_bits + 7) / 8;
   if (passes & 1) ++passes;  // even number of passes: result ends in the input buffers
+  if (n <= kBlockSort)
+    return passes <= 4 ? sort_block<uint32_t>(keys, vals, n, passes, s)
+                       : sort_block<uint64_t>(keys, vals, n, passes, s);
   uint64_t* ka = keys;
   uint32_t* va = vals;
   uint64_t* kb = kalt;
   uint32_t* vb = valt;
   for (int pass = 0; pass < passes; ++pass) {
     const int shift = 8 * pass;
-    hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(kBlock), 0, s, ka, n, shift, nb, hist);
-    int rc = scan_exclusive(hist, hist, 256 * nb, nullptr, nullptr, stemp, s);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(kBlock), 0, s, ka, va, kb, vb, n, shift,
-                       nb, hist);
+    const bool by_tile = nb <= kByTileMax;
+    hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(kBlock), 0, s, ka, n, shift, nb, by_tile, hist);
+    if (by_tile) {
+      hipLaunchKernelGGL(k_radix_scatter<true>, dim3(nb), dim3(kBlock), 0, s, ka, va, kb, vb, n,
+                         shift, nb, hist);
+    } else {
+      int rc = scan_exclusive(hist, hist, 256 * nb, nullptr, nullptr, stemp, s);
+      if (rc) return rc;
+      hipLaunchKernelGGL(k_radix_scatter<false>, dim3(nb), dim3(kBlock), 0, s, ka, va, kb, vb, n,
+                         shift, nb, hist);
+    }
     CM_LAUNCH_CHECK();
     std::swap(ka, kb);
     std::swap(va, vb);
