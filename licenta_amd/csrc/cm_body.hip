@@ -924,12 +924,16 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
   // two-pass traversal: leaves still walking after the budget's visits are finished
   // by whole waves; up to a quarter of the leaves can be handed over, the rest walk on
   // in the first pass. Off for caps above 96 (the second pass keeps at most 256 pairs
-  // per leaf). CLOTHMI_TRAV_BUDGET overrides the budget (0: one pass); the pairs are
-  // the same with any budget.
+  // per leaf). CLOTHMI_TRAV_BUDGET overrides the budget (0: one pass) and has small
+  // bodies, whose leaves groups of lanes walk, take these passes too; the pairs are the
+  // same with any budget.
   if ((rc = dalloc(b, &b->lb.spill, (size_t)t * kTravSpill))) return fail(rc);
   {
     int budget = params->pair_cap <= 96 ? 200 : 0;
-    if (const char* e = std::getenv("CLOTHMI_TRAV_BUDGET")) budget = std::max(0, std::atoi(e));
+    if (const char* e = std::getenv("CLOTHMI_TRAV_BUDGET")) {
+      budget = std::max(0, std::atoi(e));
+      b->lb.group = false;
+    }
     if (budget > 0 && t >= 2 && t < (1 << 26)) {
       b->lb.rcap = t / 4 + 1024;
       if ((rc = dalloc(b, &b->lb.trec, (size_t)b->lb.rcap * kTravRec))) return fail(rc);

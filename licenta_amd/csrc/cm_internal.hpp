@@ -140,6 +140,7 @@ struct LbvhBufs {
   int *state = nullptr, *top_list = nullptr, *top_index = nullptr, *ntop = nullptr;
   float4 *tmin = nullptr, *tmax = nullptr;  // deferred-node scratch (large trees)
   int *trm = nullptr, *tdone = nullptr;
+  bool group = true;        // few leaves may be walked by groups of lanes
   uint4* qnodes = nullptr;  // quantised record of each internal node, 2 uint4 (k_lbvh.hip)
   int* irr = nullptr;       // set when the tree has to be walked through its exact boxes
   int trav_chunk = 4;       // traversal: tiles per chunk dealt to one XCD (launch shape only)

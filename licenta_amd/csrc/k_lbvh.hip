@@ -1229,6 +1229,235 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse_lanes(
   if ((threadIdx.x & 63) == 0 && w) atomicOr(warn, w);
 }
 
+// ---- a group of lanes per leaf ----------------------------------------------------
+// On a tree of few leaves the first pass above leaves most of the chip idle behind its
+// longest walk (64^2: 124 waves on 1,024 SIMDs, 200 dependent visits of about 0.4 us).
+// Here kG lanes expand up to kG pending nodes of one leaf at once, with the keys and the
+// order of k_traverse_resume (rank 0: the root is the one subtree). The leaves they meet
+// join the hits by the quantised test alone and are tested exactly, kG at a time, when
+// there are more than the cap of them and at the end. A leaf that overflows the buffers
+// or the path bits, or could reach the stack limit, and any leaf of an irregular tree, is
+// left to k_traverse_redo. Bound by the rounds' latency (about 1,550 cycles, a third of them
+// the records' loads; 16 to 18 rounds at 64^2), on draped cloths by the instructions.
+// k_traverse -> k_traverse_group: 60^2 72 -> 17 us, 64^2 94 -> 25, 96x83 119 -> 42, flat
+// 128^2 112 -> 63, draped 131x97 164 (and 16 for k_traverse_resume) -> 134.
+constexpr int kGroup = 16;  // 8: 22, 34, 41, 64 and 143 us below
+constexpr int kGroupPend = 128, kGroupHits = 112;
+constexpr int kGroupMaxCap = kGroupHits - 1 - 2 * kGroup;
+// Up to this many leaves. A flat cloth gains beyond it (256^2 354 -> 256 us), a draped one,
+// whose leaves meet several times the cap, loses (329 -> 700).
+constexpr int kGroupLeaves = 1 << 15;
+
+template <int kG>
+__device__ __forceinline__ int group_sum(int v) {
+#pragma unroll
+  for (int o = kG / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, kG);
+  return v;
+}
+
+template <int kG>
+__global__ void __launch_bounds__(64) k_traverse_group(WalkTree T, int cap,
+                                                       int* __restrict__ chunk,
+                                                       int* __restrict__ counts,
+                                                       uint32_t* __restrict__ warn) {
+  constexpr int kPer = 64 / kG;  // leaves per wave
+  __shared__ uint64_t spk[kPer][kGroupPend], shk[kPer][kGroupHits];
+  __shared__ int spe[kPer][kGroupPend], shp[kPer][kGroupHits];  // pe: node | stack depth << 26
+  const int lane = threadIdx.x, g = lane % kG, sub = lane / kG;
+  uint64_t *pk = spk[sub], *hk = shk[sub];
+  int *pe = spe[sub], *hp = shp[sub];
+  const uint64_t mine = ((1ull << kG) - 1ull) << (sub * kG);
+  const uint64_t below_me = mine & ((1ull << lane) - 1ull);
+  // the group's kG bits of a ballot; earlier: the group's earlier lanes in two such fields
+  auto field = [&](uint64_t b) { return (uint32_t)(b >> (sub * kG)) & ((1u << kG) - 1u); };
+  const uint32_t earlier = ((1u << g) - 1u) * (1u | 1u << kG);
+  // consecutive leaves to one XCD in chunks, as in k_traverse
+  constexpr int kRun = 4 * kTravBlock / kPer;
+  const int j = blockIdx.x / kXcds, xcd = blockIdx.x % kXcds;
+  const int leaf = (((j / kRun) * kXcds + xcd) * kRun + j % kRun) * kPer + sub;
+  const int t = T.t, nin = t - 1, stride = cap;
+  // the lanes of a wave share the buffers: their accesses stay in program order
+  auto order = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+  int root = 0;
+  bool act = leaf < t, again = false;
+  if (act && T.croot) {  // a batch: the root of the leaf's cloth, its cap
+    const int c = T.slot_cloth[leaf];
+    root = T.croot[c];
+    cap = T.ccap[c];
+    act = root >= 0;  // a one-triangle cloth has no pairs
+  }
+  if (act && *T.irr != 0) {
+    act = false;
+    again = true;
+  }
+  f3 mn = mk3(0, 0, 0), mx = mk3(0, 0, 0);
+  uint3 q = make_uint3(0, 0, 0);
+  int np = 0, nh = 0, nv = 0;  // pending, hits, hits tested (the first nv)
+  if (act) {
+    mn = xyz(T.amin[nin + leaf]);
+    mx = xyz(T.amax[nin + leaf]);
+    q = q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn);
+    if (g == 0) {
+      pe[0] = root;
+      pk[0] = 0;
+    }
+    np = 1;
+  }
+  // tests hits nv to nh exactly and closes the gaps
+  auto test_hits = [&] {
+    for (int k0 = nv; k0 < nh; k0 += kG) {
+      const int k = k0 + g;
+      int c = 0;
+      uint64_t key = 0;
+      bool keep = false;
+      if (k < nh) {
+        c = hp[k];
+        key = hk[k];
+        keep = overlap(mn, mx, xyz(T.amin[nin + c]), xyz(T.amax[nin + c]));
+      }
+      const uint64_t m = __ballot(keep);
+      if (keep) {
+        const int at = nv + __popcll(m & below_me);
+        hp[at] = c;
+        hk[at] = key;
+      }
+      nv += __popcll(m & mine);
+      order();
+    }
+    nh = nv;
+  };
+  while (act) {
+    order();
+    const int take = min(kG, np), base = np - take;
+    bool tl = false, tr = false, hl = false, hr = false, deep = false;
+    int split = 0, sd = 0;
+    uint64_t key = 0, kl = 0;
+    if (g < take) {
+      const uint32_t e = (uint32_t)pe[np - 1 - g];
+      key = pk[np - 1 - g];
+      const QNode v = q_visit(T.qnodes, (int)(e & kSplitMask), leaf, q);
+      split = v.split;
+      sd = (int)(e >> 26);
+      hl = v.l & v.lleaf;
+      hr = v.r & v.rleaf;
+      tl = v.l & !v.lleaf;
+      tr = v.r & !v.rleaf;
+      const int d = (int)((key >> 1) & 127ull);
+      deep = (tl | tr) & ((d + 1 > kPathBits) | (tl & tr & (sd >= kStack)));
+      kl = (key & ~0xffull) | ((uint64_t)(d + 1) << 1);
+    }
+    // children and hits of the group's earlier lanes
+    const uint32_t c2 = field(__ballot(tl)) | field(__ballot(tr)) << kG;
+    const uint32_t h2 = field(__ballot(hl)) | field(__ballot(hr)) << kG;
+    const int totc = __popc(c2), tote = __popc(h2);
+    if (field(__ballot(deep)) || base + totc > kGroupPend) {
+      again = true;
+      break;
+    }
+    order();
+    const int ca = base + totc - 1 - __popc(c2 & earlier), ha = nh + __popc(h2 & earlier);
+    if (tl) {
+      pe[ca] = split | (((tl & tr) ? sd + 1 : sd) << 26);
+      pk[ca] = kl;
+    }
+    if (tr) {
+      pe[ca - tl] = (split + 1) | (sd << 26);
+      pk[ca - tl] = kl | (1ull << (57 - (int)((key >> 1) & 127ull)));
+    }
+    if (hl) {
+      hp[ha] = split;
+      hk[ha] = key;
+    }
+    if (hr) {
+      hp[ha + hl] = split + 1;
+      hk[ha + hl] = key | 1ull;
+    }
+    np = base + totc;
+    nh += tote;
+    order();
+    if (nh > cap) test_hits();
+    if (nh > cap) {
+      // more than the cap of pairs are final: their keys are below every pending node's
+      const uint64_t bound = np > 0 ? pk[np - 1] : ~0ull;
+      int below = 0;
+      for (int k = g; k < nh; k += kG) below += hk[k] < bound;
+      if (group_sum<kG>(below) > cap) break;
+      if (nh + 2 * kG > kGroupHits) {
+        // keep the cap + 1 smallest keys: a larger one can only move further back
+        constexpr int kMine = (kGroupHits + kG - 1) / kG;
+        uint64_t kk[kMine];
+        int kp[kMine], rk[kMine];
+#pragma unroll
+        for (int u = 0; u < kMine; ++u) {
+          const int k = g + kG * u;
+          rk[u] = kGroupHits;
+          if (k < nh) {
+            kk[u] = hk[k];
+            kp[u] = hp[k];
+            int rank = 0;
+            for (int k2 = 0; k2 < nh; ++k2) rank += hk[k2] < kk[u];
+            rk[u] = rank;
+          }
+        }
+        order();
+#pragma unroll
+        for (int u = 0; u < kMine; ++u)
+          if (rk[u] <= cap) {
+            hk[rk[u]] = kk[u];
+            hp[rk[u]] = kp[u];
+          }
+        nh = nv = min(nh, cap + 1);
+        order();
+      }
+    }
+    act = np > 0;
+  }
+  order();
+  bool over = false;
+  if (leaf < t && !again) {
+    test_hits();
+    // each pair's place is the number of smaller keys (keys are distinct)
+    int* out = chunk + (int64_t)leaf * stride;
+    for (int k = g; k < nh; k += kG) {
+      const uint64_t key = hk[k];
+      int rank = 0;
+      for (int k2 = 0; k2 < nh; ++k2) rank += hk[k2] < key;
+      if (rank < cap) out[rank] = hp[k];
+    }
+    over = nh > cap;
+  }
+  if (leaf < t && g == 0) counts[leaf] = again ? -1 : min(nh, cap);
+  if (__any(over) && lane == 0) atomicOr(warn, (uint32_t)CM_WARN_PAIR_CAP);
+}
+
+// The leaves the groups left (count -1), walked exactly by one lane each, and the tiles'
+// sums (added up here: an atomic a leaf to the tiles' two cache lines took 40 us at 64^2).
+__global__ void __launch_bounds__(kTravBlock) k_traverse_redo(WalkTree T, int cap,
+                                                              int* __restrict__ chunk,
+                                                              int* __restrict__ counts,
+                                                              uint32_t* __restrict__ warn,
+                                                              int* __restrict__ tile_sum,
+                                                              int* __restrict__ spill) {
+  __shared__ int sstk[kLdsStack][kTravBlock];
+  __shared__ int wsum[kTravBlock / 64];
+  const int leaf = blockIdx.x * kTravBlock + threadIdx.x;
+  int n = leaf < T.t ? counts[leaf] : 0;
+  if (n < 0) {
+    const int me = T.t - 1 + leaf, c = T.croot ? T.slot_cloth[leaf] : 0;
+    uint32_t w = 0;
+    n = walk_exact<kTravBlock, kLdsStack>(T, leaf, T.croot ? T.croot[c] : 0, xyz(T.amin[me]),
+                                          xyz(T.amax[me]), T.croot ? T.ccap[c] : cap,
+                                          chunk + (int64_t)leaf * cap, w, sstk, threadIdx.x,
+                                          spill + (int64_t)leaf * kSpill);
+    counts[leaf] = n;
+    if (w) atomicOr(warn, w);
+  }
+  n = wave_sum(n);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) tile_sum[blockIdx.x] = wsum[0] + wsum[1];
+}
+
 __global__ void k_clear_records(int* __restrict__ hctl) {
   if (threadIdx.x == 0) hctl[0] = 0;
 }
@@ -1440,6 +1669,15 @@ static int launch_traverse(const LbvhBufs& b, int cap, int* chunk, int* counts, 
   const WalkTree T{t,      t < kQuantLeaves ? b.qnodes : nullptr, b.irr, b.lefts, b.rights, b.rmll,
                    b.rmlr, b.amin, b.amax, b.ncloth ? b.slot_cloth : nullptr,
                    b.ncloth ? b.croot : nullptr, b.ccap};
+  if (b.group && T.qnodes && t <= kGroupLeaves && cap <= kGroupMaxCap) {
+    const int per = 64 / kGroup, nb = (t + per - 1) / per, rnd = kXcds * 4 * kTravBlock / per;
+    hipLaunchKernelGGL(k_traverse_group<kGroup>, dim3((nb + rnd - 1) / rnd * rnd), dim3(64), 0, s,
+                       T, cap, chunk, counts, b.warn);
+    hipLaunchKernelGGL(k_traverse_redo, dim3(nt), dim3(kTravBlock), 0, s, T, cap, chunk, counts,
+                       b.warn, offsets, b.spill);
+    CM_LAUNCH_CHECK();
+    return CM_OK;
+  }
   const bool few = t <= kFewLeaves;
   hipLaunchKernelGGL((few ? k_traverse<66, 8> : k_traverse<16, 4>),
                      dim3((nt + round - 1) / round * round), dim3(kTravBlock), 0, s, T, cap, chunk,
