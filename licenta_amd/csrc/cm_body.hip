@@ -89,6 +89,7 @@ struct cm_body {
   hipStream_t stream = nullptr;
   std::vector<void*> allocs;
   // state
+  float4* sphere = nullptr;  // centre, radius
   float4 *x = nullptr, *p = nullptr, *q0 = nullptr, *q1 = nullptr, *v = nullptr;
   uint8_t* pinned = nullptr;
   float* mass = nullptr;
@@ -522,6 +523,7 @@ PbdBufs pbd_bufs(cm_body* b) {
   pb.S = b->S;
   pb.B = b->B;
   pb.F = b->F;
+  pb.sphere = b->sphere;
   pb.x = b->x;
   pb.p = b->p;
   pb.q0 = b->q0;
@@ -557,8 +559,6 @@ PbdParams pbd_params(const cm_body* b) {
   pp.ref_compat = P.ref_compat;
   pp.wmin = mk3(P.world_min[0], P.world_min[1], P.world_min[2]);
   pp.wmax = mk3(P.world_max[0], P.world_max[1], P.world_max[2]);
-  pp.sc = mk3(P.sphere_center[0], P.sphere_center[1], P.sphere_center[2]);
-  pp.sr = P.sphere_radius;
   pp.kg = P.global_vel_damp;
   pp.kd = P.k_damp;
   pp.kf = P.k_friction;
@@ -660,6 +660,13 @@ int record_substep(cm_body* b, hipEvent_t* ev = nullptr, const TapeSlot* tape = 
   if (!rc && (P.flags & CM_F_FRICTION)) rc = launch_friction(pb, pp, nb, s);
   mark(CM_NUM_STAGES);
   return rc;
+}
+
+void drop_graph(cm_body* b) {
+  if (b->exec) hipGraphExecDestroy(b->exec);
+  if (b->graph) hipGraphDestroy(b->graph);
+  b->exec = nullptr;
+  b->graph = nullptr;
 }
 
 int ensure_graph(cm_body* b) {
@@ -838,7 +845,10 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
     mass[i] = b->pinned_h[i] ? params->pinned_mass
                              : (inv_mass[i] > 0 ? 1.f / inv_mass[i] : params->pinned_mass);
   }
-  if ((rc = upload(b, &b->x, x4)) || (rc = upload(b, &b->p, x4)) || (rc = dalloc(b, &b->q0, n)) ||
+  const cm_params& P = b->prm;
+  const std::vector<float4> sphere{make_float4(P.sphere_center[0], P.sphere_center[1],
+                                               P.sphere_center[2], P.sphere_radius)};
+  if ((rc = upload(b, &b->sphere, sphere)) || (rc = upload(b, &b->x, x4)) || (rc = upload(b, &b->p, x4)) || (rc = dalloc(b, &b->q0, n)) ||
       (rc = dalloc(b, &b->q1, n)) ||
       (rc = upload(b, &b->v, v4)) || (rc = upload(b, &b->pinned, b->pinned_h)) ||
       (rc = upload(b, &b->mass, mass)) || (rc = upload(b, &b->sid, h.sid)) ||
@@ -1018,9 +1028,6 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
   }
   CM_HIP(hipMemset(nb.dprefix, 0, sizeof(int) * ((size_t)n + 1)));
   CM_HIP(hipMemset(nb.dcount, 0, sizeof(int) * ((size_t)n + 1)));  // kept zero between substeps
-  if (params->flags & CM_F_SPHERE) {
-    b->prm.flags |= CM_F_SPHERE;
-  }
   b->topo = std::move(h);
   CM_HIP(hipDeviceSynchronize());
   *out = b;
@@ -1204,20 +1211,23 @@ int cm_read_vertices(cm_body* b, float* verts) {
 int cm_set_sphere(cm_body* b, const float center[3], float radius) {
   int rc = body_check(b);
   if (rc) return rc;
-  CM_HIP(hipStreamSynchronize(b->stream));
+  // in stream order: substeps already launched keep the sphere they had. Recording the
+  // substep again for a moved sphere took 0.5 ms of host work and a synchronisation.
+  rc = launch_set_sphere(b->sphere, make_float4(center[0], center[1], center[2], radius),
+                         b->stream);
+  if (rc) return rc;
   b->prm.sphere_center[0] = center[0];
   b->prm.sphere_center[1] = center[1];
   b->prm.sphere_center[2] = center[2];
   b->prm.sphere_radius = radius;
-  b->prm.flags |= CM_F_SPHERE;
   // a recorded forward ran without this sphere: its adjoint would recompute the
   // segments with it, so the record is dropped
   b->adj.ready = false;
-  // kernel arguments changed: re-record the substep graph
-  if (b->exec) hipGraphExecDestroy(b->exec);
-  if (b->graph) hipGraphDestroy(b->graph);
-  b->exec = nullptr;
-  b->graph = nullptr;
+  if (!(b->prm.flags & CM_F_SPHERE)) {  // the first sphere joins the recorded substep
+    CM_HIP(hipStreamSynchronize(b->stream));
+    b->prm.flags |= CM_F_SPHERE;
+    drop_graph(b);
+  }
   return CM_OK;
 }
 
@@ -1713,13 +1723,6 @@ void free_alloc(cm_body* b, void* ptr) {
       b->allocs.erase(b->allocs.begin() + k);
       return;
     }
-}
-
-void drop_graph(cm_body* b) {
-  if (b->exec) hipGraphExecDestroy(b->exec);
-  if (b->graph) hipGraphDestroy(b->graph);
-  b->exec = nullptr;
-  b->graph = nullptr;
 }
 
 // Jacobi tiles of tile_v vertices: rebuilt on the host and uploaded in place of the

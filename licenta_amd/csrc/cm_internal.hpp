@@ -284,6 +284,9 @@ struct TileBufs {
 };
 
 struct PbdBufs {
+  // collision sphere, centre and radius: in memory, so that moving it leaves the captured
+  // substep as it is
+  const float4* sphere = nullptr;
   int n = 0, S = 0, B = 0, F = 0;
   float4 *x = nullptr, *p = nullptr, *v = nullptr;  // .w of x/p = inverse mass
   float4 *q0 = nullptr, *q1 = nullptr;  // the solver's iterates, in solver order
@@ -309,11 +312,10 @@ struct PbdParams {
   int iters;
   uint32_t flags, ref_compat;
   f3 wmin, wmax;
-  f3 sc;
-  float sr;
   float kg, kd, kf;
 };
 int launch_predict(const PbdBufs& b, const PbdParams& pp, hipStream_t s);
+int launch_set_sphere(float4* sphere, float4 value, hipStream_t s);
 int launch_solver(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, hipStream_t s);
 int launch_solve_only(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, int iters,
                       hipStream_t s);

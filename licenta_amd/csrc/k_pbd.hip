@@ -194,10 +194,16 @@ __global__ void __launch_bounds__(kBlock) k_setup(int n, const float4* __restric
   }
 }
 
+__global__ void k_set_sphere(float4* __restrict__ sphere, float4 value) { *sphere = value; }
+
 __global__ void __launch_bounds__(kBlock) k_sphere(int n, float4* __restrict__ x,
-                                                   float4* __restrict__ p, f3 c, float rad) {
+                                                   float4* __restrict__ p,
+                                                   const float4* __restrict__ sphere, float th) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
+  const float4 s = *sphere;
+  const f3 c = xyz(s);
+  const float rad = s.w + th;
   const float4 xi = x[i], pi = p[i];
   const f3 a = xyz(xi), b = xyz(pi);
   f3 dir = sub(b, a);
@@ -1414,6 +1420,12 @@ int launch_tile_stiffness(const PbdBufs& b, hipStream_t s) {
   return CM_OK;
 }
 
+int launch_set_sphere(float4* sphere, float4 value, hipStream_t s) {
+  hipLaunchKernelGGL(k_set_sphere, dim3(1), dim3(1), 0, s, sphere, value);
+  CM_LAUNCH_CHECK();
+  return CM_OK;
+}
+
 int launch_solver(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, hipStream_t s) {
   const int g = nblocks(b.n);
   const int ground_on = (pp.flags & CM_F_GROUND) ? 1 : 0;
@@ -1422,7 +1434,7 @@ int launch_solver(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, h
     hipLaunchKernelGGL(k_setup, dim3(g), dim3(kBlock), 0, s, b.n, b.x, b.p, pp.gh, pp.th,
                        ground_on, b.ground, F, b.lra_fixed, b.lra_l0, b.pinned, b.lra_flag);
   if (pp.flags & CM_F_SPHERE)
-    hipLaunchKernelGGL(k_sphere, dim3(g), dim3(kBlock), 0, s, b.n, b.x, b.p, pp.sc, pp.sr + pp.th);
+    hipLaunchKernelGGL(k_sphere, dim3(g), dim3(kBlock), 0, s, b.n, b.x, b.p, b.sphere, pp.th);
   CM_LAUNCH_CHECK();
   return launch_iterations(b, solve_args(b, pp, nb), pp.iters, s);
 }
@@ -1488,7 +1500,7 @@ int launch_solver_rec(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& n
     hipLaunchKernelGGL(k_setup, dim3(g), dim3(kBlock), 0, s, b.n, b.x, b.p, pp.gh, pp.th,
                        ground_on, b.ground, F, b.lra_fixed, b.lra_l0, b.pinned, b.lra_flag);
   if (pp.flags & CM_F_SPHERE)
-    hipLaunchKernelGGL(k_sphere, dim3(g), dim3(kBlock), 0, s, b.n, b.x, b.p, pp.sc, pp.sr + pp.th);
+    hipLaunchKernelGGL(k_sphere, dim3(g), dim3(kBlock), 0, s, b.n, b.x, b.p, b.sphere, pp.th);
   CM_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_to_order, dim3(g), dim3(kBlock), 0, s, b.n, b.tl.order, b.p, pk);
   const SolveArgs a = solve_args(b, pp, nb);
