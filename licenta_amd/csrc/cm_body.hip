@@ -608,14 +608,15 @@ int record_substep(cm_body* b, hipEvent_t* ev = nullptr, const TapeSlot* tape = 
   if (coll) {
     rc = radix_sort(b->keys, b->perm, b->t, b->key_bits, b->sort_temp, s);
     if (rc) return rc;
-    rc = launch_gather_tris(b->t, b->perm, b->tri, b->tri_alt,
-                            (P.ref_compat & CM_RC_STALE_LEAF_AABB) ? 0 : 1, b->lb.amin,
-                            b->lb.amax, b->tmp_min, b->tmp_max, s);
+    rc = launch_gather_tris(b->lb, b->perm, b->tri, b->tri_alt,
+                            (P.ref_compat & CM_RC_STALE_LEAF_AABB) ? 0 : 1, b->tmp_min,
+                            b->tmp_max, s);
     if (rc) return rc;
   }
   mark(CM_STAGE_TREE);
   if (coll) {
-    rc = launch_build(b->lb, b->keys, (P.ref_compat & CM_RC_MIDPOINT_SPLIT) ? 1 : 0, s);
+    rc = launch_build(b->lb, b->keys, (P.ref_compat & CM_RC_MIDPOINT_SPLIT) ? 1 : 0, true,
+                      b->tri_alt, b->tri, s);
     if (rc) return rc;
     rc = launch_refit(b->lb, s);
     if (rc) return rc;
@@ -639,8 +640,6 @@ int record_substep(cm_body* b, hipEvent_t* ev = nullptr, const TapeSlot* tape = 
       rc = launch_revert_toc(pb, b->nb, s);
       if (rc) return rc;
     }
-    rc = launch_copy_i4(b->t, b->tri_alt, b->tri, s);
-    if (rc) return rc;
     if (tape) {
       CM_HIP(hipMemcpyAsync(tape->dpre, b->nb.dprefix, sizeof(int) * ((size_t)b->n + 1),
                             hipMemcpyDeviceToDevice, s));

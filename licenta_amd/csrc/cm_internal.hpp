@@ -173,7 +173,10 @@ int launch_tri_update(int n, int t, const float4* x, const float4* p, const int4
 int launch_tri_update_batch(const LbvhBufs& b, const float4* x, const float4* p, const int4* tri,
                             float th, uint64_t* keys, uint32_t* vals, float4* centroid_tmp,
                             hipStream_t s);
-int launch_build(const LbvhBufs& b, const uint64_t* keys, int midpoint, hipStream_t s);
+// cleared: launch_gather_tris has cleared what the build starts from. tri_from (or null):
+// copied to tri_to on the way.
+int launch_build(const LbvhBufs& b, const uint64_t* keys, int midpoint, bool cleared,
+                 const int4* tri_from, int4* tri_to, hipStream_t s);
 int launch_refit(const LbvhBufs& b, hipStream_t s);
 // the traversal's node records; from_caller: check the caller's tree first
 int launch_pack_nodes(const LbvhBufs& b, bool from_caller, hipStream_t s);
@@ -184,10 +187,8 @@ int launch_pairs(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offse
 // the traversal kernel alone on the current tree (it rewrites the same pair chunk)
 int launch_traverse_only(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offsets,
                          hipStream_t s);
-int launch_gather_tris(int t, const uint32_t* perm, const int4* tri_in, int4* tri_out,
-                       int fix_leaves, float4* amin, float4* amax, float4* tmp_min,
-                       float4* tmp_max, hipStream_t s);
-int launch_copy_i4(int64_t n, const int4* src, int4* dst, hipStream_t s);
+int launch_gather_tris(const LbvhBufs& b, const uint32_t* perm, const int4* tri_in, int4* tri_out,
+                       int fix_leaves, float4* tmp_min, float4* tmp_max, hipStream_t s);
 
 // ---- narrow phase (k_narrow.hip) ------------------------------------------
 // A contact record in vertex order, self-contained for the Jacobi kernel: the

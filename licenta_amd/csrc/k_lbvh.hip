@@ -85,7 +85,8 @@ __global__ void __launch_bounds__(kBlock) k_tri_update(
 }
 
 // single block: reduce the per-block boxes; result in box[2*nb], box[2*nb+1]
-__global__ void __launch_bounds__(kBlock) k_box_reduce(float4* __restrict__ box, int nb) {
+// The box of nb block boxes (min, max in turn), in every thread of the workgroup.
+__device__ __forceinline__ void box_of(const float4* __restrict__ box, int nb, f3& lo, f3& hi) {
   __shared__ float smin[3][kBlock], smax[3][kBlock];
   const float inf = __builtin_huge_valf();
   float mn[3] = {inf, inf, inf}, mx[3] = {-inf, -inf, -inf};
@@ -107,19 +108,35 @@ __global__ void __launch_bounds__(kBlock) k_box_reduce(float4* __restrict__ box,
       }
     __syncthreads();
   }
+  lo = mk3(smin[0][0], smin[1][0], smin[2][0]);
+  hi = mk3(smax[0][0], smax[1][0], smax[2][0]);
+}
+
+__global__ void __launch_bounds__(kBlock) k_box_reduce(float4* __restrict__ box, int nb) {
+  f3 lo, hi;
+  box_of(box, nb, lo, hi);
   if (threadIdx.x == 0) {
-    box[2 * nb] = make_float4(smin[0][0], smin[1][0], smin[2][0], 0.f);
-    box[2 * nb + 1] = make_float4(smax[0][0], smax[1][0], smax[2][0], 0.f);
+    box[2 * nb] = make_float4(lo.x, lo.y, lo.z, 0.f);
+    box[2 * nb + 1] = make_float4(hi.x, hi.y, hi.z, 0.f);
   }
 }
 
+// kReduce: every workgroup reduces the block boxes itself, which up to kFewBoxes of them
+// (16 KB from the L2) costs it less than k_box_reduce's launch of 3 to 4.5 us.
+constexpr int kFewBoxes = 512;
+template <bool kReduce>
 __global__ void __launch_bounds__(kBlock) k_keys30(int t, const float4* __restrict__ centroid,
                                                    const float4* __restrict__ box, int nb,
                                                    uint64_t* __restrict__ keys) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= t) return;
-  const f3 lo = xyz(box[2 * nb]), hi = xyz(box[2 * nb + 1]);
-  keys[i] = morton30(xyz(centroid[i]), lo, hi);
+  f3 lo, hi;
+  if (kReduce) {
+    box_of(box, nb, lo, hi);
+  } else {
+    lo = xyz(box[2 * nb]);
+    hi = xyz(box[2 * nb + 1]);
+  }
+  if (i < t) keys[i] = morton30(xyz(centroid[i]), lo, hi);
 }
 
 // ---- per-cloth centroid boxes of a batch -------------------------------------------
@@ -205,21 +222,26 @@ __device__ __forceinline__ int delta(const uint64_t* __restrict__ k, int i, int 
 }
 __device__ __forceinline__ int sgn(int a) { return signbit((float)a) ? -1 : 1; }
 
-__global__ void __launch_bounds__(kBlock) k_build_init(int t, int* __restrict__ cnt,
-                                                       int* __restrict__ hi,
-                                                       int* __restrict__ ntop,
-                                                       int* __restrict__ irr, int ncloth,
-                                                       int* __restrict__ croot) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < 2 * t - 1) {
-    cnt[i] = 0;
-    hi[i] = -1;
+// What the build and the refit start from; thread i of at least max(2t - 1, ncloth).
+struct BuildInit {
+  int t;
+  int *cnt, *hi, *ntop, *irr;
+  int ncloth;
+  int* croot;
+};
+__device__ __forceinline__ void build_init(const BuildInit& b, int i) {
+  if (i < 2 * b.t - 1) {
+    b.cnt[i] = 0;
+    b.hi[i] = -1;
   }
-  if (i < ncloth) croot[i] = -1;
+  if (i < b.ncloth) b.croot[i] = -1;
   if (i == 0) {
-    *ntop = 0;  // deferred-node count of the refit
-    *irr = 0;
+    *b.ntop = 0;  // deferred-node count of the refit
+    *b.irr = 0;
   }
+}
+__global__ void __launch_bounds__(kBlock) k_build_init(BuildInit b) {
+  build_init(b, blockIdx.x * kBlock + threadIdx.x);
 }
 
 __global__ void __launch_bounds__(kBlock) k_build(int t, const uint64_t* __restrict__ k,
@@ -278,8 +300,11 @@ __global__ void __launch_bounds__(kBlock) k_build(int t, const uint64_t* __restr
 
 __global__ void __launch_bounds__(kBlock) k_parents(int t, const int* __restrict__ cnt,
                                                     const int* __restrict__ hi,
-                                                    int* __restrict__ parents) {
+                                                    int* __restrict__ parents,
+                                                    const int4* __restrict__ tri_from,
+                                                    int4* __restrict__ tri_to) {
   const int c = blockIdx.x * kBlock + threadIdx.x;
+  if (tri_from && c < t) tri_to[c] = tri_from[c];
   if (c >= 2 * t - 1) return;
   if (cnt[c] > 0) parents[c] = hi[c];
 }
@@ -1507,19 +1532,38 @@ __global__ void __launch_bounds__(kBlock) k_pack_nodes(int t, const int* __restr
 // leaves' counts, then the workgroup writes the tile's pairs in order, kBlock
 // consecutive output slots at a time (each thread finds its slot's leaf by binary
 // search over the tile's prefixes), so reads and writes are contiguous runs.
+// A tile's pairs are shared by gridDim.y workgroups, so that a few tiles fill the chip, and
+// a thread looks up kAhead pairs at once: the searches and the loads after them are chains
+// of latencies. kScan: the workgroup adds up the sums of the tiles before its own, and the
+// last one writes the total (at most pair_cap), in place of a scan's launch of 5 us.
+// k_compact_pairs with that scan, one workgroup a tile and one pair a thread at a time ->
+// now: 64^2 17 -> 4.9 us, draped 131x97 31 -> 5.8, draped 256^2 39 -> 19; without it, 96
+// cloths 66 -> 44, 2 M leaves 147 -> 105, crumpled 1024^2 125 -> 97.
+constexpr int kAhead = 4;
+constexpr int kScanMax = 1024;  // tiles; every workgroup reads the sums of all before its own
+template <bool kScan>
 __global__ void __launch_bounds__(kBlock) k_compact_pairs(int t, int stride,
                                                           const int* __restrict__ chunk,
                                                           const int* __restrict__ counts,
                                                           const int* __restrict__ tile_pre,
                                                           int2* __restrict__ pairs,
-                                                          int* __restrict__ hctl) {
+                                                          int* __restrict__ hctl,
+                                                          int64_t pair_cap,
+                                                          int* __restrict__ d_npairs) {
   static_assert(kTravBlock == 128, "two leaves per lane of the first wave");
   // the traversal's hand-over record count, read by its second pass, starts the next
   // substep at zero
-  if (hctl && blockIdx.x == 0 && threadIdx.x == 0) hctl[0] = 0;
+  if (hctl && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) hctl[0] = 0;
   __shared__ int pre[kTravBlock + 1];
+  __shared__ int wsum[kBlock / 64];
   const int tile = blockIdx.x, tid = threadIdx.x;
   const int l0 = tile * kTravBlock;
+  if (kScan) {
+    int v = 0;
+    for (int k = tid; k < tile; k += kBlock) v += tile_pre[k];
+    v = wave_sum(v);
+    if ((tid & 63) == 0) wsum[tid >> 6] = v;
+  }
   if (tid < 64) {
     const int i0 = l0 + 2 * tid, i1 = i0 + 1;
     const int c0 = i0 < t ? counts[i0] : 0, c1 = i1 < t ? counts[i1] : 0;
@@ -1536,26 +1580,48 @@ __global__ void __launch_bounds__(kBlock) k_compact_pairs(int t, int stride,
   }
   __syncthreads();
   const int total = pre[kTravBlock];
-  const int out0 = tile_pre[tile];
-  for (int k = tid; k < total; k += kBlock) {
-    int lo = 0, hi = kTravBlock - 1;  // the last leaf whose prefix is <= k holds slot k
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (pre[mid] <= k) lo = mid;
-      else hi = mid - 1;
+  int out0 = 0;
+  if (kScan) {
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) out0 += wsum[w];
+    if (tile == (int)gridDim.x - 1 && blockIdx.y == 0 && tid == 0)
+      *d_npairs = (int)min((int64_t)out0 + total, pair_cap);
+  } else {
+    out0 = tile_pre[tile];
+  }
+  const int step = kBlock * gridDim.y;
+  for (int k0 = blockIdx.y * kBlock + tid; k0 < total; k0 += kAhead * step) {
+    // the last leaf whose prefix is <= k holds slot k
+    int lo[kAhead], c[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) lo[u] = 0;
+#pragma unroll
+    for (int h = kTravBlock / 2; h >= 1; h >>= 1)
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+        if (pre[lo[u] + h] <= k0 + u * step) lo[u] += h;
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int k = min(k0 + u * step, total - 1);
+      c[u] = k0 + u * step < total ? chunk[(int64_t)(l0 + lo[u]) * stride + (k - pre[lo[u]])] : 0;
     }
-    pairs[out0 + k] = make_int2(l0 + lo, chunk[(int64_t)(l0 + lo) * stride + (k - pre[lo])]);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (k0 + u * step < total) pairs[out0 + k0 + u * step] = make_int2(l0 + lo[u], c[u]);
   }
 }
 
-__global__ void __launch_bounds__(kBlock) k_gather_tris(int t, const uint32_t* __restrict__ perm,
+// Also clears what the build starts from (a launch of its own otherwise).
+__global__ void __launch_bounds__(kBlock) k_gather_tris(BuildInit init,
+                                                        const uint32_t* __restrict__ perm,
                                                         const int4* __restrict__ tin,
                                                         int4* __restrict__ tout, int fix,
                                                         const float4* __restrict__ amin,
                                                         const float4* __restrict__ amax,
                                                         float4* __restrict__ tmin,
                                                         float4* __restrict__ tmax) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const int i = blockIdx.x * kBlock + threadIdx.x, t = init.t;
+  build_init(init, i);
   if (i >= t) return;
   const uint32_t s = perm[i];
   tout[i] = tin[s];
@@ -1573,12 +1639,6 @@ __global__ void __launch_bounds__(kBlock) k_put_leaves(int t, const float4* __re
   amin[t - 1 + i] = tmin[i];
   amax[t - 1 + i] = tmax[i];
 }
-__global__ void __launch_bounds__(kBlock) k_copy_i4(int64_t n, const int4* __restrict__ s,
-                                                    int4* __restrict__ d) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) d[i] = s[i];
-}
-
 }  // namespace
 
 // ---- launchers --------------------------------------------------------------
@@ -1592,8 +1652,10 @@ int launch_tri_update(int n, int t, const float4* x, const float4* p, const int4
   hipLaunchKernelGGL(k_tri_update, dim3(nb), dim3(kBlock), 0, s, t, x, p, tri, th, bits, amin,
                      amax, keys, vals, norm ? centroid_tmp : nullptr, norm ? box_tmp : nullptr);
   if (norm) {
-    hipLaunchKernelGGL(k_box_reduce, dim3(1), dim3(kBlock), 0, s, box_tmp, nb);
-    hipLaunchKernelGGL(k_keys30, dim3(nb), dim3(kBlock), 0, s, t, centroid_tmp, box_tmp, nb, keys);
+    if (nb > kFewBoxes)
+      hipLaunchKernelGGL(k_box_reduce, dim3(1), dim3(kBlock), 0, s, box_tmp, nb);
+    hipLaunchKernelGGL((nb > kFewBoxes ? k_keys30<false> : k_keys30<true>), dim3(nb), dim3(kBlock),
+                       0, s, t, centroid_tmp, box_tmp, nb, keys);
   }
   CM_LAUNCH_CHECK();
   return CM_OK;
@@ -1616,16 +1678,23 @@ int launch_tri_update_batch(const LbvhBufs& b, const float4* x, const float4* p,
   return CM_OK;
 }
 
-int launch_build(const LbvhBufs& b, const uint64_t* keys, int midpoint, hipStream_t s) {
+static BuildInit build_init_args(const LbvhBufs& b) {
+  return {b.t, b.claim_cnt, b.claim_hi, b.ntop, b.irr, b.ncloth, b.croot};
+}
+static int build_init_grid(const LbvhBufs& b) { return nblocks(std::max(2 * b.t - 1, b.ncloth)); }
+
+int launch_build(const LbvhBufs& b, const uint64_t* keys, int midpoint, bool cleared,
+                 const int4* tri_from, int4* tri_to, hipStream_t s) {
   const int t = b.t;
   if (t < 2) return CM_OK;
-  hipLaunchKernelGGL(k_build_init, dim3(nblocks(std::max(2 * t - 1, b.ncloth))), dim3(kBlock), 0,
-                     s, t, b.claim_cnt, b.claim_hi, b.ntop, b.irr, b.ncloth, b.croot);
+  if (!cleared)
+    hipLaunchKernelGGL(k_build_init, dim3(build_init_grid(b)), dim3(kBlock), 0, s,
+                       build_init_args(b));
   hipLaunchKernelGGL(k_build, dim3(nblocks(t - 1)), dim3(kBlock), 0, s, t, keys, midpoint, b.lefts,
                      b.rights, b.claim_cnt, b.claim_hi, b.ranges, b.warn,
                      b.ncloth ? b.tstart : nullptr, b.croot);
   hipLaunchKernelGGL(k_parents, dim3(nblocks(2 * t - 1)), dim3(kBlock), 0, s, t, b.claim_cnt,
-                     b.claim_hi, b.parents);
+                     b.claim_hi, b.parents, tri_from, tri_to);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
@@ -1705,10 +1774,18 @@ int launch_pairs(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offse
   const int nt = (t + kTravBlock - 1) / kTravBlock;
   int rc = launch_traverse(b, cap, chunk, counts, offsets, s);
   if (rc) return rc;
-  rc = scan_tiles(nt, offsets, offsets + nt, 0, (int64_t)t * cap, 0, d_npairs, nullptr, scan_temp, s);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_compact_pairs, dim3(nt), dim3(kBlock), 0, s, t, cap, chunk,
-                     counts, offsets + nt, pairs, two_passes(b) ? b.hctl : nullptr);
+  const dim3 grid(nt, std::max(1, std::min(8, 2048 / nt)));
+  int* hctl = two_passes(b) ? b.hctl : nullptr;
+  if (nt <= kScanMax) {
+    hipLaunchKernelGGL(k_compact_pairs<true>, grid, dim3(kBlock), 0, s, t, cap, chunk, counts,
+                       offsets, pairs, hctl, (int64_t)t * cap, d_npairs);
+  } else {
+    rc = scan_tiles(nt, offsets, offsets + nt, 0, (int64_t)t * cap, 0, d_npairs, nullptr, scan_temp,
+                    s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_compact_pairs<false>, grid, dim3(kBlock), 0, s, t, cap, chunk, counts,
+                       offsets + nt, pairs, hctl, (int64_t)t * cap, d_npairs);
+  }
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
@@ -1733,22 +1810,16 @@ int launch_pack_nodes(const LbvhBufs& b, bool from_caller, hipStream_t s) {
   return CM_OK;
 }
 
-int launch_gather_tris(int t, const uint32_t* perm, const int4* tri_in, int4* tri_out,
-                       int fix_leaves, float4* amin, float4* amax, float4* tmp_min,
-                       float4* tmp_max, hipStream_t s) {
+int launch_gather_tris(const LbvhBufs& b, const uint32_t* perm, const int4* tri_in, int4* tri_out,
+                       int fix_leaves, float4* tmp_min, float4* tmp_max, hipStream_t s) {
+  const int t = b.t;
   if (t <= 0) return CM_OK;
-  hipLaunchKernelGGL(k_gather_tris, dim3(nblocks(t)), dim3(kBlock), 0, s, t, perm, tri_in, tri_out,
-                     fix_leaves, amin, amax, tmp_min, tmp_max);
+  hipLaunchKernelGGL(k_gather_tris, dim3(build_init_grid(b)), dim3(kBlock), 0, s,
+                     build_init_args(b), perm, tri_in, tri_out, fix_leaves, b.amin, b.amax,
+                     tmp_min, tmp_max);
   if (fix_leaves)
     hipLaunchKernelGGL(k_put_leaves, dim3(nblocks(t)), dim3(kBlock), 0, s, t, tmp_min, tmp_max,
-                       amin, amax);
-  CM_LAUNCH_CHECK();
-  return CM_OK;
-}
-
-int launch_copy_i4(int64_t n, const int4* src, int4* dst, hipStream_t s) {
-  if (n <= 0) return CM_OK;
-  hipLaunchKernelGGL(k_copy_i4, dim3(nblocks(n)), dim3(kBlock), 0, s, n, src, dst);
+                       b.amin, b.amax);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
@@ -1853,7 +1924,7 @@ extern "C" int cm_lbvh_build(int32_t t, const uint64_t* d_keys, int32_t midpoint
   b.parents = d_parents;
   b.warn = d_warn;
   carve_build(t, d_temp, &b);
-  return launch_build(b, d_keys, midpoint_split, (hipStream_t)stream);
+  return launch_build(b, d_keys, midpoint_split, false, nullptr, nullptr, (hipStream_t)stream);
 }
 
 // d_temp must be the same buffer that the preceding cm_lbvh_build used (claim records).
