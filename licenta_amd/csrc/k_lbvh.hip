@@ -84,7 +84,6 @@ __global__ void __launch_bounds__(kBlock) k_tri_update(
   }
 }
 
-// single block: reduce the per-block boxes; result in box[2*nb], box[2*nb+1]
 // The box of nb block boxes (min, max in turn), in every thread of the workgroup.
 __device__ __forceinline__ void box_of(const float4* __restrict__ box, int nb, f3& lo, f3& hi) {
   __shared__ float smin[3][kBlock], smax[3][kBlock];
@@ -112,6 +111,7 @@ __device__ __forceinline__ void box_of(const float4* __restrict__ box, int nb, f
   hi = mk3(smax[0][0], smax[1][0], smax[2][0]);
 }
 
+// single block: reduce the per-block boxes; result in box[2*nb], box[2*nb+1]
 __global__ void __launch_bounds__(kBlock) k_box_reduce(float4* __restrict__ box, int nb) {
   f3 lo, hi;
   box_of(box, nb, lo, hi);
@@ -164,35 +164,63 @@ __device__ __forceinline__ uint32_t wave_max_u(uint32_t v) {
   return v;
 }
 
-// centroid box of each cloth; a wave whose triangles all belong to one cloth
-// reduces first and issues one atomic per bound
+// Centroid box of each cloth.
+// A wave takes kBoxRun chunks of 64 consecutive slots and keeps one cloth's box in its lanes
+// until the cloth changes, then adds it to the cloth's with 6 atomics: they all go to a few
+// cache lines and bound the pass (6 for each 64 slots, 6 for each slot of a chunk with two
+// cloths: 108 us for 96 cloths of 938 k triangles, now 18). A chunk of more than kBoxCloths
+// cloths, tiny ones, goes by one atomic a bound and slot.
+constexpr int kBoxRun = 16, kBoxCloths = 4;
 __global__ void __launch_bounds__(kBlock) k_cloth_box(int t, const float4* __restrict__ cen,
                                                       const int* __restrict__ slot_cloth,
                                                       uint32_t* __restrict__ cbox) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  const bool valid = i < t;
-  const int c = valid ? slot_cloth[i] : -1;
-  const f3 p = valid ? xyz(cen[i]) : mk3(0, 0, 0);
+  const int lane = threadIdx.x & 63;
+  const int64_t base = ((int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * 64 * kBoxRun;
+  int cur = -1;  // the cloth whose box e holds
   uint32_t e[6];
-  e[0] = valid ? ford(p.x) : 0xffffffffu;
-  e[1] = valid ? ford(p.y) : 0xffffffffu;
-  e[2] = valid ? ford(p.z) : 0xffffffffu;
-  e[3] = valid ? ford(p.x) : 0u;
-  e[4] = valid ? ford(p.y) : 0u;
-  e[5] = valid ? ford(p.z) : 0u;
-  const int c0 = __shfl(c, 0, 64);
-  const int cmax = (int)wave_max_u((uint32_t)(c + 1)) - 1, cmin = (int)wave_min_u((uint32_t)(c + 1)) - 1;
-  const bool uniform = c0 >= 0 && cmin == c0 && cmax == c0;
-  if (uniform) {
-    for (int a = 0; a < 3; ++a) e[a] = wave_min_u(e[a]);
-    for (int a = 3; a < 6; ++a) e[a] = wave_max_u(e[a]);
-    if ((threadIdx.x & 63) == 0)
-      for (int a = 0; a < 6; ++a)
-        if (a < 3) atomicMin(&cbox[6 * c0 + a], e[a]); else atomicMax(&cbox[6 * c0 + a], e[a]);
-  } else if (valid) {
-    for (int a = 0; a < 6; ++a)
-      if (a < 3) atomicMin(&cbox[6 * c + a], e[a]); else atomicMax(&cbox[6 * c + a], e[a]);
+  auto flush = [&] {
+    if (cur >= 0) {
+#pragma unroll
+      for (int a = 0; a < 6; ++a) e[a] = a < 3 ? wave_min_u(e[a]) : wave_max_u(e[a]);
+      if (lane == 0)
+        for (int a = 0; a < 6; ++a)
+          if (a < 3) atomicMin(&cbox[6 * cur + a], e[a]); else atomicMax(&cbox[6 * cur + a], e[a]);
+    }
+#pragma unroll
+    for (int a = 0; a < 6; ++a) e[a] = a < 3 ? 0xffffffffu : 0u;
+  };
+  for (int j = 0; j < kBoxRun && base + j * 64 < t; ++j) {
+    const int64_t i = base + j * 64 + lane;
+    const bool valid = i < t;
+    const int c = valid ? slot_cloth[i] : -1;
+    const f3 p = valid ? xyz(cen[i]) : mk3(0, 0, 0);
+    const uint32_t o[3] = {ford(p.x), ford(p.y), ford(p.z)};
+    uint64_t left = __ballot(valid);
+    const int before = __shfl_up(c, 1, 64);
+    if (__popcll(__ballot(valid && lane > 0 && c != before)) >= kBoxCloths) {
+      if (valid)
+        for (int a = 0; a < 3; ++a) {
+          atomicMin(&cbox[6 * c + a], o[a]);
+          atomicMax(&cbox[6 * c + 3 + a], o[a]);
+        }
+      continue;
+    }
+    while (left) {  // once for each cloth of the chunk
+      const int cc = __shfl(c, __ffsll((long long)left) - 1, 64);
+      if (cc != cur) {
+        flush();
+        cur = cc;
+      }
+      const bool mine = c == cc;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        e[a] = min(e[a], mine ? o[a] : 0xffffffffu);
+        e[3 + a] = max(e[3 + a], mine ? o[a] : 0u);
+      }
+      left &= ~__ballot(mine);
+    }
   }
+  flush();
 }
 
 __global__ void __launch_bounds__(kBlock) k_keys30_cloth(int t, const float4* __restrict__ cen,
@@ -1687,7 +1715,7 @@ int launch_tri_update_batch(const LbvhBufs& b, const float4* x, const float4* p,
                      b.cbox);
   hipLaunchKernelGGL(k_tri_update, dim3(nblocks(t)), dim3(kBlock), 0, s, t, x, p, tri, th, 30,
                      b.amin, b.amax, keys, vals, centroid_tmp, nullptr);
-  hipLaunchKernelGGL(k_cloth_box, dim3(nblocks(t)), dim3(kBlock), 0, s, t, centroid_tmp,
+  hipLaunchKernelGGL(k_cloth_box, dim3(nblocks(t, kBlock * kBoxRun)), dim3(kBlock), 0, s, t, centroid_tmp,
                      b.slot_cloth, b.cbox);
   hipLaunchKernelGGL(k_keys30_cloth, dim3(nblocks(t)), dim3(kBlock), 0, s, t, centroid_tmp,
                      b.slot_cloth, b.cbox, keys);
