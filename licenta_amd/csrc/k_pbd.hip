@@ -1401,13 +1401,14 @@ size_t tile_lds_bytes(int max_local, int lds_slots, bool adjoint) {
 }
 
 // more than 64 KiB of LDS per workgroup has to be asked for (meshes with a vertex of
-// very many constraints)
+// very many constraints); all of a CU's, so that no body takes it away from another
 int tile_lds_allow(size_t bytes) {
+  constexpr int kMaxLds = 160 << 10;
   if (bytes <= (64u << 10)) return CM_OK;
   for (const void* f :
        {(const void*)k_solve<true, 256>, (const void*)k_solve<false, 256>,
         (const void*)k_solve<true, 512>, (const void*)k_solve<false, 512>, (const void*)k_adj_iter})
-    CM_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    CM_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
   return CM_OK;
 }
 

@@ -771,8 +771,10 @@ int radix_sort_dev(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t*
 template <typename K>
 static int sort_block(uint64_t* keys, uint32_t* vals, int n, int passes, hipStream_t s) {
   const size_t lds = kSortHead + (sizeof(K) + 2) * (size_t)n;
+  // the most that any call needs, whatever this one does: other threads sort too
   CM_HIP(hipFuncSetAttribute((const void*)k_sort_block<K>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)(kSortHead + (sizeof(K) + 2) * kBlockSort)));
   hipLaunchKernelGGL(k_sort_block<K>, dim3(1), dim3(kSortThreads), lds, s, keys, vals, n,
                      passes);
   CM_LAUNCH_CHECK();
