@@ -573,15 +573,22 @@ __device__ __forceinline__ T sum_run(T acc, const T* c, int k, int e) {
 
 // LDS of a tile workgroup: positions (kPos arrays), four slot arrays (x, y, z and, for
 // the records, whether the correction counts), and the tile's slot and record prefixes
+// Component k of the slots is c(k): an array of three pointers indexed by a wave's component
+// was kept in scratch memory, 48 bytes a thread and launch (18 MB at 256^2), and what was
+// read through it by generic loads (a launch at 64^2 6.5 -> 5.8 us, 128^2 9.7 -> 8.2,
+// draped 256^2 23.0 -> 20.9, crumpled 1024^2 120 -> 113).
 struct TileLds {
-  float *c[3];
+  float* c0;
+  int stride;
   int *cn, *sp, *rp;
+  __device__ __forceinline__ float* c(int k) const { return c0 + k * stride; }
 };
 template <int kPos>
 __device__ __forceinline__ TileLds tile_lds(float4* base, int max_local, int lds_slots) {
   TileLds l;
   float* f = (float*)(base + kPos * max_local);
-  for (int k = 0; k < 3; ++k) l.c[k] = f + k * lds_slots;
+  l.c0 = f;
+  l.stride = lds_slots;
   l.cn = (int*)(f + 3 * lds_slots);
   l.sp = l.cn + lds_slots;
   l.rp = l.sp + kBlock + 1;
@@ -621,8 +628,8 @@ __device__ __forceinline__ void tile_jobs(int nv, F f) {
 // and 2.34 (bend) per constraint to 1.13 and 1.24 and the entries from 32 to 16 and 24
 // bytes; one wave per component of the sums took the records' chains (up to 182 on the
 // draped 256^2 cloth, each with a branch) off one wave. Per launch, before -> now:
-// 1024^2 236 -> 122 us, 96 cloths 147 -> 91, 192x301 without contacts 15.9 -> 11.9,
-// draped 256^2 31.3 -> 23.2, draped 131x97 27.9 -> 14.5, 64^2 9.1 -> 6.0. More waves per
+// 1024^2 236 -> 113 us, 96 cloths 147 -> 89, 192x301 without contacts 15.9 -> 10.7,
+// draped 256^2 31.3 -> 20.9, draped 131x97 27.9 -> 13.7, 64^2 9.1 -> 5.8. More waves per
 // SIMD (96 registers: five) spill and are slower (1024^2: 43 against 30 ms a pass).
 template <bool kFirst, int kT>
 __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float4* __restrict__ pin,
@@ -659,10 +666,10 @@ __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float
     else
       bend_all<float>(lpos[t.x & 0xffffu], lpos[t.x >> 16], lpos[t.y & 0xffffu], lpos[t.y >> 16],
                       par, a.abs_mode, cr);
-    tile_put(l.c[0], l.c[1], l.c[2], t.z & 0xffffu, cr[0]);
-    tile_put(l.c[0], l.c[1], l.c[2], t.z >> 16, cr[1]);
-    tile_put(l.c[0], l.c[1], l.c[2], t.w & 0xffffu, cr[2]);
-    tile_put(l.c[0], l.c[1], l.c[2], t.w >> 16, cr[3]);
+    tile_put(l.c(0), l.c(1), l.c(2), t.z & 0xffffu, cr[0]);
+    tile_put(l.c(0), l.c(1), l.c(2), t.z >> 16, cr[1]);
+    tile_put(l.c(0), l.c(1), l.c(2), t.w & 0xffffu, cr[2]);
+    tile_put(l.c(0), l.c(1), l.c(2), t.w >> 16, cr[3]);
   }
   // the distance entries are dealt to the waves in reverse: the last waves, which the
   // bends' remainder leaves idle, take the first of them
@@ -671,8 +678,8 @@ __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float
     f3 c0, c1;
     stretch_both(lpos[t.x & 0xffffu], lpos[t.x >> 16],
                  make_float2(__uint_as_float(t.z), __uint_as_float(t.w)), c0, c1);
-    tile_put(l.c[0], l.c[1], l.c[2], t.y & 0xffffu, c0);
-    tile_put(l.c[0], l.c[1], l.c[2], t.y >> 16, c1);
+    tile_put(l.c(0), l.c(1), l.c(2), t.y & 0xffffu, c0);
+    tile_put(l.c(0), l.c(1), l.c(2), t.y >> 16, c1);
   }
   __syncthreads();
   float accs[kJobs], accd[kJobs];  // of this thread's jobs: slots, records
@@ -683,19 +690,19 @@ __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float
     accn[u] = 0;
   }
   tile_jobs<kT>(nv, [&](int u, int comp, int v) {
-    if (comp < 3) accs[u] = sum_run(0.f, l.c[comp], l.sp[v], l.sp[v + 1]);
+    if (comp < 3) accs[u] = sum_run(0.f, l.c(comp), l.sp[v], l.sp[v + 1]);
   });
   __syncthreads();
   for (int c0 = r0; c0 < r1; c0 += a.lds_slots) {
     const int c1 = min(c0 + a.lds_slots, r1);
     eval_records<kT>(a, c0, c1, at, [&](int q, f3 c) {
-      lds_put(l.c[0], l.c[1], l.c[2], q, c);
+      lds_put(l.c(0), l.c(1), l.c(2), q, c);
       l.cn[q] = is_zero(c) ? 0 : 1;
     });
     __syncthreads();
     tile_jobs<kT>(nv, [&](int u, int comp, int v) {
       const int k = max(l.rp[v], c0) - c0, e = min(l.rp[v + 1], c1) - c0;
-      if (comp < 3) accd[u] = sum_run(accd[u], l.c[comp], k, e);
+      if (comp < 3) accd[u] = sum_run(accd[u], l.c(comp), k, e);
       else accn[u] = sum_run(accn[u], l.cn, k, e);
     });
     __syncthreads();
@@ -703,8 +710,8 @@ __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float
   // the sums to LDS, component by component: slots at [0, kBlock), records after them
   tile_jobs<kT>(nv, [&](int u, int comp, int v) {
     if (comp < 3) {
-      l.c[comp][v] = accs[u];
-      l.c[comp][kBlock + v] = accd[u];
+      l.c(comp)[v] = accs[u];
+      l.c(comp)[kBlock + v] = accd[u];
     } else {
       l.cn[v] = accn[u];
     }
@@ -719,10 +726,10 @@ __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float
     ground_lra(a, a.order[i], pi,
                [&](int j) { return pin[kFirst ? a.lra_fixed[j] : a.rank[a.lra_fixed[j]]]; },
                total, cnt);
-  total = add(total, mk3(l.c[0][tid], l.c[1][tid], l.c[2][tid]));
+  total = add(total, mk3(l.c(0)[tid], l.c(1)[tid], l.c(2)[tid]));
   cnt += l.sp[tid + 1] - l.sp[tid];
   if (l.rp[tid + 1] > l.rp[tid]) {
-    total = add(total, mk3(l.c[0][kBlock + tid], l.c[1][kBlock + tid], l.c[2][kBlock + tid]));
+    total = add(total, mk3(l.c(0)[kBlock + tid], l.c(1)[kBlock + tid], l.c(2)[kBlock + tid]));
     cnt += l.cn[tid];
   }
   pout[i] = f4(add(xyz(pi), divs(total, (float)cnt)), pi.w);
@@ -1187,9 +1194,9 @@ struct AdjArgs {
 // once, its vertex cotangents go to the tile's slots, and each vertex adds its slots in
 // slot order, then its dynamic records in record order: la = lp + sum over slots and
 // records. The tile holding a constraint's role-0 vertex adds its dL/dkp (one owner per
-// constraint). Bound by the FP64 bend VJP at two waves per SIMD (246 registers). 128^2:
-// 13.7 us a launch (21.1 in strips of 128 ids, plus 4.2 for a scaling launch of its
-// own), 24 cloths of 64^2: 29 us (38 + 5).
+// constraint). Bound by the FP64 bend VJP at two waves per SIMD (246 registers; three
+// with spills: 24 us at 128^2). 128^2: 13.4 us a launch (21.1 in strips of 128 ids, plus
+// 4.2 for a scaling launch of its own), 24 cloths of 64^2: 26.6 us (38 + 5).
 __global__ void __launch_bounds__(kBlock) k_adj_iter(AdjArgs a, const float4* __restrict__ ps,
                                                      const int* __restrict__ cnt,
                                                      const float4* __restrict__ lp,
@@ -1230,12 +1237,12 @@ __global__ void __launch_bounds__(kBlock) k_adj_iter(AdjArgs a, const float4* __
     else
       bend_vjp<float>(P, G, par.x, par.y, a.abs_mode, o, gkp);
     if ((t.z & 0xffffu) != 0xffffu) {
-      lds_put(l.c[0], l.c[1], l.c[2], t.z & 0xffffu, o[0]);
+      lds_put(l.c(0), l.c(1), l.c(2), t.z & 0xffffu, o[0]);
       a.gkb[a.tl.bcid[h1.z + q]] += (double)gkp;
     }
-    tile_put(l.c[0], l.c[1], l.c[2], t.z >> 16, o[1]);
-    tile_put(l.c[0], l.c[1], l.c[2], t.w & 0xffffu, o[2]);
-    tile_put(l.c[0], l.c[1], l.c[2], t.w >> 16, o[3]);
+    tile_put(l.c(0), l.c(1), l.c(2), t.z >> 16, o[1]);
+    tile_put(l.c(0), l.c(1), l.c(2), t.w & 0xffffu, o[2]);
+    tile_put(l.c(0), l.c(1), l.c(2), t.w >> 16, o[3]);
   }
   for (int q = tid ^ (kBlock - 64); q < h1.y; q += kBlock) {
     const uint4 t = a.tl.sent[h1.x + q];
@@ -1244,17 +1251,17 @@ __global__ void __launch_bounds__(kBlock) k_adj_iter(AdjArgs a, const float4* __
     const f3 gd = stretch_vjp(lpos[i0], lpos[i1], lav[i0], lav[i1], __uint_as_float(t.z),
                               __uint_as_float(t.w), gkp);
     if ((t.y & 0xffffu) != 0xffffu) {
-      lds_put(l.c[0], l.c[1], l.c[2], t.y & 0xffffu, gd);
+      lds_put(l.c(0), l.c(1), l.c(2), t.y & 0xffffu, gd);
       a.gks[a.tl.scid[h1.x + q]] += (double)gkp;
     }
-    tile_put(l.c[0], l.c[1], l.c[2], t.y >> 16, neg(gd));
+    tile_put(l.c(0), l.c(1), l.c(2), t.y >> 16, neg(gd));
   }
   __syncthreads();
   float acc[kJobs];
 #pragma unroll
   for (int u = 0; u < kJobs; ++u) acc[u] = 0.f;
   tile_jobs<kBlock>(nv, [&](int u, int comp, int v) {
-    if (comp < 3) acc[u] = sum_run(0.f, l.c[comp], l.sp[v], l.sp[v + 1]);
+    if (comp < 3) acc[u] = sum_run(0.f, l.c(comp), l.sp[v], l.sp[v + 1]);
   });
   __syncthreads();
   if (a.dprefix) {
@@ -1266,22 +1273,22 @@ __global__ void __launch_bounds__(kBlock) k_adj_iter(AdjArgs a, const float4* __
         const int id0 = rp.ids.x & 0x1fffffff;
         const float4 P[4] = {ps[id0], ps[rp.ids.y], ps[rp.ids.z], ps[rp.ids.w]};
         const float4 G[4] = {scaled(id0), scaled(rp.ids.y), scaled(rp.ids.z), scaled(rp.ids.w)};
-        lds_put(l.c[0], l.c[1], l.c[2], q - c0, rec_vjp(rp, P, G, a.th));
+        lds_put(l.c(0), l.c(1), l.c(2), q - c0, rec_vjp(rp, P, G, a.th));
       }
       __syncthreads();
       tile_jobs<kBlock>(nv, [&](int u, int comp, int v) {
         if (comp < 3)
-          acc[u] = sum_run(acc[u], l.c[comp], max(l.rp[v], c0) - c0, min(l.rp[v + 1], c1) - c0);
+          acc[u] = sum_run(acc[u], l.c(comp), max(l.rp[v], c0) - c0, min(l.rp[v + 1], c1) - c0);
       });
       __syncthreads();
     }
   }
   tile_jobs<kBlock>(nv, [&](int u, int comp, int v) {
-    if (comp < 3) l.c[comp][v] = acc[u];
+    if (comp < 3) l.c(comp)[v] = acc[u];
   });
   __syncthreads();
   if (tid < nv)
-    la[v0 + tid] = f4(add(xyz(lp[v0 + tid]), mk3(l.c[0][tid], l.c[1][tid], l.c[2][tid])), 0.f);
+    la[v0 + tid] = f4(add(xyz(lp[v0 + tid]), mk3(l.c(0)[tid], l.c(1)[tid], l.c(2)[tid])), 0.f);
 }
 
 // Tape of a recorded substep's contact set: slot `slot` of ctl ([0] records used, [1]
