@@ -1539,8 +1539,10 @@ __device__ __forceinline__ bool holds(f3 amn, f3 amx, f3 bmn, f3 bmx) {
 }
 // The quantised node records, and whether they can be walked: every node's box has to
 // hold its children's. kCaller (unit-level pair query, the caller's own tree): also its
-// children have to lie side by side as the build lays them, and its rightmost leaves
-// must not shrink upwards.
+// children have to lie side by side as the build lays them, its rightmost leaves must not
+// shrink upwards, and no leaf below its left child may lie beyond a right child that is a
+// leaf itself: the record's one rightmost leaf would let that right leaf pass for leaves at
+// and past it (the build's right leaf is the last of its parent's range).
 template <bool kCaller>
 __global__ void __launch_bounds__(kBlock) k_pack_nodes(int t, const int* __restrict__ lefts,
                                                        const int* __restrict__ rights,
@@ -1561,7 +1563,7 @@ __global__ void __launch_bounds__(kBlock) k_pack_nodes(int t, const int* __restr
   bool ok = holds(mn, mx, lmn, lmx) && holds(mn, mx, rmn, rmx);
   if (kCaller && ok)
     ok = sp + 1 == (rl ? r - nin : r) && (ll ? a == l : a >= max(rmll[l], rmlr[l])) &&
-         (rl ? b == r : b >= max(rmll[r], rmlr[r]));
+         (rl ? b == r && a <= b : b >= max(rmll[r], rmlr[r]));
   if (!ok) atomicOr(irr, 1);
   const Quant q = quant_frame(amin[0], amax[0]);
   const uint3 bl = q_box(q, lmn, lmx), br = q_box(q, rmn, rmx);

@@ -1,0 +1,54 @@
+"""cm_lbvh_pairs on trees that no build of the library makes: children side by side and
+boxes that hold what lies below, as the quantised walk takes them, but leaves in any order
+and nodes with several parents or none. The oracle's walk gives the pairs."""
+import numpy as np
+import pytest
+
+from test_gpu_quant_walk import _gpu_pairs
+
+pytestmark = pytest.mark.gpu
+
+
+def _refit(oracle_mod, left, right, lo, hi):
+    t = len(left) + 1
+    left, right = np.array(left, np.int32), np.array(right, np.int32)
+    mn, mx = np.zeros((2 * t - 1, 3), np.float32), np.zeros((2 * t - 1, 3), np.float32)
+    mn[t - 1:], mx[t - 1:] = lo, hi
+    return (left, right) + oracle_mod.refit(left, right, mn, mx)
+
+
+def _check(oracle_mod, tree, cap):
+    want, warn = oracle_mod.pairs(*tree, cap)
+    got, gwarn = _gpu_pairs(*tree, cap)
+    assert np.array_equal(got, want)
+    assert gwarn == warn
+
+
+@pytest.mark.parametrize("cap", [1, 8, 79, 80])
+def test_leaf_right_of_its_right_neighbour(oracle_mod, cap):
+    """Node 0 = (node 1, leaf 2), node 1 = (node 2, leaf 3), node 2 = (leaf 0, leaf 1): the
+    left subtree's rightmost leaf lies beyond the right leaf."""
+    print(f"leaf order, cap {cap}", flush=True)
+    tree = _refit(oracle_mod, [1, 2, 3], [5, 6, 4], np.zeros((4, 3)), np.ones((4, 3)))
+    _check(oracle_mod, tree, cap)
+
+
+def _random_tree(oracle_mod, rng):
+    """Up to 8 leaves; a child is the leaf or the later node of its number."""
+    t = int(rng.integers(2, 9))
+    left, right = [], []
+    for i in range(t - 1):
+        sp = int(rng.integers(0, t - 1))
+        kids = [c if i < c < t - 1 and rng.integers(0, 2) else t - 1 + c for c in (sp, sp + 1)]
+        left.append(kids[0])
+        right.append(kids[1])
+    lo = rng.uniform(0, 1, (t, 3))
+    return _refit(oracle_mod, left, right, lo, lo + rng.uniform(0, 1.5, (t, 3)))
+
+
+@pytest.mark.parametrize("cap", [2, 16, 80])
+def test_random_small_trees(oracle_mod, cap):
+    rng = np.random.default_rng(cap)
+    for k in range(60):
+        print(f"random tree {k}, cap {cap}", flush=True)
+        _check(oracle_mod, _random_tree(oracle_mod, rng), cap)
