@@ -1306,9 +1306,10 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse_lanes(
 // order of k_traverse_resume (rank 0: the root is the one subtree). The leaves they meet
 // join the hits by the quantised test alone and are tested exactly, kG at a time, when
 // there are more than the cap of them and at the end. A leaf that overflows the buffers
-// or the path bits, or could reach the stack limit, and any leaf of an irregular tree, is
-// left to k_traverse_redo. Bound by the rounds' latency (about 1,550 cycles, a third of them
-// the records' loads; 16 to 18 rounds at 64^2), on draped cloths by the instructions.
+// or the path bits, or could reach the stack limit or the visit limit (on a caller's tree
+// of shared nodes: each path to a node is a visit), and any leaf of an irregular tree, is
+// left to k_traverse_redo. Bound by the rounds' latency (about 1,550 cycles, a third of
+// them the records' loads; 16 to 18 rounds at 64^2), on draped cloths by the instructions.
 // k_traverse -> k_traverse_group: 60^2 72 -> 17 us, 64^2 94 -> 25, 96x83 119 -> 42, flat
 // 128^2 112 -> 63, draped 131x97 164 (and 16 for k_traverse_resume) -> 134.
 constexpr int kGroup = 16;  // 8: 22, 34, 41, 64 and 143 us below
@@ -1362,7 +1363,9 @@ __global__ void __launch_bounds__(64) k_traverse_group(WalkTree T, int cap,
   }
   f3 mn = mk3(0, 0, 0), mx = mk3(0, 0, 0);
   uint3 q = make_uint3(0, 0, 0);
+  const int limit = visit_limit(t);
   int np = 0, nh = 0, nv = 0;  // pending, hits, hits tested (the first nv)
+  int seen = 0;                // nodes visited
   if (act) {
     mn = xyz(T.amin[nin + leaf]);
     mx = xyz(T.amax[nin + leaf]);
@@ -1399,6 +1402,7 @@ __global__ void __launch_bounds__(64) k_traverse_group(WalkTree T, int cap,
   while (act) {
     order();
     const int take = min(kG, np), base = np - take;
+    seen += take;
     bool tl = false, tr = false, hl = false, hr = false, deep = false;
     int split = 0, sd = 0;
     uint64_t key = 0, kl = 0;
@@ -1420,7 +1424,7 @@ __global__ void __launch_bounds__(64) k_traverse_group(WalkTree T, int cap,
     const uint32_t c2 = field(__ballot(tl)) | field(__ballot(tr)) << kG;
     const uint32_t h2 = field(__ballot(hl)) | field(__ballot(hr)) << kG;
     const int totc = __popc(c2), tote = __popc(h2);
-    if (field(__ballot(deep)) || base + totc > kGroupPend) {
+    if (field(__ballot(deep)) || base + totc > kGroupPend || seen > limit) {
       again = true;
       break;
     }

@@ -52,3 +52,36 @@ def test_random_small_trees(oracle_mod, cap):
     for k in range(60):
         print(f"random tree {k}, cap {cap}", flush=True)
         _check(oracle_mod, _random_tree(oracle_mod, rng), cap)
+
+
+def _shared(oracle_mod, levels, chain):
+    """`levels` pairs of nodes, each node of a pair above both of the next, then a chain: the
+    chain is walked once for each of the 2^levels paths to it. The leaves of low numbers lie
+    in no node, between the chain's leaves, which the last but one of them meets."""
+    b = 2 * levels + 1
+    t = b + chain + 1
+    left, right = list(range(1, t)), list(range(2, t + 1))
+    for k in range(1, levels):  # nodes 2k - 1 and 2k have the children 2k + 1 and 2k + 2
+        left[2 * k - 1], right[2 * k - 1] = 2 * k + 1, 2 * k + 2
+        left[2 * k], right[2 * k] = 2 * k + 1, 2 * k + 2
+    for i in range(b - 2, t - 1):  # leaf s, then node s + 1
+        s = max(i, b - 1)
+        left[i], right[i] = t - 1 + s, s + 1
+    right[t - 2] = 2 * t - 2
+    lo = np.zeros((t, 3))
+    lo[:b - 1, 0] = 5.0
+    lo[b - 2, 0] = 0.5
+    lo[t - 1, 0] = 10.0
+    return _refit(oracle_mod, left, right, lo, lo + 1.0)
+
+
+@pytest.mark.parametrize("levels,chain,cap", [(8, 24, 16), (8, 25, 16), (8, 40, 79), (11, 38, 79),
+                                              (11, 38, 80)])
+def test_visit_limit(oracle_mod, levels, chain, cap):
+    """Trees whose shared nodes make fewer visits than the limit, a few more and many more."""
+    print(f"visit limit: {levels} levels, chain {chain}, cap {cap}", flush=True)
+    tree = _shared(oracle_mod, levels, chain)
+    want, warn = oracle_mod.pairs(*tree, cap)
+    limited = (2 << levels) - 1 + (chain << levels) > 64 * (len(tree[0]) + 1) + 4096
+    assert bool(warn & 2) == limited
+    _check(oracle_mod, tree, cap)
