@@ -683,6 +683,16 @@ struct WalkTree {
   const int *slot_cloth, *croot, *ccap;  // batch (null: one cloth)
 };
 
+// box b lies in box a (false when a bound is NaN)
+__device__ __forceinline__ bool holds(f3 amn, f3 amx, f3 bmn, f3 bmx) {
+  return amn.x <= bmn.x && amn.y <= bmn.y && amn.z <= bmn.z && amx.x >= bmx.x &&
+         amx.y >= bmx.y && amx.z >= bmx.z;
+}
+// whether a leaf's own box can be quantised: one with a NaN bound overlaps every box by the
+// exact test, and where no node holds its leaf (midpoint split on tied codes) the tree is
+// regular all the same
+__device__ __forceinline__ bool box_ordered(f3 mn, f3 mx) { return holds(mn, mx, mn, mx); }
+
 // DFS of one leaf (Collision/CudaBVH.cu:23-113) from the root through the exact boxes:
 // the second leaves of its pairs in the reference's order into out (at most cap); the
 // stack is sstk[k][col]. Returns their number.
@@ -980,7 +990,7 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap,
     mn = xyz(T.amin[me]);
     mx = xyz(T.amax[me]);
     end = kRedo;
-    if (T.qnodes && *T.irr == 0) {
+    if (T.qnodes && *T.irr == 0 && box_ordered(mn, mx)) {
       q = q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn);
       end = walk_quant<kCand, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out,
                                    budget > 0 && rec ? budget : INT_MAX, st, w, sstk, cand,
@@ -1375,6 +1385,8 @@ __global__ void __launch_bounds__(64) k_traverse_group(WalkTree T, int cap,
       pk[0] = 0;
     }
     np = 1;
+    again = !box_ordered(mn, mx);
+    act = !again;
   }
   // tests hits nv to nh exactly and closes the gaps
   auto test_hits = [&] {
@@ -1536,11 +1548,6 @@ __global__ void k_clear_records(int* __restrict__ hctl) {
   if (threadIdx.x == 0) hctl[0] = 0;
 }
 
-// box b lies in box a (false when a bound is NaN)
-__device__ __forceinline__ bool holds(f3 amn, f3 amx, f3 bmn, f3 bmx) {
-  return amn.x <= bmn.x && amn.y <= bmn.y && amn.z <= bmn.z && amx.x >= bmx.x &&
-         amx.y >= bmx.y && amx.z >= bmx.z;
-}
 // The quantised node records, and whether they can be walked: every node's box has to
 // hold its children's. kCaller (unit-level pair query, the caller's own tree): also its
 // children have to lie side by side as the build lays them, its rightmost leaves must not

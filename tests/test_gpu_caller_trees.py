@@ -4,7 +4,7 @@ and nodes with several parents or none. The oracle's walk gives the pairs."""
 import numpy as np
 import pytest
 
-from test_gpu_quant_walk import _gpu_pairs
+from test_gpu_quant_walk import _gpu_pairs, _keys, _tree
 
 pytestmark = pytest.mark.gpu
 
@@ -84,4 +84,21 @@ def test_visit_limit(oracle_mod, levels, chain, cap):
     want, warn = oracle_mod.pairs(*tree, cap)
     limited = (2 << levels) - 1 + (chain << levels) > 64 * (len(tree[0]) + 1) + 4096
     assert bool(warn & 2) == limited
+    _check(oracle_mod, tree, cap)
+
+
+@pytest.mark.parametrize("t,cap", [(4, 2), (4, 80), (300, 16), (300, 90), (40000, 8)])
+def test_unheld_leaf_with_nan_box(oracle_mod, t, cap):
+    """Leaf 0 belongs to no node (its parent holds leaves 1 and 2) and its box is NaN, which
+    overlaps every box: its pairs are the leaves of the tree up to the cap."""
+    print(f"NaN leaf beside a tree of {t} leaves, cap {cap}", flush=True)
+    left, right, mn, mx, _, _ = _tree(oracle_mod, _keys("unique", t), 0.05, t)
+    lo, hi = np.array(mn[t - 1:]), np.array(mx[t - 1:])
+    lo[0] = hi[0] = np.nan
+    left, right = np.array(left), np.array(right)
+    parent = np.flatnonzero(left == t - 1)[0]
+    left[parent], right[parent] = t, t + 1
+    tree = _refit(oracle_mod, left, right, lo, hi)
+    want, _ = oracle_mod.pairs(*tree, cap)
+    assert (want[:, 0] == 0).sum() >= min(cap, t - 1)
     _check(oracle_mod, tree, cap)
