@@ -529,15 +529,15 @@ __device__ __forceinline__ unsigned long long unpack31(unsigned long long st) {
 }
 
 __global__ void __launch_bounds__(kBlock) k_scan_tiles(
-    const int* __restrict__ d_items, TileRule rule, int n_max, const int* sums, int* pre, int packed,
+    const int* __restrict__ d_items, TileRule rule, int64_t n_max, const int* sums, int* pre, int packed,
     int64_t cap0, int64_t cap1, int* __restrict__ d_tot0, int* __restrict__ d_tot1,
     int* __restrict__ ctr, unsigned long long* __restrict__ state) {
   __shared__ unsigned long long lds[kBlock / 64 + 1];
   __shared__ unsigned long long s_prefix;
   __shared__ int s_tile, s_last;
-  int n = n_max;  // tiles; with d_items, the tiles of at most n_max items
+  int n = (int)n_max;  // tiles; with d_items, the tiles of at most n_max items
   if (d_items) {
-    const int items = min(max(0, *d_items), n_max);
+    const int items = (int)min((int64_t)max(0, *d_items), n_max);
     const int per = 64 * tile_lanes(rule, items);
     n = items / per + (items % per != 0);
   }
@@ -694,8 +694,8 @@ int scan_exclusive(const int* in, int* out, int n_max, const int* d_n, int* d_to
   return CM_OK;
 }
 
-static int scan_tiles_grid(const int* d_items, TileRule rule, int n_max, int64_t ntile, const int* sums,
-                    int* pre, int packed, int64_t cap0, int64_t cap1, int* d_tot0, int* d_tot1,
+static int scan_tiles_grid(const int* d_items, TileRule rule, int64_t n_max, int64_t ntile,
+                    const int* sums, int* pre, int packed, int64_t cap0, int64_t cap1, int* d_tot0, int* d_tot1,
                     void* temp, hipStream_t s) {
   int* ctr = (int*)temp;
   unsigned long long* state = (unsigned long long*)((char*)temp + 256);
@@ -715,7 +715,7 @@ int scan_tiles(int n, const int* sums, int* pre, int packed, int64_t cap0, int64
 int scan_tiles_dev(const int* d_items, TileRule rule, int64_t item_cap, const int* sums, int* pre,
                    int packed, int64_t cap0, int64_t cap1, int* d_tot0, int* d_tot1, void* temp,
                    hipStream_t s) {
-  return scan_tiles_grid(d_items, rule, (int)item_cap, tile_max(rule, item_cap), sums, pre, packed,
+  return scan_tiles_grid(d_items, rule, item_cap, tile_max(rule, item_cap), sums, pre, packed,
                          cap0, cap1, d_tot0, d_tot1, temp, s);
 }
 
