@@ -531,7 +531,7 @@ constexpr int kBudget = 8, kNoBudget = 1 << 20;
 struct PlanLds {
   float root[3][64];  // secant roots of the 64 candidates under way, by interval
   int stack[128];
-  alignas(8) uint32_t near[2 * kPlanLanes];  // near mask of the tile: 2 words for each 64 candidates
+  uint32_t near[2 * kPlanLanes];  // near mask of the tile: 2 words for each 64 candidates
 };
 
 enum Plan : int { kFar, kNear, kMore };
@@ -699,7 +699,9 @@ __global__ void __launch_bounds__(kBlock) k_ccd_plan(
       depth += __popcll(more);
       if (r == kNear) atomicOr(&L.near[(id - first) >> 5], 1u << ((id - first) & 31));
     }
-    const uint64_t m = lane < chunks ? ((const uint64_t*)L.near)[lane] : 0ull;
+    const uint64_t m =
+        lane < chunks ? (uint64_t)L.near[2 * lane + 1] << 32 | L.near[2 * lane] : 0ull;
+    order();  // the next tile clears the mask
     if (lane < chunks) near_mask[tile * R + lane] = m;
     const int c = wave_sum(__popcll(m));
     if (lane == 0) tile_sum[tile] = c;
