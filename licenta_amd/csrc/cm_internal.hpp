@@ -128,7 +128,7 @@ constexpr int kTravRec = 72;
 // trees of fewer leaves are walked through their quantised nodes (26-bit ids)
 constexpr int kQuantLeaves = 1 << 26;
 // ints per leaf for the traversal stack entries below its LDS part
-constexpr int kTravSpill = 47;
+constexpr int kTravSpill = 55;
 
 struct LbvhBufs {
   int t = 0;

@@ -667,11 +667,10 @@ __global__ void __launch_bounds__(1024) k_refit_top(
 // ---- traversal ----------------------------------------------------------------
 constexpr int kTravBlock = 128;  // 2 waves
 constexpr int kStack = 63;       // usable entries, as the reference's int[64] with its -1 sentinel
-// The first kLdsStack rows of a lane's stack live in LDS (8 KiB per workgroup, so
-// LDS leaves room for 8 waves per SIMD); deeper ones, rare, go to the lane's global
-// spill row of kStack - kLdsStack ints.
-constexpr int kLdsStack = 16;
-constexpr int kSpill = kStack - kLdsStack;
+// The first rows of a lane's stack live in LDS, 8 or 12 in the lane walks (WalkShape), 16 in
+// k_traverse_redo; deeper ones, rare, go to the lane's global spill row of kSpill ints.
+constexpr int kRedoStack = 16;
+constexpr int kSpill = kStack - 8;
 static_assert(kSpill == kTravSpill, "spill row");
 
 // The tree as the traversal kernels take it
@@ -835,7 +834,7 @@ struct WalkState {
 // to the next node. The candidates are collected in LDS: a store to memory in the walk
 // would have each visit wait for it, as loads and stores share one counter. Returns
 // false when the stack limit is reached.
-template <int kRow>
+template <int kLds, int kRow>
 __device__ __forceinline__ bool quant_step(const uint4* __restrict__ qnodes, int leaf, uint3 q,
                                            WalkState& st, int& n, int (*sstk)[kRow],
                                            int (*cand)[kRow], int col, int* __restrict__ spill) {
@@ -846,8 +845,8 @@ __device__ __forceinline__ bool quant_step(const uint4* __restrict__ qnodes, int
   if (v.r & v.rleaf) cand[n++][col] = v.split + 1;
   const bool tl = v.l & !v.lleaf, tr = v.r & !v.rleaf;
   if (tl & tr) {
-    if (st.top < kLdsStack) sstk[st.top][col] = st.tos;
-    else if (st.top < kStack) spill[st.top - kLdsStack] = st.tos;
+    if (st.top < kLds) sstk[st.top][col] = st.tos;
+    else if (st.top < kStack) spill[st.top - kLds] = st.tos;
     else fits = false;
     st.tos = v.split + 1;
     ++st.top;
@@ -856,8 +855,8 @@ __device__ __forceinline__ bool quant_step(const uint4* __restrict__ qnodes, int
   if (!(tl | tr)) {
     st.node = st.top > 0 ? st.tos : -1;
     st.top = max(st.top - 1, 0);
-    st.tos = sstk[min(st.top, kLdsStack - 1)][col];
-    if (st.top >= kLdsStack) st.tos = spill[st.top - kLdsStack];
+    st.tos = sstk[min(st.top, kLds - 1)][col];
+    if (st.top >= kLds) st.tos = spill[st.top - kLds];
   }
   return fits;
 }
@@ -892,21 +891,21 @@ __device__ __forceinline__ int visit_limit(int t) {
 }
 
 // Walks on from st until it ends or `budget` visits were made; the second leaves of its
-// pairs go to out[0, st.n), at most cap.
-template <int kCand, int kVerify, int kRow>
+// pairs go to out[0, st.n), at most cap. cand has ncand rows.
+template <int kLds, int kVerify, int kRow>
 __device__ __forceinline__ WalkEnd walk_quant(const WalkTree& T, int leaf, f3 mn, f3 mx, uint3 q,
                                               int cap, int* __restrict__ out, int budget,
                                               WalkState& st, uint32_t& w, int (*sstk)[kRow],
-                                              int (*cand)[kRow], int col,
+                                              int (*cand)[kRow], int ncand, int col,
                                               int* __restrict__ spill) {
   const int limit = visit_limit(T.t);
   const int bound = min(budget, limit);
   for (;;) {
     int n = 0;
-    const int room = min(kCand - 2, cap - st.n);  // past the cap one more is looked for
+    const int room = min(ncand - 2, cap - st.n);  // past the cap one more is looked for
     bool fits = true;
     while (st.node >= 0 && st.visits < bound && n <= room && fits)
-      fits = quant_step(T.qnodes, leaf, q, st, n, sstk, cand, col, spill);
+      fits = quant_step<kLds>(T.qnodes, leaf, q, st, n, sstk, cand, col, spill);
     const int m = verify<kVerify>(T, mn, mx, n, st.n, cap, out, cand, col);
     st.n = min(m, cap);
     if (!fits) return kRedo;
@@ -930,7 +929,7 @@ constexpr int quant_budget(int budget) { return budget + budget * 7 / 10; }
 constexpr int kRec = kTravRec;
 static_assert(kRec >= 6 + kStack, "record holds the stack");
 
-template <int kRow>
+template <int kLds, int kRow>
 __device__ __forceinline__ void put_record(int* __restrict__ R, int leaf, int cap,
                                            const WalkState& st, int (*sstk)[kRow], int col,
                                            const int* __restrict__ spill) {
@@ -941,14 +940,14 @@ __device__ __forceinline__ void put_record(int* __restrict__ R, int leaf, int ca
   R[4] = cap;
   R[5] = st.visits;
   for (int k = 1; k <= st.top; ++k)
-    R[5 + k] = k == st.top ? st.tos : (k < kLdsStack ? sstk[k][col] : spill[k - kLdsStack]);
+    R[5 + k] = k == st.top ? st.tos : (k < kLds ? sstk[k][col] : spill[k - kLds]);
 }
 
 // First pass: one lane per leaf, at most `budget` visits (no budget: budget <= 0 or
 // no record buffer). A leaf still walking then takes a record slot, if one is left,
 // and counts zero pairs here; past the slots it walks on to the end.
-template <int kCand, int kVerify>
-__global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap,
+template <int kLds, int kVerify>
+__global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap, int ncand,
                                                          int* __restrict__ chunk,
                                                          int* __restrict__ counts,
                                                          uint32_t* __restrict__ warn,
@@ -959,7 +958,8 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap,
                                                          int* __restrict__ spill) {
   // Row k of every lane's stack is one LDS row, so a wave's pushes and pops at equal
   // depths hit 64 consecutive banks.
-  __shared__ int sstk[kLdsStack][kTravBlock], cand[kCand][kTravBlock];
+  extern __shared__ int walk_lds[][kTravBlock];
+  int(*sstk)[kTravBlock] = walk_lds, (*cand)[kTravBlock] = walk_lds + kLds;
   // Workgroups are dealt to the 8 XCDs in turn. Each XCD takes every eighth chunk of
   // `xchunk` consecutive tiles (Morton-ordered leaves), so its L2 serves compact
   // subtrees while the dense regions of the cloth, whose leaves visit many more
@@ -992,8 +992,8 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap,
     end = kRedo;
     if (T.qnodes && *T.irr == 0 && box_ordered(mn, mx)) {
       q = q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn);
-      end = walk_quant<kCand, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out,
-                                   budget > 0 && rec ? budget : INT_MAX, st, w, sstk, cand,
+      end = walk_quant<kLds, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out,
+                                   budget > 0 && rec ? budget : INT_MAX, st, w, sstk, cand, ncand,
                                    threadIdx.x, sp);
     }
   }
@@ -1009,18 +1009,18 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap,
     if (end == kBudget) {
       const int slot = base + __popcll(want & ((1ull << lane) - 1));
       if (slot < rcap) {
-        put_record(rec + (int64_t)slot * kRec, leaf, cap, st, sstk, threadIdx.x, sp);
+        put_record<kLds>(rec + (int64_t)slot * kRec, leaf, cap, st, sstk, threadIdx.x, sp);
         handed = true;
       } else {
-        end = walk_quant<kCand, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out, INT_MAX, st, w, sstk,
-                                     cand, threadIdx.x, sp);
+        end = walk_quant<kLds, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out, INT_MAX, st, w, sstk,
+                                     cand, ncand, threadIdx.x, sp);
       }
     }
   }
   if (walk) ncol = handed ? 0 : st.n;
   if (end == kRedo) {
     w = 0;
-    ncol = walk_exact<kTravBlock, kLdsStack>(T, leaf, root, mn, mx, cap, out, w, sstk,
+    ncol = walk_exact<kTravBlock, kLds>(T, leaf, root, mn, mx, cap, out, w, sstk,
                                              threadIdx.x, sp);
   }
   if (leaf < t) counts[leaf] = ncol;
@@ -1267,12 +1267,13 @@ __global__ void __launch_bounds__(64) k_traverse_resume(WalkTree T,
 // Second pass when there are more than kLaneModeMin records: one lane per record
 // walks on serially from the record's state (next node, stack, pairs written,
 // visits), as the first pass would have without a budget.
-template <int kCand, int kVerify>
+template <int kLds, int kVerify>
 __global__ void __launch_bounds__(kTravBlock) k_traverse_lanes(
-    WalkTree T, int* __restrict__ chunk, int stride, int* __restrict__ counts,
+    WalkTree T, int ncand, int* __restrict__ chunk, int stride, int* __restrict__ counts,
     uint32_t* __restrict__ warn, int* __restrict__ tile_sum, const int* __restrict__ rec, int rcap,
     const int* __restrict__ hctl, int* __restrict__ spill) {
-  __shared__ int sstk[kLdsStack][kTravBlock], cand[kCand][kTravBlock];
+  extern __shared__ int walk_lds[][kTravBlock];
+  int(*sstk)[kTravBlock] = walk_lds, (*cand)[kTravBlock] = walk_lds + kLds;
   const int nres = min(hctl[0], rcap);
   if (nres <= kLaneModeMin) return;  // k_traverse_resume takes them
   const int nin = T.t - 1;
@@ -1284,18 +1285,18 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse_lanes(
     int* sp = spill + (int64_t)leaf * kSpill;
     int* out = chunk + (int64_t)leaf * stride;
     for (int k = 1; k < top; ++k) {
-      if (k < kLdsStack) sstk[k][threadIdx.x] = R[5 + k];
-      else sp[k - kLdsStack] = R[5 + k];
+      if (k < kLds) sstk[k][threadIdx.x] = R[5 + k];
+      else sp[k - kLds] = R[5 + k];
     }
     const f3 mn = xyz(T.amin[nin + leaf]), mx = xyz(T.amax[nin + leaf]);
     WalkState st{R[3], top, top > 0 ? R[5 + top] : 0, R[1], R[5]};
     uint32_t wl = 0;
     int ncol;
-    if (walk_quant<kCand, kVerify, kTravBlock>(T, leaf, mn, mx, q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn),
-                               cap, out, INT_MAX, st, wl, sstk, cand, threadIdx.x, sp) == kRedo) {
+    if (walk_quant<kLds, kVerify, kTravBlock>(T, leaf, mn, mx, q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn),
+                               cap, out, INT_MAX, st, wl, sstk, cand, ncand, threadIdx.x, sp) == kRedo) {
       wl = 0;
       const int root = T.croot ? T.croot[T.slot_cloth[leaf]] : 0;
-      ncol = walk_exact<kTravBlock, kLdsStack>(T, leaf, root, mn, mx, cap, out, wl, sstk,
+      ncol = walk_exact<kTravBlock, kLds>(T, leaf, root, mn, mx, cap, out, wl, sstk,
                                                threadIdx.x, sp);
     } else {
       ncol = st.n;
@@ -1524,14 +1525,14 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse_redo(WalkTree T, int ca
                                                               uint32_t* __restrict__ warn,
                                                               int* __restrict__ tile_sum,
                                                               int* __restrict__ spill) {
-  __shared__ int sstk[kLdsStack][kTravBlock];
+  __shared__ int sstk[kRedoStack][kTravBlock];
   __shared__ int wsum[kTravBlock / 64];
   const int leaf = blockIdx.x * kTravBlock + threadIdx.x;
   int n = leaf < T.t ? counts[leaf] : 0;
   if (n < 0) {
     const int me = T.t - 1 + leaf, c = T.croot ? T.slot_cloth[leaf] : 0;
     uint32_t w = 0;
-    n = walk_exact<kTravBlock, kLdsStack>(T, leaf, T.croot ? T.croot[c] : 0, xyz(T.amin[me]),
+    n = walk_exact<kTravBlock, kRedoStack>(T, leaf, T.croot ? T.croot[c] : 0, xyz(T.amin[me]),
                                           xyz(T.amax[me]), T.croot ? T.ccap[c] : cap,
                                           chunk + (int64_t)leaf * cap, w, sstk, threadIdx.x,
                                           spill + (int64_t)leaf * kSpill);
@@ -1774,12 +1775,26 @@ int launch_refit(const LbvhBufs& b, hipStream_t s) {
   return CM_OK;
 }
 
-// Candidates a lane collects before it tests them, and how many it tests at a time: trees
-// of up to kFewLeaves leaves put at most two waves on a SIMD, so LDS and registers are
-// free, and each walk that stops to test holds up its wave (k_traverse, 66 by 8 against
-// 24 by 4: 64^2 90 against 120 us, 131x97 121 against 196); larger ones need the waves
-// (2 M leaves: 815 us with 16 by 4, 855 with 24 by 4, 1,370 with 66 by 4).
-constexpr int kFewLeaves = 1 << 18;
+// The lane walks' LDS: rows of the stack and of the candidates a lane collects before it
+// tests them, and how many it tests at a time (registers). Each walk that stops to test holds
+// up its wave, so as many candidate rows, up to 66, as leave the launch one round of
+// workgroups: a CU's 160 KB, given out by 1,280 bytes, hold four workgroups of 12 and 66 rows
+// (131,072 leaves) and ten of 12 and 17. Against 16 and 66 rows up to 262,144 leaves: 130 k
+// leaves flat 72 -> 46 us, crumpled 110 -> 70, falling 369 -> 297, draped 308 -> 309; 216 k
+// flat 107 -> 57; 258 k flat 117 -> 60, falling 735 -> 593; 156 k flat 77 -> 50 but draped
+// 343 -> 400 (49 pairs a leaf, 50 rows). Trees of more rounds want the waves: 8 and 24 rows
+// take 1,592 us for 2 M crumpled leaves and 327 for 96 cloths (16 and 16 rows 1,740 and 355,
+// 12 and 24 by 8 1,614 and 324).
+struct WalkShape {
+  int stack, cand, verify;
+};
+static WalkShape walk_shape(int nt) {
+  constexpr int kCus = 256, kLdsBytes = 160 << 10, kGrain = 1280, kRow = kTravBlock * 4;
+  const int per_cu = (nt + kCus - 1) / kCus;
+  if (per_cu > 10) return {8, 24, 4};
+  const int rows = (kLdsBytes / per_cu / kGrain * kGrain - 16) / kRow;  // 16: the tile sums
+  return {12, std::min(66, rows - 12), per_cu > 8 ? 4 : 8};
+}
 
 // the second pass needs a budget, record buffers and quantised nodes
 static bool two_passes(const LbvhBufs& b) {
@@ -1805,19 +1820,25 @@ static int launch_traverse(const LbvhBufs& b, int cap, int* chunk, int* counts, 
     CM_LAUNCH_CHECK();
     return CM_OK;
   }
-  const bool few = t <= kFewLeaves;
-  hipLaunchKernelGGL((few ? k_traverse<66, 8> : k_traverse<16, 4>),
-                     dim3((nt + round - 1) / round * round), dim3(kTravBlock), 0, s, T, cap, chunk,
-                     counts, b.warn, offsets, xchunk, two ? quant_budget(b.trav_budget) : 0,
-                     two ? b.trec : nullptr, b.rcap, b.hctl, b.spill);
+  const WalkShape ws = walk_shape(nt);
+  const size_t lds = sizeof(int) * kTravBlock * (ws.stack + ws.cand);
+  hipLaunchKernelGGL((ws.stack == 8    ? k_traverse<8, 4>
+                      : ws.verify == 4 ? k_traverse<12, 4>
+                                       : k_traverse<12, 8>),
+                     dim3((nt + round - 1) / round * round), dim3(kTravBlock), lds, s, T, cap,
+                     ws.cand, chunk, counts, b.warn, offsets, xchunk,
+                     two ? quant_budget(b.trav_budget) : 0, two ? b.trec : nullptr, b.rcap, b.hctl,
+                     b.spill);
   if (two) {  // one of the two finishes the records, the other returns at once
     hipLaunchKernelGGL(k_traverse_resume, dim3(std::min(b.rcap, kResumeBlocks)), dim3(64), 0, s, T,
                        chunk, cap, counts, b.warn, offsets, b.trec, b.rcap, b.hctl);
     if (b.rcap > kLaneModeMin)
-      hipLaunchKernelGGL((few ? k_traverse_lanes<66, 8> : k_traverse_lanes<16, 4>),
+      hipLaunchKernelGGL((ws.stack == 8    ? k_traverse_lanes<8, 4>
+                          : ws.verify == 4 ? k_traverse_lanes<12, 4>
+                                           : k_traverse_lanes<12, 8>),
                          dim3(std::min((b.rcap + kTravBlock - 1) / kTravBlock, 8192)),
-                         dim3(kTravBlock), 0, s, T, chunk, cap, counts, b.warn, offsets, b.trec,
-                         b.rcap, b.hctl, b.spill);
+                         dim3(kTravBlock), lds, s, T, ws.cand, chunk, cap, counts, b.warn, offsets,
+                         b.trec, b.rcap, b.hctl, b.spill);
   }
   CM_LAUNCH_CHECK();
   return CM_OK;
