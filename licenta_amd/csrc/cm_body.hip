@@ -952,6 +952,7 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
   }
   CM_HIP(hipMemset(b->sort_temp, 0, radix_sort_temp_bytes(t)));
   carve_build(t, b->lb_temp, &b->lb);
+  if (batch && (rc = dalloc(b, &b->lb.irr, (size_t)b->lb.ncloth))) return fail(rc);
   CM_HIP(hipMemset(b->lb_temp, 0, lbvh_build_temp_bytes(t)));
   CM_HIP(hipMemset(b->lb.parents, 0, sizeof(int) * m));
   CM_HIP(hipMemset(b->lb.amin, 0, sizeof(float4) * m));

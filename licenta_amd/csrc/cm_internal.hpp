@@ -142,7 +142,7 @@ struct LbvhBufs {
   int *trm = nullptr, *tdone = nullptr;
   bool group = true;        // few leaves may be walked by groups of lanes
   uint4* qnodes = nullptr;  // quantised record of each internal node, 2 uint4 (k_lbvh.hip)
-  int* irr = nullptr;       // set when the tree has to be walked through its exact boxes
+  int* irr = nullptr;       // per cloth: from 2 on its tree is walked through its exact boxes
   int trav_chunk = 4;       // traversal: tiles per chunk dealt to one XCD (launch shape only)
   // traversal: visits a leaf makes in the first pass before a wave takes it over (0:
   // one pass); records of kTravRec ints for up to rcap such leaves; hctl[0] their

@@ -263,10 +263,8 @@ __device__ __forceinline__ void build_init(const BuildInit& b, int i) {
     b.hi[i] = -1;
   }
   if (i < b.ncloth) b.croot[i] = -1;
-  if (i == 0) {
-    *b.ntop = 0;  // deferred-node count of the refit
-    *b.irr = 0;
-  }
+  if (i < max(b.ncloth, 1)) b.irr[i] = 0;
+  if (i == 0) *b.ntop = 0;  // deferred-node count of the refit
 }
 __global__ void __launch_bounds__(kBlock) k_build_init(BuildInit b) {
   build_init(b, blockIdx.x * kBlock + threadIdx.x);
@@ -341,6 +339,7 @@ __global__ void __launch_bounds__(kBlock) k_parents(int t, const int* __restrict
 constexpr int kRefitCH = 1024;  // leaves (and node ids) per refit workgroup
 constexpr int kTopCap = 2048;   // deferred nodes the top pass keeps in LDS
 constexpr int kTopList = 8192;  // pending deferred nodes the top pass lists in LDS
+constexpr int kIrregular = 2;   // irr from which on a tree is walked through its exact boxes
 
 // Whether any thread changed something in this pass (1, 2, ...), for all threads, with the
 // one barrier that a pass needs anyway: three flags in turn, the next one cleared while this
@@ -548,7 +547,7 @@ __global__ void __launch_bounds__(1024) k_refit_top(
     int* __restrict__ rmlr, const int* __restrict__ state,
     const int* __restrict__ top_list, const int* __restrict__ top_index, int* __restrict__ ntop,
     float4* __restrict__ gmin, float4* __restrict__ gmax, int* __restrict__ grm,
-    int* __restrict__ gdone, uint32_t* __restrict__ warn, int* __restrict__ irr) {
+    int* __restrict__ gdone, uint32_t* __restrict__ warn, int* __restrict__ irr, int ncloth) {
   __shared__ float4 smin[kTopCap], smax[kTopCap];
   __shared__ int srm[kTopCap], sdone[kTopCap];
   __shared__ int plist[kTopList];
@@ -657,9 +656,10 @@ __global__ void __launch_bounds__(1024) k_refit_top(
     for (int k = tid; k < nloop; k += 1024)
       if (gdone[listed ? plist[k] : k] == 0) left_over = true;
   }
-  if (__syncthreads_or(left_over) && tid == 0) {
-    atomicOr(warn, (uint32_t)CM_WARN_REFIT_LIMIT);
-    atomicOr(irr, 1);  // an unfinished node's box need not hold its children's
+  if (__syncthreads_or(left_over)) {
+    if (tid == 0) atomicOr(warn, (uint32_t)CM_WARN_REFIT_LIMIT);
+    // an unfinished node's box need not hold its children's
+    for (int c = tid; c < max(ncloth, 1); c += 1024) irr[c] = kIrregular;
   }
   if (tid == 0) *ntop = 0;
 }
@@ -677,9 +677,9 @@ static_assert(kSpill == kTravSpill, "spill row");
 struct WalkTree {
   int t;
   const uint4* qnodes;  // null: the exact walk
-  const int *irr, *lefts, *rights, *rmll, *rmlr;
+  const int *irr, *lefts, *rights, *rmll, *rmlr;  // irr: per cloth
   const float4 *amin, *amax;
-  const int *slot_cloth, *croot, *ccap;  // batch (null: one cloth)
+  const int *slot_cloth, *croot, *ccap, *tstart;  // batch (null: one cloth)
 };
 
 // box b lies in box a (false when a bound is NaN)
@@ -757,15 +757,16 @@ __device__ __forceinline__ int walk_exact(const WalkTree& T, int leaf, int root,
 //       parents it can be another: then bit 28 is set and .y is the larger of the two)
 //   then three words per child: its box in 16 bits a bound, (min x, min y),
 //       (min z, 65535 - max x), (65535 - max y, 65535 - max z)
-// Bounds are quantised by one monotone function over the root's box, the leaf's own box
-// by the same one as (max x, max y), (max z, 65535 - min x), ..., so boxes that overlap
+// Bounds are quantised by one monotone function over the root's box (in a batch the box of
+// the cloth's root: cloths may lie far apart), the leaf's own box by the same one as (max x, max y), (max z, 65535 - min x), ..., so boxes that overlap
 // have no word larger than the leaf's: three saturating 16-bit subtractions, an or and a
 // compare. The test can pass boxes that do not overlap, so the leaves it finds are
 // candidates: their exact boxes are tested after the walk (by 8 at a time, off its chain
 // of loads), in order, and those that fail are dropped. The pairs and their order are
-// walk_exact's: where a node's box holds its children's (irr clear), a leaf whose exact
+// walk_exact's: where a node's box holds its children's (irr small), a leaf whose exact
 // box passes has ancestors that pass. A walk that reaches the stack limit or the visit
-// limit is given up (kRedo) and done exactly.
+// limit is given up (kRedo) and done exactly, and so is the whole tree where the root's box
+// is so large that leaves apart from each other fall together (coarse_frame).
 // k_traverse with what finishes its long walks, exact records of 64 bytes and pairs
 // stored as they are found -> now: flat 256^2 614 -> 353 us, draped 319 -> 331, draped
 // 131x97 217 -> 179, 64^2 134 -> 100, 2 M leaves 1,070 -> 815, crumpled 1024^2 1,825 ->
@@ -972,10 +973,10 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap, in
   const int stride = cap;  // every leaf's chunk holds the body's cap (a cloth's may be less)
   uint32_t w = 0;
   const int me = t - 1 + leaf;
-  int root = 0, ncol = 0;
+  int root = 0, c = 0, ncol = 0;
   bool walk = leaf < t;
   if (walk && T.croot) {  // a batch: the root of the leaf's cloth, its cap
-    const int c = T.slot_cloth[leaf];
+    c = T.slot_cloth[leaf];
     root = T.croot[c];
     cap = T.ccap[c];
     walk = root >= 0;  // a one-triangle cloth has no pairs
@@ -990,8 +991,8 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap, in
     mn = xyz(T.amin[me]);
     mx = xyz(T.amax[me]);
     end = kRedo;
-    if (T.qnodes && *T.irr == 0 && box_ordered(mn, mx)) {
-      q = q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn);
+    if (T.qnodes && T.irr[c] < kIrregular && box_ordered(mn, mx)) {
+      q = q_box(quant_frame(T.amin[root], T.amax[root]), mx, mn);
       end = walk_quant<kLds, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out,
                                    budget > 0 && rec ? budget : INT_MAX, st, w, sstk, cand, ncand,
                                    threadIdx.x, sp);
@@ -1113,9 +1114,10 @@ __global__ void __launch_bounds__(64) k_traverse_resume(WalkTree T,
   for (int rid = blockIdx.x; rid < nres; rid += gridDim.x) {
     const int* R = rec + (int64_t)rid * kRec;
     const int leaf = R[0], ncol0 = R[1], top0 = R[2], cur = R[3], cap = R[4];
+    const int root = T.croot ? T.croot[T.slot_cloth[leaf]] : 0;
     const long long visits0 = R[5];
     const f3 mn = xyz(T.amin[nin + leaf]), mx = xyz(T.amax[nin + leaf]);
-    const uint3 q = q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn);
+    const uint3 q = q_box(quant_frame(T.amin[root], T.amax[root]), mx, mn);
     const int capr = cap - ncol0;  // pairs still to find (0: only whether one more exists)
     int* out = chunk + (int64_t)leaf * stride;
     // pending: the stack entries bottom-up, then the next node on top
@@ -1237,7 +1239,6 @@ __global__ void __launch_bounds__(64) k_traverse_resume(WalkTree T,
       __syncthreads();
       nout = 0;
       if (lane == 0) {
-        const int root = T.croot ? T.croot[T.slot_cloth[leaf]] : 0;
         nout = walk_exact<1, kStack>(T, leaf, root, mn, mx, cap, out, w, fstk, 0, nullptr);
       }
     } else {
@@ -1282,6 +1283,7 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse_lanes(
        rid += gridDim.x * kTravBlock) {
     const int* R = rec + (int64_t)rid * kRec;
     const int leaf = R[0], top = R[2], cap = R[4];
+    const int root = T.croot ? T.croot[T.slot_cloth[leaf]] : 0;
     int* sp = spill + (int64_t)leaf * kSpill;
     int* out = chunk + (int64_t)leaf * stride;
     for (int k = 1; k < top; ++k) {
@@ -1292,10 +1294,9 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse_lanes(
     WalkState st{R[3], top, top > 0 ? R[5 + top] : 0, R[1], R[5]};
     uint32_t wl = 0;
     int ncol;
-    if (walk_quant<kLds, kVerify, kTravBlock>(T, leaf, mn, mx, q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn),
+    if (walk_quant<kLds, kVerify, kTravBlock>(T, leaf, mn, mx, q_box(quant_frame(T.amin[root], T.amax[root]), mx, mn),
                                cap, out, INT_MAX, st, wl, sstk, cand, ncand, threadIdx.x, sp) == kRedo) {
       wl = 0;
-      const int root = T.croot ? T.croot[T.slot_cloth[leaf]] : 0;
       ncol = walk_exact<kTravBlock, kLds>(T, leaf, root, mn, mx, cap, out, wl, sstk,
                                                threadIdx.x, sp);
     } else {
@@ -1360,15 +1361,15 @@ __global__ void __launch_bounds__(64) k_traverse_group(WalkTree T, int cap,
   const int t = T.t, nin = t - 1, stride = cap;
   // the lanes of a wave share the buffers: their accesses stay in program order
   auto order = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
-  int root = 0;
+  int root = 0, c = 0;
   bool act = leaf < t, again = false;
   if (act && T.croot) {  // a batch: the root of the leaf's cloth, its cap
-    const int c = T.slot_cloth[leaf];
+    c = T.slot_cloth[leaf];
     root = T.croot[c];
     cap = T.ccap[c];
     act = root >= 0;  // a one-triangle cloth has no pairs
   }
-  if (act && *T.irr != 0) {
+  if (act && T.irr[c] >= kIrregular) {
     act = false;
     again = true;
   }
@@ -1380,7 +1381,7 @@ __global__ void __launch_bounds__(64) k_traverse_group(WalkTree T, int cap,
   if (act) {
     mn = xyz(T.amin[nin + leaf]);
     mx = xyz(T.amax[nin + leaf]);
-    q = q_box(quant_frame(T.amin[0], T.amax[0]), mx, mn);
+    q = q_box(quant_frame(T.amin[root], T.amax[root]), mx, mn);
     if (g == 0) {
       pe[0] = root;
       pk[0] = 0;
@@ -1549,35 +1550,58 @@ __global__ void k_clear_records(int* __restrict__ hctl) {
   if (threadIdx.x == 0) hctl[0] = 0;
 }
 
+// Whether leaf i and another leaf of its cloth, drawn by a hash, fall together in the frame
+// though they are apart by half the leaf's extent. One vertex far away, or a piece that falls
+// without end, makes the root's box so large that the cloth is a few cells, and a walk then
+// passes a share of all nodes: with a vertex 1e5 m off 1,770 us at 150^2 (45 through the
+// exact boxes), 6,200 at 256^2 (56), growing with the square of the leaves. A fourth of the
+// leaves draw, so the pairs found are a fourth of the leaves that a walk meets in vain: from
+// kIrregular on the tree is left to the exact walk.
+constexpr int kDraw = 4;
+__device__ __forceinline__ bool coarse_frame(const WalkTree& T, int i, int c, Quant q) {
+  const int nin = T.t - 1, first = T.croot ? T.tstart[c] : 0;
+  const uint32_t n = (uint32_t)((T.croot ? T.tstart[c + 1] : T.t) - first);
+  uint32_t h = (uint32_t)i * 0x9e3779b1u;
+  h = (h ^ (h >> 15)) * 0x85ebca77u;
+  const int j = first + (int)__umulhi(h ^ (h >> 13), n);
+  const f3 amn = xyz(T.amin[nin + i]), amx = xyz(T.amax[nin + i]);
+  const f3 bmn = xyz(T.amin[nin + j]), bmx = xyz(T.amax[nin + j]);
+  const f3 e = sub(amx, amn);
+  const float half = 0.5f * fmaxf(e.x, fmaxf(e.y, e.z));
+  const float gap = fmaxf(fmaxf(fmaxf(bmn.x - amx.x, amn.x - bmx.x),
+                                fmaxf(bmn.y - amx.y, amn.y - bmx.y)),
+                          fmaxf(bmn.z - amx.z, amn.z - bmx.z));
+  const uint3 o = q_box(q, bmn, bmx);
+  return gap > half && q_overlap(o.x, o.y, o.z, q_box(q, amx, amn));
+}
+
 // The quantised node records, and whether they can be walked: every node's box has to
-// hold its children's. kCaller (unit-level pair query, the caller's own tree): also its
+// hold its children's, and the frame be fine enough. kCaller (unit-level pair query, the caller's own tree): also its
 // children have to lie side by side as the build lays them, its rightmost leaves must not
 // shrink upwards, and no leaf below its left child may lie beyond a right child that is a
 // leaf itself: the record's one rightmost leaf would let that right leaf pass for leaves at
 // and past it (the build's right leaf is the last of its parent's range).
 template <bool kCaller>
-__global__ void __launch_bounds__(kBlock) k_pack_nodes(int t, const int* __restrict__ lefts,
-                                                       const int* __restrict__ rights,
-                                                       const float4* __restrict__ amin,
-                                                       const float4* __restrict__ amax,
-                                                       const int* __restrict__ rmll,
-                                                       const int* __restrict__ rmlr,
-                                                       uint4* __restrict__ qnodes,
+__global__ void __launch_bounds__(kBlock) k_pack_nodes(WalkTree T, uint4* __restrict__ qnodes,
                                                        int* __restrict__ irr) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
-  const int nin = t - 1;
+  const int nin = T.t - 1;
   if (i >= nin) return;
-  const int l = lefts[i], r = rights[i], a = rmll[i], b = rmlr[i];
-  const f3 lmn = xyz(amin[l]), lmx = xyz(amax[l]), rmn = xyz(amin[r]), rmx = xyz(amax[r]);
-  const f3 mn = xyz(amin[i]), mx = xyz(amax[i]);
+  const int l = T.lefts[i], r = T.rights[i], a = T.rmll[i], b = T.rmlr[i];
+  const f3 lmn = xyz(T.amin[l]), lmx = xyz(T.amax[l]), rmn = xyz(T.amin[r]), rmx = xyz(T.amax[r]);
+  const f3 mn = xyz(T.amin[i]), mx = xyz(T.amax[i]);
   const bool ll = l >= nin, rl = r >= nin;
   const int sp = ll ? l - nin : l;
   bool ok = holds(mn, mx, lmn, lmx) && holds(mn, mx, rmn, rmx);
   if (kCaller && ok)
-    ok = sp + 1 == (rl ? r - nin : r) && (ll ? a == l : a >= max(rmll[l], rmlr[l])) &&
-         (rl ? b == r && a <= b : b >= max(rmll[r], rmlr[r]));
-  if (!ok) atomicOr(irr, 1);
-  const Quant q = quant_frame(amin[0], amax[0]);
+    ok = sp + 1 == (rl ? r - nin : r) && (ll ? a == l : a >= max(T.rmll[l], T.rmlr[l])) &&
+         (rl ? b == r && a <= b : b >= max(T.rmll[r], T.rmlr[r]));
+  // in a batch, a node that is walked and the leaf of its number belong to one cloth
+  const int c = T.croot ? T.slot_cloth[i] : 0, root = T.croot ? max(T.croot[c], 0) : 0;
+  const Quant q = quant_frame(T.amin[root], T.amax[root]);
+  const int found = !ok ? kIrregular : (i % kDraw == 0 && coarse_frame(T, i, c, q)) ? 1 : 0;
+  if (found && __hip_atomic_load(&irr[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kIrregular)
+    atomicAdd(&irr[c], found);
   const uint3 bl = q_box(q, lmn, lmx), br = q_box(q, rmn, rmx);
   const bool other = a != nin + sp;
   qnodes[2 * (int64_t)i] =
@@ -1770,7 +1794,7 @@ int launch_refit(const LbvhBufs& b, hipStream_t s) {
                        b.top_list, b.top_index, b.ntop, b.tmin, b.tmax, b.trm, b.tdone);
   hipLaunchKernelGGL(k_refit_top, dim3(1), dim3(1024), 0, s, t, b.lefts, b.rights, b.amin, b.amax,
                      b.rmll, b.rmlr, b.state, b.top_list, b.top_index, b.ntop, b.tmin,
-                     b.tmax, b.trm, b.tdone, b.warn, b.irr);
+                     b.tmax, b.trm, b.tdone, b.warn, b.irr, b.ncloth);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
@@ -1796,6 +1820,12 @@ static WalkShape walk_shape(int nt) {
   return {12, std::min(66, rows - 12), per_cu > 8 ? 4 : 8};
 }
 
+static WalkTree walk_tree(const LbvhBufs& b) {
+  return {b.t,    b.t < kQuantLeaves ? b.qnodes : nullptr, b.irr, b.lefts, b.rights, b.rmll,
+          b.rmlr, b.amin, b.amax, b.ncloth ? b.slot_cloth : nullptr,
+          b.ncloth ? b.croot : nullptr, b.ccap, b.tstart};
+}
+
 // the second pass needs a budget, record buffers and quantised nodes
 static bool two_passes(const LbvhBufs& b) {
   return b.t < kQuantLeaves && b.trav_budget > 0 && b.trec && b.hctl && b.rcap > 0;
@@ -1808,9 +1838,7 @@ static int launch_traverse(const LbvhBufs& b, int cap, int* chunk, int* counts, 
   const int xchunk = b.trav_chunk > 0 ? b.trav_chunk : 4;
   const int round = kXcds * xchunk;
   const bool two = two_passes(b);
-  const WalkTree T{t,      t < kQuantLeaves ? b.qnodes : nullptr, b.irr, b.lefts, b.rights, b.rmll,
-                   b.rmlr, b.amin, b.amax, b.ncloth ? b.slot_cloth : nullptr,
-                   b.ncloth ? b.croot : nullptr, b.ccap};
+  const WalkTree T = walk_tree(b);
   if (b.group && T.qnodes && t <= kGroupLeaves && cap <= kGroupMaxCap) {
     const int per = 64 / kGroup, nb = (t + per - 1) / per, rnd = kXcds * 4 * kTravBlock / per;
     hipLaunchKernelGGL(k_traverse_group<kGroup>, dim3((nb + rnd - 1) / rnd * rnd), dim3(64), 0, s,
@@ -1883,8 +1911,7 @@ int launch_pack_nodes(const LbvhBufs& b, bool from_caller, hipStream_t s) {
   const int t = b.t;
   if (t < 2 || t >= kQuantLeaves) return CM_OK;
   hipLaunchKernelGGL(from_caller ? k_pack_nodes<true> : k_pack_nodes<false>, dim3(nblocks(t - 1)),
-                     dim3(kBlock), 0, s, t, b.lefts, b.rights, b.amin, b.amax, b.rmll, b.rmlr,
-                     b.qnodes, b.irr);
+                     dim3(kBlock), 0, s, walk_tree(b), b.qnodes, b.irr);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
