@@ -142,6 +142,7 @@ struct LbvhBufs {
   int *trm = nullptr, *tdone = nullptr;
   bool group = true;        // few leaves may be walked by groups of lanes
   uint4* qnodes = nullptr;  // quantised record of each internal node, 2 uint4 (k_lbvh.hip)
+  float4* nodes = nullptr;  // exact records of a caller's irregular tree, 4 float4 a node
   int* irr = nullptr;       // per cloth: from 2 on its tree is walked through its exact boxes
   int trav_chunk = 4;       // traversal: tiles per chunk dealt to one XCD (launch shape only)
   // traversal: visits a leaf makes in the first pass before a wave takes it over (0:

@@ -677,6 +677,7 @@ static_assert(kSpill == kTravSpill, "spill row");
 struct WalkTree {
   int t;
   const uint4* qnodes;  // null: the exact walk
+  const float4* nodes;  // records of the exact walk of an irregular tree (k_pack_exact) or null
   const int *irr, *lefts, *rights, *rmll, *rmlr;  // irr: per cloth
   const float4 *amin, *amax;
   const int *slot_cloth, *croot, *ccap, *tstart;  // batch (null: one cloth)
@@ -695,7 +696,7 @@ __device__ __forceinline__ bool box_ordered(f3 mn, f3 mx) { return holds(mn, mx,
 // DFS of one leaf (Collision/CudaBVH.cu:23-113) from the root through the exact boxes:
 // the second leaves of its pairs in the reference's order into out (at most cap); the
 // stack is sstk[k][col]. Returns their number.
-template <int kRow, int kLds>
+template <int kRow, int kLds, bool kPacked = false>
 __device__ __forceinline__ int walk_exact(const WalkTree& T, int leaf, int root, f3 mn, f3 mx, int cap,
                           int* __restrict__ out, uint32_t& w, int (*sstk)[kRow], int col,
                           int* __restrict__ spill) {
@@ -707,9 +708,21 @@ __device__ __forceinline__ int walk_exact(const WalkTree& T, int leaf, int root,
       w |= CM_WARN_TRAVERSAL_LIMIT;
       break;
     }
-    const int l = T.lefts[node], r = T.rights[node];
-    const bool ol = (T.rmll[node] > me) & overlap(mn, mx, xyz(T.amin[l]), xyz(T.amax[l]));
-    const bool orr = (T.rmlr[node] > me) & overlap(mn, mx, xyz(T.amin[r]), xyz(T.amax[r]));
+    int l, r;
+    bool ol, orr;
+    if (kPacked) {
+      const float4* n = T.nodes + 4 * (int64_t)node;
+      const float4 ids = n[0], a = n[1], b = n[2], c = n[3];
+      l = __float_as_int(ids.x);
+      r = __float_as_int(ids.y);
+      ol = (__float_as_int(ids.z) > me) & overlap(mn, mx, xyz(a), mk3(a.w, b.x, b.y));
+      orr = (__float_as_int(ids.w) > me) & overlap(mn, mx, mk3(b.z, b.w, c.x), mk3(c.y, c.z, c.w));
+    } else {
+      l = T.lefts[node];
+      r = T.rights[node];
+      ol = (T.rmll[node] > me) & overlap(mn, mx, xyz(T.amin[l]), xyz(T.amax[l]));
+      orr = (T.rmlr[node] > me) & overlap(mn, mx, xyz(T.amin[r]), xyz(T.amax[r]));
+    }
     const bool el = ol & (l >= nin), er = orr & (r >= nin);
     // Past the cap the reference keeps walking but drops every further pair, so
     // stopping at the first dropped pair yields the same list.
@@ -944,6 +957,15 @@ __device__ __forceinline__ void put_record(int* __restrict__ R, int leaf, int ca
     R[5 + k] = k == st.top ? st.tos : (k < kLds ? sstk[k][col] : spill[k - kLds]);
 }
 
+// Workgroups are dealt to the 8 XCDs in turn. Each XCD takes every eighth chunk of
+// `xchunk` consecutive tiles (Morton-ordered leaves), so its L2 serves compact
+// subtrees while the dense regions of the cloth, whose leaves visit many more
+// nodes, are shared evenly between the XCDs. The grid is padded to whole rounds.
+__device__ __forceinline__ int walk_tile(int xchunk) {
+  const int j = blockIdx.x / kXcds, xcd = blockIdx.x % kXcds;
+  return ((j / xchunk) * kXcds + xcd) * xchunk + j % xchunk;
+}
+
 // First pass: one lane per leaf, at most `budget` visits (no budget: budget <= 0 or
 // no record buffer). A leaf still walking then takes a record slot, if one is left,
 // and counts zero pairs here; past the slots it walks on to the end.
@@ -961,14 +983,10 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap, in
   // depths hit 64 consecutive banks.
   extern __shared__ int walk_lds[][kTravBlock];
   int(*sstk)[kTravBlock] = walk_lds, (*cand)[kTravBlock] = walk_lds + kLds;
-  // Workgroups are dealt to the 8 XCDs in turn. Each XCD takes every eighth chunk of
-  // `xchunk` consecutive tiles (Morton-ordered leaves), so its L2 serves compact
-  // subtrees while the dense regions of the cloth, whose leaves visit many more
-  // nodes, are shared evenly between the XCDs. The grid is padded to whole rounds.
-  const int j = blockIdx.x / kXcds, xcd = blockIdx.x % kXcds;
-  const int tile = ((j / xchunk) * kXcds + xcd) * xchunk + j % xchunk;
+  const int tile = walk_tile(xchunk);
   const int t = T.t;
   if (tile >= (t + kTravBlock - 1) / kTravBlock) return;
+  if (T.nodes && *T.irr >= kIrregular) return;  // k_traverse_exact takes the tree
   const int leaf = tile * kTravBlock + threadIdx.x;
   const int stride = cap;  // every leaf's chunk holds the body's cap (a cloth's may be less)
   uint32_t w = 0;
@@ -1546,6 +1564,38 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse_redo(WalkTree T, int ca
   if (threadIdx.x == 0) tile_sum[blockIdx.x] = wsum[0] + wsum[1];
 }
 
+// A caller's irregular tree of many leaves through its exact records: one lane per leaf, and
+// no more LDS than the stack's, so that eight waves a SIMD hide the gathers.
+__global__ void __launch_bounds__(kTravBlock) k_traverse_exact(WalkTree T, int cap, int xchunk,
+                                                               int* __restrict__ chunk,
+                                                               int* __restrict__ counts,
+                                                               uint32_t* __restrict__ warn,
+                                                               int* __restrict__ tile_sum,
+                                                               int* __restrict__ spill) {
+  __shared__ int sstk[kRedoStack][kTravBlock];
+  __shared__ int wsum[kTravBlock / 64];
+  const int tile = walk_tile(xchunk), leaf = tile * kTravBlock + threadIdx.x;
+  if (tile >= (T.t + kTravBlock - 1) / kTravBlock || *T.irr < kIrregular) return;
+  int n = 0;
+  uint32_t w = 0;
+  if (leaf < T.t) {
+    const int me = T.t - 1 + leaf;
+    n = walk_exact<kTravBlock, kRedoStack, true>(T, leaf, 0, xyz(T.amin[me]), xyz(T.amax[me]), cap,
+                                                 chunk + (int64_t)leaf * cap, w, sstk, threadIdx.x,
+                                                 spill + (int64_t)leaf * kSpill);
+    counts[leaf] = n;
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) w |= __shfl_xor(w, o, 64);
+  n = wave_sum(n);
+  if ((threadIdx.x & 63) == 0) {
+    wsum[threadIdx.x >> 6] = n;
+    if (w) atomicOr(warn, w);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) tile_sum[tile] = wsum[0] + wsum[1];
+}
+
 __global__ void k_clear_records(int* __restrict__ hctl) {
   if (threadIdx.x == 0) hctl[0] = 0;
 }
@@ -1587,6 +1637,10 @@ __global__ void __launch_bounds__(kBlock) k_pack_nodes(WalkTree T, uint4* __rest
   const int i = blockIdx.x * kBlock + threadIdx.x;
   const int nin = T.t - 1;
   if (i >= nin) return;
+  // a tree that others have found irregular needs no records
+  if (kCaller &&
+      __hip_atomic_load(irr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= kIrregular)
+    return;
   const int l = T.lefts[i], r = T.rights[i], a = T.rmll[i], b = T.rmlr[i];
   const f3 lmn = xyz(T.amin[l]), lmx = xyz(T.amax[l]), rmn = xyz(T.amin[r]), rmx = xyz(T.amax[r]);
   const f3 mn = xyz(T.amin[i]), mx = xyz(T.amax[i]);
@@ -1599,7 +1653,11 @@ __global__ void __launch_bounds__(kBlock) k_pack_nodes(WalkTree T, uint4* __rest
   // in a batch, a node that is walked and the leaf of its number belong to one cloth
   const int c = T.croot ? T.slot_cloth[i] : 0, root = T.croot ? max(T.croot[c], 0) : 0;
   const Quant q = quant_frame(T.amin[root], T.amax[root]);
-  const int found = !ok ? kIrregular : (i % kDraw == 0 && coarse_frame(T, i, c, q)) ? 1 : 0;
+  int found = !ok ? kIrregular : (i % kDraw == 0 && coarse_frame(T, i, c, q)) ? 1 : 0;
+  if (!T.croot) {  // one cloth: one lane adds for the wave
+    const uint64_t any = __ballot(found), bad = __ballot(found == kIrregular);
+    found = (threadIdx.x & 63) == __ffsll((long long)any) - 1 ? (bad ? kIrregular : __popcll(any)) : 0;
+  }
   if (found && __hip_atomic_load(&irr[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kIrregular)
     atomicAdd(&irr[c], found);
   const uint3 bl = q_box(q, lmn, lmx), br = q_box(q, rmn, rmx);
@@ -1609,6 +1667,24 @@ __global__ void __launch_bounds__(kBlock) k_pack_nodes(WalkTree T, uint4* __rest
                      (other ? kOtherRight : 0u),
                  (uint32_t)((other ? max(a, b) : b) - nin), bl.x, bl.y);
   qnodes[2 * (int64_t)i + 1] = make_uint4(bl.z, br.x, br.y, br.z);
+}
+
+// 64-byte records of an irregular tree for the exact walk: children, rightmost leaves, both
+// boxes. A caller's nodes may be numbered in any order, and four words and four boxes from as
+// many places a visit then cost several times the record's one (500 k renumbered leaves 2,296
+// us, with the records 5XX; 2 M 10,735 and 1,9XX). Up to kGroupLeaves leaves the caches hold
+// the tree (30,000: 132 us, 137 by records), and a body's nodes lie as the build numbers them.
+__global__ void __launch_bounds__(kBlock) k_pack_exact(WalkTree T, float4* __restrict__ nodes) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= T.t - 1 || *T.irr < kIrregular) return;
+  const int l = T.lefts[i], r = T.rights[i];
+  const f3 lmn = xyz(T.amin[l]), lmx = xyz(T.amax[l]), rmn = xyz(T.amin[r]), rmx = xyz(T.amax[r]);
+  float4* o = nodes + 4 * (int64_t)i;
+  o[0] = make_float4(__int_as_float(l), __int_as_float(r), __int_as_float(T.rmll[i]),
+                     __int_as_float(T.rmlr[i]));
+  o[1] = make_float4(lmn.x, lmn.y, lmn.z, lmx.x);
+  o[2] = make_float4(lmx.y, lmx.z, rmn.x, rmn.y);
+  o[3] = make_float4(rmn.z, rmx.x, rmx.y, rmx.z);
 }
 
 // One workgroup per traversal tile of kTravBlock leaves: the first wave scans the
@@ -1821,7 +1897,7 @@ static WalkShape walk_shape(int nt) {
 }
 
 static WalkTree walk_tree(const LbvhBufs& b) {
-  return {b.t,    b.t < kQuantLeaves ? b.qnodes : nullptr, b.irr, b.lefts, b.rights, b.rmll,
+  return {b.t,    b.t < kQuantLeaves ? b.qnodes : nullptr, b.nodes, b.irr, b.lefts, b.rights, b.rmll,
           b.rmlr, b.amin, b.amax, b.ncloth ? b.slot_cloth : nullptr,
           b.ncloth ? b.croot : nullptr, b.ccap, b.tstart};
 }
@@ -1857,6 +1933,9 @@ static int launch_traverse(const LbvhBufs& b, int cap, int* chunk, int* counts, 
                      ws.cand, chunk, counts, b.warn, offsets, xchunk,
                      two ? quant_budget(b.trav_budget) : 0, two ? b.trec : nullptr, b.rcap, b.hctl,
                      b.spill);
+  if (b.nodes)
+    hipLaunchKernelGGL(k_traverse_exact, dim3((nt + round - 1) / round * round), dim3(kTravBlock),
+                       0, s, T, cap, xchunk, chunk, counts, b.warn, offsets, b.spill);
   if (two) {  // one of the two finishes the records, the other returns at once
     hipLaunchKernelGGL(k_traverse_resume, dim3(std::min(b.rcap, kResumeBlocks)), dim3(64), 0, s, T,
                        chunk, cap, counts, b.warn, offsets, b.trec, b.rcap, b.hctl);
@@ -1912,6 +1991,9 @@ int launch_pack_nodes(const LbvhBufs& b, bool from_caller, hipStream_t s) {
   if (t < 2 || t >= kQuantLeaves) return CM_OK;
   hipLaunchKernelGGL(from_caller ? k_pack_nodes<true> : k_pack_nodes<false>, dim3(nblocks(t - 1)),
                      dim3(kBlock), 0, s, walk_tree(b), b.qnodes, b.irr);
+  if (b.nodes)
+    hipLaunchKernelGGL(k_pack_exact, dim3(nblocks(t - 1)), dim3(kBlock), 0, s, walk_tree(b),
+                       b.nodes);
   CM_LAUNCH_CHECK();
   return CM_OK;
 }
@@ -1959,10 +2041,15 @@ size_t carve_build(int t, void* d_temp, LbvhBufs* b) {
 }
 
 size_t lbvh_build_temp_bytes(int t) { return carve_build(t, nullptr, nullptr); }
+// bytes of the exact walk's records for a caller's tree
+static size_t exact_bytes(int t) {
+  return t > kGroupLeaves && t < kQuantLeaves ? align_up(4 * sizeof(float4) * (size_t)t) : 0;
+}
 size_t lbvh_pairs_temp_bytes(int t, int cap) {
   return align_up(sizeof(int) * (size_t)t * cap) +
          2 * align_up(sizeof(int) * (size_t)t) + align_up(2 * sizeof(uint4) * (size_t)t) +
-         align_up(sizeof(int) * kSpill * (size_t)t) + align_up(sizeof(int)) + scan_temp_bytes(t);
+         exact_bytes(t) + align_up(sizeof(int) * kSpill * (size_t)t) + align_up(sizeof(int)) +
+         scan_temp_bytes(t);
 }
 
 }  // namespace cm
@@ -2090,6 +2177,8 @@ extern "C" int cm_lbvh_pairs(int32_t t, const int32_t* d_lefts, const int32_t* d
   tp += align_up(sizeof(int) * (size_t)t);
   b.qnodes = (uint4*)tp;
   tp += align_up(2 * sizeof(uint4) * (size_t)t);
+  if (exact_bytes(t)) b.nodes = (float4*)tp;
+  tp += exact_bytes(t);
   b.spill = (int*)tp;
   tp += align_up(sizeof(int) * kSpill * (size_t)t);
   b.irr = (int*)tp;

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from test_gpu_quant_walk import _gpu_pairs, _keys, _tree
+from test_gpu_walk_shapes import _sheet
 
 pytestmark = pytest.mark.gpu
 
@@ -101,4 +102,19 @@ def test_unheld_leaf_with_nan_box(oracle_mod, t, cap):
     tree = _refit(oracle_mod, left, right, lo, hi)
     want, _ = oracle_mod.pairs(*tree, cap)
     assert (want[:, 0] == 0).sum() >= min(cap, t - 1)
+    _check(oracle_mod, tree, cap)
+
+
+@pytest.mark.parametrize("t,cap", [(32768, 16), (32769, 16), (32769, 100), (150001, 24)])
+def test_renumbered_nodes(oracle_mod, t, cap):
+    """The build's tree with its nodes in another order (the root stays node 0), up to the
+    leaves from which on the exact walk takes records of its own; lists cut at the cap."""
+    print(f"renumbered tree of {t} leaves, cap {cap}", flush=True)
+    left, right, mn, mx, rl, rr = _sheet(oracle_mod, t, 4.0 if cap > 24 else 8.0)
+    rng = np.random.default_rng(t)
+    new = np.concatenate([[0], 1 + rng.permutation(t - 2)])
+    at = np.concatenate([new, np.arange(t - 1, 2 * t - 1)])
+    tree = [np.empty_like(a) for a in (left, right, mn, mx, rl, rr)]
+    tree[0][new], tree[1][new], tree[4][new], tree[5][new] = at[left], at[right], rl, rr
+    tree[2][at], tree[3][at] = mn, mx
     _check(oracle_mod, tree, cap)
