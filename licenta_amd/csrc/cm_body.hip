@@ -404,20 +404,23 @@ void build_tiles(int n, HostTopo& h, int tile_v, int sub) {
   }
 }
 
-// The tile shape of a body, from k_solve's launches measured on the draped 256^2 and
-// 131x97 cloths (contacts) and on cloths without contacts:
-// - from 2,048 tiles of 128 up, or without self-collision, plain 128-vertex patches
-//   with 256 threads: the fewest repeated evaluations, and the tiles per CU even out
-//   their contacts (1024^2: 122 us, 180 as below; 96 cloths: 91 against 101 us);
-// - smaller colliding cloths: 512 threads and tiles of 32-vertex patches from all over
-//   the cloth (draped 256^2: 23 us; 41 us as plain patches of 256 threads, whose
-//   heaviest tile holds 5,800 of the 344,000 records; without contacts 13.6 against
-//   11.8 us);
-// - fewer vertices per tile where the tiles would not fill the CUs (131x97: 14.5 us
-//   with 64, 15.4 with 128; 64^2: 6.0 us with 32, 7.0 with 64, 8.4 with 128).
+// The tile shape of a body, from an iteration's time (k_solve):
+// - fewer vertices a tile where larger tiles would leave CUs idle behind the longest one:
+//   without collisions 64^2 8.2 us with 128, 6.5 with 64, 5.4 with 32, 16^2 7.4, 5.2 and 4.7;
+//   128^2 8.4, 6.7 and 6.4; 181^2 8.6, 7.9 and 9.7; 192x301 10.7, 12.4 and 15.1; draped cloths
+//   of 110^2 14.6, 13.4 and 12.2, 131x97 13.8, 11.1 and 11.7, 181^2 13.3, 11.8 and 16.0;
+// - 512 threads for tiles of 32 (64^2 5.4 -> 5.1 us, 16^2 5.2 -> 4.8), and for 64 vertices one
+//   tile (8^2 4.3 us, 4.7 in two);
+// - plain patches without contacts and from 2,048 tiles up, 256 threads for 64 and more: the
+//   fewest repeated evaluations, and the tiles per CU even out their contacts (1024^2 107 us,
+//   151 as below; 96 cloths 81 and 81);
+// - smaller colliding cloths: 512 threads and tiles of 32-vertex patches from all over the cloth
+//   (draped 256^2 19.3 us; 39.1 as plain patches of 256 threads, whose heaviest tile holds
+//   5,800 of the 344,000 records; without contacts 12.0 against 10.8).
 TileShape default_shape(int n, bool collides) {
-  if (!collides || n >= 262144) return {128, 0, 256};
-  return {n < 12288 ? 32 : (n < 32768 ? 64 : 128), kSubPatch, 512};
+  const int tile_v = n <= 64 ? 64 : (n < 12288 ? 32 : (n < 32768 ? 64 : 128));
+  const bool plain = !collides || n >= 262144;
+  return {tile_v, plain ? 0 : kSubPatch, plain && n >= 12288 ? 256 : 512};
 }
 
 int build_topology(const cm_params& P, const float* xyz, int n, const uint32_t* tri, int t,

@@ -66,3 +66,16 @@ def test_iteration_of_tiny_cloths():
         us.append(_solve_us(body))
         body.close()
     assert us[1] < 2 * us[0], us
+
+
+def test_iteration_of_a_small_cloth():
+    """Small cloths without collisions take tiles of their size too: 16x16 took longer than
+    with the solver's strips of 128 vertices, 24x24 in 5 tiles as long as 90x90 in 64."""
+    from licenta_amd.body import ClothBody
+    us = []
+    for n, collide in ((24, False), (24, True)):
+        print(f"{n}x{n}, collide={collide}", flush=True)
+        body = ClothBody.from_scene(_scene(n, n, 0, collide))
+        us.append(_solve_us(body))
+        body.close()
+    assert us[0] < 1.3 * us[1], us
