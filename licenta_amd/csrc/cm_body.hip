@@ -1009,9 +1009,9 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
   // two-pass traversal: leaves still walking after the budget's visits are finished
   // by whole waves; up to a quarter of the leaves can be handed over, the rest walk on
   // in the first pass. Off for caps above 96 (the second pass keeps at most 256 pairs
-  // per leaf). CLOTHMI_TRAV_BUDGET overrides the budget (0: one pass) and has small
-  // bodies, whose leaves groups of lanes walk, take these passes too; the pairs are the
-  // same with any budget.
+  // per leaf) and for small bodies, whose leaves groups of lanes walk. CLOTHMI_TRAV_BUDGET
+  // overrides the budget (0: one pass) and has small bodies take these passes too; the
+  // pairs are the same with any budget.
   if ((rc = dalloc(b, &b->lb.spill, (size_t)t * kTravSpill))) return fail(rc);
   {
     int budget = params->pair_cap <= 96 ? 200 : 0;
@@ -1019,7 +1019,7 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
       budget = std::max(0, std::atoi(e));
       b->lb.group = false;
     }
-    if (budget > 0 && t >= 2 && t < (1 << 26)) {
+    if (budget > 0 && t >= 2 && t < kQuantLeaves && !walked_by_groups(b->lb, b->cap)) {
       b->lb.rcap = t / 4 + 1024;
       if ((rc = dalloc(b, &b->lb.trec, (size_t)b->lb.rcap * kTravRec))) return fail(rc);
       b->lb.hctl = b->counters + 8;  // zeroed above
@@ -1913,7 +1913,7 @@ int cm_autotune(cm_body* b, int32_t substeps, int32_t* chosen) {
     }
     if ((rc = set_tiles(b, best))) return fail(rc);
   }
-  {
+  if (!walked_by_groups(b->lb, b->cap)) {
     const int cand[4] = {1, 2, 4, 8};
     int best = b->lb.trav_chunk;
     float best_ms = 1e30f;

@@ -185,6 +185,8 @@ int launch_pack_nodes(const LbvhBufs& b, bool from_caller, hipStream_t s);
 // then compaction.
 int launch_pairs(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offsets,
                  int2* pairs, int* d_npairs, void* scan_temp, hipStream_t s);
+// whether groups of lanes walk the tree (k_traverse_group), without tile chunks or a budget
+bool walked_by_groups(const LbvhBufs& b, int cap);
 // the traversal kernel alone on the current tree (it rewrites the same pair chunk)
 int launch_traverse_only(const LbvhBufs& b, int cap, int* chunk, int* counts, int* offsets,
                          hipStream_t s);

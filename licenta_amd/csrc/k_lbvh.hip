@@ -1902,6 +1902,10 @@ static WalkTree walk_tree(const LbvhBufs& b) {
           b.ncloth ? b.croot : nullptr, b.ccap, b.tstart};
 }
 
+bool walked_by_groups(const LbvhBufs& b, int cap) {
+  return b.group && b.t <= kGroupLeaves && cap <= kGroupMaxCap;
+}
+
 // the second pass needs a budget, record buffers and quantised nodes
 static bool two_passes(const LbvhBufs& b) {
   return b.t < kQuantLeaves && b.trav_budget > 0 && b.trec && b.hctl && b.rcap > 0;
@@ -1915,7 +1919,7 @@ static int launch_traverse(const LbvhBufs& b, int cap, int* chunk, int* counts, 
   const int round = kXcds * xchunk;
   const bool two = two_passes(b);
   const WalkTree T = walk_tree(b);
-  if (b.group && T.qnodes && t <= kGroupLeaves && cap <= kGroupMaxCap) {
+  if (walked_by_groups(b, cap)) {
     const int per = 64 / kGroup, nb = (t + per - 1) / per, rnd = kXcds * 4 * kTravBlock / per;
     hipLaunchKernelGGL(k_traverse_group<kGroup>, dim3((nb + rnd - 1) / rnd * rnd), dim3(64), 0, s,
                        T, cap, chunk, counts, b.warn);
