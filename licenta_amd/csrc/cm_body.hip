@@ -53,7 +53,7 @@ struct HostTopo {
   std::vector<int4> hdr;
   std::vector<uint4> sent, bent;
   std::vector<float2> bpar;
-  int max_local = 0, lds_slots = 0;
+  int max_local = 0, lds_slots = 0, mem_tiles = 0;
   std::vector<float> k_dist, k_bend;  // stiffness per constraint (before the kp mapping)
 };
 
@@ -227,6 +227,7 @@ int upload_tiles(cm_body* b, const HostTopo& h) {
   t.nsent = (int)h.sent.size();
   t.nbent = (int)h.bent.size();
   t.n = (int)h.hdr.size() / 2;
+  t.n_mem = h.mem_tiles;
   t.threads = b->shape.threads;
   b->tl = t;
   b->nb.rank = t.rank;
@@ -350,7 +351,7 @@ void build_tiles(int n, HostTopo& h, int tile_v, int sub) {
   h.bpar.clear();
   h.scid.clear();
   h.bcid.clear();
-  h.max_local = h.lds_slots = 0;
+  h.max_local = h.lds_slots = h.mem_tiles = 0;
   for (int v = 0; v < n; ++v)
     if (h.prefix[v + 1] - h.prefix[v] > kTileSlots) return;
   std::vector<int> ts{0};
@@ -448,20 +449,32 @@ void build_tiles(int n, HostTopo& h, int tile_v, int sub) {
         }
       }
     }
-    const int nh = (int)h.halo.size() - h_base;
-    h.max_local = std::max(h.max_local, v1 - v0 + nh);
     h.lds_slots = std::max(h.lds_slots, h.sprefix[v1] - slot0);
-    h.hdr.push_back(make_int4(v0, v1 - v0, h_base, nh));
+    h.hdr.push_back(make_int4(v0, v1 - v0, h_base, (int)h.halo.size() - h_base));
     h.hdr.push_back(make_int4(s_base, (int)h.sent.size() - s_base, b_base,
                               (int)h.bent.size() - b_base));
   }
   // dynamic records pass through the same LDS, 1,024 of them or more at a time
   h.lds_slots = std::max((h.lds_slots + 3) & ~3, 1024);
-  if (h.max_local > 0xffff ||
-      tile_lds_bytes(h.max_local, h.lds_slots, true) > (size_t)(150 << 10)) {
-    if (tile_v > 1) return build_tiles(n, h, tile_v / 2, 0);
-    h.hdr.clear();
+  // tiles whose positions (two a vertex for the adjoint) don't fit beside the slots come last,
+  // where CUs hold several tiles also those that would leave room for one only (a local id is
+  // at most tile_v + 3 * kTileSlots, below 0xffff)
+  const size_t room = nt <= 256 ? 150 << 10 : 80 << 10;
+  std::vector<int4> mem;
+  size_t at = 0;
+  for (size_t k = 0; k < h.hdr.size(); k += 2) {
+    const int local = h.hdr[k].y + h.hdr[k].w;
+    if (tile_lds_bytes(local, h.lds_slots, true) > room) {
+      mem.insert(mem.end(), {h.hdr[k], h.hdr[k + 1]});
+      continue;
+    }
+    h.max_local = std::max(h.max_local, local);
+    h.hdr[at] = h.hdr[k];
+    h.hdr[at + 1] = h.hdr[k + 1];
+    at += 2;
   }
+  std::copy(mem.begin(), mem.end(), h.hdr.begin() + at);
+  h.mem_tiles = (int)mem.size() / 2;
 }
 
 // The tile shape of a body, from an iteration's time (k_solve):

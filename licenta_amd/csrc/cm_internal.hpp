@@ -271,6 +271,7 @@ constexpr int kTileSlots = 3072;
 constexpr int kSubPatch = 32;
 struct TileBufs {
   int n = 0;  // 0: no tiles (a vertex has more slots than a tile holds)
+  int n_mem = 0;  // the last of them: halo too large for the LDS
   int threads = 256;                 // of a workgroup (256 or 512)
   int max_local = 0, lds_slots = 0;  // LDS per workgroup: positions and slots
   int* order = nullptr;   // n vertices (null: solver numbering = vertex ids)

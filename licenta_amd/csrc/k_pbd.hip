@@ -621,7 +621,8 @@ __device__ __forceinline__ void tile_jobs(int nv, F f) {
 // rounding. The dynamic records follow the same way, their positions from memory; only
 // non-zero corrections are counted (adding a zero one changes nothing: a sum that
 // starts at +0 is never -0). kFirst: pin is in vertex order; else, and pout always, in
-// solver order.
+// solver order. Tiles with more vertices about them than the LDS holds (a vertex in over a
+// thousand bends that share none) are launched apart and read them from memory (kStaged off).
 // The launch is bound by the bends' FP64 chains (about 540 instructions each) and, with
 // contacts, by the tile with the most records. Evaluating from LDS-staged patches
 // instead of strips of 128 vertex ids cut the repeated evaluations from 1.75 (distance)
@@ -631,12 +632,12 @@ __device__ __forceinline__ void tile_jobs(int nv, F f) {
 // 1024^2 236 -> 113 us, 96 cloths 147 -> 89, 192x301 without contacts 15.9 -> 10.7,
 // draped 256^2 31.3 -> 20.9, draped 131x97 27.9 -> 13.7, 64^2 9.1 -> 5.8. More waves per
 // SIMD (96 registers: five) spill and are slower (1024^2: 43 against 30 ms a pass).
-template <bool kFirst, int kT>
+template <bool kFirst, int kT, bool kStaged>
 __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float4* __restrict__ pin,
                                                   float4* __restrict__ pout) {
   constexpr int kJobs = tile_job_count<kT>();
   extern __shared__ float4 lpos[];
-  const TileLds l = tile_lds<1>(lpos, a.max_local, a.lds_slots);
+  const TileLds l = tile_lds<1>(lpos, kStaged ? a.max_local : 0, a.lds_slots);
   // each XCD takes a contiguous range of tiles, so the positions that neighbouring
   // tiles share are fetched into one L2
   const int tile = xcd_block(blockIdx.x, gridDim.x);
@@ -644,7 +645,10 @@ __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float
   const int v0 = h0.x, nv = h0.y, nh = h0.w;
   const int tid = threadIdx.x;
   auto at = [&](int k) { return pin[kFirst ? a.order[k] : k]; };
-  for (int k = tid; k < nv + nh; k += kT) lpos[k] = at(k < nv ? v0 + k : a.halo[h0.z + k - nv]);
+  auto local = [&](int k) { return at(k < nv ? v0 + k : a.halo[h0.z + k - nv]); };
+  auto pos = [&](int k) { return kStaged ? lpos[k] : local(k); };
+  if (kStaged)
+    for (int k = tid; k < nv + nh; k += kT) lpos[k] = local(k);
   const int s0 = a.vprefix[v0];
   int r0 = 0, r1 = 0;
   if (a.dprefix) {
@@ -661,10 +665,10 @@ __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float
     const float2 par = a.bpar[h1.z + q];
     f3 cr[4];
     if (a.bend_fp64)
-      bend_all<double>(lpos[t.x & 0xffffu], lpos[t.x >> 16], lpos[t.y & 0xffffu], lpos[t.y >> 16],
+      bend_all<double>(pos(t.x & 0xffffu), pos(t.x >> 16), pos(t.y & 0xffffu), pos(t.y >> 16),
                        par, a.abs_mode, cr);
     else
-      bend_all<float>(lpos[t.x & 0xffffu], lpos[t.x >> 16], lpos[t.y & 0xffffu], lpos[t.y >> 16],
+      bend_all<float>(pos(t.x & 0xffffu), pos(t.x >> 16), pos(t.y & 0xffffu), pos(t.y >> 16),
                       par, a.abs_mode, cr);
     tile_put(l.c(0), l.c(1), l.c(2), t.z & 0xffffu, cr[0]);
     tile_put(l.c(0), l.c(1), l.c(2), t.z >> 16, cr[1]);
@@ -676,7 +680,7 @@ __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float
   for (int q = tid ^ (kT - 64); q < h1.y; q += kT) {
     const uint4 t = a.sent[h1.x + q];
     f3 c0, c1;
-    stretch_both(lpos[t.x & 0xffffu], lpos[t.x >> 16],
+    stretch_both(pos(t.x & 0xffffu), pos(t.x >> 16),
                  make_float2(__uint_as_float(t.z), __uint_as_float(t.w)), c0, c1);
     tile_put(l.c(0), l.c(1), l.c(2), t.y & 0xffffu, c0);
     tile_put(l.c(0), l.c(1), l.c(2), t.y >> 16, c1);
@@ -719,7 +723,7 @@ __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float
   __syncthreads();
   if (tid >= nv) return;
   const int i = v0 + tid;
-  const float4 pi = lpos[tid];
+  const float4 pi = pos(tid);
   f3 total = mk3(0, 0, 0);
   int cnt = 0;
   if (a.ground_on | a.F)
@@ -1197,6 +1201,7 @@ struct AdjArgs {
 // constraint). Bound by the FP64 bend VJP at two waves per SIMD (246 registers; three
 // with spills: 24 us at 128^2). 128^2: 13.4 us a launch (21.1 in strips of 128 ids, plus
 // 4.2 for a scaling launch of its own), 24 cloths of 64^2: 26.6 us (38 + 5).
+template <bool kStaged>
 __global__ void __launch_bounds__(kBlock) k_adj_iter(AdjArgs a, const float4* __restrict__ ps,
                                                      const int* __restrict__ cnt,
                                                      const float4* __restrict__ lp,
@@ -1204,7 +1209,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_iter(AdjArgs a, const float4* __
   constexpr int kJobs = tile_job_count<kBlock>();
   extern __shared__ float4 lpos[];
   float4* lav = lpos + a.max_local;
-  const TileLds l = tile_lds<2>(lpos, a.max_local, a.lds_slots);
+  const TileLds l = tile_lds<2>(lpos, kStaged ? a.max_local : 0, a.lds_slots);
   const int tile = xcd_block(blockIdx.x, gridDim.x);  // contiguous tiles per XCD
   const int4 h0 = a.tl.hdr[2 * tile], h1 = a.tl.hdr[2 * tile + 1];
   const int v0 = h0.x, nv = h0.y, nh = h0.w;
@@ -1213,11 +1218,15 @@ __global__ void __launch_bounds__(kBlock) k_adj_iter(AdjArgs a, const float4* __
     const int c = cnt[k];
     return c ? f4(divs(xyz(lp[k]), (float)c), 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
   };
-  for (int k = tid; k < nv + nh; k += kBlock) {
-    const int v = k < nv ? v0 + k : a.tl.halo[h0.z + k - nv];
-    lpos[k] = ps[v];
-    lav[k] = scaled(v);
-  }
+  auto at = [&](int k) { return k < nv ? v0 + k : a.tl.halo[h0.z + k - nv]; };
+  auto pos = [&](int k) { return kStaged ? lpos[k] : ps[at(k)]; };
+  auto cot = [&](int k) { return kStaged ? lav[k] : scaled(at(k)); };
+  if (kStaged)
+    for (int k = tid; k < nv + nh; k += kBlock) {
+      const int v = at(k);
+      lpos[k] = ps[v];
+      lav[k] = scaled(v);
+    }
   const int s0 = a.tl.prefix[v0];
   for (int k = tid; k <= nv; k += kBlock) {
     l.sp[k] = a.tl.prefix[v0 + k] - s0;
@@ -1228,8 +1237,8 @@ __global__ void __launch_bounds__(kBlock) k_adj_iter(AdjArgs a, const float4* __
     const uint4 t = a.tl.bent[h1.z + q];
     const float2 par = a.tl.bpar[h1.z + q];
     const uint32_t id[4] = {t.x & 0xffffu, t.x >> 16, t.y & 0xffffu, t.y >> 16};
-    const float4 P[4] = {lpos[id[0]], lpos[id[1]], lpos[id[2]], lpos[id[3]]};
-    const float4 G[4] = {lav[id[0]], lav[id[1]], lav[id[2]], lav[id[3]]};
+    const float4 P[4] = {pos(id[0]), pos(id[1]), pos(id[2]), pos(id[3])};
+    const float4 G[4] = {cot(id[0]), cot(id[1]), cot(id[2]), cot(id[3])};
     f3 o[4];
     float gkp;
     if (a.bend_fp64)
@@ -1248,7 +1257,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_iter(AdjArgs a, const float4* __
     const uint4 t = a.tl.sent[h1.x + q];
     const uint32_t i0 = t.x & 0xffffu, i1 = t.x >> 16;
     float gkp;
-    const f3 gd = stretch_vjp(lpos[i0], lpos[i1], lav[i0], lav[i1], __uint_as_float(t.z),
+    const f3 gd = stretch_vjp(pos(i0), pos(i1), cot(i0), cot(i1), __uint_as_float(t.z),
                               __uint_as_float(t.w), gkp);
     if ((t.y & 0xffffu) != 0xffffu) {
       lds_put(l.c(0), l.c(1), l.c(2), t.y & 0xffffu, gd);
@@ -1379,14 +1388,20 @@ static void launch_iteration(const PbdBufs& b, const SolveArgs& a, bool first, c
                        src, dst);
     return;
   }
-  const size_t lds = tile_lds_bytes(b.tl.max_local, b.tl.lds_slots, false);
-  const dim3 grid(b.tl.n), wg(b.tl.threads);
-  if (b.tl.threads == 512) {
-    if (first) hipLaunchKernelGGL((k_solve<true, 512>), grid, wg, lds, s, a, src, dst);
-    else hipLaunchKernelGGL((k_solve<false, 512>), grid, wg, lds, s, a, src, dst);
-  } else {
-    if (first) hipLaunchKernelGGL((k_solve<true, 256>), grid, wg, lds, s, a, src, dst);
-    else hipLaunchKernelGGL((k_solve<false, 256>), grid, wg, lds, s, a, src, dst);
+  const bool wide = b.tl.threads == 512;
+  auto launch = [&](bool staged, int tiles, const SolveArgs& args) {
+    const size_t lds = tile_lds_bytes(staged ? b.tl.max_local : 0, b.tl.lds_slots, false);
+    auto f = staged ? (wide ? (first ? k_solve<true, 512, true> : k_solve<false, 512, true>)
+                            : (first ? k_solve<true, 256, true> : k_solve<false, 256, true>))
+                    : (wide ? (first ? k_solve<true, 512, false> : k_solve<false, 512, false>)
+                            : (first ? k_solve<true, 256, false> : k_solve<false, 256, false>));
+    hipLaunchKernelGGL(f, dim3(tiles), dim3(b.tl.threads), lds, s, args, src, dst);
+  };
+  if (b.tl.n > b.tl.n_mem) launch(true, b.tl.n - b.tl.n_mem, a);
+  if (b.tl.n_mem) {
+    SolveArgs m = a;
+    m.hdr += 2 * (b.tl.n - b.tl.n_mem);
+    launch(false, b.tl.n_mem, m);
   }
 }
 
@@ -1413,8 +1428,9 @@ int tile_lds_allow(size_t bytes) {
   constexpr int kMaxLds = 160 << 10;
   if (bytes <= (64u << 10)) return CM_OK;
   for (const void* f :
-       {(const void*)k_solve<true, 256>, (const void*)k_solve<false, 256>,
-        (const void*)k_solve<true, 512>, (const void*)k_solve<false, 512>, (const void*)k_adj_iter})
+       {(const void*)k_solve<true, 256, true>, (const void*)k_solve<false, 256, true>,
+        (const void*)k_solve<true, 512, true>, (const void*)k_solve<false, 512, true>,
+        (const void*)k_adj_iter<true>})
     CM_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
   return CM_OK;
 }
@@ -1553,11 +1569,20 @@ int launch_adj_substep(const PbdBufs& b, const PbdParams& pp, const AdjBufs& ab,
     hipLaunchKernelGGL(k_adj_counts, dim3(1024), dim3(kBlock), 0, s, b.n, pp.iters, dprefix, rec,
                        pk, ab.cnt, pp.th);
   const size_t lds = tile_lds_bytes(b.tl.max_local, b.tl.lds_slots, true);
+  const int n_lds = b.tl.n - b.tl.n_mem;
   float4* src = ab.lp;
   float4* dst = ab.la;
   for (int it = pp.iters - 1; it >= 0; --it) {
-    hipLaunchKernelGGL(k_adj_iter, dim3(b.tl.n), dim3(kBlock), lds, s, a, pk + (int64_t)it * b.n,
-                       ab.cnt + (int64_t)it * b.n, src, dst);
+    if (n_lds)
+      hipLaunchKernelGGL(k_adj_iter<true>, dim3(n_lds), dim3(kBlock), lds, s, a,
+                         pk + (int64_t)it * b.n, ab.cnt + (int64_t)it * b.n, src, dst);
+    if (b.tl.n_mem) {
+      AdjArgs m = a;
+      m.tl.hdr += 2 * n_lds;
+      hipLaunchKernelGGL(k_adj_iter<false>, dim3(b.tl.n_mem), dim3(kBlock),
+                         tile_lds_bytes(0, b.tl.lds_slots, true), s, m, pk + (int64_t)it * b.n,
+                         ab.cnt + (int64_t)it * b.n, src, dst);
+    }
     std::swap(src, dst);
   }
   hipLaunchKernelGGL(k_adj_predict, dim3(g), dim3(kBlock), 0, s, b.n, b.tl.rank, ab.lx, ab.lv, src,
