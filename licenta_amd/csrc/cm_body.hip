@@ -1095,7 +1095,7 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
       (rc = dalloc(b, &nb.vf_w, nb.vf_out_cap)) || (rc = dalloc(b, &nb.vf_tn, nb.vf_out_cap)) ||
       (rc = dalloc(b, &nb.ee_v, nb.ee_out_cap)) || (rc = dalloc(b, &nb.ee_w, nb.ee_out_cap)) ||
       (rc = dalloc(b, &nb.ee_tn, nb.ee_out_cap)) || (rc = dalloc(b, &nb.dcount, (size_t)n + 1)) ||
-      (rc = dalloc(b, &nb.dprefix, (size_t)n + 1)) || (rc = dalloc(b, &nb.dcursor, n)) ||
+      (rc = dalloc(b, &nb.dprefix, (size_t)n + 1)) ||
       (rc = dalloc(b, &nb.drec, 4 * (size_t)(nb.vf_out_cap + nb.ee_out_cap))) ||
       (rc = dalloc(b, &nb.dtmp, 4 * (size_t)(nb.vf_out_cap + nb.ee_out_cap))) ||
       (rc = dalloc(b, &nb.rec, 4 * (size_t)(nb.vf_out_cap + nb.ee_out_cap))) ||

@@ -231,7 +231,7 @@ struct NarrowBufs {
   // per-vertex dynamic record CSR, in solver order (rank: solver position of a vertex,
   // null: its id); the payloads' vertex ids are solver positions too
   const int* rank = nullptr;
-  int *dcount = nullptr, *dprefix = nullptr, *dcursor = nullptr;  // n + 1, n + 1, n
+  int *dcount = nullptr, *dprefix = nullptr;  // n + 1 each
   uint32_t* drec = nullptr;  // 4 * (vf_out_cap + ee_out_cap)
   uint32_t* dtmp = nullptr;  // same size: staging for very long record lists
   // same size: record payloads in drec order; between the solver's last read and

@@ -1076,11 +1076,6 @@ __global__ void __launch_bounds__(kBlock) k_rec_place(int n, const uint32_t* __r
   }
 }
 
-__global__ void k_copy_i32(const int* __restrict__ s, int* __restrict__ d, int n) {
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) d[i] = s[i];
-}
-
-
 }  // namespace
 
 static int grid_for(int64_t cap) {
