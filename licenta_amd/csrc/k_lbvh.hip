@@ -1387,16 +1387,13 @@ __global__ void __launch_bounds__(64) k_traverse_group(WalkTree T, int cap,
     cap = T.ccap[c];
     act = root >= 0;  // a one-triangle cloth has no pairs
   }
-  if (act && T.irr[c] >= kIrregular) {
-    act = false;
-    again = true;
-  }
   f3 mn = mk3(0, 0, 0), mx = mk3(0, 0, 0);
   uint3 q = make_uint3(0, 0, 0);
-  const int limit = visit_limit(t);
   int np = 0, nh = 0, nv = 0;  // pending, hits, hits tested (the first nv)
-  int seen = 0;                // nodes visited
+  const int limit = visit_limit(t);
+  int seen = 0;
   if (act) {
+    const int irr = T.irr[c];
     mn = xyz(T.amin[nin + leaf]);
     mx = xyz(T.amax[nin + leaf]);
     q = q_box(quant_frame(T.amin[root], T.amax[root]), mx, mn);
@@ -1405,7 +1402,7 @@ __global__ void __launch_bounds__(64) k_traverse_group(WalkTree T, int cap,
       pk[0] = 0;
     }
     np = 1;
-    again = !box_ordered(mn, mx);
+    again = irr >= kIrregular || !box_ordered(mn, mx);
     act = !again;
   }
   // tests hits nv to nh exactly and closes the gaps
@@ -1642,18 +1639,20 @@ __global__ void __launch_bounds__(kBlock) k_pack_nodes(WalkTree T, uint4* __rest
       __hip_atomic_load(irr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= kIrregular)
     return;
   const int l = T.lefts[i], r = T.rights[i], a = T.rmll[i], b = T.rmlr[i];
-  const f3 lmn = xyz(T.amin[l]), lmx = xyz(T.amax[l]), rmn = xyz(T.amin[r]), rmx = xyz(T.amax[r]);
   const f3 mn = xyz(T.amin[i]), mx = xyz(T.amax[i]);
+  // in a batch, a node that is walked and the leaf of its number belong to one cloth
+  const int c = T.croot ? T.slot_cloth[i] : 0, root = T.croot ? max(T.croot[c], 0) : 0;
+  const Quant q = quant_frame(T.amin[root], T.amax[root]);
+  // before the children's boxes, whose loads wait for their numbers
+  const bool coarse = i % kDraw == 0 && coarse_frame(T, i, c, q);
+  const f3 lmn = xyz(T.amin[l]), lmx = xyz(T.amax[l]), rmn = xyz(T.amin[r]), rmx = xyz(T.amax[r]);
   const bool ll = l >= nin, rl = r >= nin;
   const int sp = ll ? l - nin : l;
   bool ok = holds(mn, mx, lmn, lmx) && holds(mn, mx, rmn, rmx);
   if (kCaller && ok)
     ok = sp + 1 == (rl ? r - nin : r) && (ll ? a == l : a >= max(T.rmll[l], T.rmlr[l])) &&
          (rl ? b == r && a <= b : b >= max(T.rmll[r], T.rmlr[r]));
-  // in a batch, a node that is walked and the leaf of its number belong to one cloth
-  const int c = T.croot ? T.slot_cloth[i] : 0, root = T.croot ? max(T.croot[c], 0) : 0;
-  const Quant q = quant_frame(T.amin[root], T.amax[root]);
-  int found = !ok ? kIrregular : (i % kDraw == 0 && coarse_frame(T, i, c, q)) ? 1 : 0;
+  int found = !ok ? kIrregular : coarse ? 1 : 0;
   if (!T.croot) {  // one cloth: one lane adds for the wave
     const uint64_t any = __ballot(found), bad = __ballot(found == kIrregular);
     found = (threadIdx.x & 63) == __ffsll((long long)any) - 1 ? (bad ? kIrregular : __popcll(any)) : 0;
