@@ -378,7 +378,8 @@ void build_tiles(int n, HostTopo& h, int tile_v, int sub) {
     const int nsub = (len + unit - 1) / unit, per = tile_v / unit, nt = (nsub + per - 1) / per;
     for (int t = 0; t < nt; ++t) {
       for (int u = t; u < nsub; u += nt)
-        for (int k = u * unit; k < std::min(len, (u + 1) * unit); ++k) tile.push_back(h.patch[b + k]);
+        for (int k = u * unit; k < std::min(len, (u + 1) * unit); ++k)
+          tile.push_back(h.patch[b + k]);
       if ((int)tile.size() == tile_v) {
         emit(tile);
         continue;

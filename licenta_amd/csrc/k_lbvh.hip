@@ -771,9 +771,9 @@ __device__ __forceinline__ int walk_exact(const WalkTree& T, int leaf, int root,
 //   then three words per child: its box in 16 bits a bound, (min x, min y),
 //       (min z, 65535 - max x), (65535 - max y, 65535 - max z)
 // Bounds are quantised by one monotone function over the root's box (in a batch the box of
-// the cloth's root: cloths may lie far apart), the leaf's own box by the same one as (max x, max y), (max z, 65535 - min x), ..., so boxes that overlap
-// have no word larger than the leaf's: three saturating 16-bit subtractions, an or and a
-// compare. The test can pass boxes that do not overlap, so the leaves it finds are
+// the cloth's root: cloths may lie far apart), the leaf's own box by the same one as
+// (max x, max y), (max z, 65535 - min x), ..., so boxes that overlap have no word larger
+// than the leaf's: three saturating 16-bit subtractions, an or and a compare. The test can pass boxes that do not overlap, so the leaves it finds are
 // candidates: their exact boxes are tested after the walk (by 8 at a time, off its chain
 // of loads), in order, and those that fail are dropped. The pairs and their order are
 // walk_exact's: where a node's box holds its children's (irr small), a leaf whose exact
@@ -781,10 +781,10 @@ __device__ __forceinline__ int walk_exact(const WalkTree& T, int leaf, int root,
 // limit is given up (kRedo) and done exactly, and so is the whole tree where the root's box
 // is so large that leaves apart from each other fall together (coarse_frame).
 // k_traverse with what finishes its long walks, exact records of 64 bytes and pairs
-// stored as they are found -> now: flat 256^2 614 -> 353 us, draped 319 -> 331, draped
-// 131x97 217 -> 179, 64^2 134 -> 100, 2 M leaves 1,070 -> 815, crumpled 1024^2 1,825 ->
-// 1,860 (there 65 vector and 30 scalar instructions a visit at 43% of the lanes bound
-// it; refilling the lanes that finish early from a wave's queue of leaves was slower,
+// stored as they are found -> now (walk_shape's rows): falling 256^2 614 -> 295 us, flat
+// 54 -> 46, draped 319 -> 305, draped 131x97 217 -> 157, 64^2 134 -> 94, 2 M leaves
+// 1,070 -> 850, crumpled 1024^2 1,740 -> 1,597 (there 65 vector and 30 scalar instructions
+// a visit at 43% of the lanes bound it; refilling the lanes that finish early from a wave's queue of leaves was slower,
 // 2,320, as is stepping two levels at a time: 650 instructions a step, or loading both
 // children's records ahead).
 constexpr uint32_t kSplitMask = (1u << 26) - 1, kLeftLeaf = 1u << 26, kRightLeaf = 1u << 27,
@@ -934,7 +934,7 @@ __device__ __forceinline__ WalkEnd walk_quant(const WalkTree& T, int leaf, f3 mn
 
 // The first pass's budget is given in exact visits; quantised ones are cheaper, and 1.7
 // for one give the shortest two passes (draped 256^2: 342 us at 200 visits, 331 at 340,
-// 362 at 400; flat 256^2: 500, 353, 320).
+// 362 at 400; falling 256^2: 500, 353, 320; all with 16 rows of stack and 66 of candidates).
 constexpr int quant_budget(int budget) { return budget + budget * 7 / 10; }
 
 // A leaf whose walk outlasts the first pass's visit budget leaves its state in a
@@ -1031,8 +1031,8 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(WalkTree T, int cap, in
         put_record<kLds>(rec + (int64_t)slot * kRec, leaf, cap, st, sstk, threadIdx.x, sp);
         handed = true;
       } else {
-        end = walk_quant<kLds, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out, INT_MAX, st, w, sstk,
-                                     cand, ncand, threadIdx.x, sp);
+        end = walk_quant<kLds, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out, INT_MAX, st, w,
+                                                    sstk, cand, ncand, threadIdx.x, sp);
       }
     }
   }
@@ -1312,8 +1312,9 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse_lanes(
     WalkState st{R[3], top, top > 0 ? R[5 + top] : 0, R[1], R[5]};
     uint32_t wl = 0;
     int ncol;
-    if (walk_quant<kLds, kVerify, kTravBlock>(T, leaf, mn, mx, q_box(quant_frame(T.amin[root], T.amax[root]), mx, mn),
-                               cap, out, INT_MAX, st, wl, sstk, cand, ncand, threadIdx.x, sp) == kRedo) {
+    const uint3 q = q_box(quant_frame(T.amin[root], T.amax[root]), mx, mn);
+    if (walk_quant<kLds, kVerify, kTravBlock>(T, leaf, mn, mx, q, cap, out, INT_MAX, st, wl, sstk,
+                                              cand, ncand, threadIdx.x, sp) == kRedo) {
       wl = 0;
       ncol = walk_exact<kTravBlock, kLds>(T, leaf, root, mn, mx, cap, out, wl, sstk,
                                                threadIdx.x, sp);
@@ -1340,13 +1341,15 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse_lanes(
 // of shared nodes: each path to a node is a visit), and any leaf of an irregular tree, is
 // left to k_traverse_redo. Bound by the rounds' latency (about 1,550 cycles, a third of
 // them the records' loads; 16 to 18 rounds at 64^2), on draped cloths by the instructions.
-// k_traverse -> k_traverse_group: 60^2 72 -> 17 us, 64^2 94 -> 25, 96x83 119 -> 42, flat
-// 128^2 112 -> 63, draped 131x97 164 (and 16 for k_traverse_resume) -> 134.
-constexpr int kGroup = 16;  // 8: 22, 34, 41, 64 and 143 us below
+// k_traverse, with what finishes its long walks -> k_traverse_group: 60^2 72 -> 17 us, 64^2
+// 94 -> 25, 96x83 119 -> 43, falling 128^2 174 -> 68, fit 128^2 64 -> 58, draped 131x97
+// 157 -> 128. Where few boxes overlap the lanes of a group idle and it is the slower one:
+// flat 128^2 33 -> 54, a crumpled ball of 128^2 139 -> 173, a batch of four 67 -> 44.
+constexpr int kGroup = 16;  // 8: 22, 34, 41 us for 60^2, 64^2 and 96x83, 143 draped 131x97
 constexpr int kGroupPend = 128, kGroupHits = 112;
 constexpr int kGroupMaxCap = kGroupHits - 1 - 2 * kGroup;
-// Up to this many leaves. A flat cloth gains beyond it (256^2 354 -> 256 us), a draped one,
-// whose leaves meet several times the cap, loses (329 -> 700).
+// Up to this many leaves. Beyond it a falling cloth gains little (256^2 295 -> 271 us), and a
+// draped one, whose leaves meet several times the cap, loses (305 -> 655).
 constexpr int kGroupLeaves = 1 << 15;
 
 template <int kG>
@@ -1623,11 +1626,12 @@ __device__ __forceinline__ bool coarse_frame(const WalkTree& T, int i, int c, Qu
 }
 
 // The quantised node records, and whether they can be walked: every node's box has to
-// hold its children's, and the frame be fine enough. kCaller (unit-level pair query, the caller's own tree): also its
-// children have to lie side by side as the build lays them, its rightmost leaves must not
-// shrink upwards, and no leaf below its left child may lie beyond a right child that is a
-// leaf itself: the record's one rightmost leaf would let that right leaf pass for leaves at
-// and past it (the build's right leaf is the last of its parent's range).
+// hold its children's, and the frame be fine enough. kCaller (unit-level pair query, the
+// caller's own tree): also its children have to lie side by side as the build lays them,
+// its rightmost leaves must not shrink upwards, and no leaf below its left child may lie
+// beyond a right child that is a leaf itself: the record's one rightmost leaf would let that
+// right leaf pass for leaves at and past it (the build's right leaf is the last of its
+// parent's range).
 template <bool kCaller>
 __global__ void __launch_bounds__(kBlock) k_pack_nodes(WalkTree T, uint4* __restrict__ qnodes,
                                                        int* __restrict__ irr) {
@@ -1655,7 +1659,8 @@ __global__ void __launch_bounds__(kBlock) k_pack_nodes(WalkTree T, uint4* __rest
   int found = !ok ? kIrregular : coarse ? 1 : 0;
   if (!T.croot) {  // one cloth: one lane adds for the wave
     const uint64_t any = __ballot(found), bad = __ballot(found == kIrregular);
-    found = (threadIdx.x & 63) == __ffsll((long long)any) - 1 ? (bad ? kIrregular : __popcll(any)) : 0;
+    const bool adds = (threadIdx.x & 63) == __ffsll((long long)any) - 1;
+    found = adds ? (bad ? kIrregular : __popcll(any)) : 0;
   }
   if (found && __hip_atomic_load(&irr[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kIrregular)
     atomicAdd(&irr[c], found);
@@ -1671,7 +1676,7 @@ __global__ void __launch_bounds__(kBlock) k_pack_nodes(WalkTree T, uint4* __rest
 // 64-byte records of an irregular tree for the exact walk: children, rightmost leaves, both
 // boxes. A caller's nodes may be numbered in any order, and four words and four boxes from as
 // many places a visit then cost several times the record's one (500 k renumbered leaves 2,296
-// us, with the records 5XX; 2 M 10,735 and 1,9XX). Up to kGroupLeaves leaves the caches hold
+// us, with the records 535; 2 M 10,735 and 1,883). Up to kGroupLeaves leaves the caches hold
 // the tree (30,000: 132 us, 137 by records), and a body's nodes lie as the build numbers them.
 __global__ void __launch_bounds__(kBlock) k_pack_exact(WalkTree T, float4* __restrict__ nodes) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
@@ -1896,9 +1901,14 @@ static WalkShape walk_shape(int nt) {
 }
 
 static WalkTree walk_tree(const LbvhBufs& b) {
-  return {b.t,    b.t < kQuantLeaves ? b.qnodes : nullptr, b.nodes, b.irr, b.lefts, b.rights, b.rmll,
-          b.rmlr, b.amin, b.amax, b.ncloth ? b.slot_cloth : nullptr,
-          b.ncloth ? b.croot : nullptr, b.ccap, b.tstart};
+  return {b.t,      b.t < kQuantLeaves ? b.qnodes : nullptr,
+          b.nodes,  b.irr,
+          b.lefts,  b.rights,
+          b.rmll,   b.rmlr,
+          b.amin,   b.amax,
+          b.ncloth ? b.slot_cloth : nullptr,
+          b.ncloth ? b.croot : nullptr,
+          b.ccap,   b.tstart};
 }
 
 bool walked_by_groups(const LbvhBufs& b, int cap) {

@@ -629,8 +629,8 @@ __device__ __forceinline__ void tile_jobs(int nv, F f) {
 // and 2.34 (bend) per constraint to 1.13 and 1.24 and the entries from 32 to 16 and 24
 // bytes; one wave per component of the sums took the records' chains (up to 182 on the
 // draped 256^2 cloth, each with a branch) off one wave. Per launch, before -> now:
-// 1024^2 236 -> 113 us, 96 cloths 147 -> 89, 192x301 without contacts 15.9 -> 10.7,
-// draped 256^2 31.3 -> 20.9, draped 131x97 27.9 -> 13.7, 64^2 9.1 -> 5.8. More waves per
+// 1024^2 236 -> 107 us, 96 cloths 147 -> 81, 192x301 without contacts 15.9 -> 10.7,
+// draped 256^2 31.3 -> 19.3, draped 131x97 27.9 -> 11.1, 64^2 9.1 -> 5.1. More waves per
 // SIMD (96 registers: five) spill and are slower (1024^2: 43 against 30 ms a pass).
 template <bool kFirst, int kT, bool kStaged>
 __global__ void __launch_bounds__(kT, kT / 128) k_solve(SolveArgs a, const float4* __restrict__ pin,

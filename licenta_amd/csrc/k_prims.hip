@@ -529,8 +529,8 @@ __device__ __forceinline__ unsigned long long unpack31(unsigned long long st) {
 }
 
 __global__ void __launch_bounds__(kBlock) k_scan_tiles(
-    const int* __restrict__ d_items, TileRule rule, int64_t n_max, const int* sums, int* pre, int packed,
-    int64_t cap0, int64_t cap1, int* __restrict__ d_tot0, int* __restrict__ d_tot1,
+    const int* __restrict__ d_items, TileRule rule, int64_t n_max, const int* sums, int* pre,
+    int packed, int64_t cap0, int64_t cap1, int* __restrict__ d_tot0, int* __restrict__ d_tot1,
     int* __restrict__ ctr, unsigned long long* __restrict__ state) {
   __shared__ unsigned long long lds[kBlock / 64 + 1];
   __shared__ unsigned long long s_prefix;
@@ -695,8 +695,8 @@ int scan_exclusive(const int* in, int* out, int n_max, const int* d_n, int* d_to
 }
 
 static int scan_tiles_grid(const int* d_items, TileRule rule, int64_t n_max, int64_t ntile,
-                    const int* sums, int* pre, int packed, int64_t cap0, int64_t cap1, int* d_tot0, int* d_tot1,
-                    void* temp, hipStream_t s) {
+                    const int* sums, int* pre, int packed, int64_t cap0, int64_t cap1,
+                    int* d_tot0, int* d_tot1, void* temp, hipStream_t s) {
   int* ctr = (int*)temp;
   unsigned long long* state = (unsigned long long*)((char*)temp + 256);
   const int grid = std::min(lookback_tiles(ntile), kScanMaxGrid);
