@@ -1042,7 +1042,12 @@ int create_impl(const cm_params* params, const float* xyz, int32_t n, const uint
   }
   CM_HIP(hipMemset(b->sort_temp, 0, radix_sort_temp_bytes(t)));
   carve_build(t, b->lb_temp, &b->lb);
-  if (batch && (rc = dalloc(b, &b->lb.irr, (size_t)b->lb.ncloth))) return fail(rc);
+  if (batch) {
+    // no roots until the first build: the tree can be timed before a step
+    if ((rc = dalloc(b, &b->lb.irr, (size_t)b->lb.ncloth))) return fail(rc);
+    CM_HIP(hipMemset(b->lb.irr, 0, sizeof(int) * b->lb.ncloth));
+    CM_HIP(hipMemset(b->lb.croot, 0xff, sizeof(int) * b->lb.ncloth));
+  }
   CM_HIP(hipMemset(b->lb_temp, 0, lbvh_build_temp_bytes(t)));
   CM_HIP(hipMemset(b->lb.parents, 0, sizeof(int) * m));
   CM_HIP(hipMemset(b->lb.amin, 0, sizeof(float4) * m));
