@@ -773,20 +773,21 @@ __device__ __forceinline__ int walk_exact(const WalkTree& T, int leaf, int root,
 // Bounds are quantised by one monotone function over the root's box (in a batch the box of
 // the cloth's root: cloths may lie far apart), the leaf's own box by the same one as
 // (max x, max y), (max z, 65535 - min x), ..., so boxes that overlap have no word larger
-// than the leaf's: three saturating 16-bit subtractions, an or and a compare. The test can pass boxes that do not overlap, so the leaves it finds are
-// candidates: their exact boxes are tested after the walk (by 8 at a time, off its chain
-// of loads), in order, and those that fail are dropped. The pairs and their order are
-// walk_exact's: where a node's box holds its children's (irr small), a leaf whose exact
-// box passes has ancestors that pass. A walk that reaches the stack limit or the visit
-// limit is given up (kRedo) and done exactly, and so is the whole tree where the root's box
-// is so large that leaves apart from each other fall together (coarse_frame).
+// than the leaf's: three saturating 16-bit subtractions, an or and a compare. The test can
+// pass boxes that do not overlap, so the leaves it finds are candidates: their exact boxes
+// are tested after the walk (by 8 at a time, off its chain of loads), in order, and those
+// that fail are dropped. The pairs and their order are walk_exact's: where a node's box
+// holds its children's (irr small), a leaf whose exact box passes has ancestors that pass. A
+// walk that reaches the stack limit or the visit limit is given up (kRedo) and done exactly,
+// and so is the whole tree where the root's box is so large that leaves apart from each other
+// fall together (coarse_frame).
 // k_traverse with what finishes its long walks, exact records of 64 bytes and pairs
 // stored as they are found -> now (walk_shape's rows): falling 256^2 614 -> 295 us, flat
 // 54 -> 46, draped 319 -> 305, draped 131x97 217 -> 157, 64^2 134 -> 94, 2 M leaves
 // 1,070 -> 850, crumpled 1024^2 1,740 -> 1,597 (there 65 vector and 30 scalar instructions
-// a visit at 43% of the lanes bound it; refilling the lanes that finish early from a wave's queue of leaves was slower,
-// 2,320, as is stepping two levels at a time: 650 instructions a step, or loading both
-// children's records ahead).
+// a visit at 43% of the lanes bound it; refilling the lanes that finish early from a wave's
+// queue of leaves was slower, 2,320, as is stepping two levels at a time: 650 instructions a
+// step, or loading both children's records ahead).
 constexpr uint32_t kSplitMask = (1u << 26) - 1, kLeftLeaf = 1u << 26, kRightLeaf = 1u << 27,
                    kOtherRight = 1u << 28;
 struct Quant {
@@ -1342,9 +1343,9 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse_lanes(
 // left to k_traverse_redo. Bound by the rounds' latency (about 1,550 cycles, a third of
 // them the records' loads; 16 to 18 rounds at 64^2), on draped cloths by the instructions.
 // k_traverse, with what finishes its long walks -> k_traverse_group: 60^2 72 -> 17 us, 64^2
-// 94 -> 25, 96x83 119 -> 43, falling 128^2 174 -> 68, fit 128^2 64 -> 58, draped 131x97
-// 157 -> 128. Where few boxes overlap the lanes of a group idle and it is the slower one:
-// flat 128^2 33 -> 54, a crumpled ball of 128^2 139 -> 173, a batch of four 67 -> 44.
+// 94 -> 25, 96x83 119 -> 43, four of 64^2 67 -> 44, falling 128^2 174 -> 68, fit 128^2
+// 64 -> 58, draped 131x97 157 -> 128. Where few boxes overlap the lanes of a group idle and
+// it is the slower one: flat 128^2 33 -> 54, a crumpled ball of 128^2 139 -> 173.
 constexpr int kGroup = 16;  // 8: 22, 34, 41 us for 60^2, 64^2 and 96x83, 143 draped 131x97
 constexpr int kGroupPend = 128, kGroupHits = 112;
 constexpr int kGroupMaxCap = kGroupHits - 1 - 2 * kGroup;
